@@ -41,25 +41,25 @@ def listed():
         # a toy or test model, one token: launches and the call itself are all there is
         case("small layer", "mlp", 512, 1024, 1, "fp16"),
         # single-stream decoding of a 7B model, the headline layer
-        case("7B layer, 1 row", "mlp", 4096, 11008, 1, "fp16"),
+        case("7B layer - 1 row", "mlp", 4096, 11008, 1, "fp16"),
         # the same in the layout and the call that need no prepared weights, in a checkpoint's fp32
-        case("7B layer, 1 row, fp32, HF layout", "inner", 4096, 11008, 1, "fp32"),
+        case("7B layer - 1 row - fp32 - HF layout", "inner", 4096, 11008, 1, "fp32"),
         # the reference's own decode path (gate by the module, sparse up / down) with a wider, heavy-tailed layer
-        case("wide 7B layer, 1 row, module", "module2", 4096, 14336, 1, "bf16", 0.7, heavy=True),
+        case("wide 7B layer - 1 row - module", "module2", 4096, 14336, 1, "bf16", 0.7, heavy=True),
         # the reference's index-list baseline, which its users compare with
-        case("7B layer, 1 row, index list", "list", 4096, 11008, 1, "fp16"),
+        case("7B layer - 1 row - index list", "list", 4096, 11008, 1, "fp16"),
         # a handful of streams or beams: the union of the masks is nearly dense
-        case("7B layer, 4 rows", "mlp", 4096, 11008, 4, "fp16"),
+        case("7B layer - 4 rows", "mlp", 4096, 11008, 4, "fp16"),
         # a small server's batch over weights as they come from a checkpoint
-        case("wide 7B layer, 8 rows, HF layout", "inner", 4096, 14336, 8, "bf16", 0.7, heavy=True),
+        case("wide 7B layer - 8 rows - HF layout", "inner", 4096, 14336, 8, "bf16", 0.7, heavy=True),
         # the largest batch the path takes
-        case("wide 7B layer, 16 rows", "mlp", 4096, 14336, 16, "bf16"),
+        case("wide 7B layer - 16 rows", "mlp", 4096, 14336, 16, "bf16"),
         # sizes no kernel was shaped for: a row that is no whole number of blocks, an odd number of neurons, odd batch
-        case("ragged layer, 3 rows", "mlp", 3080, 8191, 3, "bf16", 0.6),
+        case("ragged layer - 3 rows", "mlp", 3080, 8191, 3, "bf16", 0.6),
         # a 70B layer, a server's batch: the largest matrices
-        case("70B layer, 8 rows", "mlp", 8192, 28672, 8, "fp16", 0.7),
+        case("70B layer - 8 rows", "mlp", 8192, 28672, 8, "fp16", 0.7),
         # the prompt of a 7B model goes through the same module before decoding starts
-        case("7B layer, prompt", "prefill", 4096, 11008, 512, "fp16"),
+        case("7B layer - prompt", "prefill", 4096, 11008, 512, "fp16"),
         # one token of a 7B-architecture model, four of its layers with attention, norms and the output head around them
         case("7B model step", "decode", 4096, 11008, 1, "fp16", layers=4, heads=32, vocab=32000, context=256),
     ]
