@@ -63,28 +63,71 @@ struct MmaLaunch {
 };
 template <class DT>
 struct MmaLaunch16 {
+  typedef void (*Kernel)(RowsArgs);
+  enum Which { kGateOnly, kGateAndUp, kUpOnly };
+  template <int STEPS, int CH, int NG>
+  static Kernel kernel(Which w) {
+    return w == kUpOnly ? rows_mma_up_kernel<DT, STEPS, CH, NG> : w == kGateAndUp ? rows_mma_kernel<DT, STEPS, CH, true, NG> : rows_mma_kernel<DT, STEPS, CH, false, NG>;
+  }
+  // One instance per number of steps, so that no load or MFMA sits behind a branch on the row length.
+  template <int NG>
+  static Kernel kernel_for(Which w, MmaSplit sp) {
+    if (sp.chunks == 2) {
+      if constexpr (NG == 1) {  // two groups of x operands of such rows do not fit in LDS
+        switch (sp.steps) {
+          case 5: return kernel<5, 2, NG>(w);
+          case 6: return kernel<6, 2, NG>(w);
+          case 7: return kernel<7, 2, NG>(w);
+          case 8: return kernel<8, 2, NG>(w);
+          case 9: return kernel<9, 2, NG>(w);
+        }
+      }
+      return nullptr;
+    }
+    switch (sp.steps) {
+      case 1: return kernel<1, 1, NG>(w);
+      case 2: return kernel<2, 1, NG>(w);
+      case 3: return kernel<3, 1, NG>(w);
+      case 4: return kernel<4, 1, NG>(w);
+      case 5: return kernel<5, 1, NG>(w);
+      case 6: return kernel<6, 1, NG>(w);
+      case 7: return kernel<7, 1, NG>(w);
+      case 8: return kernel<8, 1, NG>(w);
+      case 9: return kernel<9, 1, NG>(w);
+    }
+    return nullptr;
+  }
   static bool supported(const RowsArgs& a, int ng = 1) {
-    const int steps = rows_mma_steps(a.K);
+    const MmaSplit sp = rows_mma_split(a);
     if (a.mask_out && !a.ubytes_out) return false;  // this kernel writes the union of the flags as bytes only
-    return (steps == 4 || steps == 8) && rows_mma_lds_bytes(a.K, ng) <= 160 * 1024;
+    return sp.steps > 0 && (ng == 1 || sp.chunks == 1) && rows_mma_lds_bytes(a, ng) <= kMmaMaxLds;
   }
-  // gate + up (a.w2 set) or the gate pass alone for 9..16 batch rows in one pass over the weights
-  static hipError_t run16(const RowsArgs& a, hipStream_t stream) {
-    const int cus = current_device_cus();
-    const bool s8 = rows_mma_steps(a.K) == 8;
-    auto kern = a.w2 ? (s8 ? rows_mma_kernel<DT, 8, true, 2> : rows_mma_kernel<DT, 4, true, 2>)
-                     : (s8 ? rows_mma_kernel<DT, 8, false, 2> : rows_mma_kernel<DT, 4, false, 2>);
-    const size_t lds = rows_mma_lds_bytes(a.K, 2);
+  static constexpr size_t kMmaMaxLds = 160 * 1024 - 256;  // the kernels' static LDS takes the rest
+  static hipError_t launch(Which w, const RowsArgs& a_in, int ng, size_t lds, hipStream_t stream) {
+    RowsArgs a = a_in;
+    const int grid = rows_mma_layout(a, current_device_cus());
+    const MmaSplit sp = rows_mma_split(a);
+    Kernel kern = ng == 2 ? kernel_for<2>(w, sp) : kernel_for<1>(w, sp);
+    if (!kern) return hipErrorInvalidValue;
+    a.mma_front = sp.front;
+    a.mma_slots = sp.slots;
     if (hipError_t e = ensure_dynamic_lds((const void*)kern, lds); e != hipSuccess) return e;
-    const int ntiles = (a.N + kMmaTileRows - 1) / kMmaTileRows;
-    return launch_kernel(kern, dim3(ntiles < cus ? ntiles : cus), dim3(kMmaThreads), lds, stream, a);
+    return launch_kernel(kern, dim3(grid), dim3(kMmaThreads), lds, stream, a);
   }
-  // the up pass alone, gate activations given (kUp)
+  // one persistent workgroup per CU, or per tile where there are fewer tiles
   static int up_grid(const RowsArgs& a) {
     const int cus = current_device_cus();
     const int ntiles = (a.N + kMmaTileRows - 1) / kMmaTileRows;
     return ntiles < cus ? ntiles : cus;
   }
+  static hipError_t run(const RowsArgs& a, bool up, hipStream_t stream) {
+    return launch(up ? kGateAndUp : kGateOnly, a, 1, rows_mma_lds_bytes(a), stream);
+  }
+  // gate + up (a.w2 set) or the gate pass alone for 9..16 batch rows in one pass over the weights
+  static hipError_t run16(const RowsArgs& a, hipStream_t stream) {
+    return launch(a.w2 ? kGateAndUp : kGateOnly, a, 2, rows_mma_lds_bytes(a, 2), stream);
+  }
+  // the up pass alone, gate activations given (kUp)
   static int up_rows_pad(const RowsArgs& a) {
     const int grid = up_grid(a);
     return ((a.N + grid - 1) / grid + kMmaTileRows - 1) / kMmaTileRows * kMmaTileRows;
@@ -92,16 +135,11 @@ struct MmaLaunch16 {
   static bool supported_up(const RowsArgs& a) {
     const int ng = a.nb > 8 ? 2 : 1;
     return supported(a, ng) && a.a_in && (a.z32_out || a.zt_out) && !a.norm_w && a.nb <= 16 &&
-           rows_mma_up_lds_bytes(a.K, up_rows_pad(a), ng) <= 160 * 1024;
+           rows_mma_up_lds_bytes(a, up_rows_pad(a), ng) <= kMmaMaxLds;
   }
   static hipError_t run_up(const RowsArgs& a, hipStream_t stream) {
     const int ng = a.nb > 8 ? 2 : 1;
-    const bool s8 = rows_mma_steps(a.K) == 8;
-    auto kern = ng == 2 ? (s8 ? rows_mma_up_kernel<DT, 8, 2> : rows_mma_up_kernel<DT, 4, 2>)
-                        : (s8 ? rows_mma_up_kernel<DT, 8, 1> : rows_mma_up_kernel<DT, 4, 1>);
-    const size_t lds = rows_mma_up_lds_bytes(a.K, up_rows_pad(a), ng);
-    if (hipError_t e = ensure_dynamic_lds((const void*)kern, lds); e != hipSuccess) return e;
-    return launch_kernel(kern, dim3(up_grid(a)), dim3(kMmaThreads), lds, stream, a);
+    return launch(kUpOnly, a, ng, rows_mma_up_lds_bytes(a, up_rows_pad(a), ng), stream);
   }
   // dense GEMV out = x . w^T (kGemv): any row length, 3..16 batch rows, up to 64 rows of w per workgroup
   static bool supported_gemv(const RowsArgs& a) {
@@ -116,22 +154,15 @@ struct MmaLaunch16 {
     return launch_kernel(kern, dim3(up_grid(a)), dim3(kMmaThreads), lds, stream, a);
   }
   static hipError_t run_gemv(const RowsArgs& a, hipStream_t stream) { return a.nb > 8 ? run_gemv_ng<2>(a, stream) : run_gemv_ng<1>(a, stream); }
-  static hipError_t run(const RowsArgs& a, bool up, hipStream_t stream) {
-    const int cus = current_device_cus();  // one workgroup per CU
-    const bool s8 = rows_mma_steps(a.K) == 8;
-    auto kern = up ? (s8 ? rows_mma_kernel<DT, 8, true> : rows_mma_kernel<DT, 4, true>)
-                   : (s8 ? rows_mma_kernel<DT, 8, false> : rows_mma_kernel<DT, 4, false>);
-    const size_t lds = rows_mma_lds_bytes(a.K);
-    if (hipError_t e = ensure_dynamic_lds((const void*)kern, lds); e != hipSuccess) return e;
-    const int ntiles = (a.N + kMmaTileRows - 1) / kMmaTileRows;
-    return launch_kernel(kern, dim3(ntiles < cus ? ntiles : cus), dim3(kMmaThreads), lds, stream, a);
-  }
 };
 template <> struct MmaLaunch<F16> : MmaLaunch16<F16> {};
 template <> struct MmaLaunch<BF16> : MmaLaunch16<BF16> {};
 
 // Whether a call goes to the matrix-core kernel.  Measured on Llama-7B shapes: at 2 batch rows the wave-per-row kernel is
-// still the faster one (28.4 vs 29.4 us).  The plain gate pass goes the same way as gate + up, so a gate call and a fused
+// still the faster one (28.4 vs 29.4 us).  From three rows on it wins at every row length (gate + up, wave-per-row against
+// matrix cores: 255 against 129 us for 28672 rows of 8192 elements at 8 batch rows; whole MLP calls: 22.0 against 15.7 us for 3000
+// rows of 1024 at 4, 162 against 75 us for 13824 rows of 5120 at 8, 57 against 21 us for 3931 rows of 1264 at 11, where the
+// other way is two passes).  The plain gate pass goes the same way as gate + up, so a gate call and a fused
 // call produce the same activations bit for bit.
 template <class DT>
 bool takes_mma(int mode, int bt, const RowsArgs& a) {

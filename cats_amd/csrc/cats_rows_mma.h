@@ -1,4 +1,4 @@
-// Gate and fused gate + up pass for batches of 3..8 rows in 16-bit types, on the matrix cores.
+// Gate and fused gate + up pass for batches of 3..16 rows in 16-bit types, on the matrix cores.
 //
 // Why not the wave-per-row kernel: with B batch rows every 16-byte weight vector costs 4 * B v_dot2 and B / 2
 // LDS reads of x per lane.  From B = 4 on, that arithmetic plus the LDS traffic takes as long as the HBM stream
@@ -13,8 +13,8 @@
 // two quadrants pair mismatched halves and are dropped.
 //
 // Work split.  One persistent workgroup per CU: x is staged once in LDS in operand order (one linear 16-byte
-// read per lane per step).  A workgroup owns ceil(N / grid) consecutive rows -- the same number of weight bytes for
-// every CU; dealing whole tiles instead leaves 96 of 256 workgroups with 6 tiles against 5 at N = 11008 and spreads their
+// read per lane per step).  A workgroup owns ceil(N / grid) rows, consecutive ones where the rows start on cache lines --
+// the same number of weight bytes for every CU; dealing whole tiles instead leaves 96 of 256 workgroups with 6 tiles against 5 at N = 11008 and spreads their
 // ends over 4-6 us instead of 1.3-2 (the kernel's duration is the same: the memory system is the limit) -- cut into
 // tiles of eight, the last one partial (its missing rows fetch nothing).  The rows of a range do not end on multiples of eight, so the union of the flags goes out as one byte
 // per row (ubytes_out) rather than as bits.  The waves of a workgroup split K.  Tiles move through a software
@@ -53,81 +53,203 @@ constexpr int kMmaThreads = kMmaWaves * kWave;
 constexpr int kMmaTileRows = 8;
 constexpr int kMmaPart = 128;    // floats per wave in a partial buffer (the two useful quadrants)
 
-// dynamic LDS: x operands, gate partials, up partials -- each once per group of eight batch rows (ng = 1 or 2)
-inline size_t rows_mma_lds_bytes(int K, int ng = 1) {
-  return (size_t)ng * ((size_t)(K / 64) * kWave * sizeof(u32x4) + 2u * kMmaWaves * kMmaPart * sizeof(float));
+// How a row of K elements is cut.  A step is 64 elements = 128 bytes, a whole cache line: where the pitch of the rows is no multiple
+// of 128 bytes the steps of a row start at the line its first element lies in, "phase" 16-byte vectors before it (phase =
+// address / 16 mod 8), and the lanes in front of the row are padding like those behind it.  All rows of a tile need the same
+// phase, because they share the x operand; rows eight apart have it, so a workgroup then owns every eighth row of a block
+// (rows_mma_layout).  Steps cut at the row start instead straddle two lines each: 22.3 against 19.8 us for 8191 rows of 3080
+// and 3072 elements, 78.7 against 63.5 us for 16000 rows of 6152 and 6144.
+// The steps of a row are dealt to the eight waves as contiguous runs, the last waves one more if they do not divide evenly.  A
+// register set holds up to nine steps of one tile; longer rows take two sets per tile ("chunks") and add both into the same
+// accumulator.  steps: per wave and chunk (the kernels' template argument), chunks: 1 or 2; all 0 if the row is too long.
+// slots: steps of an x operand in LDS -- those of the row with the largest phase; where there are phases one of zeros in front
+// (`front`), and behind what the last wave's register sets can have past the end of its run: the rounding up to two chunks, and
+// one for a phase that needs a step less or for a row that does not fill its steps.
+struct MmaSplit {
+  int steps, chunks, front, slots;
+};
+inline MmaSplit rows_mma_split(const RowsArgs& a) {
+  const bool shifted = a.row_vecs % 8 != 0 || (((uintptr_t)a.w | (uintptr_t)a.w2) & 127u) != 0;
+  const int total = (a.row_vecs + (shifted ? 7 : 0) + 7) / 8;
+  const int per_wave = (total + kMmaWaves - 1) / kMmaWaves;
+  if (per_wave > 18) return {0, 0, 0, 0};
+  const int chunks = per_wave > 9 ? 2 : 1;
+  const int steps = (per_wave + chunks - 1) / chunks, front = shifted ? 1 : 0;
+  return {steps, chunks, front, front + total + (steps * chunks - per_wave) + (shifted || total < kMmaWaves * per_wave ? 1 : 0)};
 }
-// STEPS = 64-element k steps per wave per tile; the row length must be exactly kMmaWaves * STEPS * 64 so that no
-// load or MFMA sits behind a bounds check (control flow around loads in flight makes the compiler wait for them).
-inline int rows_mma_steps(int K) { return K % (kMmaWaves * 64) == 0 ? K / (kMmaWaves * 64) : 0; }
+// Which rows a workgroup owns, and the grid: about one persistent workgroup per CU.  Workgroup i owns rows base + q * stride for q <
+// rows_per: `rows_per` consecutive rows (stride 1), or, where the rows' phases differ, every eighth row of the block of
+// 8 * rows_per rows that it shares with seven others.
+inline int rows_mma_layout(RowsArgs& a, int cus) {
+  const int ntiles = (a.N + kMmaTileRows - 1) / kMmaTileRows;
+  const int grid = ntiles < cus ? ntiles : cus;
+  a.rows_per = (a.N + grid - 1) / grid;
+  a.row_stride = a.row_vecs % 8 != 0 ? 8 : 1;
+  return a.row_stride == 1 ? (a.N + a.rows_per - 1) / a.rows_per : 8 * ((a.N + 8 * a.rows_per - 1) / (8 * a.rows_per));
+}
+// dynamic LDS: x operands, gate partials, up partials -- each once per group of eight batch rows (ng = 1 or 2)
+inline size_t rows_mma_lds_bytes(const RowsArgs& a, int ng = 1) {
+  return (size_t)ng * ((size_t)rows_mma_split(a).slots * kWave * sizeof(u32x4) + 2u * kMmaWaves * kMmaPart * sizeof(float));
+}
+
+// This lane's view of one weight matrix: its place in a tile (weight row lane % 8, 16-byte piece `piece` of the row's 128-byte
+// steps), its first vector of a row, the end of those it reads, and where it finds the x operand of its wave's first step.
+// STEPS, CH: as MmaSplit.
+template <class DT, int STEPS, int CH, int NG>
+struct MmaRows {
+  const u32x4* __restrict__ w;
+  int row_vecs, vec0, vend;
+  const u32x4* xs;   // x operands of this lane, first step of its wave
+  int xgroup;        // operand vectors between the two groups of eight batch rows
+
+  // Only a wave's first step can start in front of a row.  Only its last two can be missing or reach past the end (the last wave
+  // has the longest run, one step less where this phase needs one step less than the largest), or three where two chunks
+  // round the run up.  The checks of all others fold away.
+  static __device__ __forceinline__ constexpr bool edge(int c, int s) { return (c == 0 && s == 0) || (c == CH - 1 && s >= STEPS - 1 - CH); }
+  __device__ __forceinline__ bool outside(int c, int s) const { return edge(c, s) && ((unsigned)vec(c, s) >= (unsigned)vend); }
+  __device__ __forceinline__ int vec(int c, int s) const { return vec0 + (c * STEPS + s) * 8; }
+
+  // row: any row this workgroup owns (they share a phase)
+  __device__ __forceinline__ MmaRows(const u32x4* w_, int row, int row_vecs_, const u32x4* xs_, int xgroup_, int front, int lane, int wave)
+      : w(w_), row_vecs(row_vecs_), xgroup(xgroup_) {
+    const int phase = (int)((((uintptr_t)w_ >> 4) + (size_t)row * row_vecs_) & 7u);
+    const int steps = (row_vecs + phase + 7) >> 3;
+    const int longer = kMmaWaves - steps % kMmaWaves;  // the first wave whose run is one step longer
+    const int first = wave * (steps / kMmaWaves) + max(wave - longer, 0);
+    const int count = steps / kMmaWaves + (wave >= longer ? 1 : 0);
+    const int piece = ((lane >> 3) & 1) * 4 + (lane >> 4);
+    vec0 = first * 8 + piece - phase;
+    vend = max(0, min(row_vecs, (first + count) * 8 - phase));  // 0: a wave without steps
+    xs = xs_ + slot(vec0 + 8 * front, lane & 7);
+  }
+  // x operands in LDS: vector v of batch row b (of a group of eight) sits at slot(v + 8 * front, b), so that the eight vectors of a step,
+  // whatever the phase, are 64 slots with distinct banks in every quarter wave.
+  static __device__ __forceinline__ int slot(int v, int b) { return (v >> 3) * kWave + (v & 3) * 16 + ((v >> 2) & 1) * 8 + b; }
+
+  // Loads of chunk c of this lane's row, never predicated: a lane with nothing to fetch (mine false: rows past the end of the
+  // range or without a flag; or outside the row) reads the first vector of the matrix over and over, which stays in
+  // cache and moves nothing from HBM.
+  __device__ __forceinline__ void issue(int row, bool mine, int c, u32x4 (&dst)[STEPS]) const {
+    const u32x4* src = mine ? w + ((ptrdiff_t)row * row_vecs + vec(c, 0)) : w;
+    const int stride = mine ? 8 : 0;
+#pragma unroll
+    for (int s = 0; s < STEPS; s++) dst[s] = load_stream(outside(c, s) ? w : src + s * stride);
+  }
+  // acc += chunk c of the tile times the staged x rows.  What a load outside the row brought are weights of another
+  // place, perhaps infinities: replaced by zeros before they meet the zeros of the x padding.
+  __device__ __forceinline__ void multiply(const u32x4 (&src)[STEPS], int c, f32x4 (&acc)[NG]) const {
+#pragma unroll
+    for (int g = 0; g < NG; g++)
+#pragma unroll
+      for (int s = 0; s < STEPS; s++)
+        acc[g] = Mma<DT>::run(outside(c, s) ? zero4() : src[s], xs[g * xgroup + (c * STEPS + s) * kWave], acc[g]);
+  }
+};
+
+constexpr int kMmaPartGroup = kMmaWaves * kMmaPart;  // partial-sum floats of one group of eight batch rows
+
+// The two useful quadrants of the accumulators -> this wave's part of a partial buffer.
+template <int NG>
+__device__ __forceinline__ void mma_store_partials(const f32x4 (&acc)[NG], float* part, int lane, int wave) {
+  const int ncol = lane & 15;
+  const bool keep = (lane < 32) ? (ncol < 8) : (ncol >= 8);
+  const int slot = (lane >> 5) * 16 + ((lane >> 4) & 1) * 8 + (ncol & 7);
+  if (keep) {
+#pragma unroll
+    for (int g = 0; g < NG; g++) {
+      float* dst = part + g * kMmaPartGroup + wave * kMmaPart + slot;
+#pragma unroll
+      for (int i = 0; i < 4; i++) dst[i * 32] = acc[g][i];
+    }
+  }
+}
+// One thread per (row rj of the tile, batch row rb): adds the waves' partials of group g in wave order.
+__device__ __forceinline__ float mma_reduce(const float* part, int g, int rj, int rb) {
+  const float* src = part + g * kMmaPartGroup + (rj & 3) * 32 + (rj >> 2) * 8 + rb;
+  float s = 0.f;
+#pragma unroll
+  for (int w = 0; w < kMmaWaves; w++) s += src[w * kMmaPart] + src[w * kMmaPart + 16];
+  return s;
+}
+
+// Staging of x: thread tid takes vectors tid + k * 512 of the nb rows, row by row in groups of eight; the loads of all are in flight together.
+// The padding steps and the batch rows past nb are zero.  NV: vectors per thread, at least those of a whole operand.
+template <int NV, int NG>
+struct MmaX {
+  u32x4 v[NG][NV];
+  int tid, front;
+  // Slot i of an operand holds vector(i), counted from the row's first, of batch row gb * 8 + i % 8.  No branches (x is
+  // what everything waits for): a slot without one fetches the first vector of x and stores zeros.
+  __device__ __forceinline__ int vector(int i) const { return (i >> 6) * 8 + ((i >> 3) & 1) * 4 + ((i >> 4) & 3) - 8 * front; }
+  __device__ __forceinline__ bool in(const RowsArgs& p, int gb, int i) const {
+    return (gb * 8 + (i & 7) < p.nb) & ((unsigned)vector(i) < (unsigned)p.row_vecs);
+  }
+  __device__ __forceinline__ void fetch(const RowsArgs& p) {
+#pragma unroll
+    for (int gb = 0; gb < NG; gb++)
+#pragma unroll
+      for (int k = 0; k < NV; k++) {
+        const int i = front * kWave + tid + k * kMmaThreads;
+        const unsigned o = (gb * 8 + (i & 7)) * p.row_vecs + vector(i);
+        v[gb][k] = p.x[in(p, gb, i) ? o : 0u];
+      }
+  }
+  // xgroup: slots of one group's operand; the last one is padding where fewer than NV * 512 are needed
+  __device__ __forceinline__ void store(const RowsArgs& p, u32x4* xs, int xgroup) const {
+#pragma unroll
+    for (int gb = 0; gb < NG; gb++) {
+      if (front && tid < kWave) xs[gb * xgroup + tid] = zero4();
+#pragma unroll
+      for (int k = 0; k < NV; k++) {
+        const int i = front * kWave + tid + k * kMmaThreads;
+        u32x4 o;
+        const bool ok = in(p, gb, i);
+#pragma unroll
+        for (int e = 0; e < 4; e++) o[e] = ok ? v[gb][k][e] : 0u;
+        xs[gb * xgroup + min(i, xgroup - 1)] = o;
+      }
+      for (int i = front * kWave + tid + NV * kMmaThreads; i < xgroup; i += kMmaThreads) xs[gb * xgroup + i] = zero4();
+    }
+  }
+};
 
 // UP = false is the gate pass alone (activations, flags and union bits out; no up rows, no z).
 // NG = 2 takes 9..16 batch rows in one pass over the weights: the second group of eight rows is a second x operand in
 // LDS and a second MFMA on the weight registers the first one just used, so the weights are still read once.
-template <class DT, int STEPS, bool UP, int NG = 1>
+// CH = 2 (rows of more than 4096 elements; their x fills 128 KiB of LDS at 8192): a tile is two register sets, so the gate ring
+// holds one tile ahead instead of two, and the up sums of tile r - 1 are taken before the up rows of tile r overwrite their set.
+template <class DT, int STEPS, int CH, bool UP, int NG = 1>
 __global__ __launch_bounds__(kMmaThreads) void rows_mma_kernel(RowsArgs p) {
   typedef typename DT::st st;
-  extern __shared__ u32x4 xs[];  // [nsteps][64] x operands, then the partial buffers
+  typedef MmaRows<DT, STEPS, CH, NG> Rows;
+  extern __shared__ u32x4 xs[];  // [NG][mma_slots][64] x operands, then the partial buffers
   __shared__ uint32_t s_any;
 
   const int tid = threadIdx.x;
   const int lane = tid & (kWave - 1);
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  constexpr int kMmaSteps = STEPS;
-  constexpr int nsteps = kMmaWaves * STEPS;
-  constexpr int kXGroup = nsteps * kWave;             // operand vectors of one group of eight batch rows
-  constexpr int kPartGroup = kMmaWaves * kMmaPart;    // partial-sum floats of one group
-  float* part_g = (float*)(xs + (size_t)NG * kXGroup);
-  float* part_u = part_g + NG * kPartGroup;
+  const int xgroup = p.mma_slots * kWave;
+  float* part_g = (float*)(xs + (size_t)NG * xgroup);
+  float* part_u = part_g + NG * kMmaPartGroup;
 
-  const int rows_per = (p.N + (int)gridDim.x - 1) / (int)gridDim.x;
-  const int r0 = min((int)blockIdx.x * rows_per, p.N);  // this workgroup's rows: [r0, r1)
-  const int r1 = min(r0 + rows_per, p.N);
-  const int my_tiles = (r1 - r0 + kMmaTileRows - 1) / kMmaTileRows;
+  // this workgroup's rows: base + q * stride, q < nrows
+  const int base = p.row_stride == 1 ? (int)blockIdx.x * p.rows_per : (int)(blockIdx.x >> 3) * 8 * p.rows_per + (int)(blockIdx.x & 7);
+  const int nrows = max(0, min(p.rows_per, (p.N - base + p.row_stride - 1) / p.row_stride));
+  const int my_tiles = (nrows + kMmaTileRows - 1) / kMmaTileRows;
+  const int jl = lane & 7;  // this lane's weight row in a tile
+  const Rows gate(p.w, base, p.row_vecs, xs, xgroup, p.mma_front, lane, wave);
+  const Rows up(UP ? p.w2 : p.w, base, p.row_vecs, xs, xgroup, p.mma_front, lane, wave);
 
-  const int s0 = wave * STEPS;  // this wave's first k step
-  // this lane's weight row inside a tile and its 16-byte piece of the 128-byte step
-  const int jl = lane & 7;
-  const int piece = ((lane >> 3) & 1) * 4 + (lane >> 4);
-  // slot of this lane's accumulators in a partial buffer; the two mismatched quadrants are not stored
-  const int ncol = lane & 15;
-  const bool keep = (lane < 32) ? (ncol < 8) : (ncol >= 8);
-  const int slot = (lane >> 5) * 16 + ((lane >> 4) & 1) * 8 + (ncol & 7);
-
-  // Loads of tile number `it` of this workgroup, never predicated: lanes with nothing to fetch -- rows past the end of
-  // the range, and with use_any the rows whose union bit is clear -- read the first bytes of the matrix over and over,
-  // which stay in cache and move nothing from HBM (their sums are dropped).
-  auto issue = [&](const u32x4* __restrict__ w, int it, u32x4 (&dst)[kMmaSteps], bool use_any) {
-    const int row = r0 + it * kMmaTileRows + jl;
-    bool mine = row < r1;
-    if (use_any) mine = mine && ((s_any >> jl) & 1u);
-    const u32x4* src = mine ? w + (size_t)row * p.row_vecs + piece + (size_t)s0 * 8 : w + piece;
-    const int stride = mine ? 8 : 0;
-#pragma unroll
-    for (int c = 0; c < kMmaSteps; c++) dst[c] = load_stream(src + c * stride);
+  auto issue_gate = [&](int it, int c, u32x4 (&dst)[STEPS]) {
+    const int q = it * kMmaTileRows + jl;
+    gate.issue(base + q * p.row_stride, q < nrows, c, dst);
   };
-  auto multiply = [&](const u32x4 (&src)[kMmaSteps], float* part) {
-#pragma unroll
-    for (int g = 0; g < NG; g++) {
-      f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-      for (int c = 0; c < kMmaSteps; c++) acc = Mma<DT>::run(src[c], xs[g * kXGroup + (s0 + c) * kWave + lane], acc);
-      if (keep) {
-        float* dst = part + g * kPartGroup + wave * kMmaPart + slot;
-#pragma unroll
-        for (int i = 0; i < 4; i++) dst[i * 32] = acc[i];
-      }
-    }
+  auto issue_up = [&](int it, int c, u32x4 (&dst)[STEPS]) {  // only the rows of the tile that some batch row keeps
+    const int q = it * kMmaTileRows + jl;
+    up.issue(base + q * p.row_stride, q < nrows && ((s_any >> jl) & 1u), c, dst);
   };
-  // wave 0, one thread per (row j of the tile, batch row b): adds the waves' partials in wave order
+  // wave 0, one thread per (row rj of the tile, batch row rb)
   const int rj = (lane >> 3), rb = lane & 7;
-  auto reduce = [&](const float* part) -> float {
-    const float* src = part + (rj & 3) * 32 + (rj >> 2) * 8 + rb;
-    float s = 0.f;
-#pragma unroll
-    for (int w = 0; w < kMmaWaves; w++) s += src[w * kMmaPart] + src[w * kMmaPart + 16];
-    return s;
-  };
 
   // wave 0 carries the gate results of the previous tile until its up sums arrive
   float prev_a[NG];
@@ -140,9 +262,22 @@ __global__ __launch_bounds__(kMmaThreads) void rows_mma_kernel(RowsArgs p) {
   uint32_t prev_bits = 0u;
   int prev_row = 0;
 
-  auto round_body = [&](int r, u32x4 (&gcur)[kMmaSteps], u32x4 (&ucur)[kMmaSteps], u32x4 (&uprev)[kMmaSteps]) {
-    multiply(gcur, part_g);
-    issue(p.w, r + 2, gcur, false);
+  // gbuf, ubuf, uprev: the register sets of the round.  One chunk: gbuf[0] is the tile's set, ubuf[0] takes its up rows, uprev[0]
+  // holds those of the tile before.  Two chunks: gbuf[0..1] and ubuf[0..1] are the tile's two sets, uprev is ubuf.
+  auto round_body = [&](int r, u32x4 (&ga)[STEPS], u32x4 (&gb)[STEPS], u32x4 (&ucur)[STEPS], u32x4 (&uprev)[STEPS]) {
+    f32x4 acc[NG];
+#pragma unroll
+    for (int g = 0; g < NG; g++) acc[g] = f32x4{0.f, 0.f, 0.f, 0.f};
+    gate.multiply(ga, 0, acc);
+    if constexpr (CH == 2) {
+      issue_gate(r + 1, 0, ga);
+      gate.multiply(gb, 1, acc);
+      mma_store_partials<NG>(acc, part_g, lane, wave);
+      issue_gate(r + 1, 1, gb);
+    } else {
+      mma_store_partials<NG>(acc, part_g, lane, wave);
+      issue_gate(r + 2, 0, ga);
+    }
     __syncthreads();
     float a[NG];
     bool act[NG], valid[NG];
@@ -152,14 +287,15 @@ __global__ __launch_bounds__(kMmaThreads) void rows_mma_kernel(RowsArgs p) {
       act[g] = valid[g] = false;
     }
     uint32_t bits8 = 0u;
-    const int row = r0 + r * kMmaTileRows + rj;
+    const int row = base + (r * kMmaTileRows + rj) * p.row_stride;
+    const bool row_in = r * kMmaTileRows + rj < nrows;
     if (wave == 0 && r < my_tiles) {
       uint64_t bal = 0ull;
 #pragma unroll
       for (int g = 0; g < NG; g++) {
         const int b = g * 8 + rb;  // batch row of this thread in group g
-        valid[g] = row < r1 && b < p.nb;
-        const float gr = DT::rnd(reduce(part_g + g * kPartGroup));
+        valid[g] = row_in && b < p.nb;
+        const float gr = DT::rnd(mma_reduce(part_g, g, rj, rb));
         a[g] = DT::rnd(gr / (1.f + expf(-gr)));
         act[g] = valid[g] && fabsf(a[g]) > p.t;
         bal |= __ballot(act[g]);
@@ -169,18 +305,28 @@ __global__ __launch_bounds__(kMmaThreads) void rows_mma_kernel(RowsArgs p) {
 #pragma unroll
       for (int j = 0; j < 8; j++) bits8 |= ((bal >> (8 * j)) & 0xffull) ? (1u << j) : 0u;
       if (lane == 0) s_any = bits8;
-      if (p.ubytes_out && rb == 0 && row < r1) p.ubytes_out[row] = (uint8_t)((bits8 >> rj) & 1u);
+      if (p.ubytes_out && rb == 0 && row_in) p.ubytes_out[row] = (uint8_t)((bits8 >> rj) & 1u);
     }
     __syncthreads();
     if (!UP) return;
-    issue(p.w2, r, ucur, true);
-    multiply(uprev, part_u);
+#pragma unroll
+    for (int g = 0; g < NG; g++) acc[g] = f32x4{0.f, 0.f, 0.f, 0.f};
+    if constexpr (CH == 2) {
+      up.multiply(ucur, 0, acc);
+      issue_up(r, 0, ucur);
+      up.multiply(uprev, 1, acc);
+      issue_up(r, 1, uprev);
+    } else {
+      issue_up(r, 0, ucur);
+      up.multiply(uprev, 0, acc);
+    }
+    mma_store_partials<NG>(acc, part_u, lane, wave);
     __syncthreads();
     if (wave == 0) {
 #pragma unroll
       for (int g = 0; g < NG; g++) {
         if (r >= 1 && prev_valid[g]) {
-          const float u = reduce(part_u + g * kPartGroup);
+          const float u = mma_reduce(part_u, g, rj, rb);
           const float z = prev_act[g] ? DT::rnd(prev_a[g] * DT::rnd(u)) : 0.f;
           const size_t o = (size_t)(g * 8 + rb) * p.N + prev_row;
           if (p.z32_out && ((prev_bits >> rj) & 1u)) p.z32_out[o] = z;
@@ -195,62 +341,47 @@ __global__ __launch_bounds__(kMmaThreads) void rows_mma_kernel(RowsArgs p) {
   CATS_RSTAMP(0);
   // ---- prologue.  x is requested before the first weight load goes out, so that its read does not queue behind
   // the weight requests of the whole machine. ---------------------------------------------------------------------
-  u32x4 g0[kMmaSteps], g1[kMmaSteps], u0[kMmaSteps], u1[kMmaSteps];
+  u32x4 g0[STEPS], g1[STEPS], u0[STEPS], u1[STEPS];
   {
-    // nsteps * 64 operand vectors over kMmaThreads threads = STEPS per thread, all loads in flight together;
-    // batch rows past nb read row 0 and store zeros
-    u32x4 xv[NG][STEPS];
-#pragma unroll
-    for (int gb = 0; gb < NG; gb++)
-#pragma unroll
-      for (int k = 0; k < STEPS; k++) {
-        const int i = tid + k * kMmaThreads;
-        const int step = i >> 6, l = i & 63;
-        const int n = l & 15, g = l >> 4, b = gb * 8 + (n & 7), kh = n >> 3;
-        xv[gb][k] = p.x[(size_t)(b < p.nb ? b : 0) * p.row_vecs + step * 8 + kh * 4 + g];
-      }
-    // the first gate tile goes out behind x, before x is waited for: it is a memory round trip ahead when the staging is done
+    MmaX<STEPS * CH, NG> x;
+    x.tid = tid;
+    x.front = p.mma_front;
+    x.fetch(p);
+    // the first gate set goes out behind x, before x is waited for: it is a memory round trip ahead when the staging is done
     __builtin_amdgcn_sched_barrier(0);
-    issue(p.w, 0, g0, false);
+    issue_gate(0, 0, g0);
     __builtin_amdgcn_sched_barrier(0);
+    x.store(p, xs, xgroup);
 #pragma unroll
-    for (int gb = 0; gb < NG; gb++)
+    for (int c = 0; c < STEPS; c++) u1[c] = zero4();  // defined before the first (unused) up product
+    if constexpr (CH == 2) {
 #pragma unroll
-      for (int k = 0; k < STEPS; k++) {
-        const int i = tid + k * kMmaThreads;
-        const int b = gb * 8 + (i & 7);
-        xs[gb * kXGroup + i] = b < p.nb ? xv[gb][k] : zero4();
-      }
-#pragma unroll
-    for (int c = 0; c < kMmaSteps; c++) u1[c] = zero4();  // defined before the first (unused) up product
+      for (int c = 0; c < STEPS; c++) u0[c] = zero4();
+    }
   }
   // a barrier for LDS only: __syncthreads() would also wait for the gate loads in flight
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
   __builtin_amdgcn_s_barrier();
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-  // The second gate tile goes out after the barrier: a wave blocks at issue once the CU's miss queue is full, so
+  // The second gate set goes out after the barrier: a wave blocks at issue once the CU's miss queue is full, so
   // everything issued before the barrier delays the moment the staged x becomes usable.
-  issue(p.w, 1, g1, false);
+  issue_gate(CH == 2 ? 0 : 1, CH == 2 ? 1 : 0, g1);
   if (p.norm_w) {
-    // RMS norm in place.  Operand slot i = step * 64 + l holds batch row l % 8, vector step * 8 + (l % 16 / 8) * 4 + l / 16.
-    // Wave b adds the squares of batch row b (kMmaWaves == 8 rows), in a fixed order.
+    // RMS norm in place.  Wave b adds the squares of batch row b (kMmaWaves == 8 rows), in a fixed order.
     __shared__ float s_scale[NG * 8];
 #pragma unroll
     for (int gb = 0; gb < NG; gb++) {
       float ss = 0.f;
-      for (int q = lane; q < nsteps * 8; q += kWave) ss = vec_sumsq<DT>(xs[gb * kXGroup + q * 8 + wave], ss);
+      for (int q = lane; q < xgroup / 8; q += kWave) ss = vec_sumsq<DT>(xs[gb * xgroup + q * 8 + wave], ss);
       ss = wave_sum(ss);
       if (lane == 0) s_scale[gb * 8 + wave] = rsqrtf(ss / (float)p.K + p.norm_eps);
     }
     __syncthreads();
 #pragma unroll
     for (int gb = 0; gb < NG; gb++)
-#pragma unroll
-      for (int k = 0; k < STEPS; k++) {
-        const int i = tid + k * kMmaThreads;
-        const int step = i >> 6, l = i & 63;
-        const int n = l & 15, g = l >> 4, b = gb * 8 + (n & 7), kh = n >> 3;
-        if (b < p.nb) xs[gb * kXGroup + i] = vec_norm_apply<DT>(xs[gb * kXGroup + i], s_scale[b], p.norm_w[step * 8 + kh * 4 + g]);
+      for (int i = p.mma_front * kWave + tid; i < xgroup; i += kMmaThreads) {
+        const int b = gb * 8 + (i & 7), v = (i >> 6) * 8 + ((i >> 3) & 1) * 4 + ((i >> 4) & 3) - 8 * p.mma_front;
+        if (b < p.nb && v < p.row_vecs) xs[gb * xgroup + i] = vec_norm_apply<DT>(xs[gb * xgroup + i], s_scale[b], p.norm_w[v]);
       }
     __syncthreads();
   }
@@ -258,12 +389,21 @@ __global__ __launch_bounds__(kMmaThreads) void rows_mma_kernel(RowsArgs p) {
 
   // rounds 0 .. my_tiles: the last one only drains the up sums of the last tile
   const int last = UP ? my_tiles : my_tiles - 1;
-  for (int r = 0; r <= last; r += 2) {
-    round_body(r, g0, u0, u1);
-    if (r + 1 <= last) round_body(r + 1, g1, u1, u0);
+  if constexpr (CH == 2) {
+    for (int r = 0; r <= last; r++) {
+      round_body(r, g0, g1, u0, u1);
 #ifdef CATS_TIMING
-    if (r < 10) CATS_RSTAMP(2 + (r >> 1));
+      if (r < 10) CATS_RSTAMP(2 + (r >> 1));
 #endif
+    }
+  } else {
+    for (int r = 0; r <= last; r += 2) {
+      round_body(r, g0, g0, u0, u1);
+      if (r + 1 <= last) round_body(r + 1, g1, g1, u1, u0);
+#ifdef CATS_TIMING
+      if (r < 10) CATS_RSTAMP(2 + (r >> 1));
+#endif
+    }
   }
   CATS_RSTAMP(7);
 }
@@ -279,70 +419,52 @@ __global__ __launch_bounds__(kMmaThreads) void rows_mma_kernel(RowsArgs p) {
 // NG = 2 takes 9..16 batch rows: a second x operand in LDS and a second MFMA on the same weight registers.
 // dynamic LDS, per group of eight batch rows: x operands | two partial buffers | a of the range, [8][rows_pad] in storage
 // type | its flags, [8][rows_pad] bytes; then one byte of union bits per tile
-inline size_t rows_mma_up_lds_bytes(int K, int rows_pad, int ng) {
-  return rows_mma_lds_bytes(K, ng) + (size_t)ng * 8 * rows_pad * 3 + (size_t)(rows_pad / 8 + 15) / 16 * 16;
+inline size_t rows_mma_up_lds_bytes(const RowsArgs& a, int rows_pad, int ng) {
+  return rows_mma_lds_bytes(a, ng) + (size_t)ng * 8 * rows_pad * 3 + (size_t)(rows_pad / 8 + 15) / 16 * 16;
 }
 
-template <class DT, int STEPS, int NG>
+template <class DT, int STEPS, int CH, int NG>
 __global__ __launch_bounds__(kMmaThreads) void rows_mma_up_kernel(RowsArgs p) {
   typedef typename DT::st st;
+  typedef MmaRows<DT, STEPS, CH, NG> Rows;
   static_assert(sizeof(st) == 2, "16-bit types only");
   extern __shared__ u32x4 xs[];
   const int tid = threadIdx.x;
   const int lane = tid & (kWave - 1);
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  constexpr int nsteps = kMmaWaves * STEPS;
-  constexpr int kXGroup = nsteps * kWave;
-  constexpr int kPartGroup = kMmaWaves * kMmaPart;
+  const int xgroup = p.mma_slots * kWave;
 
-  const int rows_per = (p.N + (int)gridDim.x - 1) / (int)gridDim.x;
-  const int rows_pad = (rows_per + kMmaTileRows - 1) / kMmaTileRows * kMmaTileRows;
-  const int r0 = min((int)blockIdx.x * rows_per, p.N);
-  const int r1 = min(r0 + rows_per, p.N);
-  const int my_tiles = (r1 - r0 + kMmaTileRows - 1) / kMmaTileRows;
+  // this workgroup's rows: base + q * stride, q < nrows
+  const int base = p.row_stride == 1 ? (int)blockIdx.x * p.rows_per : (int)(blockIdx.x >> 3) * 8 * p.rows_per + (int)(blockIdx.x & 7);
+  const int nrows = max(0, min(p.rows_per, (p.N - base + p.row_stride - 1) / p.row_stride));
+  const int rows_pad = (p.rows_per + kMmaTileRows - 1) / kMmaTileRows * kMmaTileRows;
+  const int my_tiles = (nrows + kMmaTileRows - 1) / kMmaTileRows;
+  const int jl = lane & 7;
+  const Rows up(p.w, base, p.row_vecs, xs, xgroup, p.mma_front, lane, wave);
   constexpr int NB = NG * 8;                                // batch rows the kernel is laid out for
-  float* part = (float*)(xs + NG * kXGroup);                // [2][NG][kPartGroup]
-  st* s_a = (st*)(part + 2 * NG * kPartGroup);              // [NB][rows_pad]
+  float* part = (float*)(xs + NG * xgroup);                 // [2][NG][kMmaPartGroup]
+  st* s_a = (st*)(part + 2 * NG * kMmaPartGroup);           // [NB][rows_pad]
   uint8_t* s_f = (uint8_t*)(s_a + NB * rows_pad);           // [NB][rows_pad]
   uint8_t* s_bits = s_f + NB * rows_pad;                    // [rows_pad / 8]
-
-  const int s0 = wave * STEPS;
-  const int jl = lane & 7;
-  const int piece = ((lane >> 3) & 1) * 4 + (lane >> 4);
-  const int ncol = lane & 15;
-  const bool keep = (lane < 32) ? (ncol < 8) : (ncol >= 8);
-  const int slot = (lane >> 5) * 16 + ((lane >> 4) & 1) * 8 + (ncol & 7);
   const int rj = lane >> 3, rb = lane & 7;
 
   CATS_RSTAMP(0);
   // ---- prologue: x -> LDS in operand order (as rows_mma_kernel), a of the range -> LDS, the bits of every tile ----------
   {
-    u32x4 xv[NG][STEPS];
-#pragma unroll
-    for (int gb = 0; gb < NG; gb++)
-#pragma unroll
-      for (int k = 0; k < STEPS; k++) {
-        const int i = tid + k * kMmaThreads;
-        const int step = i >> 6, l = i & 63;
-        const int n = l & 15, g = l >> 4, b = gb * 8 + (n & 7), kh = n >> 3;
-        xv[gb][k] = p.x[(size_t)(b < p.nb ? b : 0) * p.row_vecs + step * 8 + kh * 4 + g];
-      }
+    MmaX<STEPS * CH, NG> x;
+    x.tid = tid;
+    x.front = p.mma_front;
+    x.fetch(p);
     const st* ain = (const st*)p.a_in;
     for (int e = tid; e < NB * rows_pad; e += kMmaThreads) {
       const int b = e / rows_pad, j = e - b * rows_pad;
-      const bool in = b < p.nb && r0 + j < r1;  // the padding of the range and of the batch is never flagged
-      const size_t o = (size_t)b * p.N + r0 + j;
+      const bool in = b < p.nb && j < nrows;  // the padding of the range and of the batch is never flagged
+      const size_t o = (size_t)b * p.N + base + j * p.row_stride;
       const st av = in ? ain[o] : DT::fromf(0.f);
       s_a[e] = av;
       s_f[e] = in && (p.flag_in ? p.flag_in[o] != 0 : fabsf(DT::tof(av)) > p.t) ? 1 : 0;
     }
-#pragma unroll
-    for (int gb = 0; gb < NG; gb++)
-#pragma unroll
-      for (int k = 0; k < STEPS; k++) {
-        const int i = tid + k * kMmaThreads;
-        xs[gb * kXGroup + i] = gb * 8 + (i & 7) < p.nb ? xv[gb][k] : zero4();
-      }
+    x.store(p, xs, xgroup);
   }
   __syncthreads();
   // one thread per row of the range: any batch row flagged?  Eight neighbouring lanes make a tile's byte.
@@ -352,7 +474,7 @@ __global__ __launch_bounds__(kMmaThreads) void rows_mma_up_kernel(RowsArgs p) {
     if (j < rows_pad) {
 #pragma unroll
       for (int b = 0; b < NB; b++) any = any || s_f[b * rows_pad + j] != 0;
-      if (p.ubytes_out && r0 + j < r1) p.ubytes_out[r0 + j] = any ? 1 : 0;
+      if (p.ubytes_out && j < nrows) p.ubytes_out[base + j * p.row_stride] = any ? 1 : 0;
     }
     const uint64_t bal = __ballot(any);
     if (j < rows_pad && (lane & 7) == 0) s_bits[j >> 3] = (uint8_t)((bal >> (lane & 56)) & 0xffull);
@@ -360,63 +482,56 @@ __global__ __launch_bounds__(kMmaThreads) void rows_mma_up_kernel(RowsArgs p) {
   __syncthreads();
   CATS_RSTAMP(1);
 
-  auto issue = [&](int it, u32x4 (&dst)[STEPS]) {
-    const int row = r0 + it * kMmaTileRows + jl;
+  auto issue = [&](int it, int c, u32x4 (&dst)[STEPS]) {
+    const int q = it * kMmaTileRows + jl;
     const uint32_t bits = it < my_tiles ? s_bits[it] : 0u;
-    const bool mine = row < r1 && ((bits >> jl) & 1u);
-    const u32x4* src = mine ? p.w + (size_t)row * p.row_vecs + piece + (size_t)s0 * 8 : p.w + piece;
-    const int stride = mine ? 8 : 0;
-#pragma unroll
-    for (int c = 0; c < STEPS; c++) dst[c] = load_stream(src + c * stride);
+    up.issue(base + q * p.row_stride, q < nrows && ((bits >> jl) & 1u), c, dst);
   };
-  auto multiply = [&](const u32x4 (&src)[STEPS], float* dst_part) {
+  // wave 0, one thread per (row rj of the tile, batch row rb): the eight waves' partials in wave order, then z = a * up
+  auto finish = [&](int r, const float* my_part) {
+    const int j = r * kMmaTileRows + rj;
+    const int row = base + j * p.row_stride;
+    const bool live = (s_bits[r] >> rj) & 1u;       // the row was read
 #pragma unroll
     for (int gb = 0; gb < NG; gb++) {
-      f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-      for (int c = 0; c < STEPS; c++) acc = Mma<DT>::run(src[c], xs[gb * kXGroup + (s0 + c) * kWave + lane], acc);
-      if (keep) {
-        float* dst = dst_part + gb * kPartGroup + wave * kMmaPart + slot;
-#pragma unroll
-        for (int i = 0; i < 4; i++) dst[i * 32] = acc[i];
+      const int b = gb * 8 + rb;
+      const float u = mma_reduce(my_part, gb, rj, rb);
+      const float a = DT::tof(s_a[b * rows_pad + j]);
+      if (j < nrows && b < p.nb) {
+        const float z = s_f[b * rows_pad + j] ? DT::rnd(a * DT::rnd(u)) : 0.f;  // u of a row that was not read is noise: never used
+        const size_t o = (size_t)b * p.N + row;
+        if (p.z32_out && (live || p.flag_in)) p.z32_out[o] = z;
+        if (p.zt_out) ((st*)p.zt_out)[o] = DT::fromf(z);
       }
     }
   };
-  auto body = [&](int r, u32x4 (&ring)[STEPS], float* my_part) {
-    multiply(ring, my_part);
-    issue(r + 2, ring);
-    __syncthreads();
-    if (wave == 0 && r < my_tiles) {
-      // one thread per (row rj of the tile, batch row rb): the eight waves' partials in wave order, then z = a * up
-      const int j = r * kMmaTileRows + rj;
-      const int row = r0 + j;
-      const bool live = (s_bits[r] >> rj) & 1u;       // the row was read
+  // one tile: ra (and with two chunks rb2) hold it; they are refilled with what follows in the ring
+  auto body = [&](int r, u32x4 (&ra)[STEPS], u32x4 (&rb2)[STEPS], float* my_part) {
+    f32x4 acc[NG];
 #pragma unroll
-      for (int gb = 0; gb < NG; gb++) {
-        const int b = gb * 8 + rb;
-        const float* src = my_part + gb * kPartGroup + (rj & 3) * 32 + (rj >> 2) * 8 + rb;
-        float u = 0.f;
-#pragma unroll
-        for (int w = 0; w < kMmaWaves; w++) u += src[w * kMmaPart] + src[w * kMmaPart + 16];
-        const float a = DT::tof(s_a[b * rows_pad + j]);
-        if (row < r1 && b < p.nb) {
-          const float z = s_f[b * rows_pad + j] ? DT::rnd(a * DT::rnd(u)) : 0.f;  // u of a row that was not read is noise: never used
-          const size_t o = (size_t)b * p.N + row;
-          if (p.z32_out && (live || p.flag_in)) p.z32_out[o] = z;
-          if (p.zt_out) ((st*)p.zt_out)[o] = DT::fromf(z);
-        }
-      }
+    for (int g = 0; g < NG; g++) acc[g] = f32x4{0.f, 0.f, 0.f, 0.f};
+    up.multiply(ra, 0, acc);
+    if constexpr (CH == 2) {
+      issue(r + 1, 0, ra);
+      up.multiply(rb2, 1, acc);
+      mma_store_partials<NG>(acc, my_part, lane, wave);
+      issue(r + 1, 1, rb2);
+    } else {
+      mma_store_partials<NG>(acc, my_part, lane, wave);
+      issue(r + 2, 0, ra);
     }
+    __syncthreads();
+    if (wave == 0 && r < my_tiles) finish(r, my_part);
   };
 
   u32x4 u0[STEPS], u1[STEPS];
-  issue(0, u0);
-  issue(1, u1);
+  issue(0, 0, u0);
+  issue(CH == 2 ? 0 : 1, CH == 2 ? 1 : 0, u1);
   // always in pairs (an odd count ends with a tile of dummy loads): a branch around the second body would leave the
   // compiler with a path on which its counted waits for the ring degrade to "wait for everything"
   for (int r = 0; r < my_tiles; r += 2) {
-    body(r, u0, part);
-    body(r + 1, u1, part + NG * kPartGroup);
+    body(r, u0, CH == 2 ? u1 : u0, part);
+    body(r + 1, CH == 2 ? u0 : u1, u1, part + NG * kMmaPartGroup);
   }
   CATS_RSTAMP(7);
 }
