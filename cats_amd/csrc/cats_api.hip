@@ -2,6 +2,7 @@
 // workspace carving, launch-shape selection and dispatch on dtype.  No allocation, no synchronisation
 // (cats_read_count excepted), everything on the caller's stream.
 #include <hip/hip_runtime.h>
+#include <math.h>
 #include <string.h>
 
 #include <mutex>
@@ -29,6 +30,12 @@ template <> hipError_t launch_down<F32>(int, bool, const DownArgs&, int, hipStre
 template <> hipError_t launch_fused<F16>(int, int, int, const FusedArgs&, const ReduceArgs&, hipStream_t);
 template <> hipError_t launch_fused<BF16>(int, int, int, const FusedArgs&, const ReduceArgs&, hipStream_t);
 template <> hipError_t launch_fused<F32>(int, int, int, const FusedArgs&, const ReduceArgs&, hipStream_t);
+template <> hipError_t launch_proj<F16>(int, int, const ProjArgs&, hipStream_t);
+template <> hipError_t launch_proj<BF16>(int, int, const ProjArgs&, hipStream_t);
+template <> hipError_t launch_proj<F32>(int, int, const ProjArgs&, hipStream_t);
+template <> hipError_t launch_attn<F16>(int, int, const AttnArgs&, hipStream_t);
+template <> hipError_t launch_attn<BF16>(int, int, const AttnArgs&, hipStream_t);
+template <> hipError_t launch_attn<F32>(int, int, const AttnArgs&, hipStream_t);
 int current_device_cus() {
   constexpr int kDevs = 64;
   static int cus[kDevs];  // 0 = not asked yet; written once per device with the same value, so a plain atomic will do
@@ -1141,6 +1148,79 @@ int cats_mlp_rowmajor_down(const void* x, const void* wgate, const void* wup, co
     return mlp_rowmajor_down_pass(at_cbytes(x, b0 * H * sz), wgate, wup, wdown, at_bytes(y_out, b0 * H * sz), nb, H, I, dtype, threshold, ws,
                                   ws_bytes, stream);
   });
+}
+
+static int do_proj(int mode, int dtype, const ProjArgs& a, hipStream_t s) {
+  const int bt = batch_template(a.r.nb);
+  const hipError_t e = dtype == CATS_F16    ? launch_proj<F16>(mode, bt, a, s)
+                       : dtype == CATS_BF16 ? launch_proj<BF16>(mode, bt, a, s)
+                                            : launch_proj<F32>(mode, bt, a, s);
+  return e == hipSuccess ? CATS_OK : CATS_ERR_LAUNCH;
+}
+
+// x of all rows is staged on chip whole
+static int check_proj(int B, int K, int N, int dtype) {
+  if (int st = check_common(B, K, N, dtype)) return st;
+  const int vecs = K / vec_elems(dtype);
+  return proj_lds_bytes(batch_template(B), (vecs + kWave - 1) / kWave) <= kProjMaxLds ? CATS_OK : CATS_ERR_SHAPE;
+}
+
+int cats_linear(const void* x, const void* norm_weight, float eps, const void* w, const void* residual, void* out, int B, int K, int N,
+                int dtype, void* stream) {
+  if (int st = check_proj(B, K, N, dtype)) return st;
+  if (!x || !w || !out) return CATS_ERR_NULL;
+  if (!aligned16(x) || !aligned16(w) || !aligned16(norm_weight)) return CATS_ERR_ALIGN;
+  ProjArgs a;
+  memset(&a, 0, sizeof(a));
+  fill_rows(a.r, x, w, K, N, B, dtype);
+  a.r.norm_w = (const u32x4*)norm_weight;
+  a.r.norm_eps = eps;
+  a.r.zt_out = out;
+  a.residual = residual;
+  return do_proj(residual ? kProjAdd : kProjPlain, dtype, a, (hipStream_t)stream);
+}
+
+int cats_attention_step(const void* h, const void* x, const void* norm_weight, float eps, const void* wq, const void* wk, const void* wv,
+                        const void* wo, void* k_cache, void* v_cache, const void* cos_table, const void* sin_table, const int64_t* position,
+                        float* q_scratch, void* attn_scratch, void* out, int B, int H, int heads, int max_len, int dtype, void* stream) {
+  if (int st = check_proj(B, H, H, dtype)) return st;
+  if (heads < 1 || max_len < 1 || H % heads != 0) return CATS_ERR_SHAPE;
+  const int hd = H / heads, lanes = hd / vec_elems(dtype);  // of a cache slot: a power of two, so that lane groups tile a wave
+  if (hd % vec_elems(dtype) != 0 || lanes < 2 || lanes > 32 || (lanes & (lanes - 1)) != 0) return CATS_ERR_SHAPE;
+  if (!h || !x || !wq || !wk || !wv || !wo || !k_cache || !v_cache || !cos_table || !sin_table || !position || !q_scratch || !attn_scratch || !out)
+    return CATS_ERR_NULL;
+  for (const void* p : {x, norm_weight, wq, wk, wv, wo, (const void*)k_cache, (const void*)v_cache, (const void*)attn_scratch})
+    if (!aligned16(p)) return CATS_ERR_ALIGN;
+  ProjArgs a;
+  memset(&a, 0, sizeof(a));
+  fill_rows(a.r, x, wq, H, H, B, dtype);
+  a.r.norm_w = (const u32x4*)norm_weight;
+  a.r.norm_eps = eps;
+  a.wk = (const u32x4*)wk;
+  a.wv = (const u32x4*)wv;
+  a.q_out = q_scratch;
+  a.k_cache = k_cache;
+  a.v_cache = v_cache;
+  a.cos_t = cos_table;
+  a.sin_t = sin_table;
+  a.pos = position;
+  a.half = hd / 2;
+  a.heads = heads;
+  a.max_len = max_len;
+  if (int st = do_proj(kProjQkv, dtype, a, (hipStream_t)stream)) return st;
+  AttnArgs t;
+  t.q = q_scratch;
+  t.k = (const u32x4*)k_cache;
+  t.v = (const u32x4*)v_cache;
+  t.pos = position;
+  t.out = attn_scratch;
+  t.scale = 1.44269504088896341f / sqrtf((float)hd);
+  t.max_len = max_len;
+  const hipError_t e = dtype == CATS_F16    ? launch_attn<F16>(B * heads, hd, t, (hipStream_t)stream)
+                       : dtype == CATS_BF16 ? launch_attn<BF16>(B * heads, hd, t, (hipStream_t)stream)
+                                            : launch_attn<F32>(B * heads, hd, t, (hipStream_t)stream);
+  if (e != hipSuccess) return CATS_ERR_LAUNCH;
+  return cats_linear(attn_scratch, nullptr, 0.f, wo, h, out, B, H, H, dtype, stream);
 }
 
 }  // extern "C"

@@ -1,0 +1,271 @@
+// The rest of a decoder layer around the MLP, for one new token per batch row:
+//
+//   proj_kernel<kProjQkv>      q, k, v = x . W{q,k,v}^T, rotary embedding on q and k, k and v into the cache      (one launch)
+//   attn_decode_kernel         softmax(q . K^T / sqrt(d)) . V over the cache slots 0..position, per batch row and head
+//   proj_kernel<kProjAdd>      out = residual + x . W^T                                              (the output projection)
+//   proj_kernel<kProjPlain>    out = x . W^T                                                         (the output head)
+//
+// x may be given before its RMS norm (norm_w), which is then applied while x is staged.  Everything between the weight
+// matrices stays in fp32 and is rounded once where it is stored.  All of it is bound by the weight stream: one wave owns two
+// rows of a matrix, whose loads are all in flight at once, as in rows_kernel.
+// One step of four layers 4096 / 11008, 32 heads, 32000 words, 256 tokens in the cache, fp16, one row: 338 us, of which the MLP
+// kernels take 160; with torch's operations in place of these kernels (about 25 launches a layer) it was 761.  Kernel trace: q, k, v
+// 18.7 us (5.4 TB/s), attention 6.6, output projection 8.4, output head 44 (5.9 TB/s).
+#pragma once
+#include "cats_rows.h"
+
+namespace cats {
+
+enum ProjMode { kProjPlain = 0, kProjAdd = 1, kProjQkv = 2 };
+
+struct ProjArgs {
+  RowsArgs r;            // x, w, K, N, nb, nch, row_vecs, norm_w, norm_eps; zt_out is the output of kProjPlain / kProjAdd
+  const void* residual;  // kProjAdd: (nb, N) dtype
+  // kProjQkv (w is Wq; N = heads * head_dim rows of each of the three matrices)
+  const u32x4* wk;
+  const u32x4* wv;
+  float* q_out;          // (nb, N) fp32, rotated
+  void* k_cache;         // (nb, heads, max_len, head_dim) dtype
+  void* v_cache;
+  const void* cos_t;     // (max_len, head_dim) dtype
+  const void* sin_t;
+  const int64_t* pos;    // one position for all batch rows; outside [0, max_len) nothing is stored
+  int half;              // head_dim / 2
+  int heads;
+  int max_len;
+};
+
+// Two rows per wave.  For kProjQkv they are the two elements of a head that the rotary embedding mixes, d and d + head_dim / 2,
+// so it is applied to the two sums where they are; the wave's number counts these pairs over the three matrices.
+template <class DT, int B, int CB, bool FULL, int MODE, int WAVES>
+__global__ __launch_bounds__(WAVES* kWave) __attribute__((amdgpu_waves_per_eu(B == 1 && WAVES == 4 && FULL ? 6 : 1, 8)))
+void proj_kernel(ProjArgs a) {
+  typedef typename DT::st st;
+  constexpr int R = 2;
+  constexpr int kThreads = WAVES * kWave;
+  const RowsArgs& p = a.r;
+  extern __shared__ u32x4 xs[];  // [B][round_up(nch, CB) * 64] vectors
+  const int lane = threadIdx.x & (kWave - 1);
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+
+  const int item = blockIdx.x * WAVES + wave;
+  int row[R];
+  bool on[R];
+  const u32x4* w = p.w;
+  int which = 0, d = 0;
+  long long pos = 0;
+  if (MODE == kProjQkv) {
+    const int pairs = p.N / 2;
+    which = item / pairs;
+    const int i = item - which * pairs;
+    const int head = i / a.half;
+    d = i - head * a.half;
+    on[0] = on[1] = which < 3;
+    row[0] = on[0] ? head * 2 * a.half + d : 0;
+    row[1] = on[0] ? row[0] + a.half : 0;
+    w = which == 1 ? a.wk : which == 2 ? a.wv : p.w;
+    pos = *a.pos;
+  } else {
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+      on[r] = item * R + r < p.N;
+      row[r] = on[r] ? item * R + r : p.N - 1;
+    }
+  }
+  const bool pos_ok = pos >= 0 && pos < (long long)a.max_len;
+
+  // x goes out first, the weights behind it, and only x is waited for before the barrier (see rows_kernel)
+  u32x4 wv[R][CB];
+  constexpr int kXPreAll = (B * 512 + kThreads - 1) / kThreads;
+  constexpr int kXPre = kXPreAll < 4 ? kXPreAll : 4;
+  const int nchv = (p.nch + CB - 1) / CB * CB * kWave;
+  u32x4 xpre[kXPre];
+#pragma unroll
+  for (int k = 0; k < kXPre; k++) {
+    const int i = threadIdx.x + k * kThreads;
+    const int b = B == 1 ? 0 : i / nchv, v = i - b * nchv;
+    xpre[k] = zero4();
+    if (i < B * nchv && b < p.nb && v < p.row_vecs) xpre[k] = p.x[(size_t)b * p.row_vecs + v];
+  }
+  rows_issue<R, CB, FULL>(w, row, on, 0, p, lane, wv);
+#pragma unroll
+  for (int k = 0; k < kXPre; k++) {
+    const int i = threadIdx.x + k * kThreads;
+    if (i < B * nchv) xs[i] = xpre[k];
+  }
+  for (int i = threadIdx.x + kXPre * kThreads; i < B * nchv; i += kThreads) {
+    const int b = i / nchv, v = i - b * nchv;
+    u32x4 val = zero4();
+    if (b < p.nb && v < p.row_vecs) val = p.x[(size_t)b * p.row_vecs + v];
+    xs[i] = val;
+  }
+  __syncthreads();
+  if (p.norm_w) {
+    __shared__ float s_scale[B];
+    for (int b = wave; b < B; b += WAVES) {
+      float ss = 0.f;
+      for (int v = lane; v < p.row_vecs; v += kWave) ss = vec_sumsq<DT>(xs[b * nchv + v], ss);
+      ss = wave_sum(ss);
+      if (lane == 0) s_scale[b] = rsqrtf(ss / (float)p.K + p.norm_eps);
+    }
+    __syncthreads();
+    for (int i = threadIdx.x; i < B * nchv; i += kThreads) {
+      const int b = B == 1 ? 0 : i / nchv, v = i - b * nchv;
+      if (b < p.nb && v < p.row_vecs) xs[i] = vec_norm_apply<DT>(xs[i], s_scale[b], p.norm_w[v]);
+    }
+    __syncthreads();
+  }
+
+  float g[R][B];
+  rows_dot<DT, B, R, CB, FULL, true>(w, row, on, xs, p.x, p, lane, wv, true, g);
+
+  if (lane != 0) return;
+  if (MODE == kProjQkv) {
+    if (!on[0]) return;
+    if (which == 0 || which == 1) {
+      const st* ct = (const st*)a.cos_t + (size_t)(pos_ok ? pos : 0) * 2 * a.half;
+      const st* sn = (const st*)a.sin_t + (size_t)(pos_ok ? pos : 0) * 2 * a.half;
+      const float c0 = DT::tof(ct[d]), c1 = DT::tof(ct[d + a.half]), s0 = DT::tof(sn[d]), s1 = DT::tof(sn[d + a.half]);
+#pragma unroll
+      for (int b = 0; b < B; b++) {
+        const float lo = g[0][b], hi = g[1][b];
+        g[0][b] = lo * c0 - hi * s0;
+        g[1][b] = hi * c1 + lo * s1;
+      }
+    }
+#pragma unroll
+    for (int r = 0; r < R; r++)
+#pragma unroll
+      for (int b = 0; b < B; b++)
+        if (b < p.nb) {
+          if (which == 0) a.q_out[(size_t)b * p.N + row[r]] = g[r][b];
+          else if (pos_ok) {
+            const int head = row[r] / (2 * a.half), e = row[r] - head * 2 * a.half;
+            st* cache = (st*)(which == 1 ? a.k_cache : a.v_cache);
+            cache[(((size_t)b * a.heads + head) * a.max_len + (size_t)pos) * 2 * a.half + e] = DT::fromf(g[r][b]);
+          }
+        }
+  } else {
+    st* out = (st*)p.zt_out;
+#pragma unroll
+    for (int r = 0; r < R; r++)
+      if (on[r]) {
+#pragma unroll
+        for (int b = 0; b < B; b++)
+          if (b < p.nb) {
+            const size_t o = (size_t)b * p.N + row[r];
+            out[o] = DT::fromf(MODE == kProjAdd ? g[r][b] + DT::tof(((const st*)a.residual)[o]) : g[r][b]);
+          }
+      }
+  }
+}
+
+struct AttnArgs {
+  const float* q;        // (nb, heads * head_dim) fp32
+  const u32x4* k;        // (nb, heads, max_len, head_dim) dtype
+  const u32x4* v;
+  const int64_t* pos;    // slots 0..pos take part; outside [0, max_len) the output is NaN
+  void* out;             // (nb, heads * head_dim) dtype
+  float scale;           // log2(e) / sqrt(head_dim)
+  int max_len;
+};
+
+// One workgroup of sixteen waves per (batch row, head).  A slot's head_dim elements sit in LPS lanes of one 16-byte vector
+// each, so a wave holds 64 / LPS slots side by side and the workgroup 16 * 64 / LPS; every lane group runs its own online
+// softmax over the slots it meets, U slots a turn with the loads of K and V of all of them in flight together (256 slots of 128
+// 16-bit elements are one turn), and the groups' results are merged at the end, in a fixed order.  What bounds it is three
+// dependent memory trips (position, q, K and V), not the bytes: 131 KiB a head at 256 slots.
+template <class DT, int LPS>
+__global__ __launch_bounds__(1024) void attn_decode_kernel(AttnArgs p) {
+  typedef typename DT::st st;
+  constexpr int VEC = DT::VEC, HD = LPS * VEC, G = kWave / LPS, WAVES = 16, S = WAVES * G, U = 4;
+  __shared__ float s_acc[WAVES][HD];
+  __shared__ float s_m[WAVES], s_l[WAVES];
+  const int lane = threadIdx.x & (kWave - 1);
+  const int wave = threadIdx.x >> 6;
+  const int sub = lane % LPS;
+  const int slot0 = wave * G + lane / LPS;
+  const long long pos = *p.pos;
+  const int n = pos >= 0 && pos < (long long)p.max_len ? (int)pos + 1 : 0;
+  const u32x4* kb = p.k + (size_t)blockIdx.x * p.max_len * LPS + sub;
+  const u32x4* vb = p.v + (size_t)blockIdx.x * p.max_len * LPS + sub;
+  float q[VEC];
+#pragma unroll
+  for (int e = 0; e < VEC; e++) q[e] = p.q[(size_t)blockIdx.x * HD + sub * VEC + e] * p.scale;
+
+  auto elem = [](u32x4 x, int e) {
+    if constexpr (sizeof(st) == 4) return __uint_as_float(x[e]);
+    else return DT::tof((st)(x[e / 2] >> (16 * (e & 1))));
+  };
+  float m = -INFINITY, l = 0.f, acc[VEC];
+#pragma unroll
+  for (int e = 0; e < VEC; e++) acc[e] = 0.f;
+  for (int s0 = 0; s0 < n; s0 += S * U) {
+    u32x4 kv[U], vv[U];
+#pragma unroll
+    for (int u = 0; u < U; u++) kv[u] = kb[(size_t)min(s0 + u * S + slot0, n - 1) * LPS];
+#pragma unroll
+    for (int u = 0; u < U; u++) vv[u] = vb[(size_t)min(s0 + u * S + slot0, n - 1) * LPS];
+    float sc[U], mu = m;
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+      float t = 0.f;
+#pragma unroll
+      for (int e = 0; e < VEC; e++) t = fmaf(q[e], elem(kv[u], e), t);
+#pragma unroll
+      for (int o = 1; o < LPS; o <<= 1) t += __shfl_xor(t, o, kWave);
+      sc[u] = s0 + u * S + slot0 < n ? t : -INFINITY;
+      mu = fmaxf(mu, sc[u]);
+    }
+    const float base = mu == -INFINITY ? 0.f : mu;  // a group that has met no slot yet keeps zeros
+    const float keep = exp2f(m - base);
+    l *= keep;
+#pragma unroll
+    for (int e = 0; e < VEC; e++) acc[e] *= keep;
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+      const bool in = s0 + u * S + slot0 < n;
+      const float pr = exp2f(sc[u] - base);
+      l += in ? pr : 0.f;
+#pragma unroll
+      for (int e = 0; e < VEC; e++) acc[e] = in ? fmaf(pr, elem(vv[u], e), acc[e]) : acc[e];
+    }
+    m = mu;
+  }
+  // the wave's groups, then the waves
+  float mw = m;
+#pragma unroll
+  for (int o = LPS; o < kWave; o <<= 1) mw = fmaxf(mw, __shfl_xor(mw, o, kWave));
+  const float f = exp2f(m - (mw == -INFINITY ? 0.f : mw));
+  l *= f;
+#pragma unroll
+  for (int o = LPS; o < kWave; o <<= 1) l += __shfl_xor(l, o, kWave);
+#pragma unroll
+  for (int e = 0; e < VEC; e++) {
+    acc[e] *= f;
+#pragma unroll
+    for (int o = LPS; o < kWave; o <<= 1) acc[e] += __shfl_xor(acc[e], o, kWave);
+  }
+  if (lane < LPS) {
+#pragma unroll
+    for (int e = 0; e < VEC; e++) s_acc[wave][sub * VEC + e] = acc[e];
+    if (lane == 0) { s_m[wave] = mw; s_l[wave] = l; }
+  }
+  __syncthreads();
+  for (int c = threadIdx.x; c < HD; c += WAVES * kWave) {
+    float mt = -INFINITY;
+#pragma unroll
+    for (int i = 0; i < WAVES; i++) mt = fmaxf(mt, s_m[i]);
+    const float base = mt == -INFINITY ? 0.f : mt;
+    float num = 0.f, den = 0.f;
+#pragma unroll
+    for (int i = 0; i < WAVES; i++) {
+      const float e = exp2f(s_m[i] - base);
+      num = fmaf(e, s_acc[i][c], num);
+      den = fmaf(e, s_l[i], den);
+    }
+    ((st*)p.out)[(size_t)blockIdx.x * HD + c] = DT::fromf(num / den);
+  }
+}
+
+}  // namespace cats

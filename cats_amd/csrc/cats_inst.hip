@@ -263,7 +263,53 @@ hipError_t launch_fused_b(int grid, const FusedArgs& a, hipStream_t stream) {
   return hipErrorInvalidValue;
 }
 
+template <class DT, int B, int MODE>
+hipError_t launch_proj_one(const ProjArgs& a, hipStream_t stream) {
+  constexpr int WAVES = WavesFor<B>::value;
+  const bool full = a.r.K % (kWave * DT::VEC * kProjCB) == 0;
+  auto kern = full ? proj_kernel<DT, B, kProjCB, true, MODE, WAVES> : proj_kernel<DT, B, kProjCB, false, MODE, WAVES>;
+  const int pairs = MODE == kProjQkv ? a.r.N / 2 * 3 : (a.r.N + 1) / 2;
+  const size_t lds = proj_lds_bytes(B, a.r.nch);
+  if (hipError_t e = ensure_dynamic_lds((const void*)kern, lds); e != hipSuccess) return e;
+  return launch_kernel(kern, dim3((pairs + WAVES - 1) / WAVES), dim3(WAVES * kWave), lds, stream, a);
+}
+
+template <class DT, int B>
+hipError_t launch_proj_b(int mode, const ProjArgs& a, hipStream_t stream) {
+  switch (mode) {
+    case kProjPlain: return launch_proj_one<DT, B, kProjPlain>(a, stream);
+    case kProjAdd: return launch_proj_one<DT, B, kProjAdd>(a, stream);
+    case kProjQkv: return launch_proj_one<DT, B, kProjQkv>(a, stream);
+  }
+  return hipErrorInvalidValue;
+}
+
 }  // namespace
+
+template <>
+hipError_t launch_proj<CATS_DT>(int mode, int bt, const ProjArgs& a, hipStream_t stream) {
+  switch (bt) {
+    case 1: return launch_proj_b<CATS_DT, 1>(mode, a, stream);
+    case 2: return launch_proj_b<CATS_DT, 2>(mode, a, stream);
+    case 4: return launch_proj_b<CATS_DT, 4>(mode, a, stream);
+    case 8: return launch_proj_b<CATS_DT, 8>(mode, a, stream);
+  }
+  return hipErrorInvalidValue;
+}
+
+template <>
+hipError_t launch_attn<CATS_DT>(int blocks, int head_dim, const AttnArgs& a, hipStream_t stream) {
+  void (*kern)(AttnArgs) = nullptr;
+  switch (head_dim / CATS_DT::VEC) {  // lanes per cache slot
+    case 2: kern = attn_decode_kernel<CATS_DT, 2>; break;
+    case 4: kern = attn_decode_kernel<CATS_DT, 4>; break;
+    case 8: kern = attn_decode_kernel<CATS_DT, 8>; break;
+    case 16: kern = attn_decode_kernel<CATS_DT, 16>; break;
+    case 32: kern = attn_decode_kernel<CATS_DT, 32>; break;
+  }
+  if (!kern) return hipErrorInvalidValue;
+  return launch_kernel(kern, dim3(blocks), dim3(1024), 0, stream, a);
+}
 
 template <>
 hipError_t launch_fused<CATS_DT>(int bt, int grid, int stage, const FusedArgs& a, const ReduceArgs& r, hipStream_t stream) {

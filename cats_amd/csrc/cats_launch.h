@@ -2,6 +2,7 @@
 // (cats_inst.hip, compiled once per dtype).
 #pragma once
 #include <hip/hip_runtime.h>
+#include "cats_decode.h"
 #include "cats_down.h"
 #include "cats_down_mma.h"
 #include "cats_gemv_mma.h"
@@ -57,5 +58,14 @@ hipError_t launch_down_mma(bool zf32, const DownArgs& a, hipStream_t stream);
 // Single-pass MLP for 1 or 2 batch rows.  stage: 0 = both launches, 1 = streaming kernel only, 2 = reduction only.
 template <class DT>
 hipError_t launch_fused(int bt, int grid, int stage, const FusedArgs& a, const ReduceArgs& r, hipStream_t stream);
+
+// Projections and attention of one decode step (cats_decode.h).  mode is a ProjMode; lds_bytes of x have to fit (proj_lds_bytes).
+constexpr size_t kProjMaxLds = 128 * 1024;
+constexpr int kProjCB = 8;
+inline size_t proj_lds_bytes(int bt, int nch) { return (size_t)bt * ((nch + kProjCB - 1) / kProjCB * kProjCB) * kWave * sizeof(u32x4); }
+template <class DT>
+hipError_t launch_proj(int mode, int bt, const ProjArgs& a, hipStream_t stream);
+template <class DT>
+hipError_t launch_attn(int blocks, int head_dim, const AttnArgs& a, hipStream_t stream);
 
 }  // namespace cats

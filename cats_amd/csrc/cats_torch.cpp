@@ -451,6 +451,69 @@ std::tuple<at::Tensor, at::Tensor, at::Tensor> cats_mlp_stats_op(const at::Tenso
   return {out, flags, count};
 }
 
+// x . w^T (+ residual): x (B, K), w (N, K); norm_weight: x is given before its RMS norm.
+at::Tensor cats_linear_op(const at::Tensor& x, const c10::optional<at::Tensor>& norm_weight, const double eps, const at::Tensor& w) {
+  check_dev(x, "x");
+  const int B = batch_rows(x, "cats_linear");
+  const int64_t K = x.size(-1), N = w.size(0);
+  check_weight(w, x, N, K, "w");
+  const bool norm = norm_weight.has_value() && norm_weight->defined();
+  if (norm) {
+    check_dev(*norm_weight, "norm_weight");
+    TORCH_CHECK(norm_weight->scalar_type() == x.scalar_type() && norm_weight->numel() == K && norm_weight->device() == x.device(),
+                "flash_gemv.cats_linear: norm_weight must be a (K,) tensor of x's dtype on x's device");
+  }
+  std::vector<int64_t> shape(x.sizes().begin(), x.sizes().end());
+  shape.back() = N;
+  at::Tensor out = at::empty(shape, x.options());
+  check_status(cats_linear(x.data_ptr(), norm ? norm_weight->data_ptr() : nullptr, (float)eps, w.data_ptr(), nullptr, out.data_ptr(), B, (int)K,
+                           (int)N, dtype_code(x), current_stream(x)),
+               "cats_linear");
+  return out;
+}
+
+// h + attention(x): one new token per row, caches updated in place.  norm_weight: x is h, given before its norm.
+at::Tensor cats_attention_step_op(const at::Tensor& h, const at::Tensor& x, const c10::optional<at::Tensor>& norm_weight, const double eps,
+                                  const at::Tensor& wq, const at::Tensor& wk, const at::Tensor& wv, const at::Tensor& wo, at::Tensor& k_cache,
+                                  at::Tensor& v_cache, const at::Tensor& cos_table, const at::Tensor& sin_table, const at::Tensor& position) {
+  check_dev(h, "h");
+  check_dev(x, "x");
+  const int B = batch_rows(h, "cats_attention_step");
+  const int64_t H = h.size(-1);
+  TORCH_CHECK(x.sizes() == h.sizes() && x.scalar_type() == h.scalar_type() && x.device() == h.device(), "flash_gemv.cats_attention_step: x must be like h");
+  for (const at::Tensor* w : {&wq, &wk, &wv, &wo}) check_weight(*w, h, H, H, "a projection");
+  const bool norm = norm_weight.has_value() && norm_weight->defined();
+  if (norm) {
+    check_dev(*norm_weight, "norm_weight");
+    TORCH_CHECK(norm_weight->scalar_type() == h.scalar_type() && norm_weight->numel() == H && norm_weight->device() == h.device(),
+                "flash_gemv.cats_attention_step: norm_weight must be a (H,) tensor of h's dtype on h's device");
+  }
+  for (const at::Tensor* c : {(const at::Tensor*)&k_cache, (const at::Tensor*)&v_cache}) {
+    check_dev(*c, "a cache");
+    TORCH_CHECK(c->dim() == 4 && c->size(0) == B && c->size(1) * c->size(3) == H && c->sizes() == k_cache.sizes() &&
+                    c->scalar_type() == h.scalar_type() && c->device() == h.device(),
+                "flash_gemv.cats_attention_step: the caches must be (B, heads, max_len, head_dim) in h's dtype, got ", c->sizes());
+  }
+  const int64_t heads = k_cache.size(1), max_len = k_cache.size(2), hd = k_cache.size(3);
+  for (const at::Tensor* t : {&cos_table, &sin_table}) {
+    check_dev(*t, "a rotary table");
+    TORCH_CHECK(t->dim() == 2 && t->size(0) == max_len && t->size(1) == hd && t->scalar_type() == h.scalar_type() && t->device() == h.device(),
+                "flash_gemv.cats_attention_step: the rotary tables must be (max_len, head_dim) in h's dtype");
+  }
+  check_dev(position, "position");
+  TORCH_CHECK(position.scalar_type() == at::kLong && position.numel() == 1 && position.device() == h.device(),
+              "flash_gemv.cats_attention_step: position must be one int64 on h's device");
+  at::Tensor out = at::empty_like(h);
+  at::Tensor q = at::empty({B, H}, h.options().dtype(at::kFloat));
+  at::Tensor att = at::empty({B, H}, h.options());
+  check_status(cats_attention_step(h.data_ptr(), x.data_ptr(), norm ? norm_weight->data_ptr() : nullptr, (float)eps, wq.data_ptr(), wk.data_ptr(),
+                                   wv.data_ptr(), wo.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(), cos_table.data_ptr(), sin_table.data_ptr(),
+                                   position.data_ptr<int64_t>(), q.data_ptr<float>(), att.data_ptr(), out.data_ptr(), B, (int)H, (int)heads,
+                                   (int)max_len, dtype_code(h), current_stream(h)),
+               "cats_attention_step");
+  return out;
+}
+
 }  // namespace
 
 TORCH_LIBRARY(flash_gemv, m) {
@@ -478,4 +541,7 @@ TORCH_LIBRARY(flash_gemv, m) {
   m.def("cats_mlp_norm_residual_norm", cats_mlp_norm_residual_norm_op);
   m.def("cats_up_down", cats_up_down_op);
   m.def("cats_mlp_stats", cats_mlp_stats_op);
+  // the rest of a decode step
+  m.def("cats_linear", cats_linear_op);
+  m.def("cats_attention_step", cats_attention_step_op);
 }

@@ -6,7 +6,8 @@ its tree spells out: decoder layer order ``h += attn(input_layernorm(h)); h += m
 (ugly_utils.py:1016-1057), rotate-half RoPE and eager attention with an fp32 softmax
 (experiments/models/sparse_mistral/sparse_silu.py:280-312, 756-832), and the timing rule of the patched
 ``generate()``: tokens 2..N only, tok/s = (N - 1) / elapsed (experiments/time_util_nofile.py:2902-2904, 2984-2994).
-Everything except the MLP uses stock PyTorch-ROCm ops, so dense-vs-CATS differences isolate the MLP path.
+Outside the MLP every mode runs the same code -- stock PyTorch-ROCm ops for a prompt, the projection and attention kernels of
+``cats_decode.h`` for one new token per row (``LlamaDecoder._takes_step``) -- so dense-vs-CATS differences isolate the MLP path.
 The decode step is shape-static (fixed-size KV cache, position kept on the device) so it can be replayed from a
 HIP graph.
 """
@@ -37,6 +38,21 @@ class DecoderConfig:
     @property
     def head_dim(self):
         return self.hidden_size // self.num_heads
+
+
+def _bare(module, cls):
+    """`module` is a plain `cls`: calling it does nothing besides the class's own forward."""
+    return (type(module) is cls and "forward" not in module.__dict__ and not module._forward_hooks and not module._forward_pre_hooks
+            and not module._backward_hooks and not module._backward_pre_hooks)
+
+
+def _nothing_watches():
+    """No autograd, tracing, autocast, transform or mode is at work that has to see the single torch operations."""
+    return not (torch.is_grad_enabled() or torch.is_autocast_enabled("cuda") or torch.jit.is_tracing() or torch.compiler.is_compiling()
+                or torch._C._len_torch_dispatch_stack() or torch._C._len_torch_function_stack()
+                or torch._C._functorch.peek_interpreter_stack() is not None or torch.autograd.forward_ad._current_level >= 0
+                or nn.modules.module._global_forward_hooks or nn.modules.module._global_forward_pre_hooks
+                or nn.modules.module._global_backward_hooks or nn.modules.module._global_backward_pre_hooks)
 
 
 class RMSNorm(nn.Module):
@@ -104,13 +120,43 @@ class DecoderLayer(nn.Module):
         module that will consume this layer's output; with fuse_next_norm the return value is (h, next_norm(h))."""
         if normed is None:
             normed = self.input_layernorm(h)
-        h = h + self.self_attn(normed, cos, sin, positions, mask)
+        return self._mlp_tail(h + self.self_attn(normed, cos, sin, positions, mask), next_norm)
+
+    def _mlp_tail(self, h, next_norm):
         if self.fuse_norm_residual and h.shape[1] == 1 and self.mlp.is_profile and self.mlp.sp_method == 3:
             n = self.post_attention_layernorm
             if self.fuse_next_norm and next_norm is not None:
                 return self.mlp.forward_norm_residual_norm(h, n.weight, n.eps, next_norm.weight, next_norm.eps)
             return self.mlp.forward_norm_residual(h, n.weight, n.eps)
         return h + self.mlp(self.post_attention_layernorm(h))
+
+    def _bare_for(self, dtype, device, tables, batch):
+        """Whether the kernels of a decode step may stand for this layer's input norm and attention."""
+        at, n = self.self_attn, self.input_layernorm
+        if not (_bare(self, DecoderLayer) and _bare(at, Attention) and _bare(n, RMSNorm) and at.k_cache is not None):
+            return False
+        H = at.cfg.hidden_size
+        lin = (at.q_proj, at.k_proj, at.v_proj, at.o_proj)
+        if not all(_bare(m, nn.Linear) and m.bias is None and m.weight.shape == (H, H) for m in lin) or n.weight.shape != (H,):
+            return False
+        shape = (batch, at.cfg.num_heads, *tables[0].shape)
+        return (all(_plain(t, dtype, device) for t in (*(m.weight for m in lin), n.weight, at.k_cache, at.v_cache))
+                and at.k_cache.shape == shape and at.v_cache.shape == shape and at.cfg.max_len == shape[2])
+
+    def _step(self, h, normed, cos_table, sin_table, positions, next_norm):
+        """forward() for one new token per row, the input norm and attention as kernels."""
+        import flash_gemv  # noqa: F401  (raises if the HIP op library is missing)
+
+        at, n = self.self_attn, self.input_layernorm
+        h = torch.ops.flash_gemv.cats_attention_step(h, h if normed is None else normed, n.weight if normed is None else None, n.eps,
+                                                     at.q_proj.weight, at.k_proj.weight, at.v_proj.weight, at.o_proj.weight,
+                                                     at.k_cache, at.v_cache, cos_table, sin_table, positions)
+        return self._mlp_tail(h, next_norm)
+
+
+def _plain(t, dtype, device):
+    """A tensor whose memory a kernel may read as it lies."""
+    return type(t) in (torch.Tensor, nn.Parameter) and t.dtype == dtype and t.device == device and t.is_contiguous() and t.data_ptr() % 16 == 0
 
 
 class LlamaDecoder(nn.Module):
@@ -143,6 +189,8 @@ class LlamaDecoder(nn.Module):
         """tokens (B, q) int64; positions (q,) int64 -> logits (B, q, vocab).  Causal over cache slots <= position."""
         cfg = self.cfg
         h = self.embed_tokens(tokens)
+        if self._takes_step(h, positions):
+            return self._forward_step(h, positions)
         cos, sin = self.cos_table[positions], self.sin_table[positions]
         slots = torch.arange(cfg.max_len, device=tokens.device)
         mask = torch.zeros(positions.numel(), cfg.max_len, dtype=self.dtype, device=tokens.device)
@@ -153,6 +201,37 @@ class LlamaDecoder(nn.Module):
             out = layer(h, cos, sin, positions, mask, normed, next_norm)
             h, normed = out if isinstance(out, tuple) else (out, None)
         return self.lm_head(normed if normed is not None else self.norm(h))
+
+    def _takes_step(self, h, positions):
+        """Whether the kernels of cats_decode.h take this call: one new token for each of up to eight rows on the GPU, heads of 2 to
+        32 (a power of two) 16-byte vectors, nothing that has to see the modules or torch operations they stand for.  With more
+        rows, or rows whose x does not fit on chip, the batch is matrix work and stays with torch's products."""
+        if not (h.is_cuda and type(h) is torch.Tensor and h.dim() == 3 and h.shape[1] == 1 and 1 <= h.shape[0] <= 8 and _nothing_watches()):
+            return False
+        if not (type(positions) is torch.Tensor and positions.dtype == torch.int64 and positions.shape == (1,) and positions.device == h.device):
+            return False
+        B, cfg, esz = h.shape[0], self.cfg, h.element_size()
+        lanes, odd = divmod(cfg.head_dim * esz, 16)
+        rows = 1 << (B - 1).bit_length()
+        if (h.dtype not in (torch.float16, torch.bfloat16, torch.float32) or odd or lanes not in (2, 4, 8, 16, 32)
+                or cfg.head_dim * cfg.num_heads != cfg.hidden_size or h.shape[2] != cfg.hidden_size
+                or rows * -(-cfg.hidden_size * esz // 8192) * 8192 > 128 * 1024):
+            return False
+        tables = (self.cos_table, self.sin_table)
+        return (all(_plain(t, h.dtype, h.device) and t.shape == (cfg.max_len, cfg.head_dim) for t in tables) and h.is_contiguous()
+                and _bare(self.norm, RMSNorm) and _plain(self.norm.weight, h.dtype, h.device) and self.norm.weight.shape == (cfg.hidden_size,)
+                and _bare(self.lm_head, nn.Linear) and self.lm_head.bias is None and _plain(self.lm_head.weight, h.dtype, h.device)
+                and all(type(layer) is DecoderLayer and layer._bare_for(h.dtype, h.device, tables, B) for layer in self.layers))
+
+    def _forward_step(self, h, positions):
+        normed = None
+        for i, layer in enumerate(self.layers):
+            next_norm = self.layers[i + 1].input_layernorm if i + 1 < len(self.layers) else self.norm
+            out = layer._step(h, normed, self.cos_table, self.sin_table, positions, next_norm)
+            h, normed = out if isinstance(out, tuple) else (out, None)
+        last = self.norm
+        return torch.ops.flash_gemv.cats_linear(h if normed is None else normed, last.weight if normed is None else None, last.eps,
+                                                self.lm_head.weight)
 
     # ---- MLP mode switches ----
     def set_mlp_mode(self, mode: str):

@@ -210,6 +210,25 @@ int cats_mlp_rowmajor_down(const void* x, const void* wgate, const void* wup, co
 int cats_mlp_noalloc(const void* x, const void* wgate, const void* wup, const void* wdown_t, void* y_out,
                      int B, int H, int I, int dtype, float threshold, void* stream);
 
+/* out = x . w^T (+ residual) for 1..8 rows: x (B,K), w (N,K) as nn.Linear holds it, residual and out (B,N), all in dtype.
+ * norm_weight (K) != NULL: x is given before its RMS norm, which is applied while x is staged (the norm of
+ * cats_mlp_norm_residual).  One rounding, after the residual.  Needs B * K * sizeof(dtype), B rounded up to a power of two and
+ * the rows to 8 KiB, to be at most 128 KiB.  The output head and the attention's output projection of a decode step. */
+int cats_linear(const void* x, const void* norm_weight, float eps, const void* w, const void* residual, void* out,
+                int B, int K, int N, int dtype, void* stream);
+
+/* The attention half of a decoder layer for one new token per row, 1..8 rows, in three launches:
+ *   q, k, v = x . W{q,k,v}^T (x normed first if norm_weight is given), rotate-half rotary embedding of q and k at *position, k and v
+ *   stored into slot *position of the caches, softmax(q . K^T / sqrt(head_dim)) . V over slots 0..*position, out = h + att . Wo^T.
+ * h, x, out (B,H); w* (H,H); caches (B, heads, max_len, head_dim); cos / sin tables (max_len, head_dim); all in dtype.  position: one
+ * device word for all rows; outside [0, max_len) nothing is stored and out is NaN.  q_scratch B*H floats, attn_scratch B*H of dtype.
+ * head_dim has to be 2..32 (a power of two) 16-byte vectors; the limit on B and H is that of cats_linear.
+ * The conventions are those of the reference's decoder layer (experiments/models/sparse_mistral/sparse_silu.py:280-312, 756-832). */
+int cats_attention_step(const void* h, const void* x, const void* norm_weight, float eps, const void* wq, const void* wk,
+                        const void* wv, const void* wo, void* k_cache, void* v_cache, const void* cos_table, const void* sin_table,
+                        const int64_t* position, float* q_scratch, void* attn_scratch, void* out, int B, int H, int heads,
+                        int max_len, int dtype, void* stream);
+
 /* One launch of cats_mlp(y_out mode) alone, for per-kernel timing and profiling: stage 1 = the streaming launch (gate, up
  * and, for 1..2 rows, down into per-workgroup partial sums), stage 2 = the launch that finishes y from what stage 1 left in
  * the workspace.  Calling stage 1 then stage 2 with the same arguments is cats_mlp.  Not in the reference. */

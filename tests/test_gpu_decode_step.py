@@ -1,0 +1,140 @@
+"""The projection and attention kernels of a decode step against the torch operations they stand for, in float64 on the CPU."""
+import math
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+EPS = {torch.float16: 2 ** -11, torch.bfloat16: 2 ** -8, torch.float32: 2 ** -24}
+
+
+def _randn(g, *shape, dtype, scale=1.0):
+    return (torch.randn(*shape, generator=g) * scale).to(dtype)
+
+
+def _check(got, want, dtype, terms):
+    """Rounding of the stored value, and fp32 sums of `terms` products of the size of the result's own scale."""
+    tol = (2 * EPS[dtype] + terms * 2 ** -24) * (want.abs() + want.std() + 1e-3)
+    assert bool((got.cpu().double() - want).abs().le(tol).all()), float(((got.cpu().double() - want).abs() / tol).max())
+
+
+@pytest.mark.parametrize("B,K,N,dtype", [
+    (1, 8, 1, torch.float16), (1, 4096, 4096, torch.float16), (1, 4096, 1001, torch.bfloat16), (2, 264, 33, torch.float16),
+    (3, 1000, 77, torch.bfloat16), (4, 4096, 515, torch.float16), (8, 3080, 130, torch.bfloat16), (1, 8200, 19, torch.float16),
+    (1, 516, 40, torch.float32), (4, 4096, 64, torch.float32), (8, 1028, 9, torch.float32)])
+@pytest.mark.parametrize("norm", [False, True])
+def test_linear(B, K, N, dtype, norm):
+    import flash_gemv  # noqa: F401
+
+    g = torch.Generator().manual_seed(B + K + N)
+    x, w, nw = _randn(g, B, 1, K, dtype=dtype, scale=2.0), _randn(g, N, K, dtype=dtype, scale=0.02), (1 + 0.1 * torch.randn(K, generator=g)).to(dtype)
+    out = torch.ops.flash_gemv.cats_linear(x.cuda(), nw.cuda() if norm else None, 1e-5, w.cuda())
+    xr = x.double()
+    if norm:
+        xr = (nw.double() * (xr * torch.rsqrt(xr.pow(2).mean(-1, keepdim=True) + 1e-5)).to(dtype).double()).to(dtype).double()
+    want = xr @ w.double().t()
+    if norm:  # a normed value that sits on a rounding tie may go either way: half a step of each term, added as random signs
+        tie = 4 * EPS[dtype] * (xr.pow(2) @ w.double().pow(2).t()).sqrt()
+        assert bool(((out.cpu().double() - want).abs() <= tie + (2 * EPS[dtype] + K * 2 ** -24) * (want.abs() + want.std() + 1e-3 if N > 1 else 1)).all())
+    else:
+        _check(out, want, dtype, K) if N > 1 else torch.testing.assert_close(out.cpu().double(), want, rtol=4 * EPS[dtype], atol=1e-3)
+
+
+def _reference(h, x, wq, wk, wv, wo, kc, vc, cos, sin, pos):
+    B, heads, _, hd = kc.shape
+    shp = (B, heads, hd)
+    d = lambda t: t.double()
+    q, k, v = (d(x).view(B, -1) @ d(w).t() for w in (wq, wk, wv))
+    q, k, v = q.view(shp), k.view(shp), v.view(shp)
+    half = lambda t: torch.cat((-t[..., hd // 2:], t[..., : hd // 2]), -1)
+    q, k = (t * d(cos)[pos] + half(t) * d(sin)[pos] for t in (q, k))
+    kc, vc = kc.clone(), vc.clone()
+    kc[:, :, pos], vc[:, :, pos] = k.to(kc.dtype), v.to(vc.dtype)
+    att = torch.softmax((d(kc[:, :, : pos + 1]) @ q.unsqueeze(-1)).squeeze(-1) / math.sqrt(hd), -1)
+    o = (att.unsqueeze(-2) @ d(vc[:, :, : pos + 1])).reshape(B, -1)
+    return d(h).view(B, -1) + o @ d(wo).t(), kc, vc
+
+
+@pytest.mark.parametrize("B,heads,hd,max_len,pos,dtype", [
+    (1, 2, 16, 4, 0, torch.float16), (1, 3, 32, 40, 39, torch.bfloat16), (2, 4, 64, 512, 63, torch.float16), (1, 2, 128, 300, 255, torch.float16),
+    (4, 8, 128, 512, 256, torch.bfloat16), (8, 2, 128, 700, 699, torch.float16), (3, 2, 256, 130, 100, torch.bfloat16),
+    (1, 4, 128, 1100, 1030, torch.float32), (2, 3, 8, 33, 32, torch.float32), (1, 32, 128, 512, 480, torch.float16)])
+def test_attention_step(B, heads, hd, max_len, pos, dtype):
+    import flash_gemv  # noqa: F401
+
+    H = heads * hd
+    g = torch.Generator().manual_seed(H + pos)
+    h, x = _randn(g, B, 1, H, dtype=dtype, scale=2.0), _randn(g, B, 1, H, dtype=dtype)
+    ws = [_randn(g, H, H, dtype=dtype, scale=1 / math.sqrt(H)) for _ in range(4)]
+    kc, vc = (_randn(g, B, heads, max_len, hd, dtype=dtype) for _ in range(2))
+    kc[:, :, pos:], vc[:, :, pos:] = float("inf"), float("nan")   # what has not been written yet takes no part
+    ang = torch.outer(torch.arange(max_len).float(), 1.0 / (10000.0 ** (torch.arange(0, hd, 2).float() / hd)))
+    emb = torch.cat((ang, ang), -1)
+    cos, sin = emb.cos().to(dtype), emb.sin().to(dtype)
+    kd, vd = kc.cuda(), vc.cuda()
+    p = torch.tensor([pos], device="cuda")
+    out = torch.ops.flash_gemv.cats_attention_step(h.cuda(), x.cuda(), None, 0.0, *[w.cuda() for w in ws], kd, vd, cos.cuda(), sin.cuda(), p)
+    want, kw, vw = _reference(h, x, *ws, kc, vc, cos, sin, pos)
+    # attention is rounded once before the output projection: half a step of each of its H terms, added as random signs
+    _check(out.view(B, H), want, dtype, 4 * H)
+    _check(kd[:, :, pos], kw[:, :, pos].double(), dtype, 2 * H)
+    _check(vd[:, :, pos], vw[:, :, pos].double(), dtype, 2 * H)
+    assert torch.equal(kd[:, :, :pos].cpu(), kc[:, :, :pos]) and torch.equal(vd[:, :, :pos].cpu(), vc[:, :, :pos])
+    assert torch.equal(kd[:, :, pos + 1:].cpu(), kc[:, :, pos + 1:])
+    for bad in (-1, max_len):   # a position outside the cache stores nothing
+        before = kd.clone()
+        out = torch.ops.flash_gemv.cats_attention_step(h.cuda(), x.cuda(), None, 0.0, *[w.cuda() for w in ws], kd, vd, cos.cuda(), sin.cuda(),
+                                                       torch.tensor([bad], device="cuda"))
+        assert bool(out.isnan().all()) and torch.equal(kd, before)
+
+
+@pytest.mark.parametrize("B,mode", [(1, "cats_fused_next"), (4, "cats_fused_next"), (2, "cats_fused"), (3, "cats"), (1, "dense")])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_step_matches_torch_operations(B, mode, dtype):
+    """The model's step through the kernels and through the torch operations (a hook on the output head keeps it there)."""
+    from cats_amd import decoder as dec
+
+    cfg = dec.DecoderConfig(hidden_size=512, intermediate_size=1000, num_layers=2, num_heads=4, vocab_size=503, max_len=64)
+    with torch.no_grad():
+        model = dec.LlamaDecoder(cfg, dtype, "cuda", seed=0, init_std=0.05).eval()
+        model.embed_tokens.weight.mul_(40)
+        model.set_mlp_mode(mode)
+        g = torch.Generator(device="cuda").manual_seed(5)
+        prompt = torch.randint(0, 503, (B, 9), generator=g, device="cuda")
+        tok, pos = prompt[:, :1].contiguous(), torch.full((1,), 9, device="cuda")
+
+        def step(hook):
+            model.reset_cache(B)
+            model(prompt, torch.arange(9, device="cuda"))
+            handle = model.lm_head.register_forward_hook(lambda *a: None) if hook else None
+            assert model._takes_step(model.embed_tokens(tok), pos) == (not hook)
+            out = model(tok, pos)
+            if handle:
+                handle.remove()
+            return out.double(), model.layers[1].self_attn.k_cache[:, :, 9].double()
+
+        for a, b in zip(step(False), step(True)):
+            assert float((a - b).norm() / b.norm()) < 16 * EPS[dtype]  # two layers of roundings, at most eight steps each
+
+
+def test_step_leaves_watched_calls_to_torch():
+    from cats_amd import decoder as dec
+
+    cfg = dec.DecoderConfig(hidden_size=256, intermediate_size=512, num_layers=1, num_heads=4, vocab_size=53, max_len=16)
+    model = dec.LlamaDecoder(cfg, torch.float16, "cuda", seed=0).eval()
+    model.reset_cache(1)
+    h, pos = torch.randn(1, 1, 256, device="cuda").half(), torch.zeros(1, dtype=torch.int64, device="cuda")
+    assert not model._takes_step(h, pos)                                       # gradients
+    with torch.no_grad():
+        assert model._takes_step(h, pos)
+        assert not model._takes_step(h.expand(9, 1, 256).contiguous(), pos)    # rows, and a cache of another batch
+        assert not model._takes_step(h.expand(2, 1, 256).contiguous(), pos)
+        assert not model._takes_step(h, pos.int()) and not model._takes_step(h.expand(1, 2, 256).contiguous(), pos)
+        with torch.autocast("cuda"):
+            assert not model._takes_step(h, pos)
+        handle = model.layers[0].self_attn.q_proj.register_forward_hook(lambda *a: None)
+        assert not model._takes_step(h, pos)
+        handle.remove()
+        model.layers[0].self_attn.q_proj.weight.data = torch.randn(256, 256, device="cuda").half().t()
+        assert not model._takes_step(h, pos)
