@@ -36,6 +36,12 @@ template <> hipError_t launch_proj<F32>(int, int, const ProjArgs&, hipStream_t);
 template <> hipError_t launch_attn<F16>(int, int, const AttnArgs&, hipStream_t);
 template <> hipError_t launch_attn<BF16>(int, int, const AttnArgs&, hipStream_t);
 template <> hipError_t launch_attn<F32>(int, int, const AttnArgs&, hipStream_t);
+template <> hipError_t launch_gate_cols<F16>(const GateColsArgs&, int, hipStream_t);
+template <> hipError_t launch_gate_cols<BF16>(const GateColsArgs&, int, hipStream_t);
+template <> hipError_t launch_gate_cols<F32>(const GateColsArgs&, int, hipStream_t);
+template <> hipError_t launch_gate_cols_finish<F16>(const GateColsArgs&, int, void*, hipStream_t);
+template <> hipError_t launch_gate_cols_finish<BF16>(const GateColsArgs&, int, void*, hipStream_t);
+template <> hipError_t launch_gate_cols_finish<F32>(const GateColsArgs&, int, void*, hipStream_t);
 int current_device_cus() {
   constexpr int kDevs = 64;
   static int cus[kDevs];  // 0 = not asked yet; written once per device with the same value, so a plain atomic will do
@@ -1148,6 +1154,57 @@ int cats_mlp_rowmajor_down(const void* x, const void* wgate, const void* wup, co
     return mlp_rowmajor_down_pass(at_cbytes(x, b0 * H * sz), wgate, wup, wdown, at_bytes(y_out, b0 * H * sz), nb, H, I, dtype, threshold, ws,
                                   ws_bytes, stream);
   });
+}
+
+int cats_mlp_gate_cols(const void* x, const void* wgate_hi, const void* wup, const void* wdown_t, void* y_out, int H, int I, int dtype,
+                       float threshold, void* ws, size_t ws_bytes, void* stream) {
+  int st = check_common(1, H, I, dtype);
+  if (st) return st;
+  if (I < vec_elems(dtype)) return CATS_ERR_SHAPE;
+  if (!x || !wgate_hi || !wup || !wdown_t || !y_out) return CATS_ERR_NULL;
+  if (!aligned16(x) || !aligned16(wup) || !aligned16(wdown_t) || ((uintptr_t)wgate_hi & (esz(dtype) - 1)) != 0) return CATS_ERR_ALIGN;
+  WsLayout l;
+  st = check_ws(ws, ws_bytes, H, I, l);
+  if (st) return st;
+  GateColsArgs g;
+  g.x = x;
+  g.w = wgate_hi;
+  g.partial = (float*)((char*)ws + l.zt);  // that region and the next, 16 * I floats: nothing else of this call uses them
+  g.H = H;
+  g.I = I;
+  const int slab = kWave * vec_elems(dtype);
+  g.nslab = (I + slab - 1) / slab;
+  int groups = current_device_cus() / g.nslab;  // one workgroup of sixteen waves per CU, all at once
+  if (groups > kGateColsMaxGroups) groups = kGateColsMaxGroups;
+  if (groups > (H + kGateColsWaves - 1) / kGateColsWaves) groups = (H + kGateColsWaves - 1) / kGateColsWaves;
+  if (groups < 1) groups = 1;
+  g.rows_per = (H + groups - 1) / groups;
+  groups = (H + g.rows_per - 1) / g.rows_per;
+  hipStream_t s = (hipStream_t)stream;
+  hipError_t e = dtype == CATS_F16    ? launch_gate_cols<F16>(g, groups, s)
+                 : dtype == CATS_BF16 ? launch_gate_cols<BF16>(g, groups, s)
+                                      : launch_gate_cols<F32>(g, groups, s);
+  if (e != hipSuccess) return CATS_ERR_LAUNCH;
+  FusedArgs f;
+  int grid = 0;
+  if (fused_eligible(1, H, I, dtype, f, grid)) {
+    f.x = (const u32x4*)x;
+    f.a_part = g.partial;
+    f.a_groups = groups;
+    f.wu = (const u32x4*)wup;
+    f.wd = (const u32x4*)wdown_t;
+    f.t = round_through(dtype, threshold);
+    return do_fused(f, grid, 0, y_out, nullptr, nullptr, dtype, (char*)ws, l, s);
+  }
+  // Rows too long for the single-pass kernel: the activations as the separate kernels take them.  They lie where the down
+  // pass, which runs after their last reader, will leave its partial sums.
+  if ((size_t)I * esz(dtype) > l.mask - l.partial) return CATS_ERR_SHAPE;
+  void* a = (char*)ws + l.partial;
+  e = dtype == CATS_F16    ? launch_gate_cols_finish<F16>(g, groups, a, s)
+      : dtype == CATS_BF16 ? launch_gate_cols_finish<BF16>(g, groups, a, s)
+                           : launch_gate_cols_finish<F32>(g, groups, a, s);
+  if (e != hipSuccess) return CATS_ERR_LAUNCH;
+  return up_down_pass(x, a, wup, wdown_t, y_out, 1, H, I, dtype, threshold, ws, ws_bytes, stream);
 }
 
 static int do_proj(int mode, int dtype, const ProjArgs& a, hipStream_t s) {

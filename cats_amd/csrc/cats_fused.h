@@ -23,6 +23,7 @@
 // producers always make progress.
 #pragma once
 #include "cats_device.h"
+#include "cats_gate_cols.h"
 
 namespace cats {
 
@@ -82,6 +83,8 @@ struct FusedArgs {
   const u32x4* wu;       // (I, H)
   const u32x4* wd;       // (I, H) neuron-major
   const void* a_in;      // optional (nb, I) dtype: gate activations; flags = |a| > t
+  const float* a_part;   // or, one row: the sums gate_cols_kernel left, [a_groups][I]
+  int a_groups;
   uint8_t* flag_out;     // optional (nb, I)
   float* partial;        // [grid][nb][H] fp32
   float* y32;            // optional (nb, H) fp32: the workgroup adds its sums here with atomics instead of storing `partial`
@@ -645,7 +648,9 @@ __global__ __launch_bounds__(kFusedThreads) void mlp_fused_kernel(FusedArgs p) {
         bool any = false;
 #pragma unroll
         for (int b = 0; b < B; b++) {
-          const float av = b < p.nb ? DT::tof(ain[(size_t)b * p.I + row0 + q]) : 0.f;
+          float av = 0.f;
+          if (p.a_part) av = B == 1 || b == 0 ? gate_cols_activation<DT>(p.a_part, p.a_groups, p.I, row0 + q) : 0.f;
+          else if (b < p.nb) av = DT::tof(ain[(size_t)b * p.I + row0 + q]);
           sl.z[q * B + b] = av;
           any = any || (b < p.nb && fabsf(av) > p.t);
         }

@@ -312,6 +312,16 @@ hipError_t launch_attn<CATS_DT>(int blocks, int head_dim, const AttnArgs& a, hip
 }
 
 template <>
+hipError_t launch_gate_cols<CATS_DT>(const GateColsArgs& a, int groups, hipStream_t stream) {
+  return launch_kernel(gate_cols_kernel<CATS_DT>, dim3(a.nslab * groups), dim3(kGateColsWaves * kWave), 0, stream, a);
+}
+
+template <>
+hipError_t launch_gate_cols_finish<CATS_DT>(const GateColsArgs& a, int groups, void* a_out, hipStream_t stream) {
+  return launch_kernel(gate_cols_finish_kernel<CATS_DT>, dim3((a.I + 255) / 256), dim3(256), 0, stream, (const float*)a.partial, groups, a.I, a_out);
+}
+
+template <>
 hipError_t launch_fused<CATS_DT>(int bt, int grid, int stage, const FusedArgs& a, const ReduceArgs& r, hipStream_t stream) {
   if (stage != 2) {
     hipError_t e = bt == 1 ? launch_fused_b<CATS_DT, 1>(grid, a, stream) : launch_fused_b<CATS_DT, 2>(grid, a, stream);

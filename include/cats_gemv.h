@@ -164,6 +164,13 @@ int cats_mlp(const void* x, const void* wgate, const void* wup, const void* wdow
 int cats_up_down(const void* x, const void* a, const void* wup, const void* wdown_t, void* y_out, int B, int H, int I,
                  int dtype, float threshold, void* ws, size_t ws_bytes, void* stream);
 
+/* Whole CATS MLP for one row with the gate weight stored (H, I) -- x . wgate_hi, as the reference's index-list and Triton composites
+ * take it -- and neuron-major wup, wdown_t (I, H).  Three launches: column sums of the gate pass, then cats_up_down's two, the
+ * first of which finishes the activations.  wgate_hi needs the alignment of its element only (any I >= one 16-byte vector).
+ * Replaces flag_gemv_gemv_dejavu and flag_gemv_gemv_triton at one row (flash_gemv/flash_gemv/__init__.py:38-54). */
+int cats_mlp_gate_cols(const void* x, const void* wgate_hi, const void* wup, const void* wdown_t, void* y_out, int H, int I,
+                       int dtype, float threshold, void* ws, size_t ws_bytes, void* stream);
+
 /* The tail of a decoder layer in two launches:  out = h + MLP(norm_weight * rms_norm(h)).
  * The RMS norm (fp32 mean of squares, rsqrt(mean + eps), result rounded to dtype, then multiplied by norm_weight in
  * dtype -- the HF LlamaRMSNorm / MistralRMSNorm order) is applied while the gate+up kernel stages h in LDS; the
