@@ -23,7 +23,7 @@ SYMBOLS = (
     "cats_version", "cats_status_string", "cats_workspace_bytes", "cats_workspace_init", "cats_gate_flag",
     "cats_gate_compact", "cats_read_count", "cats_up_flag", "cats_down_flag", "cats_gate_up", "cats_mlp",
     "cats_mlp_rowmajor_down", "cats_mlp_norm_residual", "cats_up_down", "cats_set_tuning", "cats_mlp_stage", "cats_mlp_noalloc", "cats_up_index", "cats_down_index",
-    "cats_probe_read", "cats_mlp_norm_residual_norm", "cats_linear", "cats_attention_step", "cats_mlp_gate_cols",
+    "cats_probe_read", "cats_mlp_norm_residual_norm", "cats_linear", "cats_attention_step", "cats_mlp_gate_cols", "cats_silu_mask_mul",
 )
 
 

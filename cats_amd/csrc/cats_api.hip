@@ -42,6 +42,9 @@ template <> hipError_t launch_gate_cols<F32>(const GateColsArgs&, int, hipStream
 template <> hipError_t launch_gate_cols_finish<F16>(const GateColsArgs&, int, void*, hipStream_t);
 template <> hipError_t launch_gate_cols_finish<BF16>(const GateColsArgs&, int, void*, hipStream_t);
 template <> hipError_t launch_gate_cols_finish<F32>(const GateColsArgs&, int, void*, hipStream_t);
+template <> hipError_t launch_silu_mask_mul<F16>(const SiluMaskMulArgs&, hipStream_t);
+template <> hipError_t launch_silu_mask_mul<BF16>(const SiluMaskMulArgs&, hipStream_t);
+template <> hipError_t launch_silu_mask_mul<F32>(const SiluMaskMulArgs&, hipStream_t);
 int current_device_cus() {
   constexpr int kDevs = 64;
   static int cus[kDevs];  // 0 = not asked yet; written once per device with the same value, so a plain atomic will do
@@ -1205,6 +1208,18 @@ int cats_mlp_gate_cols(const void* x, const void* wgate_hi, const void* wup, con
                            : launch_gate_cols_finish<F32>(g, groups, a, s);
   if (e != hipSuccess) return CATS_ERR_LAUNCH;
   return up_down_pass(x, a, wup, wdown_t, y_out, 1, H, I, dtype, threshold, ws, ws_bytes, stream);
+}
+
+int cats_silu_mask_mul(const void* gate, const void* up, void* z, size_t n, int dtype, float threshold, void* stream) {
+  if (dtype != CATS_F16 && dtype != CATS_BF16 && dtype != CATS_F32) return CATS_ERR_DTYPE;
+  if (n == 0) return CATS_OK;
+  if (!gate || !up || !z) return CATS_ERR_NULL;
+  if (!aligned16(gate) || !aligned16(up) || !aligned16(z)) return CATS_ERR_ALIGN;
+  SiluMaskMulArgs a = {gate, up, z, n, round_through(dtype, threshold)};
+  const hipError_t e = dtype == CATS_F16    ? launch_silu_mask_mul<F16>(a, (hipStream_t)stream)
+                       : dtype == CATS_BF16 ? launch_silu_mask_mul<BF16>(a, (hipStream_t)stream)
+                                            : launch_silu_mask_mul<F32>(a, (hipStream_t)stream);
+  return e == hipSuccess ? CATS_OK : CATS_ERR_LAUNCH;
 }
 
 static int do_proj(int mode, int dtype, const ProjArgs& a, hipStream_t s) {

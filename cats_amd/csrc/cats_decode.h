@@ -268,4 +268,37 @@ __global__ __launch_bounds__(1024) void attn_decode_kernel(AttnArgs p) {
   }
 }
 
+// Between the matrix products of a prompt:  z = a * u with a = SiLU(g), 0 where |a| <= t (a NaN is kept, as torch's mask keeps it),
+// rounded where torch's separate operations round.  One pass over the three arrays; as silu, abs, compare, masked fill and multiply
+// they were eleven: 512 x 11008 in 16 bits took 32 us.
+struct SiluMaskMulArgs {
+  const void* g;
+  const void* u;
+  void* z;
+  size_t n;
+  float t;
+};
+template <class DT>
+__global__ __launch_bounds__(256) void silu_mask_mul_kernel(SiluMaskMulArgs p) {
+  typedef typename DT::st st;
+  constexpr int VEC = DT::VEC;
+  auto one = [&](st g, st u) {
+    const float gf = DT::tof(g), a = DT::rnd(gf / (1.f + expf(-gf)));
+    return DT::fromf((fabsf(a) <= p.t ? 0.f : a) * DT::tof(u));
+  };
+  const size_t nv = p.n / VEC, i = (size_t)blockIdx.x * 256 + threadIdx.x;
+  if (i < nv) {
+    u32x4 gv = ((const u32x4*)p.g)[i], uv = ((const u32x4*)p.u)[i], zv;
+#pragma unroll
+    for (int w = 0; w < 4; w++) {
+      const uint32_t gw = gv[w], uw = uv[w];
+      if constexpr (sizeof(st) == 4) zv[w] = __float_as_uint(one(__uint_as_float(gw), __uint_as_float(uw)));
+      else zv[w] = (uint32_t)one((st)gw, (st)uw) | ((uint32_t)one((st)(gw >> 16), (st)(uw >> 16)) << 16);
+    }
+    ((u32x4*)p.z)[i] = zv;
+  } else if (i == nv) {
+    for (size_t j = nv * VEC; j < p.n; j++) ((st*)p.z)[j] = one(((const st*)p.g)[j], ((const st*)p.u)[j]);
+  }
+}
+
 }  // namespace cats

@@ -312,6 +312,13 @@ hipError_t launch_attn<CATS_DT>(int blocks, int head_dim, const AttnArgs& a, hip
 }
 
 template <>
+hipError_t launch_silu_mask_mul<CATS_DT>(const SiluMaskMulArgs& a, hipStream_t stream) {
+  const size_t blocks = (a.n / CATS_DT::VEC + 1 + 255) / 256;  // one thread more than vectors: it takes what is left
+  if (blocks > 0x7fffffffu) return hipErrorInvalidValue;
+  return launch_kernel(silu_mask_mul_kernel<CATS_DT>, dim3((unsigned)blocks), dim3(256), 0, stream, a);
+}
+
+template <>
 hipError_t launch_gate_cols<CATS_DT>(const GateColsArgs& a, int groups, hipStream_t stream) {
   return launch_kernel(gate_cols_kernel<CATS_DT>, dim3(a.nslab * groups), dim3(kGateColsWaves * kWave), 0, stream, a);
 }

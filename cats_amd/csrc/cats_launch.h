@@ -67,6 +67,8 @@ template <class DT>
 hipError_t launch_proj(int mode, int bt, const ProjArgs& a, hipStream_t stream);
 template <class DT>
 hipError_t launch_attn(int blocks, int head_dim, const AttnArgs& a, hipStream_t stream);
+template <class DT>
+hipError_t launch_silu_mask_mul(const SiluMaskMulArgs& a, hipStream_t stream);
 
 // Gate pass over an (H, I) weight, one batch row (cats_gate_cols.h), and its activations as a launch of their own.
 template <class DT>

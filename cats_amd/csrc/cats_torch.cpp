@@ -531,6 +531,19 @@ at::Tensor cats_attention_step_op(const at::Tensor& h, const at::Tensor& x, cons
   return out;
 }
 
+// SiLU(gate) * up, 0 where |SiLU(gate)| <= threshold.
+at::Tensor cats_silu_mask_mul_op(const at::Tensor& gate, const at::Tensor& up, const double threshold) {
+  check_dev(gate, "gate");
+  check_dev(up, "up");
+  TORCH_CHECK(up.sizes() == gate.sizes() && up.scalar_type() == gate.scalar_type() && up.device() == gate.device(),
+              "flash_gemv.cats_silu_mask_mul: gate and up must be alike");
+  at::Tensor z = at::empty_like(gate);
+  check_status(cats_silu_mask_mul(gate.data_ptr(), up.data_ptr(), z.data_ptr(), (size_t)gate.numel(), dtype_code(gate), (float)threshold,
+                                  current_stream(gate)),
+               "cats_silu_mask_mul");
+  return z;
+}
+
 }  // namespace
 
 TORCH_LIBRARY(flash_gemv, m) {
@@ -561,5 +574,6 @@ TORCH_LIBRARY(flash_gemv, m) {
   m.def("cats_mlp_stats", cats_mlp_stats_op);
   // the rest of a decode step
   m.def("cats_linear", cats_linear_op);
+  m.def("cats_silu_mask_mul", cats_silu_mask_mul_op);
   m.def("cats_attention_step", cats_attention_step_op);
 }

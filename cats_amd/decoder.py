@@ -21,7 +21,7 @@ import torch
 import torch.nn as nn
 import torch.nn.functional as F
 
-from .mlp import CatsMLP
+from .mlp import CatsMLP, _bare, _nothing_watches, _plain
 
 
 @dataclass
@@ -38,21 +38,6 @@ class DecoderConfig:
     @property
     def head_dim(self):
         return self.hidden_size // self.num_heads
-
-
-def _bare(module, cls):
-    """`module` is a plain `cls`: calling it does nothing besides the class's own forward."""
-    return (type(module) is cls and "forward" not in module.__dict__ and not module._forward_hooks and not module._forward_pre_hooks
-            and not module._backward_hooks and not module._backward_pre_hooks)
-
-
-def _nothing_watches():
-    """No autograd, tracing, autocast, transform or mode is at work that has to see the single torch operations."""
-    return not (torch.is_grad_enabled() or torch.is_autocast_enabled("cuda") or torch.jit.is_tracing() or torch.compiler.is_compiling()
-                or torch._C._len_torch_dispatch_stack() or torch._C._len_torch_function_stack()
-                or torch._C._functorch.peek_interpreter_stack() is not None or torch.autograd.forward_ad._current_level >= 0
-                or nn.modules.module._global_forward_hooks or nn.modules.module._global_forward_pre_hooks
-                or nn.modules.module._global_backward_hooks or nn.modules.module._global_backward_pre_hooks)
 
 
 class RMSNorm(nn.Module):
@@ -152,11 +137,6 @@ class DecoderLayer(nn.Module):
                                                      at.q_proj.weight, at.k_proj.weight, at.v_proj.weight, at.o_proj.weight,
                                                      at.k_cache, at.v_cache, cos_table, sin_table, positions)
         return self._mlp_tail(h, next_norm)
-
-
-def _plain(t, dtype, device):
-    """A tensor whose memory a kernel may read as it lies."""
-    return type(t) in (torch.Tensor, nn.Parameter) and t.dtype == dtype and t.device == device and t.is_contiguous() and t.data_ptr() % 16 == 0
 
 
 class LlamaDecoder(nn.Module):

@@ -13,7 +13,8 @@ Same attribute switches as the reference, poked onto the module by the harness
   2  ``flash_gemv.gemv_gemv_triton``: gate in torch, sparse up / down in HIP over ``wdown_t``
   3  ``flash_gemv.cats_mlp``: everything in two HIP launches over ``wdown_t`` (no reference counterpart: the
      reference has no single call with the gate fused in and neuron-major down weights)
-Prefill (``x.shape[1] > 1``) always takes the dense-masked branch, as in the reference (:900-904).
+Prefill (``x.shape[1] > 1``) always takes the dense-masked branch, as in the reference (:900-904); on the GPU its SiLU, threshold
+and product between the three matrix products are one kernel.
 """
 from __future__ import annotations
 
@@ -41,6 +42,26 @@ def get_threshold(bin_edges: torch.Tensor, histogram_counts: torch.Tensor, spars
     histogram_counts /= histogram_counts.sum()
     threshold_idx = torch.searchsorted(histogram_counts.cumsum(0), sparsity_level, side="right")
     return bin_edges[threshold_idx]
+
+
+def _bare(module, cls):
+    """`module` is a plain `cls`: calling it does nothing besides the class's own forward."""
+    return (type(module) is cls and "forward" not in module.__dict__ and not module._forward_hooks and not module._forward_pre_hooks
+            and not module._backward_hooks and not module._backward_pre_hooks)
+
+
+def _nothing_watches():
+    """No autograd, tracing, autocast, transform or mode is at work that has to see the single torch operations."""
+    return not (torch.is_grad_enabled() or torch.is_autocast_enabled("cuda") or torch.jit.is_tracing() or torch.compiler.is_compiling()
+                or torch._C._len_torch_dispatch_stack() or torch._C._len_torch_function_stack()
+                or torch._C._functorch.peek_interpreter_stack() is not None or torch.autograd.forward_ad._current_level >= 0
+                or nn.modules.module._global_forward_hooks or nn.modules.module._global_forward_pre_hooks
+                or nn.modules.module._global_backward_hooks or nn.modules.module._global_backward_pre_hooks)
+
+
+def _plain(t, dtype, device):
+    """A tensor whose memory a kernel may read as it lies."""
+    return type(t) in (torch.Tensor, nn.Parameter) and t.dtype == dtype and t.device == device and t.is_contiguous() and t.data_ptr() % 16 == 0
 
 
 class SparseSiLU(nn.SiLU):
@@ -156,10 +177,23 @@ class CatsMLP(nn.Module):
                                                       self.wdown_t, float(self.dead_threshold), next_norm_weight, float(next_eps))
 
     def _dense_masked(self, x):
-        post_act = self.act_fn(self.gate_proj(x))
+        gate = self.gate_proj(x)
+        t = self.dead_threshold
+        if (gate.is_cuda and isinstance(t, (int, float)) and _bare(self.act_fn, nn.SiLU) and _nothing_watches()
+                and gate.dtype in (torch.float16, torch.bfloat16, torch.float32) and _plain(gate, gate.dtype, gate.device)):
+            up = self.up_proj(x)
+            if up.shape == gate.shape and _plain(up, gate.dtype, gate.device):
+                import flash_gemv  # noqa: F401
+
+                return self.down_proj(torch.ops.flash_gemv.cats_silu_mask_mul(gate, up, float(t)))
+            return self._mask_and_down(gate, up)
+        return self._mask_and_down(gate, self.up_proj(x))
+
+    def _mask_and_down(self, gate, up):
+        post_act = self.act_fn(gate)
         dead_neurons = post_act.abs() <= self.dead_threshold
         post_act[dead_neurons] = 0
-        return self.down_proj(post_act * self.up_proj(x))
+        return self.down_proj(post_act * up)
 
     def forward(self, x, sp_mask: torch.Tensor = None):
         if sp_mask is not None:  # ugly_utils.py:872-875

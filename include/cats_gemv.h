@@ -236,6 +236,10 @@ int cats_attention_step(const void* h, const void* x, const void* norm_weight, f
                         const int64_t* position, float* q_scratch, void* attn_scratch, void* out, int B, int H, int heads,
                         int max_len, int dtype, void* stream);
 
+/* z = SiLU(gate) * up over n elements, 0 where |SiLU(gate)| <= threshold; a NaN is kept.  What stands between the matrix products of a
+ * prompt in the reference's dense branch (experiments/models/sparse_silu/ugly_utils.py:895-904), with its roundings. */
+int cats_silu_mask_mul(const void* gate, const void* up, void* z, size_t n, int dtype, float threshold, void* stream);
+
 /* One launch of cats_mlp(y_out mode) alone, for per-kernel timing and profiling: stage 1 = the streaming launch (gate, up
  * and, for 1..2 rows, down into per-workgroup partial sums), stage 2 = the launch that finishes y from what stage 1 left in
  * the workspace.  Calling stage 1 then stage 2 with the same arguments is cats_mlp.  Not in the reference. */
