@@ -10,7 +10,8 @@ Same attribute switches as the reference, poked onto the module by the harness
 ``sp_method`` when ``is_profile`` and the input is a decode step (``x.shape[1] == 1``):
   0  dense-masked PyTorch (the reference's own fallback and the parity oracle's formula)
   1  ``flash_gemv.flag_gemv_gemv_inner{,_fp32,_bf16}`` on the HF-layout down weight (dense down)
-  2  ``flash_gemv.gemv_gemv_triton``: gate in torch, sparse up / down in HIP over ``wdown_t``
+  2  ``flash_gemv.gemv_gemv_triton``: gate by the module, sparse up / down in HIP over ``wdown_t``; with a plain nn.Linear as the
+     gate the same in one call
   3  ``flash_gemv.cats_mlp``: everything in two HIP launches over ``wdown_t`` (no reference counterpart: the
      reference has no single call with the gate fused in and neuron-major down weights)
 Prefill (``x.shape[1] > 1``) always takes the dense-masked branch, as in the reference (:900-904); on the GPU its SiLU, threshold
@@ -211,6 +212,12 @@ class CatsMLP(nn.Module):
                 if self.wdown_t is None:
                     raise RuntimeError("CatsMLP: sp_method 2/3 need wdown_t (call prepare_decode() once after loading weights)")
                 if self.sp_method == 2:
+                    g = self.gate_proj
+                    if (_bare(g, nn.Linear) and g.bias is None and _bare(self.act_fn, nn.SiLU) and _nothing_watches()
+                            and _plain(g.weight, x.dtype, x.device)):
+                        # a plain gate projection: the same call with the gate in it (torch's product alone takes 21 us of the 51
+                        # of a 4096 / 14336 layer at one row, all of it 38)
+                        return flash_gemv.cats_mlp(x, g.weight, self.up_proj.weight, self.wdown_t, t)
                     return flash_gemv.gemv_gemv_triton(x, self.act_fn(self.gate_proj(x)), self.up_proj.weight, self.wdown_t, t)
                 if self.is_stats:
                     # decode-time sparsity bookkeeping (the reference's agg_sparsity, ugly_utils.py:929-937, for the
