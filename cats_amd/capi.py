@@ -24,6 +24,7 @@ SYMBOLS = (
     "cats_gate_compact", "cats_read_count", "cats_up_flag", "cats_down_flag", "cats_gate_up", "cats_mlp",
     "cats_mlp_rowmajor_down", "cats_mlp_norm_residual", "cats_up_down", "cats_set_tuning", "cats_mlp_stage", "cats_mlp_noalloc", "cats_up_index", "cats_down_index",
     "cats_probe_read", "cats_mlp_norm_residual_norm", "cats_linear", "cats_attention_step", "cats_mlp_gate_cols", "cats_silu_mask_mul",
+    "cats_prompt_scratch_bytes", "cats_prompt_mlp",
 )
 
 
@@ -50,6 +51,8 @@ def lib() -> ctypes.CDLL:
         L.cats_status_string.argtypes = [i32]; L.cats_status_string.restype = ctypes.c_char_p
         L.cats_workspace_bytes.argtypes = [i32, i32, i32]; L.cats_workspace_bytes.restype = sz
         L.cats_workspace_init.argtypes = [vp, sz, vp]; L.cats_workspace_init.restype = i32
+        L.cats_prompt_scratch_bytes.argtypes = [i32, i32, i32]; L.cats_prompt_scratch_bytes.restype = sz
+        L.cats_prompt_mlp.argtypes = [vp, vp, vp, vp, vp, i32, i32, i32, i32, f32, vp, sz, vp]; L.cats_prompt_mlp.restype = i32
         L.cats_gate_flag.argtypes = [vp, vp, vp, vp, i32, i32, i32, i32, f32, vp]; L.cats_gate_flag.restype = i32
         L.cats_gate_compact.argtypes = [vp, vp, vp, vp, vp, i32, i32, i32, f32, vp, sz, vp]; L.cats_gate_compact.restype = i32
         L.cats_read_count.argtypes = [vp, vp]; L.cats_read_count.restype = i32

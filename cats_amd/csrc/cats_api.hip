@@ -45,6 +45,10 @@ template <> hipError_t launch_gate_cols_finish<F32>(const GateColsArgs&, int, vo
 template <> hipError_t launch_silu_mask_mul<F16>(const SiluMaskMulArgs&, hipStream_t);
 template <> hipError_t launch_silu_mask_mul<BF16>(const SiluMaskMulArgs&, hipStream_t);
 template <> hipError_t launch_silu_mask_mul<F32>(const SiluMaskMulArgs&, hipStream_t);
+template <> hipError_t launch_prompt<F16>(bool, const PromptPlan&, PromptArgs, hipStream_t);
+template <> hipError_t launch_prompt<BF16>(bool, const PromptPlan&, PromptArgs, hipStream_t);
+template <> hipError_t launch_prompt_sum<F16>(const PromptSumArgs&, hipStream_t);
+template <> hipError_t launch_prompt_sum<BF16>(const PromptSumArgs&, hipStream_t);
 int current_device_cus() {
   constexpr int kDevs = 64;
   static int cus[kDevs];  // 0 = not asked yet; written once per device with the same value, so a plain atomic will do
@@ -1219,6 +1223,60 @@ int cats_silu_mask_mul(const void* gate, const void* up, void* z, size_t n, int 
   const hipError_t e = dtype == CATS_F16    ? launch_silu_mask_mul<F16>(a, (hipStream_t)stream)
                        : dtype == CATS_BF16 ? launch_silu_mask_mul<BF16>(a, (hipStream_t)stream)
                                             : launch_silu_mask_mul<F32>(a, (hipStream_t)stream);
+  return e == hipSuccess ? CATS_OK : CATS_ERR_LAUNCH;
+}
+
+// The plan of the second product: what it needs in the scratch decides its size.
+static PromptPlan prompt_down_plan(int M, int H, int I) { return prompt_plan(false, M, prompt_sum_pitch(H), I, current_device_cus()); }
+static size_t prompt_z_bytes(int M, int I) { return ((size_t)M * prompt_pitch(I) * 2 + 255) / 256 * 256; }
+
+size_t cats_prompt_scratch_bytes(int M, int H, int I) {
+  if (M < 1 || M > CATS_PROMPT_MAX_TOKENS || H < 8 || I < 8 || H > (1 << 28) || I > (1 << 28)) return 0;
+  const PromptPlan down = prompt_down_plan(M, H, I);
+  return prompt_z_bytes(M, I) + (down.splits > 1 ? (size_t)down.splits * M * prompt_sum_pitch(H) * sizeof(float) : 0);
+}
+
+int cats_prompt_mlp(const void* x, const void* wgate, const void* wup, const void* wdown, void* y_out, int M, int H, int I, int dtype,
+                    float threshold, void* scratch, size_t scratch_bytes, void* stream) {
+  if (dtype != CATS_F16 && dtype != CATS_BF16) return CATS_ERR_DTYPE;
+  // the kernels count a matrix's bytes in 32 bits; the tiles' rounding must not overflow either
+  const long long limit = 0xffffffffll;
+  if (M < 1 || H < 8 || I < 8 || M > CATS_PROMPT_MAX_TOKENS || I > (1 << 28) || H > (1 << 28) || 2ll * H * prompt_pitch(I) > limit ||
+      2ll * M * H > limit || 2ll * M * prompt_pitch(I) > limit)
+    return CATS_ERR_SHAPE;
+  if (!x || !wgate || !wup || !wdown || !y_out) return CATS_ERR_NULL;
+  for (const void* p : {x, wgate, wup, wdown})
+    if ((uintptr_t)p & 1u) return CATS_ERR_ALIGN;
+  if ((uintptr_t)y_out & 7u) return CATS_ERR_ALIGN;
+  if (!scratch || ((uintptr_t)scratch & 255u) || scratch_bytes < cats_prompt_scratch_bytes(M, H, I)) return CATS_ERR_WORKSPACE;
+  const hipStream_t s = (hipStream_t)stream;
+  const int pitch = prompt_pitch(I);
+  PromptArgs a;
+  memset(&a, 0, sizeof(a));
+  a.x = x;
+  a.w = wgate;
+  a.w2 = wup;
+  a.out = scratch;
+  a.M = M; a.N = I; a.K = H;
+  a.ldx = H; a.ldo = pitch;
+  a.t = round_through(dtype, threshold);
+  const PromptPlan first = prompt_plan(true, M, pitch, H, current_device_cus());
+  hipError_t e = dtype == CATS_F16 ? launch_prompt<F16>(true, first, a, s) : launch_prompt<BF16>(true, first, a, s);
+  if (e != hipSuccess) return CATS_ERR_LAUNCH;
+  const PromptPlan second = prompt_down_plan(M, H, I);
+  float* partial = (float*)((char*)scratch + prompt_z_bytes(M, I));
+  a.x = scratch;
+  a.w = wdown;
+  a.w2 = nullptr;
+  a.N = H; a.K = I;
+  a.ldx = pitch;
+  a.out = second.splits > 1 ? (void*)partial : y_out;
+  a.ldo = second.splits > 1 ? prompt_sum_pitch(H) : H;
+  e = dtype == CATS_F16 ? launch_prompt<F16>(false, second, a, s) : launch_prompt<BF16>(false, second, a, s);
+  if (e != hipSuccess) return CATS_ERR_LAUNCH;
+  if (second.splits == 1) return CATS_OK;
+  const PromptSumArgs r = {partial, y_out, M, H, prompt_sum_pitch(H), second.splits};
+  e = dtype == CATS_F16 ? launch_prompt_sum<F16>(r, s) : launch_prompt_sum<BF16>(r, s);
   return e == hipSuccess ? CATS_OK : CATS_ERR_LAUNCH;
 }
 

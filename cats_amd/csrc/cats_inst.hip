@@ -318,6 +318,50 @@ hipError_t launch_silu_mask_mul<CATS_DT>(const SiluMaskMulArgs& a, hipStream_t s
   return launch_kernel(silu_mask_mul_kernel<CATS_DT>, dim3((unsigned)blocks), dim3(256), 0, stream, a);
 }
 
+template <class DT>
+struct PromptLaunch {
+  template <class T, bool GATE_UP>
+  static hipError_t tile(const PromptArgs& a, hipStream_t stream) {
+    auto kern = prompt_kernel<DT, T, GATE_UP>;
+    if (hipError_t e = ensure_dynamic_lds((const void*)kern, T::LDS); e != hipSuccess) return e;
+    const int grid = 8 * a.mblocks * ((a.nblocks * a.splits + 7) / 8);
+    return launch_kernel(kern, dim3(grid), dim3(T::THREADS), T::LDS, stream, a);
+  }
+  template <bool GATE_UP>
+  static hipError_t run(int t, const PromptArgs& a, hipStream_t stream) {
+    switch (t) {
+      case 0: return tile<PromptTile0, GATE_UP>(a, stream);
+      case 1: return tile<PromptTile1, GATE_UP>(a, stream);
+      case 2: return tile<PromptTile2, GATE_UP>(a, stream);
+      case 3: return tile<PromptTile3, GATE_UP>(a, stream);
+      case 4: return tile<PromptTile4, GATE_UP>(a, stream);
+    }
+    return hipErrorInvalidValue;
+  }
+  static hipError_t sum(const PromptSumArgs& a, hipStream_t stream) {
+    const size_t threads = (size_t)a.M * (a.ldp / 4);
+    return launch_kernel(prompt_sum_kernel<DT>, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, stream, a);
+  }
+};
+template <>
+struct PromptLaunch<F32> {
+  template <bool GATE_UP>
+  static hipError_t run(int, const PromptArgs&, hipStream_t) { return hipErrorInvalidValue; }
+  static hipError_t sum(const PromptSumArgs&, hipStream_t) { return hipErrorInvalidValue; }
+};
+template <>
+hipError_t launch_prompt<CATS_DT>(bool gate_up, const PromptPlan& plan, PromptArgs a, hipStream_t stream) {
+  a.mblocks = plan.mblocks;
+  a.nblocks = plan.nblocks;
+  a.steps = plan.steps;
+  a.splits = plan.splits;
+  return gate_up ? PromptLaunch<CATS_DT>::run<true>(plan.tile, a, stream) : PromptLaunch<CATS_DT>::run<false>(plan.tile, a, stream);
+}
+template <>
+hipError_t launch_prompt_sum<CATS_DT>(const PromptSumArgs& a, hipStream_t stream) {
+  return PromptLaunch<CATS_DT>::sum(a, stream);
+}
+
 template <>
 hipError_t launch_gate_cols<CATS_DT>(const GateColsArgs& a, int groups, hipStream_t stream) {
   return launch_kernel(gate_cols_kernel<CATS_DT>, dim3(a.nslab * groups), dim3(kGateColsWaves * kWave), 0, stream, a);

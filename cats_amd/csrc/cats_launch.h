@@ -3,6 +3,7 @@
 #pragma once
 #include <hip/hip_runtime.h>
 #include "cats_decode.h"
+#include "cats_prompt.h"
 #include "cats_down.h"
 #include "cats_down_mma.h"
 #include "cats_gemv_mma.h"
@@ -69,6 +70,12 @@ template <class DT>
 hipError_t launch_attn(int blocks, int head_dim, const AttnArgs& a, hipStream_t stream);
 template <class DT>
 hipError_t launch_silu_mask_mul(const SiluMaskMulArgs& a, hipStream_t stream);
+
+// The products of a prompt (cats_prompt.h), 16-bit types.  launch_prompt fills in what the plan decides.
+template <class DT>
+hipError_t launch_prompt(bool gate_up, const PromptPlan& plan, PromptArgs a, hipStream_t stream);
+template <class DT>
+hipError_t launch_prompt_sum(const PromptSumArgs& a, hipStream_t stream);
 
 // Gate pass over an (H, I) weight, one batch row (cats_gate_cols.h), and its activations as a launch of their own.
 template <class DT>

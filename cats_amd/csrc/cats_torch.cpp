@@ -6,10 +6,12 @@
 // and a cached workspace, and calls one entry point of the C ABI in include/cats_gemv.h.  A non-zero
 // status becomes a c10::Error (the reference printf()s and exit()s: fuse_gemv_cmp_cuda.cu:2096-2097).
 #include <ATen/ATen.h>
+#include <c10/core/DeviceGuard.h>
 #include <c10/hip/HIPStream.h>
 #include <hip/hip_runtime_api.h>
 #include <torch/library.h>
 
+#include <climits>
 #include <map>
 #include <mutex>
 #include <tuple>
@@ -520,6 +522,7 @@ at::Tensor cats_attention_step_op(const at::Tensor& h, const at::Tensor& x, cons
   check_dev(position, "position");
   TORCH_CHECK(position.scalar_type() == at::kLong && position.numel() == 1 && position.device() == h.device(),
               "flash_gemv.cats_attention_step: position must be one int64 on h's device");
+  const c10::DeviceGuard guard(h.device());
   at::Tensor out = at::empty_like(h);
   at::Tensor q = at::empty({B, H}, h.options().dtype(at::kFloat));
   at::Tensor att = at::empty({B, H}, h.options());
@@ -537,11 +540,32 @@ at::Tensor cats_silu_mask_mul_op(const at::Tensor& gate, const at::Tensor& up, c
   check_dev(up, "up");
   TORCH_CHECK(up.sizes() == gate.sizes() && up.scalar_type() == gate.scalar_type() && up.device() == gate.device(),
               "flash_gemv.cats_silu_mask_mul: gate and up must be alike");
+  const c10::DeviceGuard guard(gate.device());
   at::Tensor z = at::empty_like(gate);
   check_status(cats_silu_mask_mul(gate.data_ptr(), up.data_ptr(), z.data_ptr(), (size_t)gate.numel(), dtype_code(gate), (float)threshold,
                                   current_stream(gate)),
                "cats_silu_mask_mul");
   return z;
+}
+
+// The dense-masked MLP over all tokens of x (..., H) with nn.Linear's weights.
+at::Tensor cats_prompt_mlp_op(const at::Tensor& x, const at::Tensor& w_gate, const at::Tensor& w_up, const at::Tensor& w_down,
+                              const double threshold) {
+  check_dev(x, "x");
+  TORCH_CHECK(x.dim() >= 1 && w_gate.dim() == 2 && x.size(-1) == w_gate.size(1), "flash_gemv.cats_prompt_mlp: x must be (..., H)");
+  const int64_t H = w_gate.size(1), I = w_gate.size(0), M = H ? x.numel() / H : 0;
+  check_weight(w_gate, x, I, H, "w_gate");
+  check_weight(w_up, x, I, H, "w_up");
+  check_weight(w_down, x, H, I, "w_down");
+  TORCH_CHECK(M >= 1 && M <= CATS_PROMPT_MAX_TOKENS && H <= INT_MAX && I <= INT_MAX, "flash_gemv.cats_prompt_mlp: 1..", CATS_PROMPT_MAX_TOKENS, " tokens");
+  const c10::DeviceGuard guard(x.device());
+  at::Tensor y = at::empty_like(x);
+  const size_t bytes = cats_prompt_scratch_bytes((int)M, (int)H, (int)I);
+  at::Tensor scratch = at::empty({(int64_t)bytes}, x.options().dtype(at::kByte));
+  check_status(cats_prompt_mlp(x.data_ptr(), w_gate.data_ptr(), w_up.data_ptr(), w_down.data_ptr(), y.data_ptr(), (int)M, (int)H, (int)I,
+                               dtype_code(x), (float)threshold, scratch.data_ptr(), bytes, current_stream(x)),
+               "cats_prompt_mlp");
+  return y;
 }
 
 }  // namespace
@@ -575,5 +599,6 @@ TORCH_LIBRARY(flash_gemv, m) {
   // the rest of a decode step
   m.def("cats_linear", cats_linear_op);
   m.def("cats_silu_mask_mul", cats_silu_mask_mul_op);
+  m.def("cats_prompt_mlp", cats_prompt_mlp_op);
   m.def("cats_attention_step", cats_attention_step_op);
 }

@@ -14,8 +14,9 @@ Same attribute switches as the reference, poked onto the module by the harness
      gate the same in one call
   3  ``flash_gemv.cats_mlp``: everything in two HIP launches over ``wdown_t`` (no reference counterpart: the
      reference has no single call with the gate fused in and neuron-major down weights)
-Prefill (``x.shape[1] > 1``) always takes the dense-masked branch, as in the reference (:900-904); on the GPU its SiLU, threshold
-and product between the three matrix products are one kernel.
+Prefill (``x.shape[1] > 1``) always takes the dense-masked branch, as in the reference (:900-904): on the GPU, in 16-bit types, as
+``cats_prompt_mlp`` up to the number of tokens where that is the faster one, else as three products of the library with the SiLU,
+threshold and product between them in one kernel.
 """
 from __future__ import annotations
 
@@ -177,7 +178,40 @@ class CatsMLP(nn.Module):
         return flash_gemv.cats_mlp_norm_residual_norm(h, norm_weight, float(eps), self.gate_proj.weight, self.up_proj.weight,
                                                       self.wdown_t, float(self.dead_threshold), next_norm_weight, float(next_eps))
 
+    def _prompt_weights(self, x):
+        """The three weights if the projections are plain and over plain 16-bit tensors that nothing else watches -- then
+        flash_gemv.cats_prompt_mlp computes the same -- else None."""
+        if not x.is_cuda or x.dtype not in (torch.float16, torch.bfloat16) or type(x) is not torch.Tensor or not x.is_contiguous():
+            return None
+        if not isinstance(self.dead_threshold, (int, float)) or not _nothing_watches() or not _bare(self.act_fn, nn.SiLU):
+            return None
+        dtype, device, weights = x.dtype, x.device, []
+        for proj in (self.gate_proj, self.up_proj, self.down_proj):
+            if not _bare(proj, nn.Linear):
+                return None
+            w = proj._parameters.get("weight")
+            if (type(w) is not nn.Parameter or w.dtype != dtype or w.device != device or not w.is_contiguous() or w.dim() != 2
+                    or proj._parameters.get("bias", self) is not None):
+                return None
+            weights.append(w)
+        shape = weights[0].shape
+        if weights[1].shape != shape or weights[2].shape != shape[::-1] or x.shape[-1] != shape[1] or min(shape) < 8:
+            return None
+        I, H = shape
+        tokens = x.numel() // H
+        # Up to 512 tokens the kernels are the faster ones at every size measured (4096 / 11008: 66 against 81 us at 2, 163 against 195 at
+        # 512; 304 / 569: 24 against 78); from there on the library's larger tiles win where there is enough work for them
+        # (700 tokens of 4096 / 11008: 266 against 231 us, 87 against 85 of 2048 / 5632, but 44 against 80 of 1024 / 2731).
+        if not (1 <= tokens <= 512 or 512 < tokens <= 4096 and tokens * H * I <= 7e9) or 2 * H * (I + 8) >= 1 << 32:
+            return None
+        return weights
+
     def _dense_masked(self, x):
+        weights = self._prompt_weights(x)
+        if weights is not None:
+            import flash_gemv  # noqa: F401
+
+            return torch.ops.flash_gemv.cats_prompt_mlp(x, *weights, float(self.dead_threshold))
         gate = self.gate_proj(x)
         t = self.dead_threshold
         if (gate.is_cuda and isinstance(t, (int, float)) and _bare(self.act_fn, nn.SiLU) and _nothing_watches()

@@ -240,6 +240,17 @@ int cats_attention_step(const void* h, const void* x, const void* norm_weight, f
  * prompt in the reference's dense branch (experiments/models/sparse_silu/ugly_utils.py:895-904), with its roundings. */
 int cats_silu_mask_mul(const void* gate, const void* up, void* z, size_t n, int dtype, float threshold, void* stream);
 
+/* The whole dense-masked MLP over the M tokens of a prompt (1..CATS_PROMPT_MAX_TOKENS), 16-bit types:
+ *   y = (a * (x . Wup^T)) . Wdown^T,  a = SiLU(x . Wgate^T), 0 where |a| <= threshold (a NaN is kept)
+ * with the roundings of the three products and of cats_silu_mask_mul.  x (M,H), wgate / wup (I,H), wdown (H,I) at any alignment of the
+ * element, H and I at least 8, no matrix of 4 GiB or more; y_out 8-byte aligned.  scratch: 256-byte aligned, at least
+ * cats_prompt_scratch_bytes(M, H, I) on the device of the call, nothing in it needs to be set.
+ * The reference's dense branch: experiments/models/sparse_silu/ugly_utils.py:895-904. */
+#define CATS_PROMPT_MAX_TOKENS 4096
+size_t cats_prompt_scratch_bytes(int M, int H, int I);
+int cats_prompt_mlp(const void* x, const void* wgate, const void* wup, const void* wdown, void* y_out, int M, int H, int I, int dtype,
+                    float threshold, void* scratch, size_t scratch_bytes, void* stream);
+
 /* One launch of cats_mlp(y_out mode) alone, for per-kernel timing and profiling: stage 1 = the streaming launch (gate, up
  * and, for 1..2 rows, down into per-workgroup partial sums), stage 2 = the launch that finishes y from what stage 1 left in
  * the workspace.  Calling stage 1 then stage 2 with the same arguments is cats_mlp.  Not in the reference. */
