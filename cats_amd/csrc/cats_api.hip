@@ -248,9 +248,14 @@ void fill_rows(RowsArgs& a, const void* x, const void* w, int K, int N, int nb, 
   a.K = K;
   a.N = N;
   a.nb = nb;
+  a.out_pitch = N;
   const int vec = vec_elems(dtype);
   a.row_vecs = K / vec;
   a.nch = (a.row_vecs + kWave - 1) / kWave;
+}
+
+bool rows_take_mma(int mode, int dtype, int bt, const RowsArgs& a) {
+  return dtype == CATS_F16 ? rows_takes_mma<F16>(mode, bt, a) : dtype == CATS_BF16 ? rows_takes_mma<BF16>(mode, bt, a) : rows_takes_mma<F32>(mode, bt, a);
 }
 
 // Whether do_rows' pass writes the union of the flags as bytes (a.ubytes_out, the matrix-core kernel) rather than as bits
@@ -258,7 +263,7 @@ void fill_rows(RowsArgs& a, const void* x, const void* w, int K, int N, int nb, 
 bool rows_mask_is_bytes(int mode, int dtype, RowsArgs a) {
   a.mma = g_tuning.gate_variant >= 0;
   const int bt = batch_template(a.nb);
-  return dtype == CATS_F16 ? rows_takes_mma<F16>(mode, bt, a) : dtype == CATS_BF16 ? rows_takes_mma<BF16>(mode, bt, a) : false;
+  return rows_take_mma(mode, dtype, bt, a);
 }
 
 int do_rows(int mode, int dtype, const RowsArgs& a_in, hipStream_t s) {
@@ -282,6 +287,62 @@ struct NextNorm {
   float eps = 0.f;
   void* out = nullptr;
 };
+
+// What follows two matrix-core GEMVs over W_gate and W_up, for fp32 rows whose x operands do not fit in LDS whole (rows_mma_kernel): flags,
+// their union and z from the sums g = x . Wgate^T and u = x . Wup^T, both (nb, N).  One thread per neuron.  z may take u's place or g's.
+// The wave-per-row kernel reads x from global memory there: 12936 rows of 4912 at 8 batch rows 570 us, this way 140.
+struct GateUpJoinArgs {
+  const float* g;
+  const float* u;
+  float* z;
+  uint8_t* flag_out;    // optional (nb, N)
+  uint8_t* ubytes_out;  // optional (N,)
+  int N, nb;
+  float t;
+};
+__global__ __launch_bounds__(256) void gate_up_join_kernel(GateUpJoinArgs p) {
+  const int j = blockIdx.x * 256 + threadIdx.x;
+  if (j >= p.N) return;
+  bool any = false;
+  for (int b = 0; b < p.nb; b++) {
+    const size_t o = (size_t)b * p.N + j;
+    const float g = p.g[o], u = p.u[o], a = g / (1.f + expf(-g));
+    const bool act = fabsf(a) > p.t;
+    any = any || act;
+    if (p.flag_out) p.flag_out[o] = act ? 1 : 0;
+    p.z[o] = act ? a * u : 0.f;
+  }
+  if (p.ubytes_out) p.ubytes_out[j] = any ? 1 : 0;
+}
+
+constexpr int kJoinRows = 32;  // weight rows a workgroup of the fp32 matrix-core GEMV takes at most
+
+// fp32 gate + up (a as for kGateUp, no norm, at least five batch rows) as two dense GEMVs and gate_up_join_kernel, where rows_mma_kernel
+// does not take all the rows of x at once.  It reads every row of W_up, which from five batch rows on is little more than their union.
+bool joined_takes(int dtype, const RowsArgs& a) {
+  if (dtype != CATS_F32 || a.nb <= 4 || a.nb > CATS_MAX_BATCH || a.norm_w || g_tuning.gate_variant < 0) return false;
+  RowsArgs one = a;
+  one.mma = 1;
+  return a.nb > kKernelBatch ? !rows_mma16_supported<F32>(one) : !rows_takes_mma<F32>(kGateUp, kKernelBatch, one);
+}
+// sums: 16 * N floats of scratch, z: (nb, N), which takes the up sums first
+int do_joined(const RowsArgs& a, float* sums, float* z, hipStream_t s) {
+  const int most = current_device_cus() * kJoinRows, parts = (a.N + most - 1) / most;
+  const int per = ((a.N + parts - 1) / parts + 7) / 8 * 8;
+  for (int m = 0; m < 2; m++)
+    for (int n0 = 0; n0 < a.N; n0 += per) {
+      RowsArgs g = a;
+      g.w = (m ? a.w2 : a.w) + (size_t)n0 * a.row_vecs;
+      g.w2 = nullptr;
+      g.N = a.N - n0 < per ? a.N - n0 : per;
+      g.zt_out = (m ? z : sums) + n0;
+      g.z32_out = nullptr;
+      g.flag_out = g.mask_out = g.ubytes_out = nullptr;
+      if (int st = do_rows(kGemv, CATS_F32, g, s)) return st;
+    }
+  GateUpJoinArgs j = {sums, z, z, a.flag_out, a.ubytes_out, a.N, a.nb, a.t};
+  return launch_kernel(gate_up_join_kernel, dim3((a.N + 255) / 256), dim3(256), 0, s, j) == hipSuccess ? CATS_OK : CATS_ERR_LAUNCH;
+}
 
 // Fills the next-norm fields of the reduction launch; CATS_ERR_SHAPE if the launch cannot carry it.
 int set_next_norm(ReduceArgs& r, const NextNorm& next, char* ws, const WsLayout& l) {
@@ -567,8 +628,9 @@ static int rows_wide(RowsArgs& a, int dtype, void* stream) {
 #ifdef CATS_TIMING
   a.tbuf = g_tbuf_rows;
 #endif
-  if (!(dtype == CATS_F16 ? rows_mma16_supported<F16>(a) : rows_mma16_supported<BF16>(a))) return kNotTaken;
-  const hipError_t e = dtype == CATS_F16 ? launch_rows_mma16<F16>(a, (hipStream_t)stream) : launch_rows_mma16<BF16>(a, (hipStream_t)stream);
+  const hipStream_t s = (hipStream_t)stream;
+  if (!(dtype == CATS_F16 ? rows_mma16_supported<F16>(a) : dtype == CATS_BF16 ? rows_mma16_supported<BF16>(a) : rows_mma16_supported<F32>(a))) return kNotTaken;
+  const hipError_t e = dtype == CATS_F16 ? launch_rows_mma16<F16>(a, s) : dtype == CATS_BF16 ? launch_rows_mma16<BF16>(a, s) : launch_rows_mma16<F32>(a, s);
   return e == hipSuccess ? CATS_OK : CATS_ERR_LAUNCH;
 }
 
@@ -576,7 +638,7 @@ static int rows_wide(RowsArgs& a, int dtype, void* stream) {
 static int gate_flag_pass(const void* x, const void* wgate, void* a_out, uint8_t* flag_out, int B, int H, int I, int dtype,
                    float threshold, void* stream) {
   const bool wide = B > kKernelBatch;
-  if (wide && (B > CATS_MAX_BATCH || dtype == CATS_F32)) return kNotTaken;
+  if (wide && B > CATS_MAX_BATCH) return kNotTaken;
   int st = check_common(wide ? kKernelBatch : B, H, I, dtype);
   if (st) return st;
   if (!x || !wgate || (!a_out && !flag_out)) return CATS_ERR_NULL;
@@ -688,7 +750,7 @@ static int down_flag_pass(const void* z, const void* wdown_t, const uint8_t* fla
 static int gate_up_pass(const void* x, const void* wgate, const void* wup, void* out, uint8_t* flag_out, int B, int H, int I,
                  int dtype, float threshold, void* stream) {
   const bool wide = B > kKernelBatch;
-  if (wide && (B > CATS_MAX_BATCH || dtype == CATS_F32)) return kNotTaken;
+  if (wide && B > CATS_MAX_BATCH) return kNotTaken;
   int st = check_common(wide ? kKernelBatch : B, H, I, dtype);
   if (st) return st;
   if (!x || !wgate || !wup || !out) return CATS_ERR_NULL;
@@ -731,9 +793,10 @@ static int mlp_pass(const void* x, const void* wgate, const void* wup, const voi
   a.ubytes_out = (uint8_t*)ws + l.ubytes;
   a.flag_out = flag_out;
   a.t = round_through(dtype, threshold);
-  l.mask_bytes = rows_mask_is_bytes(kGateUp, dtype, a);
+  const bool joined = joined_takes(dtype, a);
+  l.mask_bytes = joined || rows_mask_is_bytes(kGateUp, dtype, a);
   if (stage != 2) {
-    st = do_rows(kGateUp, dtype, a, (hipStream_t)stream);
+    st = joined ? do_joined(a, (float*)((char*)ws + l.zt), a.z32_out, (hipStream_t)stream) : do_rows(kGateUp, dtype, a, (hipStream_t)stream);
     if (st) return st;
   }
   if (stage == 1) return CATS_OK;
@@ -744,12 +807,12 @@ static int mlp_pass(const void* x, const void* wgate, const void* wup, const voi
 
 // Whole MLP for 9..16 rows with W_gate and W_up read once: one matrix-core gate + up launch over all rows (two groups of
 // eight), then the sparse down pass per group of eight rows over the union mask of all rows.  Returns kNotTaken when the
-// type or the row length rules the one-pass kernel out (fp32, rows that are not 2048 or 4096 elements, the A/B knob).
+// row length rules the one-pass kernel out (two x operands have to fit in LDS), or the A/B knob.
 // norm_weight / residual / next: the layer-tail variants (x is then h); all optional.
 static int mlp_wide(const void* x, const void* norm_weight, float eps, const void* wgate, const void* wup, const void* wdown_t, void* y_out,
                     float* y_f32, uint8_t* flag_out, int32_t* count_out, bool residual, const NextNorm& next, int B, int H, int I, int dtype,
                     float threshold, void* ws, size_t ws_bytes, void* stream) {
-  if (B <= kKernelBatch || B > CATS_MAX_BATCH || dtype == CATS_F32) return kNotTaken;
+  if (B <= kKernelBatch || B > CATS_MAX_BATCH) return kNotTaken;
   int st = check_common(kKernelBatch, H, I, dtype);
   if (st) return st;
   if (!x || !wgate || !wup || !wdown_t || ((y_f32 == nullptr) == (y_out == nullptr))) return CATS_ERR_NULL;
@@ -768,7 +831,7 @@ static int mlp_wide(const void* x, const void* norm_weight, float eps, const voi
   a.t = round_through(dtype, threshold);
   a.norm_w = (const u32x4*)norm_weight;
   a.norm_eps = eps;
-  st = rows_wide(a, dtype, stream);
+  st = joined_takes(dtype, a) ? do_joined(a, (float*)((char*)ws + l.zt), a.z32_out, (hipStream_t)stream) : rows_wide(a, dtype, stream);
   if (st) return st;  // an error, or kNotTaken
   // all rows in one pass over W_down^T where the matrix-core down kernel takes the shape, else a pass per eight rows
   st = do_down(a.z32_out, true, wdown_t, y_f32, y_out, count_out, B, H, I, dtype, (char*)ws, l, (hipStream_t)stream, residual ? x : nullptr,
@@ -889,7 +952,7 @@ static int mlp_rowmajor_down_pass(const void* x, const void* wgate, const void* 
   a.w2 = (const u32x4*)wup;
   a.zt_out = (char*)ws + l.zt;
   a.t = round_through(dtype, threshold);
-  st = do_rows(kGateUp, dtype, a, (hipStream_t)stream);
+  st = joined_takes(dtype, a) ? do_joined(a, (float*)((char*)ws + l.z32), (float*)a.zt_out, (hipStream_t)stream) : do_rows(kGateUp, dtype, a, (hipStream_t)stream);
   if (st) return st;
   RowsArgs g;
   fill_rows(g, (char*)ws + l.zt, wdown, I, H, B, dtype);
@@ -901,7 +964,7 @@ static int mlp_rowmajor_down_pass(const void* x, const void* wgate, const void* 
 // GEMV over all rows.  kNotTaken when the type or the shape rules either kernel out.
 static int mlp_rowmajor_down_wide(const void* x, const void* wgate, const void* wup, const void* wdown, void* y_out, int B, int H,
                                   int I, int dtype, float threshold, void* ws, size_t ws_bytes, void* stream) {
-  if (B <= kKernelBatch || B > CATS_MAX_BATCH || dtype == CATS_F32) return kNotTaken;
+  if (B <= kKernelBatch || B > CATS_MAX_BATCH) return kNotTaken;
   int st = check_common(kKernelBatch, H, I, dtype);
   if (st) return st;
   if (!x || !wgate || !wup || !wdown || !y_out) return CATS_ERR_NULL;
@@ -910,18 +973,19 @@ static int mlp_rowmajor_down_wide(const void* x, const void* wgate, const void* 
   WsLayout l;
   st = check_ws(ws, ws_bytes, H, I, l);
   if (st) return st;
+  char* z = (char*)ws + (dtype == CATS_F32 ? l.z32 : l.zt);  // 16 rows of a 16-bit type fill the region of 8 rows of fp32
   RowsArgs a;
   fill_rows(a, x, wgate, H, I, B, dtype);
   a.w2 = (const u32x4*)wup;
-  a.zt_out = (char*)ws + l.zt;  // 16 rows of a 16-bit type fill the region of 8 rows of fp32
+  a.zt_out = z;
   a.t = round_through(dtype, threshold);
   RowsArgs g;
-  fill_rows(g, (char*)ws + l.zt, wdown, I, H, B, dtype);
+  fill_rows(g, z, wdown, I, H, B, dtype);
   g.zt_out = y_out;
   g.mma = g_tuning.gate_variant >= 0;
   // the GEMV first: nothing may have been launched when the call falls back to two passes
-  if (!(dtype == CATS_F16 ? rows_takes_mma<F16>(kGemv, kKernelBatch, g) : rows_takes_mma<BF16>(kGemv, kKernelBatch, g))) return kNotTaken;
-  st = rows_wide(a, dtype, stream);
+  if (!rows_take_mma(kGemv, dtype, kKernelBatch, g)) return kNotTaken;
+  st = joined_takes(dtype, a) ? do_joined(a, (float*)((char*)ws + l.zt), (float*)z, (hipStream_t)stream) : rows_wide(a, dtype, stream);
   if (st) return st;  // an error, or kNotTaken
   return do_rows(kGemv, dtype, g, (hipStream_t)stream);
 }

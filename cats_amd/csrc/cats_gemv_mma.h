@@ -1,4 +1,4 @@
-// Dense GEMV for 3..16 batch rows of a 16-bit type on the matrix cores:  out[b, r] = x[b, :] . w[r, :]   (w row-major, N x K).
+// Dense GEMV for 3..16 batch rows on the matrix cores:  out[b, r] = x[b, :] . w[r, :]   (w row-major, N x K).
 // This is the down projection of the entry point that takes W_down in the (H, I) layout of nn.Linear and has to read all
 // of it; the wave-per-row kernel (rows_kernel, kGemv) is bound by its dot instructions and LDS reads from four rows on
 // (65 us for the 90 MB of a Llama-7B W_down at eight rows).
@@ -31,7 +31,6 @@ inline size_t gemv_mma_lds_bytes() { return 2u * kGemvMmaBufBytes; }
 template <class DT, int NG, int TILES>
 __global__ __launch_bounds__(kMmaThreads) void gemv_mma_kernel(RowsArgs p) {
   typedef typename DT::st st;
-  static_assert(sizeof(st) == 2, "16-bit types only");
   static_assert((size_t)kMmaWaves * TILES * NG * kMmaPart * sizeof(float) <= 2u * kGemvMmaBufBytes, "the sums fit the x buffers");
   constexpr int CS = 8 / NG;                          // steps per wave and chunk
   constexpr int R = 2;                                // items in flight per wave
@@ -48,7 +47,7 @@ __global__ __launch_bounds__(kMmaThreads) void gemv_mma_kernel(RowsArgs p) {
   const int r1 = min(r0 + rows_per, p.N);
   const int my_tiles = (r1 - r0 + kMmaTileRows - 1) / kMmaTileRows;   // <= TILES by the launch shape
 
-  const int steps_total = (p.K + 63) / 64;            // 64-element steps of a row; the last one may be partial
+  const int steps_total = (p.row_vecs + 7) / 8;       // 128-byte steps of a row; the last one may be partial
   const int per_wave = (steps_total + kMmaWaves - 1) / kMmaWaves;
   const int nchunk = (per_wave + CS - 1) / CS;
   // chunk c holds n(c) steps per wave: per_wave dealt evenly, the first chunks one more
@@ -109,11 +108,11 @@ __global__ __launch_bounds__(kMmaThreads) void gemv_mma_kernel(RowsArgs p) {
     }
   };
 
-  f32x4 acc[TILES][NG];
+  typename Mma<DT>::Acc acc[TILES][NG];
 #pragma unroll
   for (int t = 0; t < TILES; t++)
 #pragma unroll
-    for (int gb = 0; gb < NG; gb++) acc[t][gb] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int gb = 0; gb < NG; gb++) acc[t][gb] = Mma<DT>::zero();
 
   CATS_RSTAMP(0);
   u32x4 xv[NG][CS];
@@ -178,8 +177,9 @@ __global__ __launch_bounds__(kMmaThreads) void gemv_mma_kernel(RowsArgs p) {
     for (int gb = 0; gb < NG; gb++)
       if (keep) {
         float* dst = part + ((size_t)(wave * TILES + t) * NG + gb) * kMmaPart + slot;
+        const f32x4 sum = Mma<DT>::total(acc[t][gb]);
 #pragma unroll
-        for (int i = 0; i < 4; i++) dst[i * 32] = acc[t][gb][i];
+        for (int i = 0; i < 4; i++) dst[i * 32] = sum[i];
       }
   __syncthreads();
   for (int o = tid; o < TILES * NG * kWave; o += kMmaThreads) {
@@ -187,10 +187,8 @@ __global__ __launch_bounds__(kMmaThreads) void gemv_mma_kernel(RowsArgs p) {
     const int rj = l >> 3, rb = l & 7;
     const int row = r0 + t * kMmaTileRows + rj, b = gb * 8 + rb;
     const float* src = part + ((size_t)t * NG + gb) * kMmaPart + (rj & 3) * 32 + (rj >> 2) * 8 + rb;
-    float u = 0.f;
-#pragma unroll
-    for (int w = 0; w < kMmaWaves; w++) u += src[(size_t)w * TILES * NG * kMmaPart] + src[(size_t)w * TILES * NG * kMmaPart + 16];
-    if (t < my_tiles && row < r1 && b < p.nb) ((st*)p.zt_out)[(size_t)b * p.N + row] = DT::fromf(u);
+    const float u = mma_sum_waves<DT>(src, TILES * NG * kMmaPart);
+    if (t < my_tiles && row < r1 && b < p.nb) ((st*)p.zt_out)[(size_t)b * p.out_pitch + row] = DT::fromf(u);
   }
   CATS_RSTAMP(7);
 }

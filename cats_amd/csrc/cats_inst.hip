@@ -50,24 +50,17 @@ hipError_t launch_rows_one(const RowsArgs& a, hipStream_t stream) {
   return launch_kernel(kern, dim3(grid), dim3(WAVES * kWave), lds, stream, a);
 }
 
-// Matrix-core gate + up pass: one persistent workgroup per CU.
+// Matrix-core passes over weight rows: one persistent workgroup per CU.
 template <class DT>
 struct MmaLaunch {
-  static bool supported(const RowsArgs&, int = 1) { return false; }
-  static bool supported_up(const RowsArgs&) { return false; }
-  static bool supported_gemv(const RowsArgs&) { return false; }
-  static hipError_t run(const RowsArgs&, bool, hipStream_t) { return hipErrorInvalidValue; }
-  static hipError_t run_up(const RowsArgs&, hipStream_t) { return hipErrorInvalidValue; }
-  static hipError_t run_gemv(const RowsArgs&, hipStream_t) { return hipErrorInvalidValue; }
-  static hipError_t run16(const RowsArgs&, hipStream_t) { return hipErrorInvalidValue; }
-};
-template <class DT>
-struct MmaLaunch16 {
+  static constexpr bool kHasUp = sizeof(typename DT::st) == 2;  // the up pass alone takes 16-bit types
   typedef void (*Kernel)(RowsArgs);
   enum Which { kGateOnly, kGateAndUp, kUpOnly };
   template <int STEPS, int CH, int NG>
   static Kernel kernel(Which w) {
-    return w == kUpOnly ? rows_mma_up_kernel<DT, STEPS, CH, NG> : w == kGateAndUp ? rows_mma_kernel<DT, STEPS, CH, true, NG> : rows_mma_kernel<DT, STEPS, CH, false, NG>;
+    if constexpr (kHasUp)
+      if (w == kUpOnly) return rows_mma_up_kernel<DT, STEPS, CH, NG>;
+    return w == kGateAndUp ? rows_mma_kernel<DT, STEPS, CH, true, NG> : rows_mma_kernel<DT, STEPS, CH, false, NG>;
   }
   // One instance per number of steps, so that no load or MFMA sits behind a branch on the row length.
   template <int NG>
@@ -134,31 +127,31 @@ struct MmaLaunch16 {
   }
   static bool supported_up(const RowsArgs& a) {
     const int ng = a.nb > 8 ? 2 : 1;
-    return supported(a, ng) && a.a_in && (a.z32_out || a.zt_out) && !a.norm_w && a.nb <= 16 &&
+    return kHasUp && supported(a, ng) && a.a_in && (a.z32_out || a.zt_out) && !a.norm_w && a.nb <= 16 &&
            rows_mma_up_lds_bytes(a, up_rows_pad(a), ng) <= kMmaMaxLds;
   }
   static hipError_t run_up(const RowsArgs& a, hipStream_t stream) {
     const int ng = a.nb > 8 ? 2 : 1;
     return launch(kUpOnly, a, ng, rows_mma_up_lds_bytes(a, up_rows_pad(a), ng), stream);
   }
-  // dense GEMV out = x . w^T (kGemv): any row length, 3..16 batch rows, up to 64 rows of w per workgroup
+  // dense GEMV out = x . w^T (kGemv): any row length, 3..16 batch rows, up to 64 rows of w per workgroup (32 in fp32, whose sums take
+  // four times the registers)
+  static constexpr int kGemvTiles = kHasUp ? 8 : 4;
   static bool supported_gemv(const RowsArgs& a) {
-    return a.zt_out && !a.norm_w && !a.bias && !a.scale && a.nb <= 16 && a.K % DT::VEC == 0 && up_rows_pad(a) <= 8 * kMmaTileRows;
+    return a.zt_out && !a.norm_w && !a.bias && !a.scale && a.nb <= 16 && a.K % DT::VEC == 0 && up_rows_pad(a) <= kGemvTiles * kMmaTileRows;
   }
   template <int NG>
   static hipError_t run_gemv_ng(const RowsArgs& a, hipStream_t stream) {
     const int tiles = up_rows_pad(a) / kMmaTileRows;
-    auto kern = tiles <= 2 ? gemv_mma_kernel<DT, NG, 2> : tiles <= 4 ? gemv_mma_kernel<DT, NG, 4> : gemv_mma_kernel<DT, NG, 8>;
+    auto kern = tiles <= 2 ? gemv_mma_kernel<DT, NG, 2> : tiles <= 4 ? gemv_mma_kernel<DT, NG, 4> : gemv_mma_kernel<DT, NG, kGemvTiles>;
     const size_t lds = gemv_mma_lds_bytes();
     if (hipError_t e = ensure_dynamic_lds((const void*)kern, lds); e != hipSuccess) return e;
     return launch_kernel(kern, dim3(up_grid(a)), dim3(kMmaThreads), lds, stream, a);
   }
   static hipError_t run_gemv(const RowsArgs& a, hipStream_t stream) { return a.nb > 8 ? run_gemv_ng<2>(a, stream) : run_gemv_ng<1>(a, stream); }
 };
-template <> struct MmaLaunch<F16> : MmaLaunch16<F16> {};
-template <> struct MmaLaunch<BF16> : MmaLaunch16<BF16> {};
 
-// Whether a call goes to the matrix-core kernel.  Measured on Llama-7B shapes: at 2 batch rows the wave-per-row kernel is
+// Whether a call goes to the matrix-core kernel.  16-bit types, measured on Llama-7B shapes: at 2 batch rows the wave-per-row kernel is
 // still the faster one (28.4 vs 29.4 us).  From three rows on it wins at every row length (gate + up, wave-per-row against
 // matrix cores: 255 against 129 us for 28672 rows of 8192 elements at 8 batch rows; whole MLP calls: 22.0 against 15.7 us for 3000
 // rows of 1024 at 4, 162 against 75 us for 13824 rows of 5120 at 8, 57 against 21 us for 3931 rows of 1264 at 11, where the
@@ -167,6 +160,10 @@ template <> struct MmaLaunch<BF16> : MmaLaunch16<BF16> {};
 template <class DT>
 bool takes_mma(int mode, int bt, const RowsArgs& a) {
   if (bt < 4 || !a.mma) return false;
+  // fp32 up to four rows: the wave-per-row kernel keeps up with the weights (gate + up of 4096 / 11008 at 4 rows: 17 us less), as long
+  // as it finds x in LDS (dense down, K = 12936: 11 us more).  At eight rows it spends 256 fused multiply-adds a lane on 32 vectors
+  // and the matrix cores win (5632 rows of 2048: 54 against 42 us a call, 11008 of 4096: 128 against 115, with a dense down 258 against 120).
+  if (std::is_same<DT, F32>::value && bt == 4 && (mode != kGemv || (size_t)bt * a.K * 4 <= 128 * 1024)) return false;
   if (mode == kUp) return MmaLaunch<DT>::supported_up(a);
   if (mode == kGemv) return MmaLaunch<DT>::supported_gemv(a);
   return (mode == kGateUp || mode == kGate) && MmaLaunch<DT>::supported(a);

@@ -48,6 +48,7 @@ struct RowsArgs {
   const u32x4* norm_w;   // optional (K,) RMS-norm weight: x is replaced by norm_w * round(x * rsqrt(mean(x^2) + norm_eps)) while
   float norm_eps;        //   it is staged (needs x in LDS); NULL = x is used as given
   int mma;               // host side only: kGateUp with 2..8 batch rows may take the matrix-core kernel
+  int out_pitch;         // matrix-core kGemv: elements between the batch rows of zt_out (fill_rows: N)
   int rows_per, row_stride, mma_front, mma_slots;  // matrix-core kernels, set by their launcher: see rows_mma_layout, MmaSplit
 #ifdef CATS_TIMING
   long long* tbuf;       // [gridDim][8] wall-clock stamps (100 MHz) at phase boundaries, development builds only

@@ -1,4 +1,4 @@
-// Gate and fused gate + up pass for batches of 3..16 rows in 16-bit types, on the matrix cores.
+// Gate and fused gate + up pass for batches of 3..16 rows in 16-bit types and 5..16 rows of fp32, on the matrix cores.
 //
 // Why not the wave-per-row kernel: with B batch rows every 16-byte weight vector costs 4 * B v_dot2 and B / 2
 // LDS reads of x per lane.  From B = 4 on, that arithmetic plus the LDS traffic takes as long as the HBM stream
@@ -36,15 +36,44 @@ typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
+// run: one 16-byte vector of weights times one of x per lane.  Acc: the sums of a tile; total: as one register set.
 template <class DT> struct Mma;
 template <> struct Mma<F16> {
+  typedef f32x4 Acc;
+  static __device__ __forceinline__ Acc zero() { return f32x4{0.f, 0.f, 0.f, 0.f}; }
+  static __device__ __forceinline__ f32x4 total(const Acc& c) { return c; }
   static __device__ __forceinline__ f32x4 run(u32x4 a, u32x4 b, f32x4 c) {
     return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
   }
 };
-template <> struct Mma<BF16> {
+template <> struct Mma<BF16> : Mma<F16> {
   static __device__ __forceinline__ f32x4 run(u32x4 a, u32x4 b, f32x4 c) {
     return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
+  }
+};
+
+// fp32: one v_mfma_f32_16x16x4 per element of the vectors.  Each of the four keeps sums of its own, so that a chain of additions is
+// as long as a lane's in the wave-per-row kernel (K / 64 products) and the result no further off.
+template <> struct Mma<F32> {
+  struct Acc {
+    f32x4 e[4];
+  };
+  static __device__ __forceinline__ Acc zero() {
+    Acc c;
+#pragma unroll
+    for (int i = 0; i < 4; i++) c.e[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+    return c;
+  }
+  static __device__ __forceinline__ f32x4 total(const Acc& c) {
+    f32x4 s;
+#pragma unroll
+    for (int i = 0; i < 4; i++) s[i] = (c.e[0][i] + c.e[1][i]) + (c.e[2][i] + c.e[3][i]);
+    return s;
+  }
+  static __device__ __forceinline__ Acc run(u32x4 a, u32x4 b, Acc c) {
+#pragma unroll
+    for (int i = 0; i < 4; i++) c.e[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(a[i]), __uint_as_float(b[i]), c.e[i], 0, 0, 0);
+    return c;
   }
 };
 
@@ -53,7 +82,7 @@ constexpr int kMmaThreads = kMmaWaves * kWave;
 constexpr int kMmaTileRows = 8;
 constexpr int kMmaPart = 128;    // floats per wave in a partial buffer (the two useful quadrants)
 
-// How a row of K elements is cut.  A step is 64 elements = 128 bytes, a whole cache line: where the pitch of the rows is no multiple
+// How a row of K elements is cut.  A step is 128 bytes, a whole cache line (64 16-bit elements or 32 of fp32): where the pitch of the rows is no multiple
 // of 128 bytes the steps of a row start at the line its first element lies in, "phase" 16-byte vectors before it (phase =
 // address / 16 mod 8), and the lanes in front of the row are padding like those behind it.  All rows of a tile need the same
 // phase, because they share the x operand; rows eight apart have it, so a workgroup then owns every eighth row of a block
@@ -137,7 +166,8 @@ struct MmaRows {
   }
   // acc += chunk c of the tile times the staged x rows.  What a load outside the row brought are weights of another
   // place, perhaps infinities: replaced by zeros before they meet the zeros of the x padding.
-  __device__ __forceinline__ void multiply(const u32x4 (&src)[STEPS], int c, f32x4 (&acc)[NG]) const {
+  typedef typename Mma<DT>::Acc Acc;
+  __device__ __forceinline__ void multiply(const u32x4 (&src)[STEPS], int c, Acc (&acc)[NG]) const {
 #pragma unroll
     for (int g = 0; g < NG; g++)
 #pragma unroll
@@ -149,8 +179,8 @@ struct MmaRows {
 constexpr int kMmaPartGroup = kMmaWaves * kMmaPart;  // partial-sum floats of one group of eight batch rows
 
 // The two useful quadrants of the accumulators -> this wave's part of a partial buffer.
-template <int NG>
-__device__ __forceinline__ void mma_store_partials(const f32x4 (&acc)[NG], float* part, int lane, int wave) {
+template <class DT, int NG>
+__device__ __forceinline__ void mma_store_partials(const typename Mma<DT>::Acc (&acc)[NG], float* part, int lane, int wave) {
   const int ncol = lane & 15;
   const bool keep = (lane < 32) ? (ncol < 8) : (ncol >= 8);
   const int slot = (lane >> 5) * 16 + ((lane >> 4) & 1) * 8 + (ncol & 7);
@@ -158,18 +188,32 @@ __device__ __forceinline__ void mma_store_partials(const f32x4 (&acc)[NG], float
 #pragma unroll
     for (int g = 0; g < NG; g++) {
       float* dst = part + g * kMmaPartGroup + wave * kMmaPart + slot;
+      const f32x4 sum = Mma<DT>::total(acc[g]);
 #pragma unroll
-      for (int i = 0; i < 4; i++) dst[i * 32] = acc[g][i];
+      for (int i = 0; i < 4; i++) dst[i * 32] = sum[i];
     }
   }
 }
-// One thread per (row rj of the tile, batch row rb): adds the waves' partials of group g in wave order.
-__device__ __forceinline__ float mma_reduce(const float* part, int g, int rj, int rb) {
-  const float* src = part + g * kMmaPartGroup + (rj & 3) * 32 + (rj >> 2) * 8 + rb;
-  float s = 0.f;
+// Adds the eight waves' partials (two halves each) of one output, src its first wave's: in wave order, in fp32 pairwise, as the
+// wave-per-row kernel's lanes meet (its error is the measure there: sixteen additions in a row cost 2 to 6 % of it).
+template <class DT>
+__device__ __forceinline__ float mma_sum_waves(const float* src, int wave_stride) {
+  if constexpr (sizeof(typename DT::st) == 4) {
+    float v[kMmaWaves];
 #pragma unroll
-  for (int w = 0; w < kMmaWaves; w++) s += src[w * kMmaPart] + src[w * kMmaPart + 16];
-  return s;
+    for (int w = 0; w < kMmaWaves; w++) v[w] = src[w * wave_stride] + src[w * wave_stride + 16];
+    return ((v[0] + v[1]) + (v[2] + v[3])) + ((v[4] + v[5]) + (v[6] + v[7]));
+  } else {
+    float s = 0.f;
+#pragma unroll
+    for (int w = 0; w < kMmaWaves; w++) s += src[w * wave_stride] + src[w * wave_stride + 16];
+    return s;
+  }
+}
+// One thread per (row rj of the tile, batch row rb) of group g.
+template <class DT>
+__device__ __forceinline__ float mma_reduce(const float* part, int g, int rj, int rb) {
+  return mma_sum_waves<DT>(part + g * kMmaPartGroup + (rj & 3) * 32 + (rj >> 2) * 8 + rb, kMmaPart);
 }
 
 // Staging of x: thread tid takes vectors tid + k * 512 of the nb rows, row by row in groups of eight; the loads of all are in flight together.
@@ -265,17 +309,17 @@ __global__ __launch_bounds__(kMmaThreads) void rows_mma_kernel(RowsArgs p) {
   // gbuf, ubuf, uprev: the register sets of the round.  One chunk: gbuf[0] is the tile's set, ubuf[0] takes its up rows, uprev[0]
   // holds those of the tile before.  Two chunks: gbuf[0..1] and ubuf[0..1] are the tile's two sets, uprev is ubuf.
   auto round_body = [&](int r, u32x4 (&ga)[STEPS], u32x4 (&gb)[STEPS], u32x4 (&ucur)[STEPS], u32x4 (&uprev)[STEPS]) {
-    f32x4 acc[NG];
+    typename Mma<DT>::Acc acc[NG];
 #pragma unroll
-    for (int g = 0; g < NG; g++) acc[g] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int g = 0; g < NG; g++) acc[g] = Mma<DT>::zero();
     gate.multiply(ga, 0, acc);
     if constexpr (CH == 2) {
       issue_gate(r + 1, 0, ga);
       gate.multiply(gb, 1, acc);
-      mma_store_partials<NG>(acc, part_g, lane, wave);
+      mma_store_partials<DT, NG>(acc, part_g, lane, wave);
       issue_gate(r + 1, 1, gb);
     } else {
-      mma_store_partials<NG>(acc, part_g, lane, wave);
+      mma_store_partials<DT, NG>(acc, part_g, lane, wave);
       issue_gate(r + 2, 0, ga);
     }
     __syncthreads();
@@ -295,7 +339,7 @@ __global__ __launch_bounds__(kMmaThreads) void rows_mma_kernel(RowsArgs p) {
       for (int g = 0; g < NG; g++) {
         const int b = g * 8 + rb;  // batch row of this thread in group g
         valid[g] = row_in && b < p.nb;
-        const float gr = DT::rnd(mma_reduce(part_g, g, rj, rb));
+        const float gr = DT::rnd(mma_reduce<DT>(part_g, g, rj, rb));
         a[g] = DT::rnd(gr / (1.f + expf(-gr)));
         act[g] = valid[g] && fabsf(a[g]) > p.t;
         bal |= __ballot(act[g]);
@@ -310,7 +354,7 @@ __global__ __launch_bounds__(kMmaThreads) void rows_mma_kernel(RowsArgs p) {
     __syncthreads();
     if (!UP) return;
 #pragma unroll
-    for (int g = 0; g < NG; g++) acc[g] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int g = 0; g < NG; g++) acc[g] = Mma<DT>::zero();
     if constexpr (CH == 2) {
       up.multiply(ucur, 0, acc);
       issue_up(r, 0, ucur);
@@ -320,13 +364,13 @@ __global__ __launch_bounds__(kMmaThreads) void rows_mma_kernel(RowsArgs p) {
       issue_up(r, 0, ucur);
       up.multiply(uprev, 0, acc);
     }
-    mma_store_partials<NG>(acc, part_u, lane, wave);
+    mma_store_partials<DT, NG>(acc, part_u, lane, wave);
     __syncthreads();
     if (wave == 0) {
 #pragma unroll
       for (int g = 0; g < NG; g++) {
         if (r >= 1 && prev_valid[g]) {
-          const float u = mma_reduce(part_u, g, rj, rb);
+          const float u = mma_reduce<DT>(part_u, g, rj, rb);
           const float z = prev_act[g] ? DT::rnd(prev_a[g] * DT::rnd(u)) : 0.f;
           const size_t o = (size_t)(g * 8 + rb) * p.N + prev_row;
           if (p.z32_out && ((prev_bits >> rj) & 1u)) p.z32_out[o] = z;
@@ -495,7 +539,7 @@ __global__ __launch_bounds__(kMmaThreads) void rows_mma_up_kernel(RowsArgs p) {
 #pragma unroll
     for (int gb = 0; gb < NG; gb++) {
       const int b = gb * 8 + rb;
-      const float u = mma_reduce(my_part, gb, rj, rb);
+      const float u = mma_reduce<DT>(my_part, gb, rj, rb);
       const float a = DT::tof(s_a[b * rows_pad + j]);
       if (j < nrows && b < p.nb) {
         const float z = s_f[b * rows_pad + j] ? DT::rnd(a * DT::rnd(u)) : 0.f;  // u of a row that was not read is noise: never used
@@ -507,17 +551,17 @@ __global__ __launch_bounds__(kMmaThreads) void rows_mma_up_kernel(RowsArgs p) {
   };
   // one tile: ra (and with two chunks rb2) hold it; they are refilled with what follows in the ring
   auto body = [&](int r, u32x4 (&ra)[STEPS], u32x4 (&rb2)[STEPS], float* my_part) {
-    f32x4 acc[NG];
+    typename Mma<DT>::Acc acc[NG];
 #pragma unroll
-    for (int g = 0; g < NG; g++) acc[g] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int g = 0; g < NG; g++) acc[g] = Mma<DT>::zero();
     up.multiply(ra, 0, acc);
     if constexpr (CH == 2) {
       issue(r + 1, 0, ra);
       up.multiply(rb2, 1, acc);
-      mma_store_partials<NG>(acc, my_part, lane, wave);
+      mma_store_partials<DT, NG>(acc, my_part, lane, wave);
       issue(r + 1, 1, rb2);
     } else {
-      mma_store_partials<NG>(acc, my_part, lane, wave);
+      mma_store_partials<DT, NG>(acc, my_part, lane, wave);
       issue(r + 2, 0, ra);
     }
     __syncthreads();

@@ -1,0 +1,63 @@
+"""fp32 batches of 5..16 rows: the matrix-core passes (x whole in LDS up to 4608 elements at 8 rows and 2300 at 16), the two dense
+products and their join beyond that, and the dense down product over rows of any length."""
+import pytest
+import torch
+import torch.nn.functional as F
+
+pytestmark = pytest.mark.gpu
+
+# H around the limits of one and two groups of x in LDS; I odd, below a tile, over 8192 (two launches of a product)
+SIZES = [(256, 613, 5), (36, 9, 16), (1024, 515, 9), (2304, 1000, 16), (2308, 1001, 16), (4608, 515, 8), (4612, 777, 5), (4612, 777, 11),
+         (260, 8200, 7), (5120, 8204, 8), (64, 4, 12)]
+
+
+def _data(H, I, B):
+    g = torch.Generator(device="cuda").manual_seed(H + I + B)
+    x = torch.randn(B, 1, H, generator=g, device="cuda")
+    wg, wu, wd = (torch.randn(I, H, generator=g, device="cuda") * H ** -0.5 for _ in range(3))
+    X = x.double().reshape(B, H)
+    a = F.silu(X @ wg.double().t())
+    # no activation within the error of a sum from the threshold: every order of summation keeps the same neurons
+    t = 0.2
+    near = ((a.abs() - t).abs() < 1e-5).any(0)
+    wg[near] = 0
+    a = F.silu(X @ wg.double().t())
+    a[a.abs() <= t] = 0
+    return x, wg, wu, wd, t, a, a * (X @ wu.double().t())
+
+
+def _close(got, want):
+    # fp32 sums over at most 8204 products in chains of K / 64 and a short tree: about sqrt(K / 64) * 2^-24 of the result's norm, three times
+    assert float((got.double().reshape(want.shape) - want).norm()) <= 2e-6 * float(want.norm()) + 1e-12
+
+
+@pytest.mark.parametrize("H,I,B", SIZES)
+def test_fp32_rows(H, I, B):
+    import flash_gemv
+
+    x, wg, wu, wd, t, a, z = _data(H, I, B)
+    want = z @ wd.double()
+    _close(flash_gemv.cats_mlp(x, wg, wu, wd, t), want)
+    out = torch.ones(B, H, device="cuda")
+    flash_gemv.flag_gemv_gemv_atomic(x, wg, wu, wd, out, t)
+    _close(out, want + 1)
+    y, flag, fetched = flash_gemv.cats_mlp_stats(x, wg, wu, wd, t)
+    _close(y, want)
+    assert int(fetched) == int((a != 0).any(0).sum())
+    if I % 4 == 0:
+        _close(flash_gemv.flag_gemv_gemv_inner_fp32(x, wg, wu, wd.t().contiguous(), t), want)
+
+
+def test_what_is_not_kept_does_not_count():
+    """An infinite up weight of a neuron that no row keeps, and of one that only some rows keep."""
+    import flash_gemv
+
+    for H in (256, 4612):
+        x, wg, wu, wd, t, a, z = _data(H, 404, 6)
+        wg[3], wu[3, 0] = 0, float("inf")
+        a[:, 3] = 0
+        some = int((a != 0).any(0).logical_and((a == 0).any(0)).nonzero()[0])
+        wu[some, 0] = float("inf")
+        y = flash_gemv.cats_mlp(x, wg, wu, wd, t).reshape(6, H)
+        keeps = a[:, some] != 0
+        assert not y[keeps].isfinite().any() and y[~keeps].isfinite().all()
