@@ -474,7 +474,10 @@ bool fused_eligible(int B, int H, int I, int dtype, FusedArgs& f, int& grid, boo
   if (maxgrid > kFusedMaxGrid) maxgrid = kFusedMaxGrid;
   if (B == 1) maxgrid *= kFusedPerCU;  // at two rows twice the workgroups would not fit the partial-sum region
   int rpw = (I + maxgrid - 1) / maxgrid;
-  if (rpw < 2 * rw) rpw = 2 * rw;  // small matrices: fewer workgroups rather than idle row waves
+  // Small matrices: at least half as many neurons as row waves, so that a wave takes one at most -- a second neuron is one more memory
+  // trip in a chain of four.  Fewer workgroups with two neurons a wave: 13.1 against 10.8 us at 512 / 1024, 14.4 against 12.0 at
+  // 1024 / 2731, 15.1 against 12.2 at two rows of 512 / 1995; one neuron a wave and no idle wave: 11.1, 12.3, 12.1.
+  if (rpw < rw / 2) rpw = rw / 2;
   grid = (I + rpw - 1) / rpw;
   f.rpw = rpw;
   f.spw = rpw;
