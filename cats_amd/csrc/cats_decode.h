@@ -8,9 +8,9 @@
 // x may be given before its RMS norm (norm_w), which is then applied while x is staged.  Everything between the weight
 // matrices stays in fp32 and is rounded once where it is stored.  All of it is bound by the weight stream: one wave owns two
 // rows of a matrix, whose loads are all in flight at once, as in rows_kernel.
-// One step of four layers 4096 / 11008, 32 heads, 32000 words, 256 tokens in the cache, fp16, one row: 338 us, of which the MLP
-// kernels take 160; with torch's operations in place of these kernels (about 25 launches a layer) it was 761.  Kernel trace: q, k, v
-// 18.7 us (5.4 TB/s), attention 6.6, output projection 8.4, output head 44 (5.9 TB/s).
+// One step of four layers 4096 / 11008, 32 heads, 32000 words, 256 tokens in the cache, fp16, one row: 327 us, of which the MLP
+// kernels take 150; with torch's operations in place of these kernels (about 25 launches a layer) it was 761.  Kernel trace: q, k, v
+// 18.9 us with the norm (5.3 TB/s), attention 6.6, output projection 8.4, output head 44 (5.9 TB/s).
 #pragma once
 #include "cats_rows.h"
 
