@@ -15,12 +15,16 @@
 // they lie, and only the step in which K ends looks where a vector ends.
 //
 // What bounds it at 4096 / 11008: up to 64 tokens the weight stream (41 us for gate and up, 21 for down at 32 tokens: 4.4 TB/s), at
-// 512 tokens the matrix cores and LDS in turn (110 and 65 us: 840 and 710 TFLOP/s; the matrix cores are busy 40 % of the time,
-// a step's fragment reads and stores take another 30 %, no bank conflicts).  Whole module call: 162 us at 512 tokens and 66 at 16, with the
-// library's products and one kernel between them 191 and 81; 304 / 569 at 22 tokens 24 us against 78, host time mostly.
+// 512 tokens the barrier of each step and what the waves wait for around it (102 and 61 us: 900 and 760 TFLOP/s; the matrix cores are
+// busy 45 % of the time, LDS 25 %, no bank conflicts).  Whole module call: 155 us at 512 tokens and 66 at 16, with the
+// library's products and one kernel between them 191 and 81; 304 / 569 at 22 tokens 20 us against 78, host time mostly.
+// With the end of K looked for in every step, 110 and 65 us; without the dealing of the loads between the MFMAs 101 and 64, and 142
+// against 130 for the 128 x 128 tile.
 // Measured and not taken: four waves with 128 x 96 sums each (155 us), two steps of loads in registers (no change at 256 tokens
-// and more), raised wave priority around the multiplications and stores between two halves of them (no change).
+// and more), raised wave priority around the multiplications (no change).
 #pragma once
+#include <type_traits>
+
 #include "cats_rows_mma.h"
 
 namespace cats {
@@ -51,6 +55,21 @@ struct PromptTile {
   static constexpr size_t LDS = 2 * (size_t)STEP * sizeof(u32x4);
   static constexpr int PASS = THREADS / P;         // rows that the threads load at a time
   static_assert(BM % PASS == 0 && BN % PASS == 0 && PASS % 8 == 0 && BN % 32 == 0 && BK % 64 == 0, "whole passes");
+};
+
+// Asks the scheduler to place RD LDS reads, WR LDS writes and LD loads, in this order, evenly between M MFMAs.
+template <int M, int RD, int WR, int LD>
+struct PromptDeal {
+  static constexpr int N = RD + WR + LD;
+  template <int I>
+  static __device__ __forceinline__ void go() {
+    if constexpr (I < N) {
+      __builtin_amdgcn_sched_group_barrier(I < RD ? 0x100 : I < RD + WR ? 0x200 : 0x020, 1, 0);
+      constexpr int m = (I + 1) * M / N - I * M / N;
+      if constexpr (m > 0) __builtin_amdgcn_sched_group_barrier(0x008, m, 0);
+      go<I + 1>();
+    }
+  }
 };
 
 template <class DT, class T, bool GATE_UP>
@@ -106,8 +125,8 @@ __global__ __launch_bounds__(T::THREADS) void prompt_kernel(PromptArgs p) {
     return u32x4{(uint32_t)rlo, (uint32_t)(rlo >> 32), (uint32_t)rhi, (uint32_t)(rhi >> 32)};
   };
   const int put = row * P + (piece ^ (row & 7));  // PASS is a multiple of 8: the same permutation for all of a thread's rows
-  auto store = [&](int step, int buf, u32x4 (&ra)[VA], u32x4 (&rb)[VB]) {
-    if (kbegin + (step + 1) * T::BK > p.K) {  // uniform
+  auto store = [&](int step, int buf, u32x4 (&ra)[VA], u32x4 (&rb)[VB], auto ends) {
+    if (ends && kbegin + (step + 1) * T::BK > p.K) {  // uniform
       const int s = over(step);
 #pragma unroll
       for (int i = 0; i < VA; i++) ra[i] = shifted(ra[i], s);
@@ -151,12 +170,15 @@ __global__ __launch_bounds__(T::THREADS) void prompt_kernel(PromptArgs p) {
   };
   // One barrier a step, in front of its last multiplication: by then everybody has read this step's buffer to the end (which the next
   // step overwrites) and written the next step's, whose first fragments arrive during that multiplication.  Steps past the
-  // last are loaded (the end of the rows again) and stored as well, and not used: no branches here.
-  auto step = [&](int s, int buf, u32x4 (&ra)[VA], u32x4 (&rb)[VB]) {
+  // last are loaded (the end of the rows again) and stored as well, and not used.  `ends`: K may end in the step that is stored.
+  // The LDS and memory instructions are dealt out between the MFMAs: issued in one go they queue, all waves of the CU at once, while
+  // the matrix cores wait.
+  auto step = [&](int s, int buf, u32x4 (&ra)[VA], u32x4 (&rb)[VB], auto ends) {
     fetch(buf, 1);
-    store(s + 1, buf ^ 1, ra, rb);
+    store(s + 1, buf ^ 1, ra, rb, ends);
     load(s + 1 + T::AHEAD, ra, rb);
     multiply(0);
+    if constexpr (KK == 2) PromptDeal<FM * FN, FM + FN, VA + VB, VA + VB>::template go<0>();
 #pragma unroll
     for (int kk = 1; kk < KK; kk++) {
       if (kk + 1 < KK) fetch(buf, kk + 1);
@@ -167,17 +189,24 @@ __global__ __launch_bounds__(T::THREADS) void prompt_kernel(PromptArgs p) {
       }
       multiply(kk & 1);
     }
+    if constexpr (KK == 2) PromptDeal<(FM * FN < FM + FN ? FM * FN : FM + FN), FM + FN, 0, 0>::template go<0>();
     __builtin_amdgcn_sched_barrier(0);
   };
   load(0, ring_a[0], ring_b[0]);
-  store(0, 0, ring_a[0], ring_b[0]);
+  store(0, 0, ring_a[0], ring_b[0], std::true_type());
 #pragma unroll
   for (int i = 1; i <= T::AHEAD; i++) load(i, ring_a[i % T::AHEAD], ring_b[i % T::AHEAD]);
   __syncthreads();
   fetch(0, 0);
-  for (int s = 0; s < nsteps; s += 2) {  // the loads of step s + 1 are in set (s + 1) % AHEAD
-    step(s, 0, ring_a[1 % T::AHEAD], ring_b[1 % T::AHEAD]);
-    if (s + 1 < nsteps) step(s + 1, 1, ring_a[0], ring_b[0]);
+  const int whole = min(nsteps, (p.K - kbegin) / T::BK);  // steps that K does not end in
+  int s = 0;  // the loads of step s + 1 are in set (s + 1) % AHEAD
+  for (; s + 2 < whole; s += 2) {
+    step(s, 0, ring_a[1 % T::AHEAD], ring_b[1 % T::AHEAD], std::false_type());
+    step(s + 1, 1, ring_a[0], ring_b[0], std::false_type());
+  }
+  for (; s < nsteps; s += 2) {
+    step(s, 0, ring_a[1 % T::AHEAD], ring_b[1 % T::AHEAD], std::true_type());
+    if (s + 1 < nsteps) step(s + 1, 1, ring_a[0], ring_b[0], std::true_type());
   }
 
   // lane: token fr of a fragment, four consecutive weight rows fq * 4 ..
