@@ -394,6 +394,7 @@ at::Tensor cats_mlp_gate_cols_op(const at::Tensor& x, const at::Tensor& wgate, c
   check_weight(wgate, x, H, I, "wgate (H, I)");
   check_weight(wup, x, I, H, "wup");
   check_weight(wdown_t, x, I, H, "wdown_t (neuron-major)");
+  const c10::DeviceGuard guard(x.device());
   at::Tensor out = at::empty_like(x);
   hipStream_t s = current_stream(x);
   Workspace& ws = workspace(x, 1, (int)H, (int)I, s);
@@ -482,6 +483,7 @@ at::Tensor cats_linear_op(const at::Tensor& x, const c10::optional<at::Tensor>& 
     TORCH_CHECK(norm_weight->scalar_type() == x.scalar_type() && norm_weight->numel() == K && norm_weight->device() == x.device(),
                 "flash_gemv.cats_linear: norm_weight must be a (K,) tensor of x's dtype on x's device");
   }
+  const c10::DeviceGuard guard(x.device());
   std::vector<int64_t> shape(x.sizes().begin(), x.sizes().end());
   shape.back() = N;
   at::Tensor out = at::empty(shape, x.options());
