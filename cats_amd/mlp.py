@@ -8,15 +8,16 @@ Same attribute switches as the reference, poked onto the module by the harness
 ``dead_threshold``, ``is_stats``, ``is_collect_histogram``, ``kill_sparse_swish_outputs``.
 
 ``sp_method`` when ``is_profile`` and the input is a decode step (``x.shape[1] == 1``):
-  0  dense-masked PyTorch (the reference's own fallback and the parity oracle's formula)
+  0  dense-masked PyTorch (the reference's own fallback and the parity oracle's formula), for a prompt too: no kernel of this
+     package takes part
   1  ``flash_gemv.flag_gemv_gemv_inner{,_fp32,_bf16}`` on the HF-layout down weight (dense down)
   2  ``flash_gemv.gemv_gemv_triton``: gate by the module, sparse up / down in HIP over ``wdown_t``; with a plain nn.Linear as the
      gate the same in one call
   3  ``flash_gemv.cats_mlp``: everything in two HIP launches over ``wdown_t`` (no reference counterpart: the
      reference has no single call with the gate fused in and neuron-major down weights)
-Prefill (``x.shape[1] > 1``) always takes the dense-masked branch, as in the reference (:900-904): on the GPU, in 16-bit types, as
-``cats_prompt_mlp`` up to the number of tokens where that is the faster one, else as three products of the library with the SiLU,
-threshold and product between them in one kernel.
+Prefill (``x.shape[1] > 1``) always takes the dense-masked branch, as in the reference (:900-904).  With ``sp_method`` 1 to 3, on the
+GPU and while nothing records gradients, it runs in 16-bit types as ``cats_prompt_mlp`` up to the number of tokens where that
+is the faster one, else as three products of the library with the SiLU, threshold and product between them in one kernel.
 """
 from __future__ import annotations
 
@@ -207,6 +208,8 @@ class CatsMLP(nn.Module):
         return weights
 
     def _dense_masked(self, x):
+        if self.sp_method == 0:  # the formula by torch's own operations: what the kernels are compared with
+            return self._mask_and_down(self.gate_proj(x), self.up_proj(x))
         weights = self._prompt_weights(x)
         if weights is not None:
             import flash_gemv  # noqa: F401

@@ -167,7 +167,10 @@ def test_cats_mlp_module_methods_agree(oracle):
         with torch.no_grad():
             wantp = mod(xp)
             mod.prepare_decode(3)
-            torch.testing.assert_close(mod(xp), wantp)
+            # Method 3 computes it by kernels of its own, whose fp32 sums run in another order than torch's: gate, up and z of a neuron
+            # may each round to the neighbouring value, three steps of z = 0.5 in the mean square times w = 0.05 over 1024 neurons of
+            # random signs.  In fp16 (step 2^-10) that is 32 * 0.025 * 3 * 2^-10 = 2.3e-3 if every one of them did.
+            torch.testing.assert_close(mod(xp).float(), wantp.float(), **TOL[dtype])
 
 
 def test_decode_loop_graph_replay_matches_eager():

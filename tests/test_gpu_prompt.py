@@ -47,3 +47,20 @@ def test_module_routes_agree(method, rows):
     if rows > 1 or method == 0:
         assert y.requires_grad
         torch.testing.assert_close(y, b, rtol=0, atol=0)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("shape", [(3, 1, 256), (1, 7, 256), (1, 600, 256)])
+def test_sp_method_0_is_torch_bit_for_bit(shape, dtype):
+    from cats_amd.mlp import CatsMLP
+
+    with torch.no_grad():
+        torch.manual_seed(1)
+        m = CatsMLP(256, 515, dead_threshold=0.05, dtype=dtype, device="cuda").eval()
+        for p in m.parameters():
+            p.normal_(0, 0.05)
+        m.is_profile, m.sp_method = True, 0
+        x = torch.randn(shape, device="cuda").to(dtype)
+        a = F.silu(F.linear(x, m.gate_proj.weight))
+        a[a.abs() <= 0.05] = 0
+        assert torch.equal(m(x), F.linear(a * F.linear(x, m.up_proj.weight), m.down_proj.weight))

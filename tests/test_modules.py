@@ -38,6 +38,23 @@ def test_cats_mlp_dense_masked_branch_matches_oracle(oracle):
     torch.testing.assert_close(m(xp, sp_mask=mask), want)
 
 
+def test_sp_method_0_takes_no_kernel_route(monkeypatch):
+    """What the kernel methods are compared with must not lead to a kernel itself, whatever the input."""
+    m = cm.CatsMLP(64, 96, dtype=torch.float32)
+    m.is_profile, m.sp_method, m.dead_threshold = True, 0, 0.08
+
+    def asked(*args):
+        raise AssertionError("sp_method 0 asked for a kernel route")
+
+    monkeypatch.setattr(cm.CatsMLP, "_prompt_weights", asked)
+    with torch.no_grad():
+        for shape in ((2, 1, 64), (1, 5, 64)):
+            m(torch.randn(shape))
+    model = tiny_model(layers=1)
+    model.set_mlp_mode("cats_torch")
+    assert model.layers[0].mlp.is_profile and model.layers[0].mlp.sp_method == 0
+
+
 def test_kernel_methods_fail_loudly_without_gpu():
     m = cm.CatsMLP(64, 96, dtype=torch.float16).prepare_decode(3)
     with pytest.raises(RuntimeError):
