@@ -209,7 +209,7 @@ class CatsMLP(nn.Module):
 
     def _dense_masked(self, x):
         if self.sp_method == 0:  # the formula by torch's own operations: what the kernels are compared with
-            return self._mask_and_down(self.gate_proj(x), self.up_proj(x))
+            return self._mask_and_down(x, self.gate_proj(x))
         weights = self._prompt_weights(x)
         if weights is not None:
             import flash_gemv  # noqa: F401
@@ -224,14 +224,15 @@ class CatsMLP(nn.Module):
                 import flash_gemv  # noqa: F401
 
                 return self.down_proj(torch.ops.flash_gemv.cats_silu_mask_mul(gate, up, float(t)))
-            return self._mask_and_down(gate, up)
-        return self._mask_and_down(gate, self.up_proj(x))
+            return self._mask_and_down(x, gate, up)
+        return self._mask_and_down(x, gate)
 
-    def _mask_and_down(self, gate, up):
+    def _mask_and_down(self, x, gate, up=None):
+        """The rest of the formula as torch computes it; up: up_proj(x) if it is there already."""
         post_act = self.act_fn(gate)
         dead_neurons = post_act.abs() <= self.dead_threshold
         post_act[dead_neurons] = 0
-        return self.down_proj(post_act * up)
+        return self.down_proj(post_act * (self.up_proj(x) if up is None else up))
 
     def forward(self, x, sp_mask: torch.Tensor = None):
         if sp_mask is not None:  # ugly_utils.py:872-875

@@ -55,6 +55,18 @@ def test_sp_method_0_takes_no_kernel_route(monkeypatch):
     assert model.layers[0].mlp.is_profile and model.layers[0].mlp.sp_method == 0
 
 
+def test_watched_modules_are_called_in_the_formula_s_order():
+    """gate, activation, up, down: what a hook sees does not depend on the method."""
+    for method in (0, 3):
+        m = cm.CatsMLP(64, 96, dtype=torch.float32).prepare_decode(method)
+        order = []
+        for name in ("down_proj", "up_proj", "act_fn", "gate_proj"):
+            getattr(m, name).register_forward_hook(lambda *args, name=name: order.append(name))
+        with torch.no_grad():
+            m(torch.randn(1, 5, 64))
+        assert order == ["gate_proj", "act_fn", "up_proj", "down_proj"]
+
+
 def test_kernel_methods_fail_loudly_without_gpu():
     m = cm.CatsMLP(64, 96, dtype=torch.float16).prepare_decode(3)
     with pytest.raises(RuntimeError):
