@@ -67,6 +67,25 @@ def _plain(t, dtype, device):
     return type(t) in (torch.Tensor, nn.Parameter) and t.dtype == dtype and t.device == device and t.is_contiguous() and t.data_ptr() % 16 == 0
 
 
+def _prompt_kernels_faster(tokens, H, I):
+    """Whether cats_prompt_mlp is the faster way for this many tokens (against three products of the library and the join between
+    them, and against torch's single operations; both sides fp16, us).
+
+    Up to 256 tokens it is from 304 / 569 (24 against 78 at 22 tokens) to 8192 / 28672 (432 against 633 at 256, 282 against 313 at 2);
+    8192 / 22016 and 8192 / 24576 at 2 to 96 tokens are even with torch's operations (within 2 %) and up to 6 % behind the library.
+    From 257 to 512 tokens a block of 256 tokens more is paid for, most of it padding at first, and the library's products of large
+    layers catch up: 4096 / 11008 148 against 189 at 512, 4096 / 14336 177 against 187 at 320, 6656 / 17920 346 against 374 at 320 and
+    401 against 442 at 512, but 8192 / 22016 518 against 478 and 8192 / 28672 652 against 542 at 320, 736 against 710 at 512.  The line
+    lies between the last two layers that differ in sign, 119 and 180 million weights a matrix.
+    Beyond, the library's larger tiles win where there is enough work for them: 700 tokens of 4096 / 11008 266 against 231, 87 against
+    85 of 2048 / 5632, but 62 against 83 at 600 tokens of it and 56 against 83 at 2048 of 1024 / 2731."""
+    if tokens < 1 or tokens > 4096:
+        return False
+    if tokens > 512:
+        return tokens * H * I <= 7e9
+    return tokens <= 256 or H * I <= 1.5e8
+
+
 class SparseSiLU(nn.SiLU):
     """SiLU followed by a symmetric dead zone: values with |a| <= threshold become 0 (ugly_utils.py:80-92)."""
 
@@ -199,11 +218,7 @@ class CatsMLP(nn.Module):
         if weights[1].shape != shape or weights[2].shape != shape[::-1] or x.shape[-1] != shape[1] or min(shape) < 8:
             return None
         I, H = shape
-        tokens = x.numel() // H
-        # Up to 512 tokens the kernels are the faster ones at every size measured (4096 / 11008: 66 against 81 us at 2, 163 against 195 at
-        # 512; 304 / 569: 24 against 78); from there on the library's larger tiles win where there is enough work for them
-        # (700 tokens of 4096 / 11008: 266 against 231 us, 87 against 85 of 2048 / 5632, but 44 against 80 of 1024 / 2731).
-        if not (1 <= tokens <= 512 or 512 < tokens <= 4096 and tokens * H * I <= 7e9) or 2 * H * (I + 8) >= 1 << 32:
+        if not _prompt_kernels_faster(x.numel() // H, H, I) or 2 * H * (I + 8) >= 1 << 32:
             return None
         return weights
 

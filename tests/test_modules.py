@@ -55,6 +55,14 @@ def test_sp_method_0_takes_no_kernel_route(monkeypatch):
     assert model.layers[0].mlp.is_profile and model.layers[0].mlp.sp_method == 0
 
 
+@pytest.mark.parametrize("tokens,H,I,kernels", [
+    (0, 4096, 11008, False), (1, 4096, 11008, True), (512, 4096, 14336, True), (512, 6656, 17920, True),   # up to 512 tokens
+    (256, 8192, 22016, True), (257, 8192, 22016, False), (256, 8192, 28672, True), (320, 8192, 28672, False), (512, 8192, 28672, False),
+    (600, 2048, 5632, True), (700, 2048, 5632, False), (700, 4096, 11008, False), (2048, 1024, 2731, True), (4097, 64, 64, False)])
+def test_which_prompts_go_to_the_kernels(tokens, H, I, kernels):
+    assert cm._prompt_kernels_faster(tokens, H, I) == kernels
+
+
 def test_watched_modules_are_called_in_the_formula_s_order():
     """gate, activation, up, down: what a hook sees does not depend on the method."""
     for method in (0, 3):
