@@ -71,6 +71,8 @@ def lib() -> ctypes.CDLL:
         L.cats_mlp_noalloc.argtypes = [vp, vp, vp, vp, vp, i32, i32, i32, i32, f32, vp]; L.cats_mlp_noalloc.restype = i32
         L.cats_up_index.argtypes = [vp, vp, vp, i32, vp, vp, i32, vp, i32, i32, i32, i32, vp]; L.cats_up_index.restype = i32
         L.cats_down_index.argtypes = [vp, vp, vp, i32, vp, vp, i32, i32, i32, i32, vp, sz, vp]; L.cats_down_index.restype = i32
+        if hasattr(L, "cats_mlp_gate_cols"):
+            L.cats_mlp_gate_cols.argtypes = [vp, vp, vp, vp, vp, i32, i32, i32, f32, vp, sz, vp]; L.cats_mlp_gate_cols.restype = i32
         L.cats_set_tuning.argtypes = [i32, i32, i32, i32]; L.cats_set_tuning.restype = i32
         _lib = L
     return _lib

@@ -359,6 +359,17 @@ int set_next_norm(ReduceArgs& r, const NextNorm& next, char* ws, const WsLayout&
 
 constexpr int kNotTaken = -1;  // internal: the shape or type rules this way out, take the other one
 
+// Neurons (or list entries) of a group of the sparse down pass, out of zcols; 0 if a group's list and z would not fit in LDS.
+// About one workgroup per CU over all slabs.
+int down_chunk(int zcols, int nslab, int B) {
+  int ngroup = g_tuning.down_groups > 0 ? g_tuning.down_groups : 256 / nslab;
+  if (ngroup < 1) ngroup = 1;
+  if (ngroup > kMaxGroups) ngroup = kMaxGroups;
+  if (B > kKernelBatch && ngroup > kMaxGroups / 2) ngroup = kMaxGroups / 2;  // the partial sums of 16 rows take twice the room
+  const int chunk = ((zcols + ngroup - 1) / ngroup + 7) / 8 * 8;
+  return (size_t)chunk * (1 + batch_template(B < kKernelBatch ? B : kKernelBatch)) * 4 > 96 * 1024 ? 0 : chunk;
+}
+
 // Sparse down over mask words already in the workspace.  Up to kKernelBatch rows; 16-bit types with an output that goes
 // through partial sums also take up to CATS_MAX_BATCH rows in one pass over W_down^T (matrix-core kernel) -- a call with
 // more than kKernelBatch rows that cannot go that way returns kNotTaken before anything is launched.
@@ -392,14 +403,9 @@ int do_down(const void* z, bool zf32, const void* wdown_t, float* y32, void* y_o
   if (block > 1024) block = 1024;
   while (block & (block - 1)) block &= block - 1;  // the fold across waves halves their number per round
   const int bt = batch_template(B < kKernelBatch ? B : kKernelBatch);
-  // about one workgroup per CU over all slabs; more groups if a group's list and z would not fit in LDS
-  int ngroup = g_tuning.down_groups > 0 ? g_tuning.down_groups : 256 / d.nslab;
-  if (ngroup < 1) ngroup = 1;
-  if (ngroup > kMaxGroups) ngroup = kMaxGroups;
-  if (B > kKernelBatch && ngroup > kMaxGroups / 2) ngroup = kMaxGroups / 2;  // the partial sums of 16 rows take twice the room
   const int zcols = idx ? M : I;  // what the groups split: the index list, or the neuron range
-  d.chunk = ((zcols + ngroup - 1) / ngroup + 7) / 8 * 8;
-  if ((size_t)d.chunk * (1 + bt) * 4 > 96 * 1024) return B > kKernelBatch ? kNotTaken : CATS_ERR_SHAPE;  // a group's list and z must fit in LDS
+  d.chunk = down_chunk(zcols, d.nslab, B);
+  if (d.chunk == 0) return B > kKernelBatch ? kNotTaken : CATS_ERR_SHAPE;
   d.ngroup = (zcols + d.chunk - 1) / d.chunk;
 #ifdef CATS_TIMING
   d.tbuf = g_tbuf_down;
@@ -1240,6 +1246,13 @@ int cats_mlp_gate_cols(const void* x, const void* wgate_hi, const void* wup, con
   WsLayout l;
   st = check_ws(ws, ws_bytes, H, I, l);
   if (st) return st;
+  FusedArgs f;
+  int grid = 0;
+  const bool single_pass = fused_eligible(1, H, I, dtype, f, grid);
+  if (!single_pass) {  // the separate kernels, checked before anything is launched
+    const int nslab = (H / vec_elems(dtype) + kWave - 1) / kWave;
+    if (nslab > kMaxSlabs || down_chunk(I, nslab, 1) == 0 || (size_t)I * esz(dtype) > l.mask - l.partial) return CATS_ERR_SHAPE;
+  }
   GateColsArgs g;
   g.x = x;
   g.w = wgate_hi;
@@ -1259,9 +1272,7 @@ int cats_mlp_gate_cols(const void* x, const void* wgate_hi, const void* wup, con
                  : dtype == CATS_BF16 ? launch_gate_cols<BF16>(g, groups, s)
                                       : launch_gate_cols<F32>(g, groups, s);
   if (e != hipSuccess) return CATS_ERR_LAUNCH;
-  FusedArgs f;
-  int grid = 0;
-  if (fused_eligible(1, H, I, dtype, f, grid)) {
+  if (single_pass) {
     f.x = (const u32x4*)x;
     f.a_part = g.partial;
     f.a_groups = groups;
@@ -1272,7 +1283,6 @@ int cats_mlp_gate_cols(const void* x, const void* wgate_hi, const void* wup, con
   }
   // Rows too long for the single-pass kernel: the activations as the separate kernels take them.  They lie where the down
   // pass, which runs after their last reader, will leave its partial sums.
-  if ((size_t)I * esz(dtype) > l.mask - l.partial) return CATS_ERR_SHAPE;
   void* a = (char*)ws + l.partial;
   e = dtype == CATS_F16    ? launch_gate_cols_finish<F16>(g, groups, a, s)
       : dtype == CATS_BF16 ? launch_gate_cols_finish<BF16>(g, groups, a, s)

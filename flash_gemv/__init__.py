@@ -50,6 +50,14 @@ from .kernels import (  # noqa: E402
 __version__ = "0.0.1"
 
 
+def _gate_cols_fits(H, I, size):
+    """Whether cats_mlp_gate_cols takes a layer of these sizes, whatever is kept: rows of up to 16 KiB go to the single-pass kernel, longer
+    ones to a down pass whose groups hold 12288 neurons in LDS, 256 groups over the slabs of 1 KiB of a row.  The list's own groups hold
+    the kept neurons only, so a call beyond this may still be one for the list."""
+    row = H * size
+    return I <= 1 << 18 if row <= 16384 else row <= 128 * 1024 and I <= 12288 * min(64, 256 // -(-row // 1024))
+
+
 def _takes_gate_cols(x, Wgate, Wup, Wdownt, threshold):
     """Whether one call of the kernels, from the gate on, gives what the composite below gives: one row of a 16-byte aligned x,
     one type, all weights as they lie, a plain number as threshold.  Everything else keeps torch's gate."""
@@ -57,7 +65,7 @@ def _takes_gate_cols(x, Wgate, Wup, Wdownt, threshold):
         return False
     H, I = Wgate.shape
     d, sz = x.dtype, x.element_size()
-    return (d in (torch.float16, torch.bfloat16, torch.float32) and x.shape[-1] == H and H * sz % 16 == 0 and I * sz >= 16
+    return (d in (torch.float16, torch.bfloat16, torch.float32) and x.shape[-1] == H and H * sz % 16 == 0 and I * sz >= 16 and _gate_cols_fits(H, I, sz)
             and Wup.shape == (I, H) and Wdownt.shape == (I, H) and Wgate.dtype == d and Wup.dtype == d and Wdownt.dtype == d
             and Wgate.device == x.device and Wup.device == x.device and Wdownt.device == x.device
             and Wgate.is_contiguous() and Wup.is_contiguous() and Wdownt.is_contiguous()

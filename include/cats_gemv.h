@@ -167,6 +167,8 @@ int cats_up_down(const void* x, const void* a, const void* wup, const void* wdow
 /* Whole CATS MLP for one row with the gate weight stored (H, I) -- x . wgate_hi, as the reference's index-list and Triton composites
  * take it -- and neuron-major wup, wdown_t (I, H).  Three launches: column sums of the gate pass, then cats_up_down's two, the
  * first of which finishes the activations.  wgate_hi needs the alignment of its element only (any I >= one 16-byte vector).
+ * I: at most 2^18 for rows of up to 16 KiB, else 12288 * min(64, 256 / (row bytes / 1024, rounded up)); CATS_ERR_SHAPE beyond what
+ * the kernels take, before anything is launched.
  * Replaces flag_gemv_gemv_dejavu and flag_gemv_gemv_triton at one row (flash_gemv/flash_gemv/__init__.py:38-54). */
 int cats_mlp_gate_cols(const void* x, const void* wgate_hi, const void* wup, const void* wdown_t, void* y_out, int H, int I,
                        int dtype, float threshold, void* ws, size_t ws_bytes, void* stream);

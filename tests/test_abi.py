@@ -133,3 +133,23 @@ def test_argument_validation_of_the_newer_entry_points():
     assert probe(p, 0, p, None) == 3
     assert probe(p, 24, p, None) == 3
     assert probe(odd, 64, p, None) == 3
+
+
+@pytest.mark.parametrize("dtype,size", [(0, 2), (2, 4)])
+@pytest.mark.parametrize("row,most", [(16384 + 16, 12288 * 15), (32768, 12288 * 8), (65536, 12288 * 4), (100 * 1024, 12288 * 2), (128 * 1024, 12288 * 2)])
+def test_column_major_gate_is_left_to_the_list_where_it_would_be_refused(row, most, dtype, size):
+    """The list's kernels split the kept neurons only; the call that stands for them splits all of them.  What it cannot take it refuses
+    before anything is launched (the pointers are never read), and flag_gemv_gemv_dejavu does not ask it."""
+    import flash_gemv
+    from cats_amd import capi
+
+    L = capi.lib()
+    buf = (ctypes.c_char * 4096)()
+    p = ctypes.c_void_p((ctypes.addressof(buf) + 255) // 256 * 256)
+    H = row // size
+    for I in (most + 1, most + 4096, 1 << 21):
+        assert not flash_gemv._gate_cols_fits(H, I, size)
+        assert L.cats_mlp_gate_cols(p, p, p, p, p, H, I, dtype, 0.1, p, L.cats_workspace_bytes(1, H, I), None) == 2
+    assert flash_gemv._gate_cols_fits(H, most, size)
+    assert flash_gemv._gate_cols_fits(16384 // size, 1 << 18, size) and not flash_gemv._gate_cols_fits(16384 // size, (1 << 18) + 1, size)
+    assert not flash_gemv._gate_cols_fits((128 * 1024 + 16) // size, 64, size)
