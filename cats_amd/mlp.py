@@ -86,6 +86,12 @@ def _prompt_kernels_faster(tokens, H, I):
     return tokens <= 256 or H * I <= 1.5e8
 
 
+def _prompt_fits(tokens, H, I):
+    """Whether cats_prompt_mlp takes these sizes: every matrix, the padded z among them, below 4 GiB."""
+    padded = (I + 7) // 8 * 8
+    return max(H, I) <= 1 << 28 and 2 * max(H * padded, tokens * H, tokens * padded) < 1 << 32
+
+
 class SparseSiLU(nn.SiLU):
     """SiLU followed by a symmetric dead zone: values with |a| <= threshold become 0 (ugly_utils.py:80-92)."""
 
@@ -218,7 +224,8 @@ class CatsMLP(nn.Module):
         if weights[1].shape != shape or weights[2].shape != shape[::-1] or x.shape[-1] != shape[1] or min(shape) < 8:
             return None
         I, H = shape
-        if not _prompt_kernels_faster(x.numel() // H, H, I) or 2 * H * (I + 8) >= 1 << 32:
+        tokens = x.numel() // H
+        if not (_prompt_kernels_faster(tokens, H, I) and _prompt_fits(tokens, H, I)):
             return None
         return weights
 

@@ -153,3 +153,17 @@ def test_column_major_gate_is_left_to_the_list_where_it_would_be_refused(row, mo
     assert flash_gemv._gate_cols_fits(H, most, size)
     assert flash_gemv._gate_cols_fits(16384 // size, 1 << 18, size) and not flash_gemv._gate_cols_fits(16384 // size, (1 << 18) + 1, size)
     assert not flash_gemv._gate_cols_fits((128 * 1024 + 16) // size, 64, size)
+
+
+@pytest.mark.parametrize("tokens,H,I", [
+    (512, 8, 4194296), (512, 8, 4194304), (513, 8, 4194296), (256, 8, 8388600), (256, 8, 8388608), (1, 8, (1 << 28) - 8), (1, 8, 1 << 28),
+    (512, 4194304, 8), (512, 4194296, 8), (1, 46336, 46336), (1, 46341, 46341), (512, 4096, 11008), (4096, 512, 1365)])
+def test_prompt_call_takes_what_the_module_sends_it(tokens, H, I):
+    """The pointers are never read: a size the call takes ends at the missing scratch, any other at its shape."""
+    from cats_amd import capi
+    from cats_amd.mlp import _prompt_fits
+
+    buf = (ctypes.c_char * 4096)()
+    p = ctypes.c_void_p((ctypes.addressof(buf) + 255) // 256 * 256)
+    status = capi.lib().cats_prompt_mlp(p, p, p, p, p, tokens, H, I, 0, 0.1, None, 0, None)
+    assert status == (6 if _prompt_fits(tokens, H, I) else 2)
