@@ -50,6 +50,18 @@ from .kernels import (  # noqa: E402
 __version__ = "0.0.1"
 
 
+_PLAIN = {torch.Tensor, torch.nn.Parameter}
+
+
+def _watched():
+    """Whether tracing, a transform, a mode or a module hook is at work that has to see the single torch operations of a composite."""
+    m = torch.nn.modules.module
+    return (torch.jit.is_tracing() or torch.compiler.is_compiling() or torch.is_autocast_enabled("cuda")
+            or torch._C._len_torch_dispatch_stack() or torch._C._len_torch_function_stack()
+            or torch._C._functorch.peek_interpreter_stack() is not None or torch.autograd.forward_ad._current_level >= 0
+            or m._global_forward_hooks or m._global_forward_pre_hooks)
+
+
 def _gate_cols_fits(H, I, size):
     """Whether cats_mlp_gate_cols takes a layer of these sizes, whatever is kept: rows of up to 16 KiB go to the single-pass kernel, longer
     ones to a down pass whose groups hold 12288 neurons in LDS, 256 groups over the slabs of 1 KiB of a row.  The list's own groups hold
@@ -60,8 +72,10 @@ def _gate_cols_fits(H, I, size):
 
 def _takes_gate_cols(x, Wgate, Wup, Wdownt, threshold):
     """Whether one call of the kernels, from the gate on, gives what the composite below gives: one row of a 16-byte aligned x,
-    one type, all weights as they lie, a plain number as threshold.  Everything else keeps torch's gate."""
-    if not (isinstance(threshold, (int, float)) and x.is_cuda and x.numel() == x.shape[-1] and x.is_contiguous() and Wgate.dim() == 2):
+    one type, all weights as they lie, a plain number as threshold, nothing that watches the operations.  Everything else keeps
+    torch's gate."""
+    if not (isinstance(threshold, (int, float)) and {type(x), type(Wgate), type(Wup), type(Wdownt)} <= _PLAIN
+            and not _watched() and x.is_cuda and x.numel() == x.shape[-1] and x.is_contiguous() and Wgate.dim() == 2):
         return False
     H, I = Wgate.shape
     d, sz = x.dtype, x.element_size()
@@ -69,7 +83,7 @@ def _takes_gate_cols(x, Wgate, Wup, Wdownt, threshold):
             and Wup.shape == (I, H) and Wdownt.shape == (I, H) and Wgate.dtype == d and Wup.dtype == d and Wdownt.dtype == d
             and Wgate.device == x.device and Wup.device == x.device and Wdownt.device == x.device
             and Wgate.is_contiguous() and Wup.is_contiguous() and Wdownt.is_contiguous()
-            and (x.data_ptr() | Wup.data_ptr() | Wdownt.data_ptr()) % 16 == 0 and not torch.is_autocast_enabled("cuda"))
+            and (x.data_ptr() | Wup.data_ptr() | Wdownt.data_ptr()) % 16 == 0)
 
 
 def flag_gemv_gemv_triton(x, Wgate, Wup, Wdownt, threshold):

@@ -70,3 +70,34 @@ def test_what_the_kernels_do_not_take_keeps_the_composite():
         assert not fg._takes_gate_cols(*args, 0.05)
     y = fg.flag_gemv_gemv_dejavu(d["x"], d["wg"].t(), d["wu"], d["wdt"], 0.05)
     torch.testing.assert_close(y, fg.flag_gemv_gemv_dejavu(*args, 0.05), rtol=1e-2, atol=2e-3)
+
+
+def test_watched_calls_keep_the_composite():
+    """A trace made at one row is of the operations and takes other rows later; a dispatch mode sees the gate's product."""
+    import flash_gemv as fg
+    from torch.utils._python_dispatch import TorchDispatchMode
+
+    H, I = 256, 512
+    d = dev(make_mlp(H, I, 2, torch.float16, seed=5))
+    wg_t, x = d["wg"].t().contiguous(), d["x"].view(2, 1, H)
+    traced = torch.jit.trace(lambda x: fg.flag_gemv_gemv_triton(x, wg_t, d["wu"], d["wdt"], 0.05), (x[:1].clone(),))
+    assert torch.equal(traced(x), fg.flag_gemv_gemv_triton(x, wg_t, d["wu"], d["wdt"], 0.05))
+
+    class Names(TorchDispatchMode):
+        def __init__(self):
+            super().__init__()
+            self.seen = []
+
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            self.seen.append(func.overloadpacket.__name__)
+            return func(*args, **(kwargs or {}))
+
+    with Names() as names:
+        fg.flag_gemv_gemv_dejavu(x[0], wg_t, d["wu"], d["wdt"], 0.05)
+    assert "nonzero" in names.seen and "silu" in names.seen
+
+    class Sub(torch.Tensor):
+        pass
+
+    assert not fg._takes_gate_cols(x[:1].as_subclass(Sub), wg_t, d["wu"], d["wdt"], 0.05)
+    assert fg._takes_gate_cols(x[:1], torch.nn.Parameter(wg_t), d["wu"], d["wdt"], 0.05)
