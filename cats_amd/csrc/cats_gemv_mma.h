@@ -94,6 +94,7 @@ __global__ __launch_bounds__(kMmaThreads) void gemv_mma_kernel(RowsArgs p) {
         xs[(buf * NG + gb) * kXGroup + i] = in ? xv[gb][k] : zero4();
       }
   };
+  const u32x4* idle = p.w + ((size_t)p.N * p.row_vecs >= 8 ? piece : 0);  // 4 x 4 of fp32 is half a line
   // weight loads of item (chunk c, tile t): this wave's steps are local steps wave * n(c) .. + n(c) - 1 of the chunk
   auto issue = [&](int c, int t, u32x4 (&dst)[CS]) {
     const bool item = c < nchunk && t < my_tiles;  // uniform
@@ -104,7 +105,7 @@ __global__ __launch_bounds__(kMmaThreads) void gemv_mma_kernel(RowsArgs p) {
     for (int s = 0; s < CS; s++) {
       const int vec = (step0 + s) * 8 + piece;
       const bool mine = s < nc && row < r1 && vec < p.row_vecs;
-      dst[s] = load_stream(mine ? p.w + (size_t)row * p.row_vecs + vec : p.w + piece);
+      dst[s] = load_stream(mine ? p.w + (size_t)row * p.row_vecs + vec : idle);
     }
   };
 

@@ -6,9 +6,11 @@ import torch.nn.functional as F
 
 pytestmark = pytest.mark.gpu
 
+# (4, 4): every matrix is half a cache line, and what a lane without work re-reads has to lie in it;
 # H around the limits of one and two groups of x in LDS; I odd, below a tile, over 8192 (two launches of a product)
 SIZES = [(256, 613, 5), (36, 9, 16), (1024, 515, 9), (2304, 1000, 16), (2308, 1001, 16), (4608, 515, 8), (4612, 777, 5), (4612, 777, 11),
-         (260, 8200, 7), (5120, 8204, 8), (64, 4, 12)]
+         (260, 8200, 7), (5120, 8204, 8), (64, 4, 12),
+         (4, 4, 5), (4, 4, 16)]
 
 
 def _data(H, I, B):
