@@ -319,27 +319,52 @@ constexpr int kJoinRows = 32;  // weight rows a workgroup of the fp32 matrix-cor
 
 // fp32 gate + up (a as for kGateUp, no norm, at least five batch rows) as two dense GEMVs and gate_up_join_kernel, where rows_mma_kernel
 // does not take all the rows of x at once.  It reads every row of W_up, which from five batch rows on is little more than their union.
+// The gate call and the gate + up call go the same way there, so that all three agree on every activation.
 bool joined_takes(int dtype, const RowsArgs& a) {
   if (dtype != CATS_F32 || a.nb <= 4 || a.nb > CATS_MAX_BATCH || a.norm_w || g_tuning.gate_variant < 0) return false;
   RowsArgs one = a;
   one.mma = 1;
   return a.nb > kKernelBatch ? !rows_mma16_supported<F32>(one) : !rows_takes_mma<F32>(kGateUp, kKernelBatch, one);
 }
-// sums: 16 * N floats of scratch, z: (nb, N), which takes the up sums first
-int do_joined(const RowsArgs& a, float* sums, float* z, hipStream_t s) {
+// x . w^T in launches of at most kJoinRows rows a workgroup; a.zt_out, a_in, a_out and flag_out as gemv_mma_kernel takes them.
+int do_joined_product(const RowsArgs& a, const u32x4* w, hipStream_t s) {
   const int most = current_device_cus() * kJoinRows, parts = (a.N + most - 1) / most;
   const int per = ((a.N + parts - 1) / parts + 7) / 8 * 8;
-  for (int m = 0; m < 2; m++)
-    for (int n0 = 0; n0 < a.N; n0 += per) {
-      RowsArgs g = a;
-      g.w = (m ? a.w2 : a.w) + (size_t)n0 * a.row_vecs;
-      g.w2 = nullptr;
-      g.N = a.N - n0 < per ? a.N - n0 : per;
-      g.zt_out = (m ? z : sums) + n0;
-      g.z32_out = nullptr;
-      g.flag_out = g.mask_out = g.ubytes_out = nullptr;
-      if (int st = do_rows(kGemv, CATS_F32, g, s)) return st;
-    }
+  for (int n0 = 0; n0 < a.N; n0 += per) {
+    RowsArgs g = a;
+    g.w = w + (size_t)n0 * a.row_vecs;
+    g.w2 = nullptr;
+    g.N = a.N - n0 < per ? a.N - n0 : per;
+    if (g.zt_out) g.zt_out = (float*)a.zt_out + n0;
+    if (g.a_in) g.a_in = (const float*)a.a_in + n0;
+    if (g.a_out) g.a_out = (float*)a.a_out + n0;
+    if (g.flag_out) g.flag_out = a.flag_out + n0;
+    if (int st = do_rows(kGemv, CATS_F32, g, s)) return st;
+  }
+  return CATS_OK;
+}
+// The gate call (a as for kGate): the same sums and the same activations as do_joined's.
+int do_joined_gate(const RowsArgs& a, hipStream_t s) { return do_joined_product(a, a.w, s); }
+// The gate + up call (a as for kGateUp with zt_out and no mask): the activations wait in zt_out for the up sums.
+int do_joined_gate_up(const RowsArgs& a, hipStream_t s) {
+  RowsArgs g = a;
+  g.zt_out = nullptr;
+  g.a_out = a.zt_out;
+  if (int st = do_joined_product(g, a.w, s)) return st;
+  g = a;
+  g.a_in = a.zt_out;
+  g.flag_out = nullptr;
+  return do_joined_product(g, a.w2, s);
+}
+// sums: nb * N floats of scratch, z: (nb, N), which takes the up sums first
+int do_joined(const RowsArgs& a, float* sums, float* z, hipStream_t s) {
+  RowsArgs g = a;
+  g.z32_out = nullptr;
+  g.flag_out = g.mask_out = g.ubytes_out = nullptr;
+  for (int m = 0; m < 2; m++) {
+    g.zt_out = m ? z : sums;
+    if (int st = do_joined_product(g, m ? a.w2 : a.w, s)) return st;
+  }
   GateUpJoinArgs j = {sums, z, z, a.flag_out, a.ubytes_out, a.N, a.nb, a.t};
   return launch_kernel(gate_up_join_kernel, dim3((a.N + 255) / 256), dim3(256), 0, s, j) == hipSuccess ? CATS_OK : CATS_ERR_LAUNCH;
 }
@@ -657,6 +682,7 @@ static int gate_flag_pass(const void* x, const void* wgate, void* a_out, uint8_t
   a.a_out = a_out;
   a.flag_out = flag_out;
   a.t = round_through(dtype, threshold);
+  if (joined_takes(dtype, a)) return do_joined_gate(a, (hipStream_t)stream);
   return wide ? rows_wide(a, dtype, stream) : do_rows(kGate, dtype, a, (hipStream_t)stream);
 }
 
@@ -770,6 +796,7 @@ static int gate_up_pass(const void* x, const void* wgate, const void* wup, void*
   a.zt_out = out;
   a.flag_out = flag_out;
   a.t = round_through(dtype, threshold);
+  if (joined_takes(dtype, a)) return do_joined_gate_up(a, (hipStream_t)stream);
   return wide ? rows_wide(a, dtype, stream) : do_rows(kGateUp, dtype, a, (hipStream_t)stream);
 }
 

@@ -15,6 +15,8 @@
 //    two register sets addressed statically: the tile loop is unrolled).  Deeper rings measure slower at both batch widths
 //    (three and four items: +1 to +3 us): the CU's miss queue is full before that, and a wave that blocks at issue
 //    multiplies late.
+// In fp32 it also does the gate and up passes of rows that rows_mma_kernel cannot hold on chip: without zt_out it takes SiLU of the sums
+// and writes a_out and flag_out (|a| > t), with a_in it writes a_in * sum where |a_in| > t, else 0.
 // A workgroup owns ceil(N / grid) consecutive rows (16 at N = 4096 on 256 CUs) in at most TILES tiles of eight.
 // Steps past the end of a row are padding: their loads re-read the first bytes of the matrix (cached, nothing moves from
 // HBM), what they brought is replaced by zeros at its use and their x operands are zero.
@@ -189,7 +191,23 @@ __global__ __launch_bounds__(kMmaThreads) void gemv_mma_kernel(RowsArgs p) {
     const int row = r0 + t * kMmaTileRows + rj, b = gb * 8 + rb;
     const float* src = part + ((size_t)t * NG + gb) * kMmaPart + (rj & 3) * 32 + (rj >> 2) * 8 + rb;
     const float u = mma_sum_waves<DT>(src, TILES * NG * kMmaPart);
-    if (t < my_tiles && row < r1 && b < p.nb) ((st*)p.zt_out)[(size_t)b * p.out_pitch + row] = DT::fromf(u);
+    if (t < my_tiles && row < r1 && b < p.nb) {
+      const size_t at = (size_t)b * p.out_pitch + row;
+      if constexpr (sizeof(st) == 4) {
+        if (!p.zt_out) {  // the gate pass
+          const float a = u / (1.f + expf(-u));
+          if (p.a_out) ((st*)p.a_out)[at] = a;
+          if (p.flag_out) p.flag_out[at] = fabsf(a) > p.t ? 1 : 0;
+        } else if (p.a_in) {  // the up pass behind it; zt_out may be a_in
+          const float a = ((const st*)p.a_in)[at];
+          ((st*)p.zt_out)[at] = fabsf(a) > p.t ? a * u : 0.f;
+        } else {
+          ((st*)p.zt_out)[at] = u;
+        }
+      } else {
+        ((st*)p.zt_out)[at] = DT::fromf(u);
+      }
+    }
   }
   CATS_RSTAMP(7);
 }

@@ -138,7 +138,7 @@ struct MmaLaunch {
   // four times the registers)
   static constexpr int kGemvTiles = kHasUp ? 8 : 4;
   static bool supported_gemv(const RowsArgs& a) {
-    return a.zt_out && !a.norm_w && !a.bias && !a.scale && a.nb <= 16 && a.K % DT::VEC == 0 && up_rows_pad(a) <= kGemvTiles * kMmaTileRows;
+    return (a.zt_out || (!kHasUp && (a.a_out || a.flag_out))) && !a.norm_w && !a.bias && !a.scale && a.nb <= 16 && a.K % DT::VEC == 0 && up_rows_pad(a) <= kGemvTiles * kMmaTileRows;
   }
   template <int NG>
   static hipError_t run_gemv_ng(const RowsArgs& a, hipStream_t stream) {
@@ -155,8 +155,10 @@ struct MmaLaunch {
 // still the faster one (28.4 vs 29.4 us).  From three rows on it wins at every row length (gate + up, wave-per-row against
 // matrix cores: 255 against 129 us for 28672 rows of 8192 elements at 8 batch rows; whole MLP calls: 22.0 against 15.7 us for 3000
 // rows of 1024 at 4, 162 against 75 us for 13824 rows of 5120 at 8, 57 against 21 us for 3931 rows of 1264 at 11, where the
-// other way is two passes).  The plain gate pass goes the same way as gate + up, so a gate call and a fused
-// call produce the same activations bit for bit.
+// other way is two passes).  The plain gate pass goes the same way as gate + up -- in fp32 beyond this kernel's rows too, see
+// joined_takes -- so a gate call and a fused call produce the same activations bit for bit.  (Where an up matrix that starts at
+// another place of a cache line than the gate matrix takes the fused call past the last row length that fits on chip, the two differ
+// in the order of their sums; so do a call with a norm and one without from nine fp32 rows of more than 2240 elements.)
 template <class DT>
 bool takes_mma(int mode, int bt, const RowsArgs& a) {
   if (bt < 4 || !a.mma) return false;

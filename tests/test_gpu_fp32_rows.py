@@ -63,3 +63,28 @@ def test_what_is_not_kept_does_not_count():
         y = flash_gemv.cats_mlp(x, wg, wu, wd, t).reshape(6, H)
         keeps = a[:, some] != 0
         assert not y[keeps].isfinite().any() and y[~keeps].isfinite().all()
+
+
+@pytest.mark.parametrize("H,I,B", [(256, 613, 5), (4608, 515, 8), (4612, 777, 5), (4612, 777, 11), (2240, 300, 16), (2244, 515, 9), (2308, 1001, 16),
+                                   (5120, 8204, 8), (4096, 1000, 16)])
+def test_gate_call_and_fused_calls_share_their_activations(H, I, B):
+    """With a threshold that is one of the gate call's own activations, bit for bit, every call flags exactly what it flags: a sum in another
+    order moves some activation across it."""
+    from cats_amd import capi
+
+    x, wg, wu, wd, _, a64, _ = _data(H, I, B)
+    x[:, 0, 0] = 1
+    wu.zero_()
+    wu[:, 0] = 1                                     # the up sum is 1: z is the activation
+    X, ws = x.reshape(B, H), capi.Workspace(B, H, I)
+    a, flag = capi.gate_flag(X, wg, 0.2)
+    # fp32 sums over H products of unit variance in chains of K / 64: see _close; single values up to six of their deviations
+    assert float((a.double() - F.silu(X.double() @ wg.double().t())).abs().max()) < 6 * 2e-6
+    for k in range(0, a.numel(), max(1, a.numel() // 40)):
+        t = float(a.flatten()[k].abs())
+        _, flag = capi.gate_flag(X, wg, t, want_a=False)
+        assert torch.equal(flag, a.abs() > t)
+        z, flag_up = capi.gate_up(X, wg, wu, t)
+        assert torch.equal(flag_up, flag) and torch.equal(z, torch.where(flag, a, torch.zeros_like(a)))
+        _, flag_mlp, _ = capi.mlp(X, wg, wu, wd, t, ws, want_flag=True, want_count=True)
+        assert torch.equal(flag_mlp, flag)
