@@ -1085,11 +1085,12 @@ int cats_mlp(const void* x, const void* wgate, const void* wup, const void* wdow
     return st;
   const bool union_count = count_out && B > kKernelBatch;  // a pass counts its own rows only: count the union of the flags instead
   if (union_count && !flag_out) {
-    // no flags asked for: the passes write them into the workspace region of the row-major intermediate, which no MLP pass uses
+    // no flags asked for: the passes write them into `atmp`, which no pass of at most kKernelBatch rows uses (do_joined's sums of
+    // eight rows fill `zt`; those of more rows go on into `atmp`, but then there are no passes)
     WsLayout l;
     if (int st = check_common(kKernelBatch, H, I, dtype)) return st;
     if (int st = check_ws(ws, ws_bytes, H, I, l)) return st;
-    flag_out = (uint8_t*)ws + l.zt;  // 8 * I * 4 bytes hold CATS_MAX_BATCH * I flags
+    flag_out = (uint8_t*)ws + l.atmp;  // 8 * I * 4 bytes hold CATS_MAX_BATCH * I flags
   }
   int st = in_passes(B, [&](size_t b0, int nb) {
     return mlp_pass(at_cbytes(x, b0 * H * sz), wgate, wup, wdown_t, at_bytes(y_out, b0 * H * sz), (float*)at_bytes((void*)y_f32, b0 * H * 4),

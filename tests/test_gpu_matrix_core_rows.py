@@ -107,3 +107,25 @@ def test_norm_while_staging(oracle, H, I, B, dtype):
     torch.cuda.synchronize()
     want = h.float() + oracle.c_mlp(x, m["wg"], m["wu"], m["wd"], t, a_in=a.cpu(), flag_in=flag.cpu())["y"].float()
     close(out.cpu(), want, dtype)
+
+
+@pytest.mark.parametrize("H,I,B,dtype,variant", [(5128, 263, 16, torch.float16, 0), (4488, 200, 9, torch.bfloat16, 0), (4612, 777, 13, torch.float32, -1)])
+def test_count_of_a_call_in_two_passes(H, I, B, dtype, variant):
+    """Rows that no one-pass kernel takes: the count without flags, whose bytes wait in the workspace while the second pass runs, is
+    that of the flags."""
+    m = make_mlp(H, I, B, dtype, seed=H + B)
+    d = dev(m)
+    ws = capi.Workspace(B, H, I)
+    L = capi.lib()
+    t = float(capi.gate_flag(d["x"], d["wg"], -1.0)[0].float().abs().flatten().quantile(0.95))
+    count, y2 = torch.full((1,), -1, dtype=torch.int32, device="cuda"), torch.empty(B, H, dtype=dtype, device="cuda")
+    L.cats_set_tuning(variant, 0, 0, 0)
+    try:
+        y, flag, with_flags = capi.mlp(d["x"], d["wg"], d["wu"], d["wdt"], t, ws, want_flag=True, want_count=True)
+        assert L.cats_mlp(capi._p(d["x"]), capi._p(d["wg"]), capi._p(d["wu"]), capi._p(d["wdt"]), capi._p(y2), None, None, capi._p(count), B, H, I,
+                          capi.DTYPE_CODE[dtype], t, capi._p(ws.buf), ws.nbytes, capi._stream(d["x"])) == 0
+        torch.cuda.synchronize()
+    finally:
+        L.cats_set_tuning(0, 0, 0, 0)
+    want = int(flag.any(dim=0).sum())
+    assert 0 < want < I and int(count) == want and int(with_flags) == want and torch.equal(y.view_as(y2), y2)
