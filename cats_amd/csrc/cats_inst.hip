@@ -158,7 +158,7 @@ struct MmaLaunch {
 // other way is two passes).  The plain gate pass goes the same way as gate + up -- in fp32 beyond this kernel's rows too, see
 // joined_takes -- so a gate call and a fused call produce the same activations bit for bit.  (Where an up matrix that starts at
 // another place of a cache line than the gate matrix takes the fused call past the last row length that fits on chip, the two differ
-// in the order of their sums; so do a call with a norm and one without from nine fp32 rows of more than 2240 elements.)
+// in the order of their sums; so do a layer tail and a call without its norm at 9..16 fp32 rows of more than 2180 elements.)
 template <class DT>
 bool takes_mma(int mode, int bt, const RowsArgs& a) {
   if (bt < 4 || !a.mma) return false;

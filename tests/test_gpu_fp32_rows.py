@@ -1,5 +1,5 @@
-"""fp32 batches of 5..16 rows: the matrix-core passes (x whole in LDS up to 4608 elements at 8 rows and 2300 at 16), the two dense
-products and their join beyond that, and the dense down product over rows of any length."""
+"""fp32 batches of 5..16 rows: the matrix-core passes (x whole in LDS up to 4580 elements at 8 rows and 2180 at 16, and rows of whole
+128-byte lines up to 4608 and 2240), the two dense products and their join beyond that, and the dense down product over rows of any length."""
 import pytest
 import torch
 import torch.nn.functional as F
@@ -10,7 +10,7 @@ pytestmark = pytest.mark.gpu
 # H around the limits of one and two groups of x in LDS; I odd, below a tile, over 8192 (two launches of a product)
 SIZES = [(256, 613, 5), (36, 9, 16), (1024, 515, 9), (2304, 1000, 16), (2308, 1001, 16), (4608, 515, 8), (4612, 777, 5), (4612, 777, 11),
          (260, 8200, 7), (5120, 8204, 8), (64, 4, 12),
-         (4, 4, 5), (4, 4, 16)]
+         (4, 4, 5), (4, 4, 16), (2180, 301, 16), (2184, 301, 16), (2240, 300, 16), (2244, 300, 16), (4580, 201, 7), (4584, 201, 7)]
 
 
 def _data(H, I, B):
@@ -88,3 +88,22 @@ def test_gate_call_and_fused_calls_share_their_activations(H, I, B):
         assert torch.equal(flag_up, flag) and torch.equal(z, torch.where(flag, a, torch.zeros_like(a)))
         _, flag_mlp, _ = capi.mlp(X, wg, wu, wd, t, ws, want_flag=True, want_count=True)
         assert torch.equal(flag_mlp, flag)
+
+
+@pytest.mark.parametrize("H,B,steps,joined", [
+    (2180, 9, (0, 7, 33), False), (2184, 9, (0, 7, 33), True), (2240, 16, (0, 7, 33), False), (2244, 16, (0, 7, 33), True),
+    (4580, 8, (0, 17, 115), False), (4584, 8, (0, 17, 115), True), (4608, 5, (0, 17, 115), False), (4612, 5, (0, 17, 115), True)])
+def test_where_the_one_launch_kernel_ends(H, B, steps, joined):
+    """Which kernel it is, told by the order of its sums: 1 and twice t, t below half a unit in the last place of 1 and 2t above it, in three
+    steps of 32 elements.  The one-launch kernel gives a wave consecutive steps, so one wave adds both t first: 1 + 2^-23.  The joined
+    products deal the steps of a chunk to all waves: each t meets the 1, or a wave with nothing, by itself: 1."""
+    from cats_amd import capi
+
+    t = 0.75 * 2.0 ** -24
+    w, x = torch.zeros(64, H, device="cuda"), torch.ones(B, H, device="cuda")
+    for step, v in zip(steps, (t, t, 1.0)):
+        w[0, 32 * step] = v
+    a, _ = capi.gate_flag(x, w, -1.0)
+    one, more = (F.silu(torch.tensor([v], dtype=torch.float64)).item() for v in (1.0, 1.0 + 2.0 ** -23))
+    a = a[:, 0].double()
+    assert bool(((a - (one if joined else more)).abs() < (a - (more if joined else one)).abs()).all())

@@ -36,8 +36,15 @@ ROWS = [
     (5128, 263, 7, torch.bfloat16),   # 81 or 82 steps: eleven per wave, rounded up to twelve
     (8184, 200, 5, torch.float16),    # 128 steps or 129
     (8192, 520, 8, torch.float16),
-    (9152, 64, 4, torch.bfloat16),    # the longest row whose eight x operands fit in LDS
-    (9216, 64, 3, torch.float16),     # one step more than the register sets hold is the wave-per-row kernel's
+    (9152, 64, 4, torch.bfloat16),
+    (9216, 64, 3, torch.float16),     # whole lines, no phase: the longest row whose eight x operands fit in LDS
+    (9160, 65, 5, torch.float16),     # the longest one with phases
+    (9168, 65, 5, torch.float16),     # its operands do not fit any more: the wave-per-row kernel's
+    (9224, 64, 8, torch.bfloat16),    # more steps than the register sets hold
+    (4360, 65, 16, torch.float16),    # two groups of operands: the longest row with phases
+    (4368, 65, 16, torch.bfloat16),   # two passes of eight
+    (4480, 64, 16, torch.bfloat16),   # the longest row of whole lines
+    (4488, 64, 16, torch.float16),
     (1024, 256 * 8 + 1, 6, torch.float16),   # nine rows per workgroup: a full tile and one row of the next
 ]
 
@@ -129,3 +136,25 @@ def test_count_of_a_call_in_two_passes(H, I, B, dtype, variant):
         L.cats_set_tuning(0, 0, 0, 0)
     want = int(flag.any(dim=0).sum())
     assert 0 < want < I and int(count) == want and int(with_flags) == want and torch.equal(y.view_as(y2), y2)
+
+
+@pytest.mark.parametrize("H,B,dtype,matrix_cores", [
+    (9160, 5, torch.float16, True), (9168, 5, torch.float16, False), (9216, 3, torch.bfloat16, True), (9224, 3, torch.bfloat16, False),
+    (4360, 9, torch.bfloat16, True), (4368, 9, torch.bfloat16, False), (4480, 9, torch.float16, True), (4488, 9, torch.float16, False),
+    (9216, 2, torch.float16, False)])
+def test_where_the_matrix_cores_end(H, B, dtype, matrix_cores):
+    """Which kernel took the last batch row, told by the order of its sums: the products of a row cancel in pairs, so what is left of a sum
+    is its rounding errors.  With the tuning knob the row goes to the wave-per-row kernel, which adds in one order whatever B is.  Of nine
+    rows the last is a pass of its own unless all go in one."""
+    g = torch.Generator(device="cuda").manual_seed(H)
+    half = torch.randn(96, H // 2, generator=g, device="cuda").to(dtype)
+    w = torch.cat((half, -half), 1)
+    x1 = torch.randn(B, H // 2, generator=g, device="cuda").to(dtype)
+    x = torch.cat((x1, x1), 1)
+    a, _ = capi.gate_flag(x, w, -1.0)
+    capi.set_tuning(-1, 0, 0, 0)
+    try:
+        b, _ = capi.gate_flag(x, w, -1.0)
+    finally:
+        capi.set_tuning(0, 0, 0, 0)
+    assert torch.equal(a[-1], b[-1]) != matrix_cores
