@@ -11,6 +11,8 @@ pytestmark = pytest.mark.gpu
 SIZES = [  # tokens, H, I
     (1, 8, 8), (2, 8, 9), (3, 72, 17), (22, 304, 569), (31, 128, 130), (32, 136, 127), (33, 200, 1041), (64, 1024, 515), (65, 264, 2731),
     (128, 520, 1000), (129, 1288, 333), (257, 512, 4099), (300, 2048, 5461), (256, 4096, 11008), (511, 4096, 11003), (1030, 77, 91),
+    # a long K over few columns: the second product in ranges of K, whose sums have a pitch of whole quads of columns
+    (33, 77, 2731), (5, 201, 5461), (200, 333, 4099), (64, 78, 3001), (65, 9, 2731),
 ]
 
 
@@ -92,3 +94,17 @@ def test_module_takes_it_and_leaves_it():
             a = m(x)
     assert m._prompt_weights(x) is None  # gradients
     assert a.shape == x.shape and b.shape == x.shape
+
+
+@pytest.mark.parametrize("M,H,I", [(33, 77, 2731), (5, 201, 5461), (64, 78, 3001), (65, 9, 2731), (40, 13, 21)])
+def test_nothing_is_written_behind_y(M, H, I):
+    """Columns that are no whole quad: y and the scratch end where the call says they end."""
+    from cats_amd import capi
+
+    x, wg, wu, wd = _draw(M, H, I, torch.bfloat16)
+    want = torch.ops.flash_gemv.cats_prompt_mlp(x, wg, wu, wd, 0.1)
+    L = capi.lib()
+    size = L.cats_prompt_scratch_bytes(M, H, I)
+    y, scratch = torch.full((M * H + 512,), 7.0, dtype=torch.bfloat16, device="cuda"), torch.full((size + 4096,), 7, dtype=torch.uint8, device="cuda")
+    assert L.cats_prompt_mlp(*(capi._p(t) for t in (x, wg, wu, wd, y)), M, H, I, capi.BF16, 0.1, capi._p(scratch), size, capi._stream(x)) == 0
+    assert torch.equal(y[:M * H].view(M, H), want) and bool((y[M * H:] == 7).all()) and bool((scratch[size:] == 7).all())
