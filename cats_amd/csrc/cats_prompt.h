@@ -45,10 +45,10 @@ struct PromptArgs {
   float t;
 };
 
-// WM x WN waves of FM x FN fragments (16 tokens x 16 weight rows) each, steps of BK elements, AHEAD steps of loads in registers.
-template <int WM_, int WN_, int FM_, int FN_, int BK_, int AHEAD_>
+// WM x WN waves of FM x FN fragments (16 tokens x 16 weight rows) each, steps of BK elements.
+template <int WM_, int WN_, int FM_, int FN_, int BK_>
 struct PromptTile {
-  static constexpr int WM = WM_, WN = WN_, FM = FM_, FN = FN_, BK = BK_, AHEAD = AHEAD_;
+  static constexpr int WM = WM_, WN = WN_, FM = FM_, FN = FN_, BK = BK_;
   static constexpr int THREADS = WM * WN * kWave, BM = WM * FM * 16, BN = WN * FN * 16;
   static constexpr int P = BK / 8;                 // 16-byte pieces of a row
   static constexpr int STEP = (BM + BN) * P;       // vectors of one LDS buffer
@@ -109,8 +109,8 @@ __global__ __launch_bounds__(T::THREADS) void prompt_kernel(PromptArgs p) {
   // Elements of this thread's vector of a step that lie behind K.  The vector in which K ends is read so that it ends with the row
   // and shifted down before it is stored; those behind it are stored as zeros.
   auto over = [&](int step) { return max(kbegin + step * T::BK + piece * 8 + 8 - p.K, 0); };
-  u32x4 ring_a[T::AHEAD][VA], ring_b[T::AHEAD][VB];
-  auto load = [&](int step, u32x4 (&ra)[VA], u32x4 (&rb)[VB]) {
+  u32x4 ra[VA], rb[VB];  // the step that is stored next
+  auto load = [&](int step) {
     const uint32_t at = (uint32_t)(kbegin + step * T::BK - over(step)) * 2u;
 #pragma unroll
     for (int i = 0; i < VB; i++) rb[i] = *(const u32x4_elem*)((const char*)(is_up(i) ? p.w2 : p.w) + (ob[i] + at));
@@ -125,7 +125,7 @@ __global__ __launch_bounds__(T::THREADS) void prompt_kernel(PromptArgs p) {
     return u32x4{(uint32_t)rlo, (uint32_t)(rlo >> 32), (uint32_t)rhi, (uint32_t)(rhi >> 32)};
   };
   const int put = row * P + (piece ^ (row & 7));  // PASS is a multiple of 8: the same permutation for all of a thread's rows
-  auto store = [&](int step, int buf, u32x4 (&ra)[VA], u32x4 (&rb)[VB], auto ends) {
+  auto store = [&](int step, int buf, auto ends) {
     if (ends && kbegin + (step + 1) * T::BK > p.K) {  // uniform
       const int s = over(step);
 #pragma unroll
@@ -173,10 +173,10 @@ __global__ __launch_bounds__(T::THREADS) void prompt_kernel(PromptArgs p) {
   // last are loaded (the end of the rows again) and stored as well, and not used.  `ends`: K may end in the step that is stored.
   // The LDS and memory instructions are dealt out between the MFMAs: issued in one go they queue, all waves of the CU at once, while
   // the matrix cores wait.
-  auto step = [&](int s, int buf, u32x4 (&ra)[VA], u32x4 (&rb)[VB], auto ends) {
+  auto step = [&](int s, int buf, auto ends) {
     fetch(buf, 1);
-    store(s + 1, buf ^ 1, ra, rb, ends);
-    load(s + 1 + T::AHEAD, ra, rb);
+    store(s + 1, buf ^ 1, ends);
+    load(s + 2);
     multiply(0);
     if constexpr (KK == 2) PromptDeal<FM * FN, FM + FN, VA + VB, VA + VB>::template go<0>();
 #pragma unroll
@@ -192,21 +192,20 @@ __global__ __launch_bounds__(T::THREADS) void prompt_kernel(PromptArgs p) {
     if constexpr (KK == 2) PromptDeal<(FM * FN < FM + FN ? FM * FN : FM + FN), FM + FN, 0, 0>::template go<0>();
     __builtin_amdgcn_sched_barrier(0);
   };
-  load(0, ring_a[0], ring_b[0]);
-  store(0, 0, ring_a[0], ring_b[0], std::true_type());
-#pragma unroll
-  for (int i = 1; i <= T::AHEAD; i++) load(i, ring_a[i % T::AHEAD], ring_b[i % T::AHEAD]);
+  load(0);
+  store(0, 0, std::true_type());
+  load(1);
   __syncthreads();
   fetch(0, 0);
   const int whole = min(nsteps, (p.K - kbegin) / T::BK);  // steps that K does not end in
-  int s = 0;  // the loads of step s + 1 are in set (s + 1) % AHEAD
+  int s = 0;
   for (; s + 2 < whole; s += 2) {
-    step(s, 0, ring_a[1 % T::AHEAD], ring_b[1 % T::AHEAD], std::false_type());
-    step(s + 1, 1, ring_a[0], ring_b[0], std::false_type());
+    step(s, 0, std::false_type());
+    step(s + 1, 1, std::false_type());
   }
   for (; s < nsteps; s += 2) {
-    step(s, 0, ring_a[1 % T::AHEAD], ring_b[1 % T::AHEAD], std::true_type());
-    if (s + 1 < nsteps) step(s + 1, 1, ring_a[0], ring_b[0], std::true_type());
+    step(s, 0, std::true_type());
+    if (s + 1 < nsteps) step(s + 1, 1, std::true_type());
   }
 
   // lane: token fr of a fragment, four consecutive weight rows fq * 4 ..
@@ -288,11 +287,11 @@ struct PromptShape {
   int BM, BN, BK;
   float alone, shared;
 };
-typedef PromptTile<2, 2, 1, 2, 128, 1> PromptTile0;
-typedef PromptTile<2, 2, 2, 2, 128, 1> PromptTile1;
-typedef PromptTile<4, 2, 2, 4, 64, 1> PromptTile2;
-typedef PromptTile<4, 2, 4, 4, 64, 1> PromptTile3;
-typedef PromptTile<4, 2, 4, 6, 64, 1> PromptTile4;
+typedef PromptTile<2, 2, 1, 2, 128> PromptTile0;
+typedef PromptTile<2, 2, 2, 2, 128> PromptTile1;
+typedef PromptTile<4, 2, 2, 4, 64> PromptTile2;
+typedef PromptTile<4, 2, 4, 4, 64> PromptTile3;
+typedef PromptTile<4, 2, 4, 6, 64> PromptTile4;
 constexpr int kPromptTiles = 5;
 constexpr PromptShape kPromptShapes[kPromptTiles] = {
     {PromptTile0::BM, PromptTile0::BN, PromptTile0::BK, 0.8f, 0.55f}, {PromptTile1::BM, PromptTile1::BN, PromptTile1::BK, 0.9f, 0.65f},
