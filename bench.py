@@ -603,7 +603,7 @@ def entry_points(torch, F, capi, steps, warmup, only=()):
          lambda st: capi.up_index(x, st["wu"], st["idx"], None, st["a_c"])),
         ("cats_down_index", "gather_transposed_gemv, gather_transposed_gemv_indirect_index_2d (sorted index list)", act_rows,
          lambda st: capi.down_index(st["z_c"], st["wdt"], st["idx"], ws)),
-        ("flash_gemv.flag_gemv_gemv_dejavu", "the reference's index-list composite: torch gate GEMV + SiLU + nonzero (host sync), index-list up and down",
+        ("flash_gemv.flag_gemv_gemv_dejavu", "the reference's index-list composite (at one row a single call of the kernels: no list, no host sync)",
          full + 2 * act_rows, lambda st: fg.flag_gemv_gemv_dejavu(x, st["wg_t"], st["wu"], st["wdt"], t)),
         ("cats_up_down", "gemv_gemv_triton (gate activations given)", 2 * act_rows, lambda st: capi.up_down(x, st["a"], st["wu"], st["wdt"], t, ws)),
         ("cats_gate_up", "fuse_gemv_flag_gemv", full + act_rows, lambda st: capi.gate_up(x, st["wg"], st["wu"], t)),

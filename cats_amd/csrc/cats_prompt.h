@@ -14,12 +14,14 @@
 // Rows may start at any element (an odd intermediate size makes the down weight's rows do so): the vectors are read as
 // they lie, and only the step in which K ends looks where a vector ends.
 //
-// What bounds it at 4096 / 11008: up to 64 tokens the weight stream (41 us for gate and up, 21 for down at 32 tokens: 4.4 TB/s), at
-// 512 tokens the barrier of each step and what the waves wait for around it (102 and 61 us: 900 and 760 TFLOP/s; the matrix cores are
-// busy 45 % of the time, LDS 25 %, no bank conflicts).  Whole module call: 155 us at 512 tokens and 66 at 16, with the
-// library's products and one kernel between them 191 and 81; 304 / 569 at 22 tokens 20 us against 78, host time mostly.
-// With the end of K looked for in every step, 110 and 65 us; without the dealing of the loads between the MFMAs 101 and 64, and 142
-// against 130 for the 128 x 128 tile.
+// What bounds it at 4096 / 11008 in fp16 (medians of kernel traces, and counters): at 32 tokens the weight stream, 42 us for gate and up
+// and 18.5 for down (4.3 and 4.9 TB/s); at 512 tokens the barrier of each step and what the waves wait for around it, 94 and 53 us (980
+// and 880 TFLOP/s; matrix cores busy 43 and 35 % of the time, LDS 31 %, no bank conflicts).  The chip lowers its clock when
+// the matrix cores start: in a program's first 5 ms the same launches take up to 131 us.  Whole call, steady: 153 us at 512
+// tokens, 148 against 189 with the library's products and one kernel between them; 68 against 79 at 16; 304 / 569 at 22 tokens 20
+// against 78, host time mostly.
+// Against 102 and 61 us in the same trace: 110 and 65 with the end of K looked for in every step, 101 and 64 without the dealing of
+// the loads between the MFMAs, and that 142 against 130 for the 128 x 128 tile.
 // Measured and not taken: four waves with 128 x 96 sums each (155 us), two steps of loads in registers (no change at 256 tokens
 // and more), raised wave priority around the multiplications (no change).
 #pragma once
