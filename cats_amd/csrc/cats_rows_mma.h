@@ -260,7 +260,7 @@ struct MmaX {
 // UP = false is the gate pass alone (activations, flags and union bits out; no up rows, no z).
 // NG = 2 takes 9..16 batch rows in one pass over the weights: the second group of eight rows is a second x operand in
 // LDS and a second MFMA on the weight registers the first one just used, so the weights are still read once.
-// CH = 2 (rows of more than 4096 elements; their x fills 128 KiB of LDS at 8192): a tile is two register sets, so the gate ring
+// CH = 2 (rows of more than 72 steps, 4608 16-bit elements; their x fills 128 KiB of LDS at 8192): a tile is two register sets, so the gate ring
 // holds one tile ahead instead of two, and the up sums of tile r - 1 are taken before the up rows of tile r overwrite their set.
 template <class DT, int STEPS, int CH, bool UP, int NG = 1>
 __global__ __launch_bounds__(kMmaThreads) void rows_mma_kernel(RowsArgs p) {

@@ -133,7 +133,8 @@ int cats_up_index(const void* x, const void* w, const int64_t* idx, int M, const
 int cats_down_index(const void* z, const void* wdown_t, const int64_t* idx, int M, const void* bias, void* y_out,
                     int B, int H, int Z, int dtype, void* ws, size_t ws_bytes, void* stream);
 
-/* Gate + sparse up in one pass: out[b,j] = active ? round(a * up) : 0 in dtype, flag_out optional.
+/* Gate + sparse up in one call: out[b,j] = active ? round(a * up) : 0 in dtype, flag_out optional.  One launch; fp32 rows that do not
+ * fit on chip from five batch rows on take a dense product each for gate and up, out holding the activations in between.
  * Replaces fuse_gemv_flag_gemv (flash_gemv.py:9-10; fuse_gemv_cmp_cuda.cu:715-784,2006-2022). */
 int cats_gate_up(const void* x, const void* wgate, const void* wup, void* out, uint8_t* flag_out,
                  int B, int H, int I, int dtype, float threshold, void* stream);

@@ -26,7 +26,7 @@ def test_silu_mask_mul(n, dtype):
 
 
 @pytest.mark.parametrize("rows", [1, 5])
-@pytest.mark.parametrize("method", [0, 2])
+@pytest.mark.parametrize("method", [0, 2, 3])
 def test_module_routes_agree(method, rows):
     """With and without a hook on the activation, which keeps the module on torch's operations."""
     from cats_amd.mlp import CatsMLP
