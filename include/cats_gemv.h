@@ -59,8 +59,9 @@ typedef enum {
 
 #define CATS_MAX_BATCH 16  /* 1..8 rows are one pass over the weights.  9..16 rows: the whole-MLP entry points (cats_mlp, the
                             * layer-tail calls, cats_up_down, cats_mlp_rowmajor_down), cats_gate_flag, cats_gate_up and cats_up_flag
-                            * (16-bit types, rows of 2048 or 4096 elements) and cats_down_flag (16-bit types) still read
-                            * every matrix once; every other case is two passes of at most eight rows */
+                            * (16-bit types, rows of up to 4360 elements, and 4416 or 4480 on cache lines; fp32 rows of any
+                            * length in cats_mlp, cats_mlp_rowmajor_down, cats_gate_flag and cats_gate_up) and cats_down_flag (16-bit types) still
+                            * read gate and up once; every other case is two passes of at most eight rows */
 
 /* Library identification / error text.  No reference counterpart (the reference printf()s and exit()s:
  * flash_gemv/csrc/cuda/fuse_gemv_cmp_cuda.cu:25-33,2397-2400). */

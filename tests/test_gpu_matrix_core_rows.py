@@ -100,7 +100,8 @@ def test_weights_off_a_cache_line(oracle, H, I, B, dtype):
     close(y.cpu(), oracle.c_mlp(m["x"], m["wg"], m["wu"], m["wd"], t, a_in=a.cpu(), flag_in=flag.cpu())["y"], dtype)
 
 
-@pytest.mark.parametrize("H,I,B,dtype", [(520, 200, 5, torch.float16), (3104, 96, 8, torch.bfloat16), (8192, 64, 4, torch.float16), (1000, 128, 16, torch.float16)])
+@pytest.mark.parametrize("H,I,B,dtype", [(520, 200, 5, torch.float16), (3104, 96, 8, torch.bfloat16), (8192, 64, 4, torch.float16), (1000, 128, 16, torch.float16),
+                                           (520, 200, 5, torch.float32), (4096, 64, 8, torch.float32), (2180, 96, 16, torch.float32), (2184, 96, 12, torch.float32)])
 def test_norm_while_staging(oracle, H, I, B, dtype):
     """h + MLP(norm(h)): the norm works on the staged operands, padding steps included."""
     m = make_mlp(H, I, B, dtype, seed=H + 3 * I)

@@ -69,7 +69,7 @@ def check_mlp_case(oracle, m, t, *, tag, ws=None, expect_flip_free=False):
     assert torch.equal(flag, want_flag), f"{tag}: flag != (|a| > t) on the kernel's own a"
     assert torch.equal(flag2, flag), f"{tag}: the fused MLP pass and the gate pass disagree on flags"
     union = flag.any(dim=0)
-    if count is not None:  # above 8 rows (two passes) this is the union of the flags, counted by one more small kernel
+    if count is not None:  # above 8 rows too this is the union of the flags of all rows
         assert int(count.item()) == int(union.sum()), f"{tag}: active count {int(count.item())} != {int(union.sum())}"
     # the C oracle's rule on the same activations (independent of torch's scalar casting)
     tr = oracle.c_round(dtype, t)
@@ -543,8 +543,8 @@ def test_config4_small_batch_union(oracle, B):
 
 
 MATRIX_CORE = [
-    # H, I, B, dtype -- 3..8 batch rows in 16-bit types with a row length of 2048 or 4096 take the matrix-core
-    # gate / gate+up kernel (one workgroup per CU, each with ceil(I / workgroups) consecutive rows in tiles of 8)
+    # H, I, B, dtype -- 3..8 batch rows in 16-bit types take the matrix-core gate / gate+up kernel (one workgroup
+    # per CU, each with ceil(I / workgroups) consecutive rows in tiles of 8)
     (4096, 1003, 3, torch.float16),    # 4 rows per workgroup on 256 CUs: half a tile each, the last workgroup has 3 rows
     (4096, 520, 5, torch.bfloat16),
     (2048, 777, 7, torch.float16),
@@ -814,7 +814,7 @@ def test_norm_and_residual_folded_into_the_mlp(oracle, H, I, B, dtype):
 
 @pytest.mark.parametrize("H,I,B,dtype", [(4096, 11008, 1, torch.float16), (4096, 1000, 2, torch.bfloat16), (512, 768, 4, torch.float16),
                                          (1024, 640, 8, torch.bfloat16), (256, 333, 3, torch.float32), (2048, 512, 12, torch.float16),
-                                         (256, 200, 10, torch.float32), (1056, 300, 9, torch.bfloat16)])   # the last two: two passes of <= 8 rows
+                                         (256, 200, 10, torch.float32), (1056, 300, 9, torch.bfloat16)])   # above 8 rows: one gate + up pass
 def test_next_norm_written_by_the_finishing_launch(oracle, H, I, B, dtype):
     """cats_mlp_norm_residual_norm: `out` carries the bits of cats_mlp_norm_residual (same launches), and `next` is the
     RMS norm of exactly those stored values -- checked against the restated HF norm evaluated on the kernel's own `out`
@@ -871,8 +871,8 @@ def test_norm_residual_rejects_rows_that_do_not_fit_in_lds():
 @pytest.mark.parametrize("B", [1, 4])
 def test_llama70b_shape(oracle, B):
     """8192 -> 28672, the larger shape the reference smoke-tests (flash_gemv/test/test_fuse_gemv_cmp.py:662-676).
-    Rows of 16 KiB: two passes of 8 chunks per row in the wave-per-row kernel, 16 column slabs in the down kernel;
-    batch 4 stays on the wave-per-row kernel (the matrix-core one takes rows of 2048 or 4096 elements)."""
+    Rows of 16 KiB: two passes of 8 chunks per row in the single-pass kernel, two register sets per tile in the matrix-core
+    kernel of batch 4, 16 column slabs in the down kernel."""
     m = make_mlp(8192, 28672, B, torch.float16, seed=70, corr=0.5 if B > 1 else 0.0)
     t = calibrate(m["wg"], [0.5], n_vec=64)[0]
     check_mlp_case(oracle, m, t, tag=f"llama70b-fp16-B{B}")
@@ -881,9 +881,9 @@ def test_llama70b_shape(oracle, B):
 @pytest.mark.parametrize("H,I,B,dtype", [(4096, 1000, 16, torch.float16), (512, 333, 11, torch.bfloat16), (260, 96, 9, torch.float32),
                                          (2048, 1536, 9, torch.bfloat16), (4096, 11008, 12, torch.float16), (4096, 2048, 16, torch.bfloat16)])
 def test_batches_of_nine_to_sixteen_rows(oracle, H, I, B, dtype):
-    """The reference's kernels are instantiated up to 16 rows (fuse_gemv_cmp_cuda.cu:2368-2400).  Here 16-bit rows of 2048
-    or 4096 elements take one matrix-core gate + up pass and one matrix-core down pass over all rows (every matrix read
-    once, over the union mask of all rows); every other case is two passes of at most 8 rows.  Either way: the full
+    """The reference's kernels are instantiated up to 16 rows (fuse_gemv_cmp_cuda.cu:2368-2400).  Here 16-bit rows
+    take one matrix-core gate + up pass and one matrix-core down pass over all rows (every matrix read
+    once, over the union mask of all rows); fp32 takes its down pass in two of at most 8 rows.  Either way: the full
     parity case, and rows 8.. of the big batch against the same rows run as a batch of their own (same flags, bit for
     bit; outputs to the parity tolerance -- the union of sixteen rows orders the down sums differently)."""
     m = make_mlp(H, I, B, dtype, seed=B + H, corr=0.3)
@@ -927,8 +927,7 @@ def test_batch_above_sixteen_is_an_error_not_a_crash():
 
 
 def test_active_count_above_eight_rows_is_the_union_over_both_passes(oracle):
-    """9..16 rows run as two passes of 8; the count must still be the number of neurons active in any row, whether or
-    not the caller asks for the flags (without them the passes write the flags into the workspace)."""
+    """At 9..16 rows the count is the number of neurons active in any row, whether or not the caller asks for the flags."""
     for B, H, I in ((9, 512, 200), (16, 1024, 333), (12, 4096, 11008)):
         m = make_mlp(H, I, B, torch.float16, seed=B)
         d = dev(m)
