@@ -51,7 +51,7 @@ def _run(cmd: list[str]) -> None:
         print(err, file=sys.stderr)
 
 
-def build_kernels(jobs: int = 4, timing: bool = False) -> Path:
+def build_kernels(jobs: int = 7, timing: bool = False) -> Path:
     """The kernel library; with ``timing`` the instrumented twin that ``cats_amd.phase_stamps`` loads (never the product)."""
     obj = OBJ / "timing" if timing else OBJ
     out = TIMING_LIB if timing else KERNEL_LIB
@@ -63,6 +63,9 @@ def build_kernels(jobs: int = 4, timing: bool = False) -> Path:
         (CSRC / "cats_inst.hip", obj / "cats_inst_f16.o", ["-DCATS_DT=F16"]),
         (CSRC / "cats_inst.hip", obj / "cats_inst_bf16.o", ["-DCATS_DT=BF16"]),
         (CSRC / "cats_inst.hip", obj / "cats_inst_f32.o", ["-DCATS_DT=F32"]),
+        (CSRC / "cats_inst_small.hip", obj / "cats_inst_small_f16.o", ["-DCATS_DT=F16"]),
+        (CSRC / "cats_inst_small.hip", obj / "cats_inst_small_bf16.o", ["-DCATS_DT=BF16"]),
+        (CSRC / "cats_inst_small.hip", obj / "cats_inst_small_f32.o", ["-DCATS_DT=F32"]),
         (CSRC / "cats_api.hip", obj / "cats_api.o", []),
     ]
     cmds = [[HIPCC, *HIP_FLAGS, *extra, *defs, "-c", str(src), "-o", str(o)] for src, o, defs in units]

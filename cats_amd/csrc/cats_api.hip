@@ -6,6 +6,7 @@
 #include <string.h>
 
 #include <mutex>
+#include <unordered_map>
 
 #include "cats_gemv.h"
 #include "cats_launch.h"
@@ -49,6 +50,21 @@ template <> hipError_t launch_prompt<F16>(bool, const PromptPlan&, PromptArgs, h
 template <> hipError_t launch_prompt<BF16>(bool, const PromptPlan&, PromptArgs, hipStream_t);
 template <> hipError_t launch_prompt_sum<F16>(const PromptSumArgs&, hipStream_t);
 template <> hipError_t launch_prompt_sum<BF16>(const PromptSumArgs&, hipStream_t);
+hipError_t ensure_dynamic_lds(const void* kern, size_t bytes) {
+  if (bytes <= 48 * 1024) return hipSuccess;
+  static std::mutex mu;
+  static std::unordered_map<uintptr_t, size_t> granted;  // (kernel, device) -> bytes; the attribute is per device
+  int dev = 0;
+  if (hipError_t e = hipGetDevice(&dev); e != hipSuccess) return e;
+  const uintptr_t key = (uintptr_t)kern * 64u + (uintptr_t)dev;
+  std::lock_guard<std::mutex> lock(mu);
+  auto it = granted.find(key);
+  if (it != granted.end() && it->second >= bytes) return hipSuccess;
+  hipError_t e = hipFuncSetAttribute(kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
+  if (e == hipSuccess) granted[key] = bytes;
+  return e;
+}
+
 int current_device_cus() {
   constexpr int kDevs = 64;
   static int cus[kDevs];  // 0 = not asked yet; written once per device with the same value, so a plain atomic will do
@@ -75,11 +91,12 @@ constexpr int kMaxSlabs = 128;
 constexpr int kKernelBatch = 8;  // rows one launch handles; the entry points take up to CATS_MAX_BATCH rows in passes of this many
 // Head of the workspace.  [0, 4096): the neuron-pool counters of the single-pass kernel (one 128-byte line per group of
 // workgroups; pool builds only).  then the arrival counters of the reduction launch that also writes the next norm
-// (72 lines of 128 bytes).  Both are zeroed by cats_workspace_init and put back to zero by every call that uses them.
+// (144 lines of 128 bytes), and the one counter of small layers' one-launch calls.  Both are zeroed by cats_workspace_init and put back to zero by every call that uses them.
 // Last: the per-workgroup sums of squares of that launch (overwritten by every call).
 constexpr size_t kPoolCounterBytes = 4096;
 constexpr size_t kArriveOffset = kPoolCounterBytes;
-constexpr size_t kSsqOffset = kArriveOffset + (size_t)(8 * kArriveGroups + 8) * kArriveStride * 4;
+constexpr size_t kSmallArriveOffset = kArriveOffset + (size_t)(kArriveRows * kArriveGroups + kArriveRows) * kArriveStride * 4;
+constexpr size_t kSsqOffset = kSmallArriveOffset + 256;  // one counter, and whole regions of 256 bytes
 constexpr size_t kSsqFloats = 4096;  // workgroups of the reduction launch: B * H / 32
 constexpr size_t kCounterBytes = kSsqOffset + kSsqFloats * 4;
 #ifndef CATS_POOL_NUM  // share of a workgroup's neurons that goes to its group's pool (builds with -DCATS_FUSED_POOL=1 only)
@@ -155,13 +172,15 @@ WsLayout ws_layout(int H, int I) {
   const int B = kKernelBatch;
   size_t o = 0;
   l.counters = o; o += kCounterBytes;
-  l.partial = o;  o += align_up((size_t)kMaxGroups * B * ((size_t)(H + 511) / 512 * 512) * 4, 256);
+  size_t rows = (size_t)kMaxGroups * B;
+  if (I <= kSmallMaxNeurons && H <= kSmallMaxVecs * 8 && rows < (size_t)small_max_groups(I) * CATS_MAX_BATCH) rows = (size_t)small_max_groups(I) * CATS_MAX_BATCH;
+  l.partial = o;  o += align_up(rows * ((size_t)(H + 511) / 512 * 512) * 4, 256);
   l.mask = o;     o += align_up((size_t)((I + 63) / 64) * 8, 256);
   l.ubytes = o;   o += align_up((size_t)I + 8, 256);  // the same as a byte per neuron, read eight at a time
   l.z32 = o;      o += align_up((size_t)CATS_MAX_BATCH * I * 4, 256);  // 16 rows: the one-pass gate + up of 9..16 rows fills it whole
   l.zt = o;       o += align_up((size_t)B * I * 4, 256);
   l.atmp = o;     o += align_up((size_t)B * I * 4, 256);
-  l.fin = o;      o += align_up((size_t)B * H * 4, 256);  // finished columns as fp32, for the launch that also writes the next norm
+  l.fin = o;      o += align_up((size_t)CATS_MAX_BATCH * H * 4, 256);  // finished columns as fp32, for the launch that also writes the next norm
   l.total = o;
   return l;
 }
@@ -369,6 +388,11 @@ int do_joined(const RowsArgs& a, float* sums, float* z, hipStream_t s) {
   return launch_kernel(gate_up_join_kernel, dim3((a.N + 255) / 256), dim3(256), 0, s, j) == hipSuccess ? CATS_OK : CATS_ERR_LAUNCH;
 }
 
+int do_reduce(const ReduceArgs& r, int dtype, hipStream_t s) {
+  const hipError_t e = dtype == CATS_F16 ? launch_reduce<F16>(r, s) : dtype == CATS_BF16 ? launch_reduce<BF16>(r, s) : launch_reduce<F32>(r, s);
+  return e == hipSuccess ? CATS_OK : CATS_ERR_LAUNCH;
+}
+
 // Fills the next-norm fields of the reduction launch; CATS_ERR_SHAPE if the launch cannot carry it.
 int set_next_norm(ReduceArgs& r, const NextNorm& next, char* ws, const WsLayout& l) {
   if (!next.out) return CATS_OK;
@@ -382,6 +406,7 @@ int set_next_norm(ReduceArgs& r, const NextNorm& next, char* ws, const WsLayout&
   return CATS_OK;
 }
 
+constexpr int kFusedMaxGrid = 256;  // partials of 256 workgroups x 2 batch rows fit the workspace's partial-sum region
 constexpr int kNotTaken = -1;  // internal: the shape or type rules this way out, take the other one
 
 // Neurons (or list entries) of a group of the sparse down pass, out of zcols; 0 if a group's list and z would not fit in LDS.
@@ -448,34 +473,88 @@ int do_down(const void* z, bool zf32, const void* wdown_t, float* y32, void* y_o
   else e = launch_down<F32>(bt, zf32, d, block, s);
   if (e != hipSuccess) return CATS_ERR_LAUNCH;
   if (!d.partial_out) return CATS_OK;
-  // The groups' partial sums are added by the reduction launch: rounded into y_out (and the residual added), or added to
-  // y32.  One launch for all rows, unless it also writes the next norm: its arrival counters cover kKernelBatch rows.
-  const size_t sz = (size_t)elem_size(dtype);
-  const int rows_per = next.out ? kKernelBatch : B;
-  for (int b0 = 0; b0 < B; b0 += rows_per) {
-    const int nb = B - b0 < rows_per ? B - b0 : rows_per;
-    ReduceArgs r;
-    memset(&r, 0, sizeof(r));
-    r.partial = d.partial + (size_t)b0 * H;
-    r.gstride = (size_t)B * H;
-    r.y_out = y_out ? (char*)y_out + (size_t)b0 * H * sz : nullptr;
-    r.y32_acc = reduce_into_y32 ? y32 + (size_t)b0 * H : nullptr;
-    r.residual = residual ? (const char*)residual + (size_t)b0 * H * sz : nullptr;
-    r.bias = bias;
-    r.H = H;
-    r.G = d.ngroup;
-    r.BH = nb * H;
-    NextNorm nx = next;
-    if (nx.out) nx.out = (char*)nx.out + (size_t)b0 * H * sz;
-    if (int st = set_next_norm(r, nx, ws, l)) return st;
-    FusedArgs none;
-    memset(&none, 0, sizeof(none));
-    if (dtype == CATS_F16) e = launch_fused<F16>(1, 0, 2, none, r, s);
-    else if (dtype == CATS_BF16) e = launch_fused<BF16>(1, 0, 2, none, r, s);
-    else e = launch_fused<F32>(1, 0, 2, none, r, s);
-    if (e != hipSuccess) return CATS_ERR_LAUNCH;
-  }
-  return CATS_OK;
+  // The groups' partial sums are added by the reduction launch: rounded into y_out (and the residual added), or added to y32.
+  ReduceArgs r;
+  memset(&r, 0, sizeof(r));
+  r.partial = d.partial;
+  r.y_out = y_out;
+  r.y32_acc = reduce_into_y32 ? y32 : nullptr;
+  r.residual = residual;
+  r.bias = bias;
+  r.H = H;
+  r.G = d.ngroup;
+  r.BH = B * H;
+  if (int st = set_next_norm(r, next, ws, l)) return st;
+  return do_reduce(r, dtype, s);
+}
+
+// Whether the kernels of small layers take this call (a as for kGateUp, the neurons' down rows as (I, H)), and the grid.  They read every row of
+// all three matrices and leave partial sums of sixteen neurons each, against kept rows only and one launch more, or a chain of trips more, in the other
+// kernels.  GPU time by HIP graph, those against these, us at 50 to 70 % sparsity:
+//   1 row, 16 bits    512 / 1024 9.6, 5.6   1024 / 2731 11.5, 7.9   2048 / 3072 12.2, 11.0 (at 90 % 11.1, 11.0)   2048 / 4096 13.4, 13.0 (12.0, 13.0)
+//   1 row, fp32       512 / 1024 9.6, 6.4   1024 / 3300 12.1, 11.1 (11.1, 10.8)   1024 / 4096 13.0, 12.6 (11.6, 12.5)   4 rows 19.6, 15.9
+//   4 rows            512 / 1024 12.5, 7.3   1024 / 2731 15.3, 10.4   2048 / 3072 18.4, 16.1   8 rows 20.3, 19.5
+//   8 rows            1024 / 4096 16.5, 14.6 (8.4 MB of sums)   1536 / 4096 19.1, 19.3 (12.6 MB)
+//   16 rows           1024 / 1600 15.5, 14.1 (6.6 MB)   1024 / 2731 17.6, 17.1 (11.2 MB)   1400 / 3000 20.1, 22.1 (16.8 MB)
+//   16 rows, fp32     1024 / 2731 36.0, 22.6   1024 / 4096 40.0, 27.1 (16.8 MB; the other way reads the down weight twice)
+// Beyond one workgroup a CU: 512 / 8000 15.0, 9.9 at 1 row and 17.8, 15.0 at 8;  704 / 6000 17.3, 17.1 at 8 (8.4 MB);  1024 / 5000 13.4, 11.4 at 1,
+// 17.8, 19.8 at 8 (10.3 MB);  1200 / 5000 (rows of 150 vectors, one workgroup a CU at a time) 12.0, 13.3 at 1 row and 90 %.
+bool small_takes(RowsArgs& a, int dtype, bool& mma, int& grid) {
+  if (g_tuning.path == 1 || g_tuning.gate_variant != 0 || g_tuning.down_groups > 0 || g_tuning.down_block > 0) return false;
+  if (a.nb < 1 || a.nb > CATS_MAX_BATCH || a.N > kSmallMaxNeurons) return false;
+  mma = a.nb > (dtype == CATS_F32 ? 4 : 2);  // as takes_mma has it for the gate
+  grid = small_layout(a, mma);
+  if (grid <= 0 || grid > small_max_groups(a.N)) return false;
+  const size_t bytes = (size_t)a.N * a.K * elem_size(dtype), sums = (size_t)grid * a.nb * a.K * 4;
+  const bool crowded = grid > kFusedMaxGrid;  // more than one workgroup a CU: two of them fit where a row is at most 128 vectors
+  if (crowded && a.row_vecs > 128) return false;
+  if (!mma) return bytes <= (dtype == CATS_F32 && a.nb > 2 ? 17000000u : crowded ? 11000000u : 13600000u);
+  const size_t most = crowded ? 8500000u : 11000000u;
+  return sums <= (dtype == CATS_F32 && a.nb > kKernelBatch ? 2 * most : most);
+}
+
+// Sums of a batch row that one workgroup adds up sooner than a launch over all CUs and, for the layer tail, the hand-over in front of its norm
+// (tail with the next norm, one row: 512 / 1024, 131 KB, 7.8 us against 10.1; 704 / 1451, 256 KB, 11.1; 1024 / 1965, 504 KB, 13.2 against 11.8).
+constexpr size_t kSmallTailBytes = 300000;
+// One batch row up to here is one launch: the call then takes 8.0 us instead of 8.7 to 9.2 (the host's pace: 2.1 us a launch), though
+// its kernel takes 1 to 2 us more than the two; 512 / 2048, 262 KB: 10.1 against 8.6.  In a captured graph launches are cheap: two there, with the
+// sums in the same order.
+constexpr size_t kSmallOneLaunchBytes = 131072;
+
+// y32: the caller's fp32 sums, which the call adds to.
+int do_small(const RowsArgs& a, bool mma, int grid, int stage, const void* wdown_t, void* y_out, const void* residual, float* y32, int32_t* count_out,
+             int dtype, char* ws, const WsLayout& l, hipStream_t s, const NextNorm& next = NextNorm(), float* partial = nullptr, int32_t* counts = nullptr,
+             int32_t* arrive = nullptr) {
+  SmallArgs k;
+  memset(&k, 0, sizeof(k));
+  k.r = a;
+  k.wd = (const u32x4*)wdown_t;
+  k.partial = partial ? partial : (float*)(ws + l.partial);
+  k.counts = counts ? counts : (int32_t*)(ws + l.z32);
+  ReduceArgs& r = k.fin;
+  r.partial = k.partial;
+  r.counts = k.counts;
+  r.count_out = count_out;
+  r.y_out = y_out;
+  r.y32_acc = y32;
+  r.residual = residual;
+  r.H = a.K;
+  r.G = grid;
+  r.BH = a.nb * a.K;
+  if (int st = set_next_norm(r, next, ws, l)) return st;
+  const size_t row = (size_t)grid * a.K * 4;
+  const bool one = a.nb == 1 && row <= kSmallOneLaunchBytes;
+  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+  if (one && stage == 0 && hipStreamIsCapturing(s, &cap) == hipSuccess && cap == hipStreamCaptureStatusNone) k.arrive = arrive ? arrive : (int32_t*)(ws + l.counters + kSmallArriveOffset);
+  hipError_t e = hipSuccess;
+  if (stage != 2) e = dtype == CATS_F16 ? launch_small<F16>(mma, grid, k, s) : dtype == CATS_BF16 ? launch_small<BF16>(mma, grid, k, s) : launch_small<F32>(mma, grid, k, s);
+  if (e != hipSuccess) return CATS_ERR_LAUNCH;
+  if (stage == 1 || k.arrive) return CATS_OK;
+  if (!one && (!residual || row > kSmallTailBytes)) return do_reduce(r, dtype, s);
+  e = dtype == CATS_F16    ? launch_small_tail<F16>(a.nb, r, s)
+      : dtype == CATS_BF16 ? launch_small_tail<BF16>(a.nb, r, s)
+                           : launch_small_tail<F32>(a.nb, r, s);
+  return e == hipSuccess ? CATS_OK : CATS_ERR_LAUNCH;
 }
 
 int check_ws(const void* ws, size_t ws_bytes, int H, int I, WsLayout& l) {
@@ -485,7 +564,6 @@ int check_ws(const void* ws, size_t ws_bytes, int H, int I, WsLayout& l) {
 }
 
 
-constexpr int kFusedMaxGrid = 256;  // partials of 256 workgroups x 2 batch rows fit the workspace's partial-sum region
 constexpr int kFusedPerCU = 16 / kFusedWaves;  // workgroups per CU: 1, or 2 in the 512-thread experiment build (one batch row only)
 
 // Whether the single-pass kernel covers this call, and with what launch shape: one workgroup per CU, each with an
@@ -812,23 +890,26 @@ static int mlp_pass(const void* x, const void* wgate, const void* wup, const voi
   if (st) return st;
   FusedArgs f;
   int grid = 0;
+  RowsArgs a;
+  fill_rows(a, x, wgate, H, I, B, dtype);
+  a.w2 = (const u32x4*)wup;
+  a.flag_out = flag_out;
+  a.t = round_through(dtype, threshold);
+  bool mma = false;
+  if (small_takes(a, dtype, mma, grid))
+    return do_small(a, mma, grid, stage, wdown_t, y_out, nullptr, y_f32, count_out, dtype, (char*)ws, l, (hipStream_t)stream);
   if (fused_eligible(B, H, I, dtype, f, grid)) {
     f.x = (const u32x4*)x;
     f.wg = (const u32x4*)wgate;
     f.wu = (const u32x4*)wup;
     f.wd = (const u32x4*)wdown_t;
     f.flag_out = flag_out;
-    f.t = round_through(dtype, threshold);
+    f.t = a.t;
     return do_fused(f, grid, stage, y_out, nullptr, count_out, dtype, (char*)ws, l, (hipStream_t)stream, y_f32);
   }
-  RowsArgs a;
-  fill_rows(a, x, wgate, H, I, B, dtype);
-  a.w2 = (const u32x4*)wup;
   a.z32_out = (float*)((char*)ws + l.z32);
   a.mask_out = (uint8_t*)ws + l.mask;
   a.ubytes_out = (uint8_t*)ws + l.ubytes;
-  a.flag_out = flag_out;
-  a.t = round_through(dtype, threshold);
   const bool joined = joined_takes(dtype, a);
   l.mask_bytes = joined || rows_mask_is_bytes(kGateUp, dtype, a);
   if (stage != 2) {
@@ -859,14 +940,18 @@ static int mlp_wide(const void* x, const void* norm_weight, float eps, const voi
   RowsArgs a;
   fill_rows(a, x, wgate, H, I, B, dtype);
   a.w2 = (const u32x4*)wup;
-  a.z32_out = (float*)((char*)ws + l.z32);
-  a.mask_out = (uint8_t*)ws + l.mask;
-  a.ubytes_out = (uint8_t*)ws + l.ubytes;
-  l.mask_bytes = true;  // the matrix-core kernel or nothing
   a.flag_out = flag_out;
   a.t = round_through(dtype, threshold);
   a.norm_w = (const u32x4*)norm_weight;
   a.norm_eps = eps;
+  bool mma = false;
+  int grid = 0;
+  if (small_takes(a, dtype, mma, grid))
+    return do_small(a, mma, grid, 0, wdown_t, y_out, residual ? x : nullptr, y_f32, count_out, dtype, (char*)ws, l, (hipStream_t)stream, next);
+  a.z32_out = (float*)((char*)ws + l.z32);
+  a.mask_out = (uint8_t*)ws + l.mask;
+  a.ubytes_out = (uint8_t*)ws + l.ubytes;
+  l.mask_bytes = true;  // the matrix-core kernel or nothing
   st = joined_takes(dtype, a) ? do_joined(a, (float*)((char*)ws + l.zt), a.z32_out, (hipStream_t)stream) : rows_wide(a, dtype, stream);
   if (st) return st;  // an error, or kNotTaken
   // all rows in one pass over W_down^T where the matrix-core down kernel takes the shape, else a pass per eight rows
@@ -945,27 +1030,30 @@ static int mlp_norm_residual_pass(const void* h, const void* norm_weight, float 
   WsLayout l;
   st = check_ws(ws, ws_bytes, H, I, l);
   if (st) return st;
+  RowsArgs a;
+  fill_rows(a, h, wgate, H, I, B, dtype);
+  a.w2 = (const u32x4*)wup;
+  a.t = round_through(dtype, threshold);
+  a.norm_w = (const u32x4*)norm_weight;
+  a.norm_eps = eps;
   FusedArgs f;
   int grid = 0;
+  bool mma = false;
+  if (small_takes(a, dtype, mma, grid))
+    return do_small(a, mma, grid, 0, wdown_t, out, h, nullptr, nullptr, dtype, (char*)ws, l, (hipStream_t)stream, next);
   if (fused_eligible(B, H, I, dtype, f, grid)) {
     f.x = (const u32x4*)h;
     f.wg = (const u32x4*)wgate;
     f.wu = (const u32x4*)wup;
     f.wd = (const u32x4*)wdown_t;
-    f.t = round_through(dtype, threshold);
+    f.t = a.t;
     f.norm_w = (const u32x4*)norm_weight;
     f.norm_eps = eps;
     return do_fused(f, grid, 0, out, h, nullptr, dtype, (char*)ws, l, (hipStream_t)stream, nullptr, next);
   }
-  RowsArgs a;
-  fill_rows(a, h, wgate, H, I, B, dtype);
-  a.w2 = (const u32x4*)wup;
   a.z32_out = (float*)((char*)ws + l.z32);
   a.mask_out = (uint8_t*)ws + l.mask;
   a.ubytes_out = (uint8_t*)ws + l.ubytes;
-  a.t = round_through(dtype, threshold);
-  a.norm_w = (const u32x4*)norm_weight;
-  a.norm_eps = eps;
   l.mask_bytes = rows_mask_is_bytes(kGateUp, dtype, a);
   st = do_rows(kGateUp, dtype, a, (hipStream_t)stream);
   if (st) return st;
@@ -1149,13 +1237,7 @@ int cats_down_index(const void* z, const void* wdown_t, const int64_t* idx, int 
     r.H = H;
     r.G = 0;
     r.BH = B * H;
-    FusedArgs none;
-    memset(&none, 0, sizeof(none));
-    hipError_t e;
-    if (dtype == CATS_F16) e = launch_fused<F16>(1, 0, 2, none, r, (hipStream_t)stream);
-    else if (dtype == CATS_BF16) e = launch_fused<BF16>(1, 0, 2, none, r, (hipStream_t)stream);
-    else e = launch_fused<F32>(1, 0, 2, none, r, (hipStream_t)stream);
-    return e == hipSuccess ? CATS_OK : CATS_ERR_LAUNCH;
+    return do_reduce(r, dtype, (hipStream_t)stream);
   }
   return do_down(z, false, wdown_t, nullptr, y_out, nullptr, B, H, Z, dtype, (char*)ws, l, (hipStream_t)stream, nullptr, nullptr, idx, M, bias);
 }
@@ -1168,6 +1250,17 @@ int cats_mlp_noalloc(const void* x, const void* wgate, const void* wup, const vo
   if (!aligned16(x) || !aligned16(wgate) || !aligned16(wup) || !aligned16(wdown_t)) return CATS_ERR_ALIGN;
   FusedArgs f;
   int grid = 0;
+  RowsArgs a;
+  fill_rows(a, x, wgate, H, I, B, dtype);
+  a.w2 = (const u32x4*)wup;
+  a.t = round_through(dtype, threshold);
+  bool mma = false;
+  if ((size_t)B * H <= 8192 && small_takes(a, dtype, mma, grid) && !mma && B <= 2) {  // at most kFusedMaxGrid workgroups: the scratch holds them
+    void* sp = nullptr;
+    if (int e = scratch_address(&sp)) return e;
+    return do_small(a, mma, grid, 0, wdown_t, y_out, nullptr, nullptr, nullptr, dtype, nullptr, WsLayout(), (hipStream_t)stream, NextNorm(), (float*)sp,
+                    (int32_t*)((char*)sp + kScratchPartialBytes), (int32_t*)((char*)sp + kScratchPartialBytes + kScratchCountBytes));
+  }
   const bool ok = fused_eligible(B, H, I, dtype, f, grid, true);  // this entry point is the single-pass kernel or nothing
   // the stated limit (B * H <= 8192) whatever the grid turns out to be, and the actual footprint as a second check
   if (!ok || (size_t)B * H > 8192 || (size_t)grid * B * H * 4 > kScratchPartialBytes || (size_t)grid * 4 > kScratchCountBytes)

@@ -51,6 +51,7 @@ constexpr int kFusedMaxKV = 4;          // a down wave covers KV * 64 vectors of
 constexpr bool kFusedPool = CATS_FUSED_POOL != 0;
 constexpr int kFusedGroup = 8;          // consecutive workgroups (one per XCD) that share a pool of neurons
 constexpr int kPoolStride = 32;         // int32 per group in the pool counter array: ticket counter at +0, finished workgroups at +16
+constexpr int kArriveRows = 16;         // batch rows a reduction launch that also writes the next norm takes
 constexpr int kArriveGroups = 8;        // groups a batch row's workgroups of the reduction launch arrive in
 constexpr int kArriveStride = 32;       // int32 between arrival counters: one 128-byte line each
 constexpr int kReduceCols = 32;         // fp32 columns per workgroup of the reduction kernel
@@ -105,8 +106,7 @@ struct FusedArgs {
 };
 
 struct ReduceArgs {
-  const float* partial;  // [G][BH]; or [G][gstride] with the BH wanted columns at the front of each, when gstride is set
-  size_t gstride;        // 0 = BH
+  const float* partial;  // [G][BH]
   const int32_t* counts; // [G]
   void* y_out;           // (nb, H) dtype, flattened to BH
   float* y32_acc;        // instead of y_out: (nb, H) fp32 that the sums are added to, unrounded (the fp32-accumulate contract)
@@ -123,7 +123,7 @@ struct ReduceArgs {
   float norm2_eps;
   float* ssq_part;       // [gridDim] sum of squares of every workgroup's columns
   float* fin;            // [BH] the finished columns as fp32, for the workgroup that writes norm2_out
-  int32_t* arrive;       // arrival counters, zero between calls: [8 rows][kArriveGroups] then [8 rows], kArriveStride apart
+  int32_t* arrive;       // arrival counters, zero between calls: [16 rows][kArriveGroups] then [16 rows], kArriveStride apart
 };
 
 #ifdef CATS_TIMING
@@ -791,17 +791,16 @@ __global__ __launch_bounds__(256) void reduce_partials_kernel(ReduceArgs p) {
   const int col = blockIdx.x * kReduceCols + cq * 4;
   const int per = (p.G + kReduceLanes - 1) / kReduceLanes;
   const int g0 = gl * per, g1 = min(p.G, g0 + per);
-  const size_t gstride = p.gstride ? p.gstride : (size_t)p.BH;
   float4 s = {0.f, 0.f, 0.f, 0.f};
   if (col < p.BH && per == 1) {
     // at most one partial per thread (the 32 neuron groups of the sparse down kernels): one load, not a batch of eight
-    if (g0 < g1) s = *(const float4*)(p.partial + (size_t)g0 * gstride + col);
+    if (g0 < g1) s = *(const float4*)(p.partial + (size_t)g0 * p.BH + col);
   } else if (col < p.BH) {
     constexpr int U = 8;
     for (int g = g0; g < g1; g += U) {
       float4 t[U];
 #pragma unroll
-      for (int u = 0; u < U; u++) t[u] = *(const float4*)(p.partial + (size_t)min(g + u, g1 - 1) * gstride + col);
+      for (int u = 0; u < U; u++) t[u] = *(const float4*)(p.partial + (size_t)min(g + u, g1 - 1) * p.BH + col);
 #pragma unroll
       for (int u = 0; u < U; u++)
         if (g + u < g1) { s.x += t[u].x; s.y += t[u].y; s.z += t[u].z; s.w += t[u].w; }
@@ -859,7 +858,7 @@ __global__ __launch_bounds__(256) void reduce_partials_kernel(ReduceArgs p) {
         const int wi = blockIdx.x - brow * wpr, g = wi / gsize;
         const int members = min(gsize, wpr - g * gsize), ngroups = (wpr + gsize - 1) / gsize;
         int32_t* c1 = p.arrive + (size_t)(brow * kArriveGroups + g) * kArriveStride;
-        int32_t* c2 = p.arrive + (size_t)(8 * kArriveGroups + brow) * kArriveStride;
+        int32_t* c2 = p.arrive + (size_t)(kArriveRows * kArriveGroups + brow) * kArriveStride;
         int last = 0;
         if (__hip_atomic_fetch_add(c1, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == members - 1) {
           __hip_atomic_store(c1, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);  // nobody else comes to this counter in this call

@@ -1,8 +1,5 @@
 // Kernel instantiations for one dtype.  Compiled three times (-DCATS_DT=F16 / BF16 / F32) so the
 // translation units build in parallel.
-#include <mutex>
-#include <unordered_map>
-
 #include "cats_launch.h"
 #include "cats_rows_mma.h"
 
@@ -13,23 +10,6 @@
 namespace cats {
 
 namespace {
-
-// Kernels that want more than 48 KiB of dynamic LDS have to say so once per process (and again only if a later
-// launch wants more): remembered per kernel so that the launch path makes no runtime call besides the launch.
-hipError_t ensure_dynamic_lds(const void* kern, size_t bytes) {
-  if (bytes <= 48 * 1024) return hipSuccess;
-  static std::mutex mu;
-  static std::unordered_map<uintptr_t, size_t> granted;  // (kernel, device) -> bytes; the attribute is per device
-  int dev = 0;
-  if (hipError_t e = hipGetDevice(&dev); e != hipSuccess) return e;
-  const uintptr_t key = (uintptr_t)kern * 64u + (uintptr_t)dev;
-  std::lock_guard<std::mutex> lock(mu);
-  auto it = granted.find(key);
-  if (it != granted.end() && it->second >= bytes) return hipSuccess;
-  hipError_t e = hipFuncSetAttribute(kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
-  if (e == hipSuccess) granted[key] = bytes;
-  return e;
-}
 
 constexpr int kR = 2;    // rows per wave per pass
 constexpr int kCB = 8;   // 64-lane chunks whose loads are issued together: 8 x 16 B per lane per row
@@ -372,16 +352,18 @@ hipError_t launch_gate_cols_finish<CATS_DT>(const GateColsArgs& a, int groups, v
 }
 
 template <>
+hipError_t launch_reduce<CATS_DT>(const ReduceArgs& r, hipStream_t stream) {
+  const int rgrid = (r.BH + kReduceCols - 1) / kReduceCols;  // BH == 0: only the count is wanted
+  return launch_kernel(reduce_partials_kernel<CATS_DT>, dim3(rgrid > 0 ? rgrid : 1), dim3(256), 0, stream, r);
+}
+
+template <>
 hipError_t launch_fused<CATS_DT>(int bt, int grid, int stage, const FusedArgs& a, const ReduceArgs& r, hipStream_t stream) {
   if (stage != 2) {
     hipError_t e = bt == 1 ? launch_fused_b<CATS_DT, 1>(grid, a, stream) : launch_fused_b<CATS_DT, 2>(grid, a, stream);
     if (e != hipSuccess) return e;
   }
-  if (stage != 1) {
-    const int rgrid = (r.BH + kReduceCols - 1) / kReduceCols;  // BH == 0: only the count is wanted
-    return launch_kernel(reduce_partials_kernel<CATS_DT>, dim3(rgrid > 0 ? rgrid : 1), dim3(256), 0, stream, r);
-  }
-  return hipSuccess;
+  return stage != 1 ? launch_reduce<CATS_DT>(r, stream) : hipSuccess;
 }
 
 template <>

@@ -1,0 +1,66 @@
+// The kernels of small layers for one dtype.  Compiled three times (-DCATS_DT=F16 / BF16 / F32), beside cats_inst.hip.
+#include <type_traits>
+
+#include "cats_launch.h"
+
+#ifndef CATS_DT
+#error "compile with -DCATS_DT=F16|BF16|F32"
+#endif
+
+namespace cats {
+
+namespace {
+
+typedef void (*SmallKernel)(SmallArgs);
+
+template <int B, bool ONE>
+SmallKernel rows_for(int nch) {
+  switch (nch) {
+    case 1: return small_rows_kernel<CATS_DT, B, 1, ONE>;
+    case 2: return small_rows_kernel<CATS_DT, B, 2, ONE>;
+    case 3: return small_rows_kernel<CATS_DT, B, 3, ONE>;
+    case 4: return small_rows_kernel<CATS_DT, B, 4, ONE>;
+  }
+  return nullptr;
+}
+
+template <int NG>
+SmallKernel mma_for(int steps) {
+  switch (steps) {
+    case 1: return small_mma_kernel<CATS_DT, 1, NG>;
+    case 2: return small_mma_kernel<CATS_DT, 2, NG>;
+    case 3: return small_mma_kernel<CATS_DT, 3, NG>;
+    case 4: return small_mma_kernel<CATS_DT, 4, NG>;
+    case 5: return small_mma_kernel<CATS_DT, 5, NG>;
+  }
+  return nullptr;
+}
+
+}  // namespace
+
+template <>
+hipError_t launch_small<CATS_DT>(bool mma, int grid, const SmallArgs& a, hipStream_t stream) {
+  SmallKernel kern = nullptr;
+  size_t lds = 0;
+  if (mma) {
+    const int steps = rows_mma_split(a.r).steps;
+    kern = a.r.nb > 8 ? mma_for<2>(steps) : mma_for<1>(steps);
+    lds = small_mma_lds_bytes(a.r.mma_slots, a.r.nb > 8 ? 2 : 1);
+    if (hipError_t e = ensure_dynamic_lds((const void*)kern, lds); e != hipSuccess) return e;
+  } else if (a.r.nb == 1) {
+    kern = a.arrive ? rows_for<1, true>(a.r.nch) : rows_for<1, false>(a.r.nch);
+  } else if (a.r.nb == 2) {
+    kern = rows_for<2, false>(a.r.nch);
+  } else if constexpr (std::is_same<CATS_DT, F32>::value) {
+    kern = rows_for<4, false>(a.r.nch);
+  }
+  if (!kern) return hipErrorInvalidValue;
+  return launch_kernel(kern, dim3(grid), dim3(kSmallThreads), lds, stream, a);
+}
+
+template <>
+hipError_t launch_small_tail<CATS_DT>(int rows, const ReduceArgs& r, hipStream_t stream) {
+  return launch_kernel(small_tail_kernel<CATS_DT>, dim3(rows), dim3(kSmallThreads), 0, stream, r);
+}
+
+}  // namespace cats

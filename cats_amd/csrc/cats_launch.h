@@ -9,6 +9,7 @@
 #include "cats_gemv_mma.h"
 #include "cats_fused.h"
 #include "cats_rows.h"
+#include "cats_small.h"
 
 namespace cats {
 
@@ -30,6 +31,10 @@ inline hipError_t launch_kernel(K kern, dim3 grid, dim3 block, size_t lds, hipSt
   void* params[] = {(void*)&a...};
   return hipLaunchKernel((const void*)kern, grid, block, params, lds, stream);
 }
+
+// Kernels that want more than 48 KiB of dynamic LDS have to say so once per process (and again only if a later
+// launch wants more): remembered per kernel so that the launch path makes no runtime call besides the launch.
+hipError_t ensure_dynamic_lds(const void* kern, size_t bytes);
 
 // Returns hipSuccess or the launch error.  `mode` is a RowsMode; bt (1, 2, 4 or 8) the compile-time batch.
 template <class DT>
@@ -59,6 +64,18 @@ hipError_t launch_down_mma(bool zf32, const DownArgs& a, hipStream_t stream);
 // Single-pass MLP for 1 or 2 batch rows.  stage: 0 = both launches, 1 = streaming kernel only, 2 = reduction only.
 template <class DT>
 hipError_t launch_fused(int bt, int grid, int stage, const FusedArgs& a, const ReduceArgs& r, hipStream_t stream);
+
+// The kernels of a small layer (cats_small.h); a.r has been through small_layout.
+template <class DT>
+hipError_t launch_small(bool mma, int grid, const SmallArgs& a, hipStream_t stream);
+
+// Its reduction with a residual: a workgroup per batch row.
+template <class DT>
+hipError_t launch_small_tail(int rows, const ReduceArgs& r, hipStream_t stream);
+
+// The reduction launch alone.
+template <class DT>
+hipError_t launch_reduce(const ReduceArgs& r, hipStream_t stream);
 
 // Projections and attention of one decode step (cats_decode.h).  mode is a ProjMode; lds_bytes of x have to fit (proj_lds_bytes).
 constexpr size_t kProjMaxLds = 128 * 1024;
