@@ -1428,10 +1428,13 @@ int cats_silu_mask_mul(const void* gate, const void* up, void* z, size_t n, int 
 static PromptPlan prompt_down_plan(int M, int H, int I) { return prompt_plan(false, M, prompt_sum_pitch(H), I, current_device_cus()); }
 static size_t prompt_z_bytes(int M, int I) { return ((size_t)M * prompt_pitch(I) * 2 + 255) / 256 * 256; }
 
+static size_t prompt_bytes(const PromptPlan& down, int M, int H, int I) {
+  return prompt_z_bytes(M, I) + (down.splits > 1 ? (size_t)down.splits * M * prompt_sum_pitch(H) * sizeof(float) : 0);
+}
+
 size_t cats_prompt_scratch_bytes(int M, int H, int I) {
   if (M < 1 || M > CATS_PROMPT_MAX_TOKENS || H < 8 || I < 8 || H > (1 << 28) || I > (1 << 28)) return 0;
-  const PromptPlan down = prompt_down_plan(M, H, I);
-  return prompt_z_bytes(M, I) + (down.splits > 1 ? (size_t)down.splits * M * prompt_sum_pitch(H) * sizeof(float) : 0);
+  return prompt_bytes(prompt_down_plan(M, H, I), M, H, I);
 }
 
 int cats_prompt_mlp(const void* x, const void* wgate, const void* wup, const void* wdown, void* y_out, int M, int H, int I, int dtype,
@@ -1446,7 +1449,8 @@ int cats_prompt_mlp(const void* x, const void* wgate, const void* wup, const voi
   for (const void* p : {x, wgate, wup, wdown})
     if ((uintptr_t)p & 1u) return CATS_ERR_ALIGN;
   if ((uintptr_t)y_out & 7u) return CATS_ERR_ALIGN;
-  if (!scratch || ((uintptr_t)scratch & 255u) || scratch_bytes < cats_prompt_scratch_bytes(M, H, I)) return CATS_ERR_WORKSPACE;
+  const PromptPlan second = prompt_down_plan(M, H, I);
+  if (!scratch || ((uintptr_t)scratch & 255u) || scratch_bytes < prompt_bytes(second, M, H, I)) return CATS_ERR_WORKSPACE;
   const hipStream_t s = (hipStream_t)stream;
   const int pitch = prompt_pitch(I);
   PromptArgs a;
@@ -1461,7 +1465,6 @@ int cats_prompt_mlp(const void* x, const void* wgate, const void* wup, const voi
   const PromptPlan first = prompt_plan(true, M, pitch, H, current_device_cus());
   hipError_t e = dtype == CATS_F16 ? launch_prompt<F16>(true, first, a, s) : launch_prompt<BF16>(true, first, a, s);
   if (e != hipSuccess) return CATS_ERR_LAUNCH;
-  const PromptPlan second = prompt_down_plan(M, H, I);
   float* partial = (float*)((char*)scratch + prompt_z_bytes(M, I));
   a.x = scratch;
   a.w = wdown;

@@ -49,17 +49,22 @@ def get_threshold(bin_edges: torch.Tensor, histogram_counts: torch.Tensor, spars
 
 def _bare(module, cls):
     """`module` is a plain `cls`: calling it does nothing besides the class's own forward."""
-    return (type(module) is cls and "forward" not in module.__dict__ and not module._forward_hooks and not module._forward_pre_hooks
-            and not module._backward_hooks and not module._backward_pre_hooks)
+    d = module.__dict__
+    return type(module) is cls and not ("forward" in d or d["_forward_hooks"] or d["_forward_pre_hooks"] or d["_backward_hooks"] or d["_backward_pre_hooks"])
 
 
 def _nothing_watches():
     """No autograd, tracing, autocast, transform or mode is at work that has to see the single torch operations."""
-    return not (torch.is_grad_enabled() or torch.is_autocast_enabled("cuda") or torch.jit.is_tracing() or torch.compiler.is_compiling()
-                or torch._C._len_torch_dispatch_stack() or torch._C._len_torch_function_stack()
-                or torch._C._functorch.peek_interpreter_stack() is not None or torch.autograd.forward_ad._current_level >= 0
-                or nn.modules.module._global_forward_hooks or nn.modules.module._global_forward_pre_hooks
-                or nn.modules.module._global_backward_hooks or nn.modules.module._global_backward_pre_hooks)
+    c, m = torch._C, nn.modules.module
+    return not (torch.is_grad_enabled() or torch.is_autocast_enabled("cuda") or c._is_tracing() or torch.compiler.is_compiling()
+                or c._len_torch_dispatch_stack() or c._len_torch_function_stack()
+                or c._functorch.peek_interpreter_stack() is not None or torch.autograd.forward_ad._current_level >= 0
+                or m._global_forward_hooks or m._global_forward_pre_hooks or m._global_backward_hooks or m._global_backward_pre_hooks)
+
+
+def _sub(module, name):
+    """module.name, a submodule, without nn.Module's search for it."""
+    return module._modules.get(name) or getattr(module, name)
 
 
 def _plain(t, dtype, device):
@@ -209,15 +214,17 @@ class CatsMLP(nn.Module):
         flash_gemv.cats_prompt_mlp computes the same -- else None."""
         if not x.is_cuda or x.dtype not in (torch.float16, torch.bfloat16) or type(x) is not torch.Tensor or not x.is_contiguous():
             return None
-        if not isinstance(self.dead_threshold, (int, float)) or not _nothing_watches() or not _bare(self.act_fn, nn.SiLU):
+        if not isinstance(self.dead_threshold, (int, float)) or not _nothing_watches() or not _bare(_sub(self, "act_fn"), nn.SiLU):
             return None
         dtype, device, weights = x.dtype, x.device, []
-        for proj in (self.gate_proj, self.up_proj, self.down_proj):
+        for name in ("gate_proj", "up_proj", "down_proj"):
+            proj = _sub(self, name)
             if not _bare(proj, nn.Linear):
                 return None
-            w = proj._parameters.get("weight")
+            params = proj._parameters
+            w = params.get("weight")
             if (type(w) is not nn.Parameter or w.dtype != dtype or w.device != device or not w.is_contiguous() or w.dim() != 2
-                    or proj._parameters.get("bias", self) is not None):
+                    or params.get("bias", self) is not None):
                 return None
             weights.append(w)
         shape = weights[0].shape
@@ -272,12 +279,12 @@ class CatsMLP(nn.Module):
                 if self.wdown_t is None:
                     raise RuntimeError("CatsMLP: sp_method 2/3 need wdown_t (call prepare_decode() once after loading weights)")
                 if self.sp_method == 2:
-                    g = self.gate_proj
-                    if (_bare(g, nn.Linear) and g.bias is None and _bare(self.act_fn, nn.SiLU) and _nothing_watches()
-                            and _plain(g.weight, x.dtype, x.device)):
+                    g = _sub(self, "gate_proj")
+                    if (_bare(g, nn.Linear) and g._parameters.get("bias", self) is None and _bare(_sub(self, "act_fn"), nn.SiLU) and _nothing_watches()
+                            and _plain(g._parameters.get("weight"), x.dtype, x.device)):
                         # a plain gate projection: the same call with the gate in it (torch's product alone takes 21 us of the 51
                         # of a 4096 / 14336 layer at one row, all of it 38)
-                        return flash_gemv.cats_mlp(x, g.weight, self.up_proj.weight, self.wdown_t, t)
+                        return flash_gemv.cats_mlp(x, g._parameters["weight"], _sub(self, "up_proj").weight, self.wdown_t, t)
                     return flash_gemv.gemv_gemv_triton(x, self.act_fn(self.gate_proj(x)), self.up_proj.weight, self.wdown_t, t)
                 if self.is_stats:
                     # decode-time sparsity bookkeeping (the reference's agg_sparsity, ugly_utils.py:929-937, for the

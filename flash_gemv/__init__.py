@@ -55,10 +55,10 @@ _PLAIN = {torch.Tensor, torch.nn.Parameter}
 
 def _watched():
     """Whether tracing, a transform, a mode or a module hook is at work that has to see the single torch operations of a composite."""
-    m = torch.nn.modules.module
-    return (torch.jit.is_tracing() or torch.compiler.is_compiling() or torch.is_autocast_enabled("cuda")
-            or torch._C._len_torch_dispatch_stack() or torch._C._len_torch_function_stack()
-            or torch._C._functorch.peek_interpreter_stack() is not None or torch.autograd.forward_ad._current_level >= 0
+    c, m = torch._C, torch.nn.modules.module
+    return (c._is_tracing() or torch.compiler.is_compiling() or torch.is_autocast_enabled("cuda")
+            or c._len_torch_dispatch_stack() or c._len_torch_function_stack()
+            or c._functorch.peek_interpreter_stack() is not None or torch.autograd.forward_ad._current_level >= 0
             or m._global_forward_hooks or m._global_forward_pre_hooks)
 
 
@@ -77,13 +77,12 @@ def _takes_gate_cols(x, Wgate, Wup, Wdownt, threshold):
     if not (isinstance(threshold, (int, float)) and {type(x), type(Wgate), type(Wup), type(Wdownt)} <= _PLAIN
             and not _watched() and x.is_cuda and x.numel() == x.shape[-1] and x.is_contiguous() and Wgate.dim() == 2):
         return False
-    H, I = Wgate.shape
-    d, sz = x.dtype, x.element_size()
-    return (d in (torch.float16, torch.bfloat16, torch.float32) and x.shape[-1] == H and H * sz % 16 == 0 and I * sz >= 16 and _gate_cols_fits(H, I, sz)
-            and Wup.shape == (I, H) and Wdownt.shape == (I, H) and Wgate.dtype == d and Wup.dtype == d and Wdownt.dtype == d
-            and Wgate.device == x.device and Wup.device == x.device and Wdownt.device == x.device
-            and Wgate.is_contiguous() and Wup.is_contiguous() and Wdownt.is_contiguous()
-            and (x.data_ptr() | Wup.data_ptr() | Wdownt.data_ptr()) % 16 == 0)
+    H, I = shape = Wgate.shape
+    d, sz, device = x.dtype, x.element_size(), x.device
+    if not (d in (torch.float16, torch.bfloat16, torch.float32) and x.shape[-1] == H and H * sz % 16 == 0 and I * sz >= 16 and _gate_cols_fits(H, I, sz)
+            and Wup.shape == shape[::-1] and Wdownt.shape == shape[::-1] and (x.data_ptr() | Wup.data_ptr() | Wdownt.data_ptr()) % 16 == 0):
+        return False
+    return all(w.dtype == d and w.device == device and w.is_contiguous() for w in (Wgate, Wup, Wdownt))
 
 
 def flag_gemv_gemv_triton(x, Wgate, Wup, Wdownt, threshold):
