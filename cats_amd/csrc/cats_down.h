@@ -42,6 +42,7 @@ struct DownArgs {
   int H, I, nb;
   int row_vecs;           // H / VEC
   int nslab, ngroup;
+  int slab_vecs;          // down_mma_kernel: vectors of a slab, at most 64
   int chunk;              // neurons per group, a multiple of 8
 #ifdef CATS_TIMING
   long long* tbuf;        // [gridDim][8] wall-clock stamps (100 MHz) at phase boundaries, development builds only

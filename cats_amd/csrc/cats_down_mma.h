@@ -22,6 +22,8 @@
 // in flight makes the compiler wait for all of them.  Steps past the end of the list are padding: their entries are -1,
 // they re-read row 0 (cached) and their weights are replaced by zeros before use.
 #pragma once
+#include <type_traits>
+
 #include "cats_down.h"
 
 namespace cats {
@@ -65,7 +67,99 @@ inline size_t down_mma_lds_bytes(int chunk, int nb, int depth) {
   return (stream > fold ? stream : fold) + 64;
 }
 
-template <class DT, bool ZF32, int DEPTH>
+// The first 64 neurons of a range, one step of each list wave, are asked for before the flags are there (EARLY: the flags are a byte per
+// neuron, as the whole-MLP calls leave them).  They come to rest behind the mask and z in the same memory trip, in which
+// the memory would otherwise idle, and the union of three rows and more keeps most of them; dead ones are list entries -1.
+constexpr int kDownMmaEarly = kDownMmaListWaves * kDownMmaStep;
+constexpr int kDownMmaMaskLoads = 4;  // passes of 512 neurons whose flags wave 0 has in flight together
+constexpr int kDownMmaZLoads = 8;     // z values per thread in flight together
+
+// What down_stage_list_and_z leaves, from flags `m8` and z `zv` loaded before: list entries 0 .. kDownMmaEarly - 1 are the first
+// neurons of the range (-1: dead, or past its end), those behind them the live ones among the rest.
+template <class DT, bool ZF32>
+struct DownMmaStage {
+  typedef typename DT::st st;
+  typedef typename std::conditional<ZF32, float, st>::type zt;
+  uint2 m8[kDownMmaMaskLoads];
+  zt zv[kDownMmaZLoads];
+
+  // No branches: threads without a load of their own read the first one again.
+  __device__ __forceinline__ void fetch(const DownArgs& p, int j0, int j1) {
+    const int tid = threadIdx.x, span = j1 - j0, total = p.nb * span;
+#pragma unroll
+    for (int k = 0; k < kDownMmaMaskLoads; k++) {
+      const int o = (tid + k * kWave) * 8;
+      m8[k] = *(const uint2*)(p.mask + j0 + (tid < kWave && o < span ? o : 0));
+    }
+#pragma unroll
+    for (int k = 0; k < kDownMmaZLoads; k++) {
+      const int i = tid + k * kDownMmaThreads;
+      const int b = i / span, q = i - b * span;
+      zv[k] = ((const zt*)p.z)[i < total ? (size_t)b * p.I + j0 + q : (size_t)j0];
+    }
+  }
+  static __device__ __forceinline__ st cast(zt v) {
+    if constexpr (ZF32) return DT::fromf(v);
+    else return v;
+  }
+  __device__ __forceinline__ void put(const DownArgs& p, int j0, int j1, int* s_list, st* s_z, int* s_n) {
+    const int tid = threadIdx.x, lane = tid & (kWave - 1), span = j1 - j0, total = p.nb * span;
+    if (tid < kWave) {
+      int base = kDownMmaEarly;
+      auto pass = [&](int k, uint2 m) {
+        const int o = (lane + k * kWave) * 8;  // of the lane's eight neurons in the range
+        uint32_t bits = 0;
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+          bits |= ((m.x >> (8 * e)) & 0xffu) ? 1u << e : 0u;
+          bits |= ((m.y >> (8 * e)) & 0xffu) ? 16u << e : 0u;
+        }
+        const int rem = span - o;
+        if (rem < 8) bits &= rem > 0 ? (1u << rem) - 1u : 0u;
+        if (o < kDownMmaEarly) {
+#pragma unroll
+          for (int e = 0; e < 8; e++) s_list[o + e] = (bits >> e) & 1u ? j0 + o + e : -1;
+          bits = 0;
+        }
+        const int pc = __popc(bits);
+        int rank = base + wave_scan_inclusive(pc, lane) - pc;
+        while (bits) {
+          const int bit = __builtin_ctz(bits);
+          bits &= bits - 1;
+          s_list[rank++] = j0 + o + bit;
+        }
+        base = __shfl(rank, kWave - 1, kWave);
+      };
+#pragma unroll
+      for (int k = 0; k < kDownMmaMaskLoads; k++)
+        if (k * kWave * 8 < span) pass(k, m8[k]);
+      for (int k = kDownMmaMaskLoads; k * kWave * 8 < span; k++) {
+        const int o = (lane + k * kWave) * 8;
+        pass(k, *(const uint2*)(p.mask + j0 + (o < span ? o : 0)));
+      }
+      if (lane == 0) *s_n = base;
+    }
+#pragma unroll
+    for (int k = 0; k < kDownMmaZLoads; k++) {
+      const int i = tid + k * kDownMmaThreads;
+      const int b = i / span, q = i - b * span;
+      if (i < total) s_z[b * p.chunk + q] = cast(zv[k]);
+    }
+    for (int i = tid + kDownMmaZLoads * kDownMmaThreads; i < total; i += kDownMmaThreads) {
+      const int b = i / span, q = i - b * span;
+      s_z[b * p.chunk + q] = cast(((const zt*)p.z)[(size_t)b * p.I + j0 + q]);
+    }
+  }
+};
+
+// A barrier for LDS only: __syncthreads() would also wait for the weight loads in flight.
+__device__ __forceinline__ void down_mma_lds_barrier() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
+template <class DT, bool ZF32, int DEPTH, bool EARLY>
 __global__ __launch_bounds__(kDownMmaThreads) void down_mma_kernel(DownArgs p) {
   typedef typename DT::st st;
   static_assert(sizeof(st) == 2 && DT::VEC == 8, "16-bit types only");
@@ -94,15 +188,44 @@ __global__ __launch_bounds__(kDownMmaThreads) void down_mma_kernel(DownArgs p) {
   u32x2* s_zop = (u32x2*)((char*)s_z + ((size_t)p.nb * p.chunk * 2 + 15) / 16 * 16);
   CATS_STAMP(0);
 
+  // Lanes past the end of a slab or row (H not a multiple of 512) re-read its last vector; their sums are dropped below.
+  const int L = cw * 16 + c16;  // the lane's place across the slab
+  const int v = min(slab * p.slab_vecs + min(L, p.slab_vecs - 1), p.row_vecs - 1);
+  const u32x4* wbase = p.wd + v;
+  u32x4 w[DEPTH][4];
+  auto issue = [&](int4 rows, u32x4 (&dst)[4]) {
+    dst[0] = load_stream(wbase + (size_t)max(rows.x, 0) * p.row_vecs);
+    dst[1] = load_stream(wbase + (size_t)max(rows.y, 0) * p.row_vecs);
+    dst[2] = load_stream(wbase + (size_t)max(rows.z, 0) * p.row_vecs);
+    dst[3] = load_stream(wbase + (size_t)max(rows.w, 0) * p.row_vecs);
+    // keeps the four loads here, a ring ahead of their use and in ring order, which the counted waits rely on: without it the
+    // compiler carries the row numbers round the loop instead and loads each row just before it is needed
+    asm volatile("" ::: "memory");
+    // ... and keeps the next step's work behind them: scheduled ahead, its first use of a loaded register would wait
+    // for every load in flight
+    __builtin_amdgcn_sched_barrier(0);
+  };
+
   // ---- 1. list of active rows and z of the range -> LDS ---------------------------------------------------------
-  down_stage_list_and_z<DT, ZF32>(p, j0, j1, zcols, by_list, p.nb, s_list, s_z, &s_n);
+  if constexpr (EARLY) {
+    DownMmaStage<DT, ZF32> stage;
+    stage.fetch(p, j0, j1);
+    asm volatile("" ::: "memory");  // the weights go out behind the flags and z, so that these are not waited for with them
+    __builtin_amdgcn_sched_barrier(0);
+    const int first = j0 + lw * kDownMmaStep + 4 * q;
+    issue(int4{min(first, j1 - 1), min(first + 1, j1 - 1), min(first + 2, j1 - 1), min(first + 3, j1 - 1)}, w[0]);
+    stage.put(p, j0, j1, s_list, s_z, &s_n);
+  } else {
+    down_stage_list_and_z<DT, ZF32>(p, j0, j1, zcols, by_list, p.nb, s_list, s_z, &s_n);
+  }
   if (wave == 0) {
     // padding entries, up to one ring of steps past the last one that is used (its loads are issued and never read)
     const int n0 = s_n;  // written by this wave
     const int end = (down_mma_steps_per_wave(n0, DEPTH) + DEPTH) * kDownMmaListWaves * kDownMmaStep;
     for (int i = n0 + lane; i < end; i += kWave) s_list[i] = -1;
   }
-  __syncthreads();
+  if constexpr (EARLY) down_mma_lds_barrier();
+  else __syncthreads();
   const int n = s_n;
   const int spw = down_mma_steps_per_wave(n, DEPTH);            // steps every list wave runs
   const int nsteps = spw * kDownMmaListWaves;
@@ -112,21 +235,11 @@ __global__ __launch_bounds__(kDownMmaThreads) void down_mma_kernel(DownArgs p) {
   f32x4d acc[8];
 #pragma unroll
   for (int e = 0; e < 8; e++) acc[e] = f32x4d{0.f, 0.f, 0.f, 0.f};
-  // Lanes past the end of a row (H not a multiple of 512) re-read the row's last vector; their sums are dropped below.
-  const int v = min(slab * kWave + cw * 16 + c16, p.row_vecs - 1);
-  const u32x4* wbase = p.wd + v;
   const int4* s_list4 = (const int4*)s_list;
-  u32x4 w[DEPTH][4];
 #pragma unroll
-  for (int d = 0; d < DEPTH; d++) {
-    const int4 rows = s_list4[(lw + kDownMmaListWaves * d) * 4 + q];
-    w[d][0] = load_stream(wbase + (size_t)max(rows.x, 0) * p.row_vecs);
-    w[d][1] = load_stream(wbase + (size_t)max(rows.y, 0) * p.row_vecs);
-    w[d][2] = load_stream(wbase + (size_t)max(rows.z, 0) * p.row_vecs);
-    w[d][3] = load_stream(wbase + (size_t)max(rows.w, 0) * p.row_vecs);
-    asm volatile("" ::: "memory");  // in ring order, as in the loop below: the counted waits there rely on it
-    __builtin_amdgcn_sched_barrier(0);
-  }
+  for (int d = EARLY ? 1 : 0; d < DEPTH; d++) issue(s_list4[(lw + kDownMmaListWaves * d) * 4 + q], w[d]);
+  int4 early = {0, 0, 0, 0};  // the first step's entries: dead ones are below zero
+  if constexpr (EARLY) early = s_list4[lw * 4 + q];
   // z operands: entry (step s, lane l) = z[b = l % 16][list entries 16 s + 4 (l / 16) .. + 3], zero past nb or n
   for (int i = tid; i < nsteps * kWave; i += blockDim.x) {
     const int s = i >> 6, l = i & 63;
@@ -136,15 +249,15 @@ __global__ __launch_bounds__(kDownMmaThreads) void down_mma_kernel(DownArgs p) {
     for (int r = 0; r < 4; r++) {
       const int k = k0 + r;
       zz[r] = 0;
-      if (k < n && b < p.nb) zz[r] = s_z[b * p.chunk + (by_list ? k : s_list[k] - j0)];
+      if (k < n && b < p.nb) {
+        const int at = by_list ? k : s_list[k] - j0;
+        if (!EARLY || at >= 0) zz[r] = s_z[b * p.chunk + at];
+      }
     }
     u32x2 o = {zz[0] | (zz[1] << 16), zz[2] | (zz[3] << 16)};
     s_zop[i] = o;
   }
-  // a barrier for LDS only: __syncthreads() would also wait for the weight loads in flight
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-  __builtin_amdgcn_s_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+  down_mma_lds_barrier();
   for (int t0 = 0; t0 < spw; t0 += DEPTH) {
 #pragma unroll
     for (int d = 0; d < DEPTH; d++) {
@@ -153,11 +266,14 @@ __global__ __launch_bounds__(kDownMmaThreads) void down_mma_kernel(DownArgs p) {
       const int4 nxt = s_list4[(s + kDownMmaListWaves * DEPTH) * 4 + q];   // the step that takes this register set next
       const int k0 = s * kDownMmaStep + 4 * q;
       u32x4 w0 = w[d][0], w1 = w[d][1], w2 = w[d][2], w3 = w[d][3];
-      // padding entries hold whatever row 0 holds: replace by zeros, so that an infinity there cannot become a NaN
-      if (k0 + 0 >= n) w0 = zero4();
-      if (k0 + 1 >= n) w1 = zero4();
-      if (k0 + 2 >= n) w2 = zero4();
-      if (k0 + 3 >= n) w3 = zero4();
+      // padding entries hold whatever row 0 holds, dead ones of the first step their own row: replace by zeros, so that an
+      // infinity there cannot become a NaN
+      const bool head = EARLY && d == 0;
+      if (k0 + 0 >= n || (head && early.x < 0)) w0 = zero4();
+      if (k0 + 1 >= n || (head && early.y < 0)) w1 = zero4();
+      if (k0 + 2 >= n || (head && early.z < 0)) w2 = zero4();
+      if (k0 + 3 >= n || (head && early.w < 0)) w3 = zero4();
+      if (head) early = int4{0, 0, 0, 0};
 #pragma unroll
       for (int i = 0; i < 4; i++) {
         // columns 2i (low halves) and 2i + 1 (high halves) of the lane's eight, rows 0..3 of its k block
@@ -166,16 +282,7 @@ __global__ __launch_bounds__(kDownMmaThreads) void down_mma_kernel(DownArgs p) {
         acc[2 * i] = DownMma<DT>::run(zop, lo, acc[2 * i]);
         acc[2 * i + 1] = DownMma<DT>::run(zop, hi, acc[2 * i + 1]);
       }
-      w[d][0] = load_stream(wbase + (size_t)max(nxt.x, 0) * p.row_vecs);
-      w[d][1] = load_stream(wbase + (size_t)max(nxt.y, 0) * p.row_vecs);
-      w[d][2] = load_stream(wbase + (size_t)max(nxt.z, 0) * p.row_vecs);
-      w[d][3] = load_stream(wbase + (size_t)max(nxt.w, 0) * p.row_vecs);
-      // keeps the four loads here, a ring ahead of their use: without it the compiler carries the row numbers round the
-      // loop instead and loads each row just before it is needed
-      asm volatile("" ::: "memory");
-      // ... and keeps the next step's work behind them: scheduled ahead, its first use of a loaded register would wait
-      // for every load in flight
-      __builtin_amdgcn_sched_barrier(0);
+      issue(nxt, w[d]);
     }
   }
   CATS_STAMP(2);
@@ -189,7 +296,6 @@ __global__ __launch_bounds__(kDownMmaThreads) void down_mma_kernel(DownArgs p) {
   __syncthreads();  // list, z and operands are dead from here on
   CATS_STAMP(4);
   if (4 * q < p.nb) {
-    const int L = cw * 16 + c16;
     const int swz = (L >> 3) & 1;
 #pragma unroll
     for (int i = 0; i < 4; i++)
@@ -210,8 +316,8 @@ __global__ __launch_bounds__(kDownMmaThreads) void down_mma_kernel(DownArgs p) {
       const float4 v4 = s_red4[(size_t)(g * nbp + b) * 128 + r];
       s4.x += v4.x; s4.y += v4.y; s4.z += v4.z; s4.w += v4.w;
     }
-    const int col = (slab * kWave + L) * 8 + 4 * h;
-    if (col < p.H) *(float4*)&p.partial[((size_t)group * p.nb + b) * p.H + col] = s4;
+    const int col = (slab * p.slab_vecs + L) * 8 + 4 * h;
+    if (L < p.slab_vecs && col < p.H) *(float4*)&p.partial[((size_t)group * p.nb + b) * p.H + col] = s4;
   }
   CATS_STAMP(5);
   if (p.count_out && blockIdx.x == 0) {

@@ -209,9 +209,14 @@ struct DownMmaLaunch16 {
   static bool supported(const DownArgs& a) {
     return a.partial_out && a.nb >= 1 && a.nb <= 16 && down_mma_lds_bytes(a.chunk, a.nb, kDownMmaDepth) <= 150 * 1024;
   }
-  static hipError_t run(bool zf32, const DownArgs& a, hipStream_t stream) {
+  static hipError_t run(bool zf32, const DownArgs& a_in, hipStream_t stream) {
+    DownArgs a = a_in;
+    // slabs of equal width, in whole cache lines: 385 vectors are seven of 56, the last one 49, not six of 64 and one of 1
+    a.slab_vecs = ((a.row_vecs + a.nslab - 1) / a.nslab + 7) / 8 * 8;
     const size_t lds = down_mma_lds_bytes(a.chunk, a.nb, kDownMmaDepth);
-    auto kern = zf32 ? down_mma_kernel<DT, true, kDownMmaDepth> : down_mma_kernel<DT, false, kDownMmaDepth>;
+    const bool early = a.mask_bytes && !a.flags && !a.idx;
+    auto kern = early ? (zf32 ? down_mma_kernel<DT, true, kDownMmaDepth, true> : down_mma_kernel<DT, false, kDownMmaDepth, true>)
+                      : (zf32 ? down_mma_kernel<DT, true, kDownMmaDepth, false> : down_mma_kernel<DT, false, kDownMmaDepth, false>);
     if (hipError_t e = ensure_dynamic_lds((const void*)kern, lds); e != hipSuccess) return e;
     return launch_kernel(kern, dim3(a.nslab * a.ngroup), dim3(kDownMmaThreads), lds, stream, a);
   }
