@@ -22,8 +22,8 @@
 // against 78, host time mostly.
 // Against 102 and 61 us in the same trace: 110 and 65 with the end of K looked for in every step, 101 and 64 without the dealing of
 // the loads between the MFMAs, and that 142 against 130 for the 128 x 128 tile.
-// Measured and not taken: four waves with 128 x 96 sums each (155 us), two steps of loads in registers (no change at 256 tokens
-// and more), raised wave priority around the multiplications (no change).
+// Measured and not taken: four waves with 128 x 96 sums each (155 us), two steps of loads in the registers of the large tiles (no
+// change), raised wave priority around the multiplications (no change).
 #pragma once
 #include <type_traits>
 
@@ -47,10 +47,11 @@ struct PromptArgs {
   float t;
 };
 
-// WM x WN waves of FM x FN fragments (16 tokens x 16 weight rows) each, steps of BK elements.
-template <int WM_, int WN_, int FM_, int FN_, int BK_>
+// WM x WN waves of FM x FN fragments (16 tokens x 16 weight rows) each, steps of BK elements, AHEAD (1 or an even number) steps of loads in registers.
+template <int WM_, int WN_, int FM_, int FN_, int BK_, int AHEAD_>
 struct PromptTile {
-  static constexpr int WM = WM_, WN = WN_, FM = FM_, FN = FN_, BK = BK_;
+  static constexpr int WM = WM_, WN = WN_, FM = FM_, FN = FN_, BK = BK_, AHEAD = AHEAD_;
+  static_assert(AHEAD == 1 || AHEAD % 2 == 0, "sets and LDS buffers turn together");
   static constexpr int THREADS = WM * WN * kWave, BM = WM * FM * 16, BN = WN * FN * 16;
   static constexpr int P = BK / 8;                 // 16-byte pieces of a row
   static constexpr int STEP = (BM + BN) * P;       // vectors of one LDS buffer
@@ -111,8 +112,8 @@ __global__ __launch_bounds__(T::THREADS) void prompt_kernel(PromptArgs p) {
   // Elements of this thread's vector of a step that lie behind K.  The vector in which K ends is read so that it ends with the row
   // and shifted down before it is stored; those behind it are stored as zeros.
   auto over = [&](int step) { return max(kbegin + step * T::BK + piece * 8 + 8 - p.K, 0); };
-  u32x4 ra[VA], rb[VB];  // the step that is stored next
-  auto load = [&](int step) {
+  u32x4 ring_a[T::AHEAD][VA], ring_b[T::AHEAD][VB];  // the steps that are stored next
+  auto load = [&](int step, u32x4 (&ra)[VA], u32x4 (&rb)[VB]) {
     const uint32_t at = (uint32_t)(kbegin + step * T::BK - over(step)) * 2u;
 #pragma unroll
     for (int i = 0; i < VB; i++) rb[i] = *(const u32x4_elem*)((const char*)(is_up(i) ? p.w2 : p.w) + (ob[i] + at));
@@ -127,7 +128,7 @@ __global__ __launch_bounds__(T::THREADS) void prompt_kernel(PromptArgs p) {
     return u32x4{(uint32_t)rlo, (uint32_t)(rlo >> 32), (uint32_t)rhi, (uint32_t)(rhi >> 32)};
   };
   const int put = row * P + (piece ^ (row & 7));  // PASS is a multiple of 8: the same permutation for all of a thread's rows
-  auto store = [&](int step, int buf, auto ends) {
+  auto store = [&](int step, int buf, u32x4 (&ra)[VA], u32x4 (&rb)[VB], auto ends) {
     if (ends && kbegin + (step + 1) * T::BK > p.K) {  // uniform
       const int s = over(step);
 #pragma unroll
@@ -175,10 +176,11 @@ __global__ __launch_bounds__(T::THREADS) void prompt_kernel(PromptArgs p) {
   // last are loaded (the end of the rows again) and stored as well, and not used.  `ends`: K may end in the step that is stored.
   // The LDS and memory instructions are dealt out between the MFMAs: issued in one go they queue, all waves of the CU at once, while
   // the matrix cores wait.
-  auto step = [&](int s, int buf, auto ends) {
+  auto step = [&](int s, int buf, u32x4 (&ra)[VA], u32x4 (&rb)[VB], auto ends) {
     fetch(buf, 1);
-    store(s + 1, buf ^ 1, ends);
-    load(s + 2);
+    store(s + 1, buf ^ 1, ra, rb, ends);
+    // steps past the last: the last one again, which the caches hold
+    load(T::AHEAD == 1 ? s + 2 : min(s + 1 + T::AHEAD, nsteps), ra, rb);
     multiply(0);
     if constexpr (KK == 2) PromptDeal<FM * FN, FM + FN, VA + VB, VA + VB>::template go<0>();
 #pragma unroll
@@ -194,20 +196,23 @@ __global__ __launch_bounds__(T::THREADS) void prompt_kernel(PromptArgs p) {
     if constexpr (KK == 2) PromptDeal<(FM * FN < FM + FN ? FM * FN : FM + FN), FM + FN, 0, 0>::template go<0>();
     __builtin_amdgcn_sched_barrier(0);
   };
-  load(0);
-  store(0, 0, std::true_type());
-  load(1);
+  constexpr int AHEAD = T::AHEAD, TURN = AHEAD == 1 ? 2 : AHEAD;
+  load(0, ring_a[0], ring_b[0]);
+  store(0, 0, ring_a[0], ring_b[0], std::true_type());
+#pragma unroll
+  for (int i = 1; i <= AHEAD; i++) load(min(i, nsteps), ring_a[i % AHEAD], ring_b[i % AHEAD]);
   __syncthreads();
   fetch(0, 0);
   const int whole = min(nsteps, (p.K - kbegin) / T::BK);  // steps that K does not end in
-  int s = 0;
-  for (; s + 2 < whole; s += 2) {
-    step(s, 0, std::false_type());
-    step(s + 1, 1, std::false_type());
+  int s = 0;  // the loads of step s + 1 are in set (s + 1) % AHEAD
+  for (; s + TURN < whole; s += TURN) {
+#pragma unroll
+    for (int i = 0; i < TURN; i++) step(s + i, i & 1, ring_a[(i + 1) % AHEAD], ring_b[(i + 1) % AHEAD], std::false_type());
   }
-  for (; s < nsteps; s += 2) {
-    step(s, 0, std::true_type());
-    if (s + 1 < nsteps) step(s + 1, 1, std::true_type());
+  for (; s < nsteps; s += TURN) {
+#pragma unroll
+    for (int i = 0; i < TURN; i++)
+      if (s + i < nsteps) step(s + i, i & 1, ring_a[(i + 1) % AHEAD], ring_b[(i + 1) % AHEAD], std::true_type());
   }
 
   // lane: token fr of a fragment, four consecutive weight rows fq * 4 ..
@@ -289,15 +294,20 @@ struct PromptShape {
   int BM, BN, BK;
   float alone, shared;
 };
-typedef PromptTile<2, 2, 1, 2, 128> PromptTile0;
-typedef PromptTile<2, 2, 2, 2, 128> PromptTile1;
-typedef PromptTile<4, 2, 2, 4, 64> PromptTile2;
-typedef PromptTile<4, 2, 4, 4, 64> PromptTile3;
-typedef PromptTile<4, 2, 4, 6, 64> PromptTile4;
+// The small tiles have a second instance with two steps of loads in registers, taken where a CU has at most one workgroup and so too
+// few bytes in flight, from six steps on (whole call in us, one / two steps ahead: 2048 / 5461 2 tokens 28.7 / 26.3 and 192 tokens
+// 47.6 / 42.8, 4096 / 11008 96 tokens 83.7 / 74.8, 3072 / 8192 192 tokens 68.8 / 62.6, 1536 / 4096 32 tokens 23.2 / 22.2).  With more
+// workgroups a CU the registers cost more than they give (4096 / 11008 64 tokens 74.8 / 76.8), and so does the longer start of a short
+// range (512 / 1365, four steps, 192 tokens 16.3 / 17.0).  Four steps ahead: slower than two nearly everywhere (32 tokens 69.6 for 66.3).
+template <int AHEAD> using PromptTile0 = PromptTile<2, 2, 1, 2, 128, AHEAD>;
+template <int AHEAD> using PromptTile1 = PromptTile<2, 2, 2, 2, 128, AHEAD>;
+template <int AHEAD> using PromptTile2 = PromptTile<4, 2, 2, 4, 64, AHEAD>;
+typedef PromptTile<4, 2, 4, 4, 64, 1> PromptTile3;
+typedef PromptTile<4, 2, 4, 6, 64, 1> PromptTile4;
 constexpr int kPromptTiles = 5;
 constexpr PromptShape kPromptShapes[kPromptTiles] = {
-    {PromptTile0::BM, PromptTile0::BN, PromptTile0::BK, 0.8f, 0.55f}, {PromptTile1::BM, PromptTile1::BN, PromptTile1::BK, 0.9f, 0.65f},
-    {PromptTile2::BM, PromptTile2::BN, PromptTile2::BK, 0.7f, 0.65f}, {PromptTile3::BM, PromptTile3::BN, PromptTile3::BK, 1.1f, 1.1f},
+    {PromptTile0<1>::BM, PromptTile0<1>::BN, PromptTile0<1>::BK, 0.8f, 0.55f}, {PromptTile1<1>::BM, PromptTile1<1>::BN, PromptTile1<1>::BK, 0.9f, 0.65f},
+    {PromptTile2<1>::BM, PromptTile2<1>::BN, PromptTile2<1>::BK, 0.7f, 0.65f}, {PromptTile3::BM, PromptTile3::BN, PromptTile3::BK, 1.1f, 1.1f},
     {PromptTile4::BM, PromptTile4::BN, PromptTile4::BK, 1.45f, 1.45f}};
 
 struct PromptPlan {

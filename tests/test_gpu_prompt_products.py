@@ -44,6 +44,12 @@ def test_prompt_mlp(M, H, I, dtype):
     assert kept == 0 or rel < 3 * step + 0.1 / math.sqrt(kept), rel
 
 
+@pytest.mark.parametrize("M,H,I", [(2, 640, 515), (32, 641, 1000), (9, 773, 515), (48, 905, 900), (64, 1283, 515), (100, 384, 700), (128, 393, 1041), (200, 520, 2731)])
+def test_two_steps_ahead(M, H, I):
+    """Launches of at most one workgroup a CU, five steps of K and more, odd and even numbers of them, K ending inside and on a step."""
+    test_prompt_mlp(M, H, I, torch.float16)
+
+
 @pytest.mark.parametrize("M,H,I", [(5, 64, 9), (40, 304, 569), (130, 136, 1041)])
 def test_what_lies_outside_a_row_stays_outside(M, H, I):
     """Infinities and NaN in one token or one weight row: reached by the columns torch reaches, whatever vector they share with others."""
