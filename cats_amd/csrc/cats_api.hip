@@ -34,9 +34,9 @@ template <> hipError_t launch_fused<F32>(int, int, int, const FusedArgs&, const 
 template <> hipError_t launch_proj<F16>(int, int, const ProjArgs&, hipStream_t);
 template <> hipError_t launch_proj<BF16>(int, int, const ProjArgs&, hipStream_t);
 template <> hipError_t launch_proj<F32>(int, int, const ProjArgs&, hipStream_t);
-template <> hipError_t launch_attn<F16>(int, int, const AttnArgs&, hipStream_t);
-template <> hipError_t launch_attn<BF16>(int, int, const AttnArgs&, hipStream_t);
-template <> hipError_t launch_attn<F32>(int, int, const AttnArgs&, hipStream_t);
+template <> hipError_t launch_attn<F16>(int, int, AttnArgs, hipStream_t);
+template <> hipError_t launch_attn<BF16>(int, int, AttnArgs, hipStream_t);
+template <> hipError_t launch_attn<F32>(int, int, AttnArgs, hipStream_t);
 template <> hipError_t launch_gate_cols<F16>(const GateColsArgs&, int, hipStream_t);
 template <> hipError_t launch_gate_cols<BF16>(const GateColsArgs&, int, hipStream_t);
 template <> hipError_t launch_gate_cols<F32>(const GateColsArgs&, int, hipStream_t);
@@ -1547,9 +1547,14 @@ int cats_attention_step(const void* h, const void* x, const void* norm_weight, f
   t.out = attn_scratch;
   t.scale = 1.44269504088896341f / sqrtf((float)hd);
   t.max_len = max_len;
-  const hipError_t e = dtype == CATS_F16    ? launch_attn<F16>(B * heads, hd, t, (hipStream_t)stream)
-                       : dtype == CATS_BF16 ? launch_attn<BF16>(B * heads, hd, t, (hipStream_t)stream)
-                                            : launch_attn<F32>(B * heads, hd, t, (hipStream_t)stream);
+  t.pairs = B * heads;
+  t.next = (const u32x4*)wo;
+  t.piece_vecs = H / vec_elems(dtype);
+  const size_t vecs = (size_t)H * t.piece_vecs;
+  t.next_vecs = (unsigned)(vecs < kAttnAheadVecs ? vecs : kAttnAheadVecs);
+  const hipError_t e = dtype == CATS_F16    ? launch_attn<F16>(hd, B, t, (hipStream_t)stream)
+                       : dtype == CATS_BF16 ? launch_attn<BF16>(hd, B, t, (hipStream_t)stream)
+                                            : launch_attn<F32>(hd, B, t, (hipStream_t)stream);
   if (e != hipSuccess) return CATS_ERR_LAUNCH;
   return cats_linear(attn_scratch, nullptr, 0.f, wo, h, out, B, H, H, dtype, stream);
 }

@@ -8,7 +8,7 @@
 // x may be given before its RMS norm (norm_w), which is then applied while x is staged.  Everything between the weight
 // matrices stays in fp32 and is rounded once where it is stored.  All of it is bound by the weight stream: one wave owns two
 // rows of a matrix, whose loads are all in flight at once, as in rows_kernel.
-// One step of four layers 4096 / 11008, 32 heads, 32000 words, 256 tokens in the cache, fp16, one row: 327 us, of which the MLP
+// One step of four layers 4096 / 11008, 32 heads, 32000 words, 256 tokens in the cache, fp16, one row: 321 us, of which the MLP
 // kernels take 150; with torch's operations in place of these kernels (about 25 launches a layer) it was 761.  Kernel trace: q, k, v
 // 18.9 us with the norm (5.3 TB/s), attention 6.6, output projection 8.4, output head 44 (5.9 TB/s).
 #pragma once
@@ -168,13 +168,43 @@ struct AttnArgs {
   void* out;             // (nb, heads * head_dim) dtype
   float scale;           // log2(e) / sqrt(head_dim)
   int max_len;
+  int pairs;             // batch rows x heads: the workgroups that attend; those behind them fetch `next` ahead
+  const u32x4* next;     // weights of the projection that follows, in pieces of one of its workgroups each
+  unsigned next_vecs;    // less than 2^28
+  int piece_vecs;
 };
+
+// The projection that follows depends on this launch, and attention leaves most CUs and the memory idle.  So the workgroups behind the
+// attending ones read its weights into the caches: the pieces that an XCD's workgroups will ask for on this XCD (workgroups go
+// round the eight XCDs in both launches).  They start about 2 us late, when the cache slots have been asked for: at once they hold
+// those up (attention 10.1 us for 6.6), and as much is fetched as comes in meanwhile.  Step of four layers as above: 327.9 us without
+// (output projection 8.1 us); 24 MiB 320.6, started at once 325 to 335; 32 MiB 322 to 325 (output projection 4.7); 16 MiB 322.1.
+constexpr unsigned kAttnAheadVecs = (24u << 20) / 16;
+constexpr int kAttnAheadSleeps = 5;  // of 1024 clocks each
+__device__ __forceinline__ void attn_fetch_next(const AttnArgs& p) {
+  constexpr int kLoads = 10;  // in flight per thread
+  const unsigned xcd = blockIdx.x & 7, groups = (gridDim.x - p.pairs) / 8;  // workgroups on this XCD
+  const unsigned piece = p.piece_vecs, first = (blockIdx.x - p.pairs) / 8 * 1024 + threadIdx.x;
+  for (int i = 0; i < kAttnAheadSleeps; i++) __builtin_amdgcn_s_sleep(16);
+  const unsigned pieces = (p.next_vecs + piece - 1) / piece, mine = ((pieces + 7 - xcd) / 8) * piece;  // vectors for this XCD
+  for (unsigned t = first; t < mine; t += kLoads * groups * 1024) {
+    u32x4 w[kLoads];
+#pragma unroll
+    for (int i = 0; i < kLoads; i++) {
+      const unsigned at = min(t + i * groups * 1024, mine - 1), n = at / piece;
+      w[i] = p.next[min((xcd + 8 * n) * piece + (at - n * piece), p.next_vecs - 1)];
+    }
+#pragma unroll
+    for (int i = 0; i < kLoads; i++) asm volatile("" ::"v"(w[i]));
+  }
+}
 
 // One workgroup of sixteen waves per (batch row, head).  A slot's head_dim elements sit in LPS lanes of one 16-byte vector
 // each, so a wave holds 64 / LPS slots side by side and the workgroup 16 * 64 / LPS; every lane group runs its own online
 // softmax over the slots it meets, U slots a turn with the loads of K and V of all of them in flight together (256 slots of 128
-// 16-bit elements are one turn), and the groups' results are merged at the end, in a fixed order.  What bounds it is three
-// dependent memory trips (position, q, K and V), not the bytes: 131 KiB a head at 256 slots.
+// 16-bit elements are one turn), and the groups' results are merged at the end, in a fixed order.  What bounds it is dependent
+// memory trips, not the bytes (131 KiB a head at 256 slots): so the first turn's slots are asked for with the position, whatever it is
+// (slots behind it hold anything and are masked), and the next turn's before this one's are used.
 template <class DT, int LPS>
 __global__ __launch_bounds__(1024) void attn_decode_kernel(AttnArgs p) {
   typedef typename DT::st st;
@@ -185,10 +215,10 @@ __global__ __launch_bounds__(1024) void attn_decode_kernel(AttnArgs p) {
   const int wave = threadIdx.x >> 6;
   const int sub = lane % LPS;
   const int slot0 = wave * G + lane / LPS;
-  const long long pos = *p.pos;
-  const int n = pos >= 0 && pos < (long long)p.max_len ? (int)pos + 1 : 0;
+  if ((int)blockIdx.x >= p.pairs) return attn_fetch_next(p);
   const u32x4* kb = p.k + (size_t)blockIdx.x * p.max_len * LPS + sub;
   const u32x4* vb = p.v + (size_t)blockIdx.x * p.max_len * LPS + sub;
+  const long long pos = *p.pos;
   float q[VEC];
 #pragma unroll
   for (int e = 0; e < VEC; e++) q[e] = p.q[(size_t)blockIdx.x * HD + sub * VEC + e] * p.scale;
@@ -197,15 +227,20 @@ __global__ __launch_bounds__(1024) void attn_decode_kernel(AttnArgs p) {
     if constexpr (sizeof(st) == 4) return __uint_as_float(x[e]);
     else return DT::tof((st)(x[e / 2] >> (16 * (e & 1))));
   };
+  u32x4 kv[U], vv[U], kn[U], vn[U];
+  auto fetch = [&](int s0, int last, u32x4 (&k)[U], u32x4 (&v)[U]) {
+#pragma unroll
+    for (int u = 0; u < U; u++) k[u] = kb[(size_t)min(s0 + u * S + slot0, last) * LPS];
+#pragma unroll
+    for (int u = 0; u < U; u++) v[u] = vb[(size_t)min(s0 + u * S + slot0, last) * LPS];
+  };
+  fetch(0, p.max_len - 1, kv, vv);
+  const int n = pos >= 0 && pos < (long long)p.max_len ? (int)pos + 1 : 0;
   float m = -INFINITY, l = 0.f, acc[VEC];
 #pragma unroll
   for (int e = 0; e < VEC; e++) acc[e] = 0.f;
   for (int s0 = 0; s0 < n; s0 += S * U) {
-    u32x4 kv[U], vv[U];
-#pragma unroll
-    for (int u = 0; u < U; u++) kv[u] = kb[(size_t)min(s0 + u * S + slot0, n - 1) * LPS];
-#pragma unroll
-    for (int u = 0; u < U; u++) vv[u] = vb[(size_t)min(s0 + u * S + slot0, n - 1) * LPS];
+    fetch(s0 + S * U, n - 1, kn, vn);  // past the last turn: the last slot again, which the caches hold
     float sc[U], mu = m;
 #pragma unroll
     for (int u = 0; u < U; u++) {
@@ -231,6 +266,11 @@ __global__ __launch_bounds__(1024) void attn_decode_kernel(AttnArgs p) {
       for (int e = 0; e < VEC; e++) acc[e] = in ? fmaf(pr, elem(vv[u], e), acc[e]) : acc[e];
     }
     m = mu;
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+      kv[u] = kn[u];
+      vv[u] = vn[u];
+    }
   }
   // the wave's groups, then the waves
   float mw = m;

@@ -282,7 +282,7 @@ hipError_t launch_proj<CATS_DT>(int mode, int bt, const ProjArgs& a, hipStream_t
 }
 
 template <>
-hipError_t launch_attn<CATS_DT>(int blocks, int head_dim, const AttnArgs& a, hipStream_t stream) {
+hipError_t launch_attn<CATS_DT>(int head_dim, int bt, AttnArgs a, hipStream_t stream) {
   void (*kern)(AttnArgs) = nullptr;
   switch (head_dim / CATS_DT::VEC) {  // lanes per cache slot
     case 2: kern = attn_decode_kernel<CATS_DT, 2>; break;
@@ -292,7 +292,11 @@ hipError_t launch_attn<CATS_DT>(int blocks, int head_dim, const AttnArgs& a, hip
     case 32: kern = attn_decode_kernel<CATS_DT, 32>; break;
   }
   if (!kern) return hipErrorInvalidValue;
-  return launch_kernel(kern, dim3(blocks), dim3(1024), 0, stream, a);
+  // the CUs that attention leaves free fetch the next projection's weights, where they are at least a quarter of the chip
+  const int cus = current_device_cus();
+  const int ahead = a.pairs <= cus - cus / 4 ? (cus - a.pairs) / 8 * 8 : 0;
+  a.piece_vecs *= kR * (bt <= 2 ? WavesFor<1>::value : WavesFor<8>::value);  // from vectors of a row to those of a workgroup of proj_kernel
+  return launch_kernel(kern, dim3(a.pairs + ahead), dim3(1024), 0, stream, a);
 }
 
 template <>

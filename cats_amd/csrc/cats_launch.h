@@ -84,7 +84,7 @@ inline size_t proj_lds_bytes(int bt, int nch) { return (size_t)bt * ((nch + kPro
 template <class DT>
 hipError_t launch_proj(int mode, int bt, const ProjArgs& a, hipStream_t stream);
 template <class DT>
-hipError_t launch_attn(int blocks, int head_dim, const AttnArgs& a, hipStream_t stream);
+hipError_t launch_attn(int head_dim, int bt, AttnArgs a, hipStream_t stream);  // a.piece_vecs: vectors of a row of a.next
 template <class DT>
 hipError_t launch_silu_mask_mul(const SiluMaskMulArgs& a, hipStream_t stream);
 

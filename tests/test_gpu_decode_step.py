@@ -89,6 +89,12 @@ def test_attention_step(B, heads, hd, max_len, pos, dtype):
         assert bool(out.isnan().all()) and torch.equal(kd, before)
 
 
+@pytest.mark.parametrize("B,heads,hd,max_len,pos", [(7, 28, 16, 40, 20), (1, 20, 128, 600, 511), (8, 24, 16, 3, 2)])
+def test_attention_with_and_without_workgroups_that_fetch_ahead(B, heads, hd, max_len, pos):
+    """196 of 256 CUs attending: none fetch the next weights; 20 and 192: the rest do, also from a number that is no multiple of eight."""
+    test_attention_step(B, heads, hd, max_len, pos, torch.float16)
+
+
 @pytest.mark.parametrize("B,mode", [(1, "cats_fused_next"), (4, "cats_fused_next"), (2, "cats_fused"), (3, "cats"), (1, "dense")])
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 def test_step_matches_torch_operations(B, mode, dtype):
