@@ -174,6 +174,22 @@ struct MmaRows {
       for (int s = 0; s < STEPS; s++)
         acc[g] = Mma<DT>::run(outside(c, s) ? zero4() : src[s], xs[g * xgroup + (c * STEPS + s) * kWave], acc[g]);
   }
+  // The same with this lane's x operands of chunk 0 in registers.  The groups of batch rows take turns: their sums are two
+  // independent chains of MFMAs.
+  __device__ __forceinline__ void hold(u32x4 (&x)[NG][STEPS]) const {
+#pragma unroll
+    for (int g = 0; g < NG; g++)
+#pragma unroll
+      for (int s = 0; s < STEPS; s++) x[g][s] = xs[g * xgroup + s * kWave];
+  }
+  __device__ __forceinline__ void multiply(const u32x4 (&src)[STEPS], const u32x4 (&x)[NG][STEPS], Acc (&acc)[NG]) const {
+#pragma unroll
+    for (int s = 0; s < STEPS; s++) {
+      const u32x4 w = outside(0, s) ? zero4() : src[s];
+#pragma unroll
+      for (int g = 0; g < NG; g++) acc[g] = Mma<DT>::run(w, x[g][s], acc[g]);
+    }
+  }
 };
 
 constexpr int kMmaPartGroup = kMmaWaves * kMmaPart;  // partial-sum floats of one group of eight batch rows
@@ -262,10 +278,15 @@ struct MmaX {
 // LDS and a second MFMA on the weight registers the first one just used, so the weights are still read once.
 // CH = 2 (rows of more than 72 steps, 4608 16-bit elements; their x fills 128 KiB of LDS at 8192): a tile is two register sets, so the gate ring
 // holds one tile ahead instead of two, and the up sums of tile r - 1 are taken before the up rows of tile r overwrite their set.
+// A wave multiplies the same steps of K for every tile, so one chunk's x operands stay in its registers (kHeld) once they are
+// staged: read from LDS for every tile they cost a CU 1 KiB (2 KiB at 9..16 rows) of LDS traffic a KiB of weights, 6 us of a 43 us
+// kernel at sixteen rows, part of it in front of the next loads (4096 / 14336 bf16 16 rows: kernel 43.7 / 41.7 us, call 70.6 / 70.0;
+// 3080 / 8191 3 rows 33.25 / 33.0; 4 and 8 rows of 4096 as before).
 template <class DT, int STEPS, int CH, bool UP, int NG = 1>
 __global__ __launch_bounds__(kMmaThreads) void rows_mma_kernel(RowsArgs p) {
   typedef typename DT::st st;
   typedef MmaRows<DT, STEPS, CH, NG> Rows;
+  constexpr bool kHeld = CH == 1 && NG * STEPS <= (sizeof(st) == 2 ? 16 : 9);  // more would not fit beside four sets of weights
   extern __shared__ u32x4 xs[];  // [NG][mma_slots][64] x operands, then the partial buffers
   __shared__ uint32_t s_any;
 
@@ -306,13 +327,20 @@ __global__ __launch_bounds__(kMmaThreads) void rows_mma_kernel(RowsArgs p) {
   uint32_t prev_bits = 0u;
   int prev_row = 0;
 
+  u32x4 held[NG][STEPS];
+  const bool one_phase = gate.xs == up.xs;  // uniform; else the two matrices start at different places of a line and take turns in `held`
   // gbuf, ubuf, uprev: the register sets of the round.  One chunk: gbuf[0] is the tile's set, ubuf[0] takes its up rows, uprev[0]
   // holds those of the tile before.  Two chunks: gbuf[0..1] and ubuf[0..1] are the tile's two sets, uprev is ubuf.
   auto round_body = [&](int r, u32x4 (&ga)[STEPS], u32x4 (&gb)[STEPS], u32x4 (&ucur)[STEPS], u32x4 (&uprev)[STEPS]) {
     typename Mma<DT>::Acc acc[NG];
 #pragma unroll
     for (int g = 0; g < NG; g++) acc[g] = Mma<DT>::zero();
-    gate.multiply(ga, 0, acc);
+    if constexpr (kHeld) {
+      if (UP && !one_phase) gate.hold(held);
+      gate.multiply(ga, held, acc);
+    } else {
+      gate.multiply(ga, 0, acc);
+    }
     if constexpr (CH == 2) {
       issue_gate(r + 1, 0, ga);
       gate.multiply(gb, 1, acc);
@@ -362,7 +390,12 @@ __global__ __launch_bounds__(kMmaThreads) void rows_mma_kernel(RowsArgs p) {
       issue_up(r, 1, uprev);
     } else {
       issue_up(r, 0, ucur);
-      up.multiply(uprev, 0, acc);
+      if constexpr (kHeld) {
+        if (!one_phase) up.hold(held);
+        up.multiply(uprev, held, acc);
+      } else {
+        up.multiply(uprev, 0, acc);
+      }
     }
     mma_store_partials<DT, NG>(acc, part_u, lane, wave);
     __syncthreads();
@@ -430,6 +463,7 @@ __global__ __launch_bounds__(kMmaThreads) void rows_mma_kernel(RowsArgs p) {
     __syncthreads();
   }
   CATS_RSTAMP(1);
+  if constexpr (kHeld) gate.hold(held);
 
   // rounds 0 .. my_tiles: the last one only drains the up sums of the last tile
   const int last = UP ? my_tiles : my_tiles - 1;
