@@ -295,20 +295,26 @@ struct PromptShape {
   float alone, shared;
 };
 // The small tiles have a second instance with two steps of loads in registers, taken where a CU has at most one workgroup and so too
-// few bytes in flight, from six steps on (whole call in us, one / two steps ahead: 2048 / 5461 2 tokens 28.7 / 26.3 and 192 tokens
+// few bytes in flight, from ten steps on (whole call in us, one / two steps ahead: 2048 / 5461 2 tokens 28.7 / 26.3 and 192 tokens
 // 47.6 / 42.8, 4096 / 11008 96 tokens 83.7 / 74.8, 3072 / 8192 192 tokens 68.8 / 62.6, 1536 / 4096 32 tokens 23.2 / 22.2).  With more
 // workgroups a CU the registers cost more than they give (4096 / 11008 64 tokens 74.8 / 76.8), and so does the longer start of a short
-// range (512 / 1365, four steps, 192 tokens 16.3 / 17.0).  Four steps ahead: slower than two nearly everywhere (32 tokens 69.6 for 66.3).
+// range (512 / 1365, four steps, 192 tokens 16.3 / 17.0; 2048 / 5461, six steps of the second product, 64 tokens 32.8 / 33.6).  Four steps ahead: slower than two nearly everywhere (32 tokens 69.6 for 66.3).
 template <int AHEAD> using PromptTile0 = PromptTile<2, 2, 1, 2, 128, AHEAD>;
 template <int AHEAD> using PromptTile1 = PromptTile<2, 2, 2, 2, 128, AHEAD>;
 template <int AHEAD> using PromptTile2 = PromptTile<4, 2, 2, 4, 64, AHEAD>;
 typedef PromptTile<4, 2, 4, 4, 64, 1> PromptTile3;
 typedef PromptTile<4, 2, 4, 6, 64, 1> PromptTile4;
-constexpr int kPromptTiles = 5;
+// Half of tile 0: two or three workgroups a CU where tile 0 has one on most and two on some, so the weights come in evenly (4096 / 11008
+// 2 tokens: gate and up 3.4 us less, down 1.6; at 32 tokens, where it reads x twice as often, 0.5 and 0.7).  Up to two blocks of tokens:
+// at 128 tokens of 512 / 1365 13.9 us without it, 14.5 with.  Whole call at 2, 16 and 32 tokens, before / now: 4096 / 11008 64.2 / 59.6,
+// 65.0 / 60.9, 66.5 / 63.7; 1024 / 2731 18.5 / 16.5, 19.0 / 17.0, 19.3 / 17.3.
+typedef PromptTile<2, 1, 1, 2, 128, 1> PromptTile5;
+constexpr int kPromptTiles = 6;
 constexpr PromptShape kPromptShapes[kPromptTiles] = {
     {PromptTile0<1>::BM, PromptTile0<1>::BN, PromptTile0<1>::BK, 0.8f, 0.55f}, {PromptTile1<1>::BM, PromptTile1<1>::BN, PromptTile1<1>::BK, 0.9f, 0.65f},
     {PromptTile2<1>::BM, PromptTile2<1>::BN, PromptTile2<1>::BK, 0.7f, 0.65f}, {PromptTile3::BM, PromptTile3::BN, PromptTile3::BK, 1.1f, 1.1f},
-    {PromptTile4::BM, PromptTile4::BN, PromptTile4::BK, 1.45f, 1.45f}};
+    {PromptTile4::BM, PromptTile4::BN, PromptTile4::BK, 1.45f, 1.45f},
+    {PromptTile5::BM, PromptTile5::BN, PromptTile5::BK, 0.6f, 0.33f}};
 
 struct PromptPlan {
   int tile, mblocks, nblocks, steps, splits;
@@ -321,6 +327,7 @@ inline PromptPlan prompt_plan(bool gate_up, int M, int N, int K, int cus) {
   for (int t = 0; t < kPromptTiles; t++) {
     const PromptShape& h = kPromptShapes[t];
     const int bn = gate_up ? h.BN / 2 : h.BN, ksteps = (K + h.BK - 1) / h.BK;
+    if (h.BN == PromptTile5::BN && M > 2 * h.BM) continue;
     const int mblocks = (M + h.BM - 1) / h.BM, nblocks = (N + bn - 1) / bn;
     for (int want = 1; want <= (gate_up ? 1 : 8); want++) {
       const int steps = (ksteps + want - 1) / want, splits = (ksteps + steps - 1) / steps;
