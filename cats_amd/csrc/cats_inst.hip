@@ -321,7 +321,7 @@ struct PromptLaunch {
     const bool alone = a.steps >= 10 && (long long)a.mblocks * a.nblocks * a.splits <= current_device_cus();
     switch (t) {
       case 0: return alone ? tile<PromptTile0<2>, GATE_UP>(a, stream) : tile<PromptTile0<1>, GATE_UP>(a, stream);
-      case 1: return alone ? tile<PromptTile1<2>, GATE_UP>(a, stream) : tile<PromptTile1<1>, GATE_UP>(a, stream);
+      case 1: return tile<PromptTile1, GATE_UP>(a, stream);
       case 2: return alone ? tile<PromptTile2<2>, GATE_UP>(a, stream) : tile<PromptTile2<1>, GATE_UP>(a, stream);
       case 3: return tile<PromptTile3, GATE_UP>(a, stream);
       case 4: return tile<PromptTile4, GATE_UP>(a, stream);

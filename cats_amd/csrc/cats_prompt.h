@@ -294,24 +294,26 @@ struct PromptShape {
   int BM, BN, BK;
   float alone, shared;
 };
-// The small tiles have a second instance with two steps of loads in registers, taken where a CU has at most one workgroup and so too
+// Tiles 0 and 2 have a second instance with two steps of loads in registers, taken where a CU has at most one workgroup and so too
 // few bytes in flight, from ten steps on (whole call in us, one / two steps ahead: 2048 / 5461 2 tokens 28.7 / 26.3 and 192 tokens
 // 47.6 / 42.8, 4096 / 11008 96 tokens 83.7 / 74.8, 3072 / 8192 192 tokens 68.8 / 62.6, 1536 / 4096 32 tokens 23.2 / 22.2).  With more
 // workgroups a CU the registers cost more than they give (4096 / 11008 64 tokens 74.8 / 76.8), and so does the longer start of a short
-// range (512 / 1365, four steps, 192 tokens 16.3 / 17.0; 2048 / 5461, six steps of the second product, 64 tokens 32.8 / 33.6).  Four steps ahead: slower than two nearly everywhere (32 tokens 69.6 for 66.3).
+// range (512 / 1365, four steps, 192 tokens 16.3 / 17.0).  Four steps ahead: slower than two nearly everywhere (32 tokens 69.6 for
+// 66.3).  Tile 1 has none: up to 5 % less on weights from HBM, 3 % more on weights that the caches hold.
 template <int AHEAD> using PromptTile0 = PromptTile<2, 2, 1, 2, 128, AHEAD>;
-template <int AHEAD> using PromptTile1 = PromptTile<2, 2, 2, 2, 128, AHEAD>;
+typedef PromptTile<2, 2, 2, 2, 128, 1> PromptTile1;
 template <int AHEAD> using PromptTile2 = PromptTile<4, 2, 2, 4, 64, AHEAD>;
 typedef PromptTile<4, 2, 4, 4, 64, 1> PromptTile3;
 typedef PromptTile<4, 2, 4, 6, 64, 1> PromptTile4;
 // Half of tile 0: two or three workgroups a CU where tile 0 has one on most and two on some, so the weights come in evenly (4096 / 11008
-// 2 tokens: gate and up 3.4 us less, down 1.6; at 32 tokens, where it reads x twice as often, 0.5 and 0.7).  Up to two blocks of tokens:
-// at 128 tokens of 512 / 1365 13.9 us without it, 14.5 with.  Whole call at 2, 16 and 32 tokens, before / now: 4096 / 11008 64.2 / 59.6,
+// 2 tokens: gate and up 3.4 us less, down 1.6; at 32 tokens, where it reads x twice as often, 0.5 and 0.7).  Up to two blocks of tokens
+// (at 128 tokens of 512 / 1365 13.9 us without it, 14.5 with), and where at most a fifth of the last round's places stay empty: 342
+// workgroups of 2048 / 5461 at 30 tokens, weights in cache, 23.7 us against 22.8.  Whole call at 2, 16 and 32 tokens, before / now: 4096 / 11008 64.2 / 59.6,
 // 65.0 / 60.9, 66.5 / 63.7; 1024 / 2731 18.5 / 16.5, 19.0 / 17.0, 19.3 / 17.3.
 typedef PromptTile<2, 1, 1, 2, 128, 1> PromptTile5;
 constexpr int kPromptTiles = 6;
 constexpr PromptShape kPromptShapes[kPromptTiles] = {
-    {PromptTile0<1>::BM, PromptTile0<1>::BN, PromptTile0<1>::BK, 0.8f, 0.55f}, {PromptTile1<1>::BM, PromptTile1<1>::BN, PromptTile1<1>::BK, 0.9f, 0.65f},
+    {PromptTile0<1>::BM, PromptTile0<1>::BN, PromptTile0<1>::BK, 0.8f, 0.55f}, {PromptTile1::BM, PromptTile1::BN, PromptTile1::BK, 0.9f, 0.65f},
     {PromptTile2<1>::BM, PromptTile2<1>::BN, PromptTile2<1>::BK, 0.7f, 0.65f}, {PromptTile3::BM, PromptTile3::BN, PromptTile3::BK, 1.1f, 1.1f},
     {PromptTile4::BM, PromptTile4::BN, PromptTile4::BK, 1.45f, 1.45f},
     {PromptTile5::BM, PromptTile5::BN, PromptTile5::BK, 0.6f, 0.33f}};
@@ -327,11 +329,13 @@ inline PromptPlan prompt_plan(bool gate_up, int M, int N, int K, int cus) {
   for (int t = 0; t < kPromptTiles; t++) {
     const PromptShape& h = kPromptShapes[t];
     const int bn = gate_up ? h.BN / 2 : h.BN, ksteps = (K + h.BK - 1) / h.BK;
-    if (h.BN == PromptTile5::BN && M > 2 * h.BM) continue;
     const int mblocks = (M + h.BM - 1) / h.BM, nblocks = (N + bn - 1) / bn;
+    if (h.BN == PromptTile5::BN && mblocks > 2) continue;
     for (int want = 1; want <= (gate_up ? 1 : 8); want++) {
       const int steps = (ksteps + want - 1) / want, splits = (ksteps + steps - 1) / steps;
-      const double per_cu = ((long long)mblocks * nblocks * splits + cus - 1) / cus * (double)h.shared;
+      const long long groups = (long long)mblocks * nblocks * splits, rounds = (groups + cus - 1) / cus;
+      if (h.BN == PromptTile5::BN && rounds > 1 && 4 * rounds * cus > 5 * groups) continue;  // see there
+      const double per_cu = rounds * (double)h.shared;
       const double us = steps * (per_cu > h.alone ? per_cu : h.alone) + (splits > 1 ? 2.5 + 8e-6 * splits * M * N / 4 : 0.);
       if (best.splits == 0 || us < best_us) {
         best_us = us;
