@@ -214,7 +214,10 @@ struct DownMmaLaunch16 {
     // slabs of equal width, in whole cache lines: 385 vectors are seven of 56, the last one 49, not six of 64 and one of 1
     a.slab_vecs = ((a.row_vecs + a.nslab - 1) / a.nslab + 7) / 8 * 8;
     const size_t lds = down_mma_lds_bytes(a.chunk, a.nb, kDownMmaDepth);
-    const bool early = a.mask_bytes && !a.flags && !a.idx;
+    // What is fetched early for nothing has to be little: nine rows and more keep most neurons (4096 / 14336 16 rows 72.4 / 70.6 us), small
+    // matrices wait for trips and not for bytes (2304 / 6144 5 rows 90 % 22.2 / 21.8, 3080 / 8191 3 rows 60 % 33.8 / 33.4).  4096 / 11008
+    // gains 50.2 / 49.6 at 4 rows and 50 % but loses 35.8 / 37.6 at 3 rows and 90 %.
+    const bool early = a.mask_bytes && !a.flags && !a.idx && (a.nb > 8 || (size_t)a.I * a.row_vecs * 16 <= (56u << 20));
     auto kern = early ? (zf32 ? down_mma_kernel<DT, true, kDownMmaDepth, true> : down_mma_kernel<DT, false, kDownMmaDepth, true>)
                       : (zf32 ? down_mma_kernel<DT, true, kDownMmaDepth, false> : down_mma_kernel<DT, false, kDownMmaDepth, false>);
     if (hipError_t e = ensure_dynamic_lds((const void*)kern, lds); e != hipSuccess) return e;
@@ -292,9 +295,10 @@ hipError_t launch_attn<CATS_DT>(int head_dim, int bt, AttnArgs a, hipStream_t st
     case 32: kern = attn_decode_kernel<CATS_DT, 32>; break;
   }
   if (!kern) return hipErrorInvalidValue;
-  // the CUs that attention leaves free fetch the next projection's weights, where they are at least a quarter of the chip
+  // the CUs that attention leaves free fetch the next projection's weights, where they are at least three quarters of the chip (half of
+  // it: steps of two layers 4096 / 11008, 4 rows of 32 heads, 228.7 / 231.2 us)
   const int cus = current_device_cus();
-  const int ahead = a.pairs <= cus - cus / 4 ? (cus - a.pairs) / 8 * 8 : 0;
+  const int ahead = a.pairs <= cus / 4 ? (cus - a.pairs) / 8 * 8 : 0;
   a.piece_vecs *= kR * (bt <= 2 ? WavesFor<1>::value : WavesFor<8>::value);  // from vectors of a row to those of a workgroup of proj_kernel
   return launch_kernel(kern, dim3(a.pairs + ahead), dim3(1024), 0, stream, a);
 }

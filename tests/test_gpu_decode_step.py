@@ -89,9 +89,9 @@ def test_attention_step(B, heads, hd, max_len, pos, dtype):
         assert bool(out.isnan().all()) and torch.equal(kd, before)
 
 
-@pytest.mark.parametrize("B,heads,hd,max_len,pos", [(7, 28, 16, 40, 20), (1, 20, 128, 600, 511), (8, 24, 16, 3, 2)])
+@pytest.mark.parametrize("B,heads,hd,max_len,pos", [(5, 13, 16, 40, 20), (1, 20, 128, 600, 511), (8, 8, 16, 3, 2)])
 def test_attention_with_and_without_workgroups_that_fetch_ahead(B, heads, hd, max_len, pos):
-    """196 of 256 CUs attending: none fetch the next weights; 20 and 192: the rest do, also from a number that is no multiple of eight."""
+    """65 of 256 CUs attending: none fetch the next weights; 20 and 64: the rest do, also from a number that is no multiple of eight."""
     test_attention_step(B, heads, hd, max_len, pos, torch.float16)
 
 

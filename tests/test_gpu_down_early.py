@@ -14,7 +14,7 @@ CASES = [
     (3080, 4095, 3, torch.bfloat16),   # seven slabs of 56 vectors, the last one of 49
     (4168, 1500, 5, torch.float16),    # nine slabs of 64, the last one of 9
     (4096, 17000, 16, torch.float16),  # more z values than a thread asks for at once
-    (8192, 33001, 3, torch.float16),   # more flags than wave 0 asks for at once: ranges of 2064
+    (8192, 33001, 3, torch.float16),   # ranges of 2064 neurons, whose rows wait for the flags
 ]
 
 
