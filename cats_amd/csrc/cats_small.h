@@ -85,7 +85,7 @@ __device__ __forceinline__ void small_finish_row(const ReduceArgs& p, int row, f
 #pragma unroll
     for (int e = 0; e < 4; e++) {
       if (p.y32_acc) {
-        p.y32_acc[col + e] += y[e];
+        unsafeAtomicAdd(p.y32_acc + col + e, y[e]);  // as in reduce_partials_kernel
       } else {
         const st o = DT::fromf(p.residual ? DT::rnd(y[e]) + DT::tof(((const st*)p.residual)[col + e]) : y[e]);
         ((st*)p.y_out)[col + e] = o;

@@ -145,9 +145,11 @@ int cats_gate_up(const void* x, const void* wgate, const void* wup, void* out, u
  *   y_out != NULL : (B,H) in dtype.  The workgroups leave fp32 partial sums and a second launch adds them in a fixed
  *                   order: the result is bitwise reproducible from run to run.
  *   y_f32 != NULL : fp32 accumulate into the caller's (B,H), which the caller has zeroed (or which holds what the result
- *                   is to be added to) -- the contract of the reference ops named below.  At 1..2 rows this is ONE launch:
- *                   the streaming kernel adds its sums into y_f32 with fp32 atomics (the order, and so the last bits,
- *                   vary from run to run).
+ *                   is to be added to) -- the contract of the reference ops named below.  Everything is added with fp32
+ *                   atomics, so calls on different streams, each with a workspace of its own, may add into one buffer.
+ *                   At 1..2 rows this is ONE launch, in which every workgroup adds its own sums (the order, and so the
+ *                   last bits, vary from run to run); small layers and more rows total their partial sums in a fixed
+ *                   order first, in a second launch where the layer needs one, and add each column once.
  * flag_out (B,I) optional.  count_out (device int32, optional) receives the number of neurons active in any row of the
  * batch (the number of neurons fetched; where 9..16 rows run as two passes one small kernel counts the union of the
  * flags afterwards).  With y_f32 and count_out at 1..2 rows a second, tiny launch totals the count.

@@ -78,3 +78,31 @@ def test_layer_tail(H, I, B, dtype):
     o = out.double()
     scale = (o.square().mean(1, keepdim=True) + 1e-6).rsqrt()
     assert float((nxt.double() - n2.double() * o * scale).norm()) <= 2.5 * UNIT[dtype] * float((n2.double() * o * scale).norm()) + 1e-12
+
+
+@pytest.mark.parametrize("H,I,B", [(512, 1000, 1), (1024, 2731, 2), (1024, 500, 4), (512, 300, 16)])
+def test_two_streams_add_into_one_buffer(H, I, B):
+    """The fp32-accumulate calls of two streams, a workspace each, add into one buffer without losing any: 1 and 2 rows in one and
+    two launches, and batches."""
+    from cats_amd import capi
+
+    n = 150
+    layers = [layer(H, I, B, torch.float16, seed) for seed in (1, 2)]
+    spaces = [capi.Workspace(B, H, I) for _ in layers]
+    once = []
+    for (x, wg, wu, wd), ws in zip(layers, spaces):
+        v = torch.zeros(B, H, device="cuda")
+        capi.mlp(x, wg, wu, wd, 0.2, ws, y_f32=v)
+        once.append(v.double())
+    out, streams = torch.zeros(B, H, device="cuda"), [torch.cuda.Stream() for _ in layers]
+    torch.cuda.synchronize()
+    for _ in range(n):
+        for (x, wg, wu, wd), ws, s in zip(layers, spaces, streams):
+            with torch.cuda.stream(s):
+                capi.mlp(x, wg, wu, wd, 0.2, ws, y_f32=out)
+    torch.cuda.synchronize()
+    # a call's totals have a fixed order, so each adds the same value every time; 2 n fp32 additions round by half a unit of a running
+    # sum of at most n (|a| + |b|) each.  One addition lost is a whole |a| or |b|, hundreds of times as much.
+    a, b = once
+    bound = 2 * n * 2.0 ** -24 * n * (a.abs() + b.abs())
+    assert bool(((out.double() - n * (a + b)).abs() <= bound + 1e-30).all())
