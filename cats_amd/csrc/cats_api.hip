@@ -11,7 +11,7 @@
 #include "cats_gemv.h"
 #include "cats_launch.h"
 
-// Built-in scratch of cats_mlp_noalloc: the per-workgroup partial sums and active counts of the single-pass kernel.
+// Built-in scratch of cats_mlp_noalloc: the per-workgroup partial sums and active counts of the single-pass kernel and of small layers'.
 // Every GPU the library runs on holds its own copy of this array, at its own address, until the process ends.
 constexpr size_t kScratchPartialBytes = (size_t)256 * 8192 * 4;  // 256 workgroups x (B * H <= 8192) fp32 partial sums
 constexpr size_t kScratchCountBytes = 4096;                      // one int32 count per workgroup
@@ -521,10 +521,10 @@ constexpr size_t kSmallTailBytes = 300000;
 // sums in the same order.
 constexpr size_t kSmallOneLaunchBytes = 131072;
 
-// y32: the caller's fp32 sums, which the call adds to.
+// y32: the caller's fp32 sums, which the call adds to.  partial, counts: instead of those in ws (then NULL), memory without an arrival
+// counter that calls keep at zero, so two launches.
 int do_small(const RowsArgs& a, bool mma, int grid, int stage, const void* wdown_t, void* y_out, const void* residual, float* y32, int32_t* count_out,
-             int dtype, char* ws, const WsLayout& l, hipStream_t s, const NextNorm& next = NextNorm(), float* partial = nullptr, int32_t* counts = nullptr,
-             int32_t* arrive = nullptr) {
+             int dtype, char* ws, const WsLayout& l, hipStream_t s, const NextNorm& next = NextNorm(), float* partial = nullptr, int32_t* counts = nullptr) {
   SmallArgs k;
   memset(&k, 0, sizeof(k));
   k.r = a;
@@ -545,7 +545,8 @@ int do_small(const RowsArgs& a, bool mma, int grid, int stage, const void* wdown
   const size_t row = (size_t)grid * a.K * 4;
   const bool one = a.nb == 1 && row <= kSmallOneLaunchBytes;
   hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-  if (one && stage == 0 && hipStreamIsCapturing(s, &cap) == hipSuccess && cap == hipStreamCaptureStatusNone) k.arrive = arrive ? arrive : (int32_t*)(ws + l.counters + kSmallArriveOffset);
+  if (one && stage == 0 && ws && hipStreamIsCapturing(s, &cap) == hipSuccess && cap == hipStreamCaptureStatusNone)
+    k.arrive = (int32_t*)(ws + l.counters + kSmallArriveOffset);
   hipError_t e = hipSuccess;
   if (stage != 2) e = dtype == CATS_F16 ? launch_small<F16>(mma, grid, k, s) : dtype == CATS_BF16 ? launch_small<BF16>(mma, grid, k, s) : launch_small<F32>(mma, grid, k, s);
   if (e != hipSuccess) return CATS_ERR_LAUNCH;
@@ -1255,16 +1256,20 @@ int cats_mlp_noalloc(const void* x, const void* wgate, const void* wup, const vo
   a.w2 = (const u32x4*)wup;
   a.t = round_through(dtype, threshold);
   bool mma = false;
-  if ((size_t)B * H <= 8192 && small_takes(a, dtype, mma, grid) && !mma && B <= 2) {  // at most kFusedMaxGrid workgroups: the scratch holds them
+  const auto scratch_holds = [&](int workgroups) {
+    return (size_t)workgroups * B * H * 4 <= kScratchPartialBytes && (size_t)workgroups * 4 <= kScratchCountBytes;
+  };
+  // Two launches, never one: calls that overlap on this GPU may spoil each other's sums, but a counter they left off zero would spoil
+  // every call after them.
+  if (B <= 2 && (size_t)B * H <= 8192 && small_takes(a, dtype, mma, grid) && scratch_holds(grid)) {
     void* sp = nullptr;
     if (int e = scratch_address(&sp)) return e;
     return do_small(a, mma, grid, 0, wdown_t, y_out, nullptr, nullptr, nullptr, dtype, nullptr, WsLayout(), (hipStream_t)stream, NextNorm(), (float*)sp,
-                    (int32_t*)((char*)sp + kScratchPartialBytes), (int32_t*)((char*)sp + kScratchPartialBytes + kScratchCountBytes));
+                    (int32_t*)((char*)sp + kScratchPartialBytes));
   }
   const bool ok = fused_eligible(B, H, I, dtype, f, grid, true);  // this entry point is the single-pass kernel or nothing
   // the stated limit (B * H <= 8192) whatever the grid turns out to be, and the actual footprint as a second check
-  if (!ok || (size_t)B * H > 8192 || (size_t)grid * B * H * 4 > kScratchPartialBytes || (size_t)grid * 4 > kScratchCountBytes)
-    return CATS_ERR_SCRATCH;
+  if (!ok || (size_t)B * H > 8192 || !scratch_holds(grid)) return CATS_ERR_SCRATCH;
   void* sp = nullptr;
   st = scratch_address(&sp);
   if (st) return st;

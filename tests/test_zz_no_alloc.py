@@ -72,3 +72,44 @@ def test_mlp_noalloc_in_a_hip_graph():
         g.replay()
         torch.cuda.synchronize()
         assert torch.equal(y, want), f"replay {rep}: max |diff| {float((y.float() - want.float()).abs().max())}"
+
+
+SMALL = [(512, 1024, 1, torch.float16), (256, 100, 1, torch.bfloat16), (512, 8000, 1, torch.float16), (256, 700, 1, torch.float32),
+         (1024, 2000, 2, torch.float16)]
+
+
+def _small_layers():
+    g = torch.Generator(device="cuda").manual_seed(5)
+    rn = lambda *s: torch.randn(*s, generator=g, device="cuda")
+    return [tuple((rn(*s) * f).to(dt) for s, f in (((B, H), 1.0), ((I, H), H ** -0.5), ((I, H), H ** -0.5), ((I, H), 0.1))) for H, I, B, dt in SMALL]
+
+
+def _check_small(layers):
+    from cats_amd import capi
+
+    for rep in range(3):
+        for (H, I, B, dtype), (x, wg, wu, wd) in zip(SMALL, layers):
+            want = capi.mlp(x, wg, wu, wd, 0.2, capi.Workspace(B, H, I))
+            got = capi.mlp_noalloc(x, wg, wu, wd, 0.2, torch.full_like(want, float("nan")))
+            assert torch.equal(got, want), (H, I, B, dtype, rep)
+
+
+def test_noalloc_on_small_layers_whose_grids_differ():
+    """Layers whose whole call with a workspace is one launch, in turn: different numbers of workgroups, the largest 500."""
+    _check_small(_small_layers())
+
+
+def test_noalloc_calls_that_overlapped_leave_nothing_behind():
+    """Overlapping calls may get each other's sums, as the header says; calls after them may not."""
+    from cats_amd import capi
+
+    layers = _small_layers()
+    outs, streams = [torch.empty_like(x) for x, *_ in layers], [torch.cuda.Stream() for _ in range(2)]
+    torch.cuda.synchronize()
+    for rep in range(100):
+        for k, s in enumerate(streams):
+            x, wg, wu, wd = layers[(rep + k) % 3]
+            with torch.cuda.stream(s):
+                capi.mlp_noalloc(x, wg, wu, wd, 0.2, outs[(rep + k) % 3])
+    torch.cuda.synchronize()
+    _check_small(layers)
