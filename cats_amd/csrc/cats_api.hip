@@ -160,10 +160,32 @@ inline size_t align_up(size_t v, size_t a) { return (v + a - 1) / a * a; }
 
 struct WsLayout {
   size_t counters, mask, ubytes, z32, zt, partial, atmp, fin, total;
+  size_t room() const { return mask - partial; }  // bytes of the partial sums
   bool mask_bytes = false;  // not part of the carving: the pass that just ran left the union of the flags in `ubytes`, not `mask`
 };
 
 constexpr int kMaxGroups = 64;  // neuron groups of the sparse down kernel; bounds the partial-sum scratch
+
+// Bytes of partial sums that small layers' kernels may leave at most in a call that small_takes lets through, by how many workgroups there are
+// (crowded: more than one a CU) and whether it is 9 to 16 rows of fp32.
+constexpr int kSmallCuGroups = 256;
+inline bool small_crowded(int groups) { return groups > kSmallCuGroups; }
+inline size_t small_sums_most(bool crowded, bool f32_wide) { return (crowded ? 8500000u : 11000000u) * (size_t)(f32_wide ? 2 : 1); }
+constexpr int kSmallCrowdedVecs = 128;  // of a row, at most
+
+// What of that a layer of (H, I) can come to over all types and batches; 0 if no call of it is a small one.
+size_t small_sum_bytes(int H, int I) {
+  if (I > kSmallMaxNeurons) return 0;
+  const int groups = small_max_groups(I);
+  const size_t all = (size_t)groups * CATS_MAX_BATCH * H * 4;
+  size_t most = 0;
+  for (const int vec : {8, 4}) {
+    if (H / vec > (small_crowded(groups) ? kSmallCrowdedVecs : kSmallMaxVecs)) continue;
+    const size_t cap = small_sums_most(small_crowded(groups), vec == 4);
+    if (most < (all < cap ? all : cap)) most = all < cap ? all : cap;
+  }
+  return most;
+}
 
 // The carving depends on (H, I) only -- every region is sized for kKernelBatch rows -- so calls with
 // different batch sizes can share one workspace.  Nothing in it has to survive from one call to the next.
@@ -172,9 +194,8 @@ WsLayout ws_layout(int H, int I) {
   const int B = kKernelBatch;
   size_t o = 0;
   l.counters = o; o += kCounterBytes;
-  size_t rows = (size_t)kMaxGroups * B;
-  if (I <= kSmallMaxNeurons && H <= kSmallMaxVecs * 8 && rows < (size_t)small_max_groups(I) * CATS_MAX_BATCH) rows = (size_t)small_max_groups(I) * CATS_MAX_BATCH;
-  l.partial = o;  o += align_up(rows * ((size_t)(H + 511) / 512 * 512) * 4, 256);
+  const size_t sums = (size_t)kMaxGroups * B * ((size_t)(H + 511) / 512 * 512) * 4, small = small_sum_bytes(H, I);
+  l.partial = o;  o += align_up(sums > small ? sums : small, 256);
   l.mask = o;     o += align_up((size_t)((I + 63) / 64) * 8, 256);
   l.ubytes = o;   o += align_up((size_t)I + 8, 256);  // the same as a byte per neuron, read eight at a time
   l.z32 = o;      o += align_up((size_t)CATS_MAX_BATCH * I * 4, 256);  // 16 rows: the one-pass gate + up of 9..16 rows fills it whole
@@ -499,18 +520,19 @@ int do_down(const void* z, bool zf32, const void* wdown_t, float* y32, void* y_o
 //   16 rows, fp32     1024 / 2731 36.0, 22.6   1024 / 4096 40.0, 27.1 (16.8 MB; the other way reads the down weight twice)
 // Beyond one workgroup a CU: 512 / 8000 15.0, 9.9 at 1 row and 17.8, 15.0 at 8;  704 / 6000 17.3, 17.1 at 8 (8.4 MB);  1024 / 5000 13.4, 11.4 at 1,
 // 17.8, 19.8 at 8 (10.3 MB);  1200 / 5000 (rows of 150 vectors, one workgroup a CU at a time) 12.0, 13.3 at 1 row and 90 %.
-bool small_takes(RowsArgs& a, int dtype, bool& mma, int& grid) {
+// room: bytes there are for the sums.
+bool small_takes(RowsArgs& a, int dtype, size_t room, bool& mma, int& grid) {
   if (g_tuning.path == 1 || g_tuning.gate_variant != 0 || g_tuning.down_groups > 0 || g_tuning.down_block > 0) return false;
   if (a.nb < 1 || a.nb > CATS_MAX_BATCH || a.N > kSmallMaxNeurons) return false;
   mma = a.nb > (dtype == CATS_F32 ? 4 : 2);  // as takes_mma has it for the gate
   grid = small_layout(a, mma);
   if (grid <= 0 || grid > small_max_groups(a.N)) return false;
   const size_t bytes = (size_t)a.N * a.K * elem_size(dtype), sums = (size_t)grid * a.nb * a.K * 4;
-  const bool crowded = grid > kFusedMaxGrid;  // more than one workgroup a CU: two of them fit where a row is at most 128 vectors
-  if (crowded && a.row_vecs > 128) return false;
+  if (sums > room) return false;
+  const bool crowded = small_crowded(grid);  // two workgroups a CU fit where a row is at most 128 vectors
+  if (crowded && a.row_vecs > kSmallCrowdedVecs) return false;
   if (!mma) return bytes <= (dtype == CATS_F32 && a.nb > 2 ? 17000000u : crowded ? 11000000u : 13600000u);
-  const size_t most = crowded ? 8500000u : 11000000u;
-  return sums <= (dtype == CATS_F32 && a.nb > kKernelBatch ? 2 * most : most);
+  return sums <= small_sums_most(crowded, dtype == CATS_F32 && a.nb > kKernelBatch);
 }
 
 // Sums of a batch row that one workgroup adds up sooner than a launch over all CUs and, for the layer tail, the hand-over in front of its norm
@@ -897,7 +919,7 @@ static int mlp_pass(const void* x, const void* wgate, const void* wup, const voi
   a.flag_out = flag_out;
   a.t = round_through(dtype, threshold);
   bool mma = false;
-  if (small_takes(a, dtype, mma, grid))
+  if (small_takes(a, dtype, l.room(), mma, grid))
     return do_small(a, mma, grid, stage, wdown_t, y_out, nullptr, y_f32, count_out, dtype, (char*)ws, l, (hipStream_t)stream);
   if (fused_eligible(B, H, I, dtype, f, grid)) {
     f.x = (const u32x4*)x;
@@ -947,7 +969,7 @@ static int mlp_wide(const void* x, const void* norm_weight, float eps, const voi
   a.norm_eps = eps;
   bool mma = false;
   int grid = 0;
-  if (small_takes(a, dtype, mma, grid))
+  if (small_takes(a, dtype, l.room(), mma, grid))
     return do_small(a, mma, grid, 0, wdown_t, y_out, residual ? x : nullptr, y_f32, count_out, dtype, (char*)ws, l, (hipStream_t)stream, next);
   a.z32_out = (float*)((char*)ws + l.z32);
   a.mask_out = (uint8_t*)ws + l.mask;
@@ -1040,7 +1062,7 @@ static int mlp_norm_residual_pass(const void* h, const void* norm_weight, float 
   FusedArgs f;
   int grid = 0;
   bool mma = false;
-  if (small_takes(a, dtype, mma, grid))
+  if (small_takes(a, dtype, l.room(), mma, grid))
     return do_small(a, mma, grid, 0, wdown_t, out, h, nullptr, nullptr, dtype, (char*)ws, l, (hipStream_t)stream, next);
   if (fused_eligible(B, H, I, dtype, f, grid)) {
     f.x = (const u32x4*)h;
@@ -1256,12 +1278,9 @@ int cats_mlp_noalloc(const void* x, const void* wgate, const void* wup, const vo
   a.w2 = (const u32x4*)wup;
   a.t = round_through(dtype, threshold);
   bool mma = false;
-  const auto scratch_holds = [&](int workgroups) {
-    return (size_t)workgroups * B * H * 4 <= kScratchPartialBytes && (size_t)workgroups * 4 <= kScratchCountBytes;
-  };
   // Two launches, never one: calls that overlap on this GPU may spoil each other's sums, but a counter they left off zero would spoil
   // every call after them.
-  if (B <= 2 && (size_t)B * H <= 8192 && small_takes(a, dtype, mma, grid) && scratch_holds(grid)) {
+  if (B <= 2 && (size_t)B * H <= 8192 && small_takes(a, dtype, kScratchPartialBytes, mma, grid) && (size_t)grid * 4 <= kScratchCountBytes) {
     void* sp = nullptr;
     if (int e = scratch_address(&sp)) return e;
     return do_small(a, mma, grid, 0, wdown_t, y_out, nullptr, nullptr, nullptr, dtype, nullptr, WsLayout(), (hipStream_t)stream, NextNorm(), (float*)sp,
@@ -1269,7 +1288,8 @@ int cats_mlp_noalloc(const void* x, const void* wgate, const void* wup, const vo
   }
   const bool ok = fused_eligible(B, H, I, dtype, f, grid, true);  // this entry point is the single-pass kernel or nothing
   // the stated limit (B * H <= 8192) whatever the grid turns out to be, and the actual footprint as a second check
-  if (!ok || (size_t)B * H > 8192 || !scratch_holds(grid)) return CATS_ERR_SCRATCH;
+  if (!ok || (size_t)B * H > 8192 || (size_t)grid * B * H * 4 > kScratchPartialBytes || (size_t)grid * 4 > kScratchCountBytes)
+    return CATS_ERR_SCRATCH;
   void* sp = nullptr;
   st = scratch_address(&sp);
   if (st) return st;

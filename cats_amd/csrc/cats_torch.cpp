@@ -65,8 +65,8 @@ struct Workspace {
 // for a shape; that first call must not happen under stream capture (the allocation would come out of the graph's
 // private pool and the fill would be recorded into the graph), so it is refused there: run one call eagerly on the
 // capturing stream first.  A captured graph keeps using the workspace of the stream it was captured on, so eager
-// calls on that stream must not overlap its replays.  Entries live until the process ends (a few MB per layer shape
-// and stream; torch hands out at most 32 pooled side streams per device) and the map is never destroyed: at exit the
+// calls on that stream must not overlap its replays.  Entries live until the process ends (up to some 20 MB per layer shape
+// and stream, mostly partial sums; torch hands out at most 32 pooled side streams per device) and the map is never destroyed: at exit the
 // HIP runtime may be gone before static destructors run.
 Workspace& workspace(const at::Tensor& like, int B, int H, int I, hipStream_t stream) {
   static std::mutex mu;

@@ -74,9 +74,9 @@ const char* cats_status_string(int status);
  * aligned), runs cats_workspace_init() once (it zero-fills with a kernel), and then passes the same buffer to
  * every call; no call relies on what an earlier call left in it (the counter words at its head are all zero
  * between calls: a call that uses them puts them back).  The size and the carving depend on (H, I)
- * only (B is checked; every region holds the 8 rows of one pass over the weights, and a call with 9..16 rows
- * reuses them pass by pass), so one workspace serves every batch size of one layer shape; for another (H, I)
- * use another workspace or initialise again.  One workspace serves one stream at a time. */
+ * only (B is checked; every region holds what any call of up to CATS_MAX_BATCH rows leaves in it), so one
+ * workspace serves every batch size of one layer shape; for another (H, I) use another workspace or initialise
+ * again.  One workspace serves one stream at a time. */
 size_t cats_workspace_bytes(int B, int H, int I);
 int cats_workspace_init(void* ws, size_t ws_bytes, void* stream);
 

@@ -68,6 +68,29 @@ def test_workspace_size_depends_on_layer_shape_only():
     assert L.cats_workspace_bytes(0, 4096, 11008) == 0
 
 
+def test_workspace_holds_what_small_layers_calls_can_leave_and_no_more():
+    """Partial sums: 64 groups of 8 rows, or what a layer's small calls leave -- at most 22 MB, and nothing where no call is one."""
+    from cats_amd import capi
+
+    L = capi.lib()
+
+    def sums(H, I):  # of a workspace with the other regions taken off
+        up = lambda n: (n + 255) // 256 * 256
+        other = 4096 + 144 * 128 + 256 + 4096 * 4 + up((I + 63) // 64 * 8) + up(I + 8) + up(64 * I) + 2 * up(32 * I) + up(64 * H)
+        return L.cats_workspace_bytes(1, H, I) - other
+
+    def streaming(H):
+        return 512 * ((H + 511) // 512 * 512) * 4
+
+    for H, I in [(2048, 8192), (2048, 5461), (2048, 4097), (1032, 4100), (4096, 11008), (2056, 1000), (512, 8193)]:
+        assert sums(H, I) == streaming(H), (H, I)
+    for H, I in [(512, 1024), (1024, 2731), (2048, 4096), (1024, 4096), (512, 8192), (1024, 8192), (8, 1), (256, 8000)]:
+        rows = 16 * ((I + 127) // 128 * 8)
+        assert streaming(H) <= sums(H, I) <= max(streaming(H), min(rows * H * 4 + 255, 22000000 + 255)), (H, I)
+    assert sums(512, 8192) >= 16 * 512 * 512 * 4  # sixteen rows of fp32: 512 workgroups
+    assert sums(1024, 4096) >= 16 * 256 * 1024 * 4
+
+
 def test_flash_gemv_package_surface():
     import flash_gemv
 
