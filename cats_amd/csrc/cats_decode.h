@@ -179,13 +179,21 @@ struct AttnArgs {
 // round the eight XCDs in both launches).  They start about 2 us late, when the cache slots have been asked for: at once they hold
 // those up (attention 10.1 us for 6.6), and as much is fetched as comes in meanwhile.  Step of four layers as above: 327.9 us without
 // (output projection 8.1 us); 24 MiB 320.6, started at once 325 to 335; 32 MiB 322 to 325 (output projection 4.7); 16 MiB 322.1.
+// Nothing is fetched where the cache slots and the weights together exceed the L2s (eight of 4 MiB): attention then needs the memory
+// itself and its slots take the weights' place.  Steps of two layers 4096 / 11008, one row, without, with, with this limit, in us: 256
+// slots 160.6, 156.5, 156.3;  480 160.9, 158.7, 159.1;  1000 168.2, 171.3, 168.4;  2000 186, 194, 187;  two rows at 480 198.9, 200.9,
+// 199.2; one row of 16 heads and 2048 / 5461 (8 MiB of weights) at 2000 slots 111.3, 109.8, 109.7.
 constexpr unsigned kAttnAheadVecs = (24u << 20) / 16;
+constexpr long long kL2Vecs = (32 << 20) / 16;
 constexpr int kAttnAheadSleeps = 5;  // of 1024 clocks each
+template <int LPS>
 __device__ __forceinline__ void attn_fetch_next(const AttnArgs& p) {
   constexpr int kLoads = 10;  // in flight per thread
   const unsigned xcd = blockIdx.x & 7, groups = (gridDim.x - p.pairs) / 8;  // workgroups on this XCD
   const unsigned piece = p.piece_vecs, first = (blockIdx.x - p.pairs) / 8 * 1024 + threadIdx.x;
+  const long long pos = *p.pos;
   for (int i = 0; i < kAttnAheadSleeps; i++) __builtin_amdgcn_s_sleep(16);
+  if (pos < 0 || pos >= (long long)p.max_len || 2 * LPS * (long long)p.pairs * (pos + 1) + p.next_vecs > kL2Vecs) return;
   const unsigned pieces = (p.next_vecs + piece - 1) / piece, mine = ((pieces + 7 - xcd) / 8) * piece;  // vectors for this XCD
   for (unsigned t = first; t < mine; t += kLoads * groups * 1024) {
     u32x4 w[kLoads];
@@ -203,9 +211,12 @@ __device__ __forceinline__ void attn_fetch_next(const AttnArgs& p) {
 // each, so a wave holds 64 / LPS slots side by side and the workgroup 16 * 64 / LPS; every lane group runs its own online
 // softmax over the slots it meets, U slots a turn with the loads of K and V of all of them in flight together (256 slots of 128
 // 16-bit elements are one turn), and the groups' results are merged at the end, in a fixed order.  What bounds it is dependent
-// memory trips, not the bytes (131 KiB a head at 256 slots): so the first turn's slots are asked for with the position, whatever it is
-// (slots behind it hold anything and are masked), and the next turn's before this one's are used.
-template <class DT, int LPS>
+// memory trips, not the bytes (131 KiB a head at 256 slots): so (AHEAD) the first turn's slots are asked for with the position, whatever
+// it is (slots behind it hold anything and are masked), and the next turn's before this one's are used.  Where the heads fill more than
+// a quarter of the chip the slots behind the position cost more than the trip (steps of two layers 4096 / 11008, 4 rows of 32 heads at 60 slots
+// 230.7 us with, 228.6 without).  The last turn asks for nothing: its registers would be waited for (one row at 480 slots 159.1 us, so
+// 156.7; 4 rows of 16 heads, 2048 / 5461, 132.8, 130.4).
+template <class DT, int LPS, bool AHEAD>
 __global__ __launch_bounds__(1024) void attn_decode_kernel(AttnArgs p) {
   typedef typename DT::st st;
   constexpr int VEC = DT::VEC, HD = LPS * VEC, G = kWave / LPS, WAVES = 16, S = WAVES * G, U = 4;
@@ -215,7 +226,7 @@ __global__ __launch_bounds__(1024) void attn_decode_kernel(AttnArgs p) {
   const int wave = threadIdx.x >> 6;
   const int sub = lane % LPS;
   const int slot0 = wave * G + lane / LPS;
-  if ((int)blockIdx.x >= p.pairs) return attn_fetch_next(p);
+  if ((int)blockIdx.x >= p.pairs) return attn_fetch_next<LPS>(p);
   const u32x4* kb = p.k + (size_t)blockIdx.x * p.max_len * LPS + sub;
   const u32x4* vb = p.v + (size_t)blockIdx.x * p.max_len * LPS + sub;
   const long long pos = *p.pos;
@@ -234,13 +245,12 @@ __global__ __launch_bounds__(1024) void attn_decode_kernel(AttnArgs p) {
 #pragma unroll
     for (int u = 0; u < U; u++) v[u] = vb[(size_t)min(s0 + u * S + slot0, last) * LPS];
   };
-  fetch(0, p.max_len - 1, kv, vv);
+  if constexpr (AHEAD) fetch(0, p.max_len - 1, kv, vv);
   const int n = pos >= 0 && pos < (long long)p.max_len ? (int)pos + 1 : 0;
   float m = -INFINITY, l = 0.f, acc[VEC];
 #pragma unroll
   for (int e = 0; e < VEC; e++) acc[e] = 0.f;
-  for (int s0 = 0; s0 < n; s0 += S * U) {
-    fetch(s0 + S * U, n - 1, kn, vn);  // past the last turn: the last slot again, which the caches hold
+  auto turn = [&](int s0) {
     float sc[U], mu = m;
 #pragma unroll
     for (int u = 0; u < U; u++) {
@@ -266,10 +276,23 @@ __global__ __launch_bounds__(1024) void attn_decode_kernel(AttnArgs p) {
       for (int e = 0; e < VEC; e++) acc[e] = in ? fmaf(pr, elem(vv[u], e), acc[e]) : acc[e];
     }
     m = mu;
+  };
+  if constexpr (AHEAD) {
+    int s0 = 0;
+    for (; s0 + S * U < n; s0 += S * U) {
+      fetch(s0 + S * U, n - 1, kn, vn);
+      turn(s0);
 #pragma unroll
-    for (int u = 0; u < U; u++) {
-      kv[u] = kn[u];
-      vv[u] = vn[u];
+      for (int u = 0; u < U; u++) {
+        kv[u] = kn[u];
+        vv[u] = vn[u];
+      }
+    }
+    if (n > 0) turn(s0);
+  } else {
+    for (int s0 = 0; s0 < n; s0 += S * U) {
+      fetch(s0, n - 1, kv, vv);
+      turn(s0);
     }
   }
   // the wave's groups, then the waves

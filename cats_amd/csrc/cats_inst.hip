@@ -284,21 +284,26 @@ hipError_t launch_proj<CATS_DT>(int mode, int bt, const ProjArgs& a, hipStream_t
   return hipErrorInvalidValue;
 }
 
+typedef void (*AttnKernel)(AttnArgs);
+template <int LPS>
+static AttnKernel attn_for(bool ahead) { return ahead ? attn_decode_kernel<CATS_DT, LPS, true> : attn_decode_kernel<CATS_DT, LPS, false>; }
+
 template <>
 hipError_t launch_attn<CATS_DT>(int head_dim, int bt, AttnArgs a, hipStream_t stream) {
-  void (*kern)(AttnArgs) = nullptr;
+  AttnKernel kern = nullptr;
+  const int cus = current_device_cus();
+  const bool spare = a.pairs <= cus / 4;
   switch (head_dim / CATS_DT::VEC) {  // lanes per cache slot
-    case 2: kern = attn_decode_kernel<CATS_DT, 2>; break;
-    case 4: kern = attn_decode_kernel<CATS_DT, 4>; break;
-    case 8: kern = attn_decode_kernel<CATS_DT, 8>; break;
-    case 16: kern = attn_decode_kernel<CATS_DT, 16>; break;
-    case 32: kern = attn_decode_kernel<CATS_DT, 32>; break;
+    case 2: kern = attn_for<2>(spare); break;
+    case 4: kern = attn_for<4>(spare); break;
+    case 8: kern = attn_for<8>(spare); break;
+    case 16: kern = attn_for<16>(spare); break;
+    case 32: kern = attn_for<32>(spare); break;
   }
   if (!kern) return hipErrorInvalidValue;
   // the CUs that attention leaves free fetch the next projection's weights, where they are at least three quarters of the chip (half of
   // it: steps of two layers 4096 / 11008, 4 rows of 32 heads, 228.7 / 231.2 us)
-  const int cus = current_device_cus();
-  const int ahead = a.pairs <= cus / 4 ? (cus - a.pairs) / 8 * 8 : 0;
+  const int ahead = spare ? (cus - a.pairs) / 8 * 8 : 0;
   a.piece_vecs *= kR * (bt <= 2 ? WavesFor<1>::value : WavesFor<8>::value);  // from vectors of a row to those of a workgroup of proj_kernel
   return launch_kernel(kern, dim3(a.pairs + ahead), dim3(1024), 0, stream, a);
 }

@@ -89,9 +89,11 @@ def test_attention_step(B, heads, hd, max_len, pos, dtype):
         assert bool(out.isnan().all()) and torch.equal(kd, before)
 
 
-@pytest.mark.parametrize("B,heads,hd,max_len,pos", [(5, 13, 16, 40, 20), (1, 20, 128, 600, 511), (8, 8, 16, 3, 2)])
+@pytest.mark.parametrize("B,heads,hd,max_len,pos", [(5, 13, 16, 40, 20), (5, 13, 128, 600, 513), (1, 20, 128, 600, 255), (1, 20, 128, 600, 256),
+                                                    (1, 20, 128, 600, 511), (8, 8, 16, 3, 2), (8, 8, 128, 1100, 900), (8, 8, 128, 1100, 1023)])
 def test_attention_with_and_without_workgroups_that_fetch_ahead(B, heads, hd, max_len, pos):
-    """65 of 256 CUs attending: none fetch the next weights; 20 and 64: the rest do, also from a number that is no multiple of eight."""
+    """65 of 256 CUs attending: none fetch the next weights or the slots of a turn ahead; 20 and 64: the rest do, also from a number that is
+    no multiple of eight, up to 960 slots of 64 heads of 128; turns of 256 slots, one to five of them, ending on and behind a turn."""
     test_attention_step(B, heads, hd, max_len, pos, torch.float16)
 
 
