@@ -63,8 +63,15 @@ def _nothing_watches():
 
 
 def _sub(module, name):
-    """module.name, a submodule, without nn.Module's search for it."""
-    return module._modules.get(name) or getattr(module, name)
+    """module.name, a submodule, without nn.Module's search for it unless a class puts something (a property) in front of it."""
+    found = None if hasattr(type(module), name) else module._modules.get(name)
+    return getattr(module, name) if found is None else found
+
+
+def _param(linear, name):
+    """linear.name of a bare nn.Linear, without nn.Module's search for it unless it is no parameter but an attribute in one's place."""
+    params = linear._parameters
+    return params[name] if name in params else getattr(linear, name)
 
 
 def _plain(t, dtype, device):
@@ -280,11 +287,11 @@ class CatsMLP(nn.Module):
                     raise RuntimeError("CatsMLP: sp_method 2/3 need wdown_t (call prepare_decode() once after loading weights)")
                 if self.sp_method == 2:
                     g = _sub(self, "gate_proj")
-                    if (_bare(g, nn.Linear) and g._parameters.get("bias", self) is None and _bare(_sub(self, "act_fn"), nn.SiLU) and _nothing_watches()
-                            and _plain(g._parameters.get("weight"), x.dtype, x.device)):
+                    if (_bare(g, nn.Linear) and _param(g, "bias") is None and _bare(_sub(self, "act_fn"), nn.SiLU) and _nothing_watches()
+                            and _plain(_param(g, "weight"), x.dtype, x.device)):
                         # a plain gate projection: the same call with the gate in it (torch's product alone takes 21 us of the 51
                         # of a 4096 / 14336 layer at one row, all of it 38)
-                        return flash_gemv.cats_mlp(x, g._parameters["weight"], _sub(self, "up_proj").weight, self.wdown_t, t)
+                        return flash_gemv.cats_mlp(x, _param(g, "weight"), _sub(self, "up_proj").weight, self.wdown_t, t)
                     return flash_gemv.gemv_gemv_triton(x, self.act_fn(self.gate_proj(x)), self.up_proj.weight, self.wdown_t, t)
                 if self.is_stats:
                     # decode-time sparsity bookkeeping (the reference's agg_sparsity, ugly_utils.py:929-937, for the

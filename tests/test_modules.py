@@ -196,3 +196,30 @@ def _greedy_cpu(model, prompt, n):
         tok = logits[:, -1].argmax(-1, keepdim=True)
         out.append(int(tok))
     return torch.tensor(out), logits
+
+
+def test_sp_method_2_sees_what_the_modules_attributes_give(monkeypatch):
+    """The one-call route of sp_method 2: a property of a subclass in front of a submodule, and a weight that is an attribute in the
+    parameter's place, are what the module's own attributes say."""
+    import flash_gemv
+
+    class Doubled(cm.CatsMLP):
+        @property
+        def up_proj(self):
+            lin = torch.nn.Linear(64, 96, bias=False)
+            lin.weight = torch.nn.Parameter(2 * self._modules["up_proj"].weight.detach())
+            return lin
+
+    calls = []
+    monkeypatch.setattr(flash_gemv, "cats_mlp", lambda x, wg, wu, wdt, t: calls.append((wg, wu)))
+    x = torch.randn(1, 1, 64)
+    with torch.no_grad():
+        m = Doubled(64, 96, dtype=torch.float32).prepare_decode(2)
+        m(x)
+        assert torch.equal(calls[-1][1], 2 * m._modules["up_proj"].weight)
+        m = cm.CatsMLP(64, 96, dtype=torch.float32).prepare_decode(2)
+        weight = m.gate_proj.weight.detach().clone()
+        del m.gate_proj.weight
+        m.gate_proj.weight = weight
+        m(x)
+        assert len(calls) == 2 and calls[-1][0] is weight and calls[-1][1] is m.up_proj.weight
