@@ -520,6 +520,24 @@ int do_down(const void* z, bool zf32, const void* wdown_t, float* y32, void* y_o
 //   16 rows, fp32     1024 / 2731 36.0, 22.6   1024 / 4096 40.0, 27.1 (16.8 MB; the other way reads the down weight twice)
 // Beyond one workgroup a CU: 512 / 8000 15.0, 9.9 at 1 row and 17.8, 15.0 at 8;  704 / 6000 17.3, 17.1 at 8 (8.4 MB);  1024 / 5000 13.4, 11.4 at 1,
 // 17.8, 19.8 at 8 (10.3 MB);  1200 / 5000 (rows of 150 vectors, one workgroup a CU at a time) 12.0, 13.3 at 1 row and 90 %.
+// What is read for nothing grows with the sparsity, so from three rows on the lines are drawn with 30, 60 and 90 % of it measured: by the sums, and by
+// a matrix and the sums together (MB of both below).  Those and these in us at 30 / 60 / 90 %:
+//   a workgroup a CU       3 rows 2048 / 3700 18.9, 17.6 / 18.7, 17.9 / 18.2, 17.3 (5.7, 20.8)   2048 / 4096 19.9, 19.2 / 19.6, 19.5 / 19.0, 19.4 (6.3, 23.1)
+//                          5 rows 1792 / 4000 18.8, 17.2 / 18.7, 17.2 / 18.1, 17.1 (9.0, 23.3)   2048 / 3700 20.0, 19.9 / - / 19.5, 19.7 (9.5, 24.7)
+//                          8 rows 1536 / 3500 17.9, 17.1 / 17.9, 17.1 / 17.5, 17.1 (10.8, 21.5)
+//     rows of more than 224 vectors are what the others are best at, four slabs of 64:
+//                          5 rows 2048 / 3300 18.6, 18.5 / 18.5, 18.5 / 18.1, 18.5 (8.4, 21.9)   2040 / 3500 20.3, 20.2 / 20.2, 20.1 / 19.6, 20.2 (8.9, 23.2)
+//                          8 rows 2048 / 2600 18.6, 18.8 / 18.7, 18.8 / 18.2, 18.7 (10.7, 21.3)
+//   two a CU               4 rows 1024 / 5000 16.5, 15.9 / 16.3, 15.9 / 15.9, 15.8 (5.1, 15.4)   6 rows 1024 / 4300 16.7, 16.6 / 16.6, 16.7 / 16.2, 16.7 (6.6, 15.4)
+//                          6 rows 840 / 5000 17.1, 17.5 / 17.0, 17.5 / 16.7, 17.5 (6.5, 14.9)   704 / 6000 16.5, 15.7 / 16.4, 15.8 / 15.9, 15.7 (6.3, 14.8)
+//     short rows, slabs that the others do not fill:   8 rows 512 / 8000 17.3, 14.9 / 17.2, 14.9 / 16.8, 14.9 (8.2, 16.4)   520 / 8000 18.1, 16.9 / 18.0,
+//                          16.9 / 17.4, 16.9 (8.3, 16.6)
+//   more than one a CU, but no place for two: more than 64 registers from three steps a wave on, at nine rows and more from two
+//                          3 rows 1000 / 4200 17.3, 16.7 / 17.1, 16.7 / 16.7, 16.7 (3.2, 11.6)   6 rows 17.9, 19.2 / - / 17.4, 19.2 (6.3, 14.7)
+//                          12 rows 520 / 5000 19.8, 19.1 / 19.8, 19.1 / 17.8, 19.1 (7.8, 13.0)   11 rows 640 / 4500 19.2, 19.3 / - / 17.6, 19.3 (7.9, 13.7)
+//   fp32                   5 rows 1024 / 4096 23.2, 20.6 / 22.6, 20.9 / 19.6, 20.9 (5.2, 22.0)   8 rows 23.9, 22.7 / - / 20.6, 23.0 (8.4, 25.2)
+//                          8 rows 512 / 5000 20.5, 19.4 / - / 18.6, 19.4 (5.1, 15.4)   512 / 8000 24.3, 22.9 / - / 20.8, 22.9 (8.2, 24.6)
+// At one and two rows the gain at low sparsity is the larger: 2048 / 3300 at one row 12.6, 11.8 at 50 % and 11.5, 11.8 at 90 %.
 // room: bytes there are for the sums.
 bool small_takes(RowsArgs& a, int dtype, size_t room, bool& mma, int& grid) {
   if (g_tuning.path == 1 || g_tuning.gate_variant != 0 || g_tuning.down_groups > 0 || g_tuning.down_block > 0) return false;
@@ -532,7 +550,12 @@ bool small_takes(RowsArgs& a, int dtype, size_t room, bool& mma, int& grid) {
   const bool crowded = small_crowded(grid);  // two workgroups a CU fit where a row is at most 128 vectors
   if (crowded && a.row_vecs > kSmallCrowdedVecs) return false;
   if (!mma) return bytes <= (dtype == CATS_F32 && a.nb > 2 ? 17000000u : crowded ? 11000000u : 13600000u);
-  return sums <= small_sums_most(crowded, dtype == CATS_F32 && a.nb > kKernelBatch);
+  const bool f32_wide = dtype == CATS_F32 && a.nb > kKernelBatch;  // the other way reads the down weight twice
+  // no place for two 16-bit workgroups a CU with more registers than these steps take; fp32 as measured
+  const bool two_fit = dtype == CATS_F32 || rows_mma_split(a).steps <= (a.nb > kKernelBatch ? 1 : 2);
+  const size_t most = !crowded ? 23500000u : two_fit ? 17000000u : 13500000u;
+  if (dtype != CATS_F32 && sums > (crowded ? (a.row_vecs > 80 ? 6400000u : 8500000u) : a.row_vecs > 224 ? 8500000u : 11000000u)) return false;
+  return sums <= small_sums_most(crowded, f32_wide) && bytes + sums <= most * (f32_wide ? 2 : 1);
 }
 
 // Sums of a batch row that one workgroup adds up sooner than a launch over all CUs and, for the layer tail, the hand-over in front of its norm

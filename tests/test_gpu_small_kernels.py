@@ -33,7 +33,9 @@ def tolerance(want, dtype):
 
 
 CASES = [(8, 1, 1), (8, 17, 3), (256, 15, 2), (512, 16, 9), (520, 1000, 4), (1024, 129, 16), (1032, 777, 5), (1536, 272, 1), (1544, 2049, 3),
-         (2040, 300, 8), (2048, 512, 2), (2048, 31, 12), (512, 4097, 1), (512, 4113, 3), (1024, 5000, 2)]
+         (2040, 300, 8), (2048, 512, 2), (2048, 31, 12), (512, 4097, 1), (512, 4113, 3), (1024, 5000, 2),
+         # both sides of the lines to the other kernels, a workgroup a CU, two, and more than one without place for two
+         (2048, 4096, 3), (2048, 4096, 4), (1024, 5000, 4), (1024, 5000, 6), (1000, 4200, 3), (1000, 4200, 4), (520, 4500, 12), (640, 4500, 11)]
 
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
