@@ -214,10 +214,19 @@ struct DownMmaLaunch16 {
     // slabs of equal width, in whole cache lines: 385 vectors are seven of 56, the last one 49, not six of 64 and one of 1
     a.slab_vecs = ((a.row_vecs + a.nslab - 1) / a.nslab + 7) / 8 * 8;
     const size_t lds = down_mma_lds_bytes(a.chunk, a.nb, kDownMmaDepth);
-    // What is fetched early for nothing has to be little: nine rows and more keep most neurons (4096 / 14336 16 rows 72.4 / 70.6 us), small
-    // matrices wait for trips and not for bytes (2304 / 6144 5 rows 90 % 22.2 / 21.8, 3080 / 8191 3 rows 60 % 33.8 / 33.4).  4096 / 11008
-    // gains 50.2 / 49.6 at 4 rows and 50 % but loses 35.8 / 37.6 at 3 rows and 90 %.
-    const bool early = a.mask_bytes && !a.flags && !a.idx && (a.nb > 8 || (size_t)a.I * a.row_vecs * 16 <= (56u << 20));
+    // Early rows save the trip in which the memory idles, 0.6 to 1.2 us, and cost 64 rows of every range, up to 16.8 MB in all whatever the matrix,
+    // times their dead share.  Without, with them in us at 30 / 60 / 90 % sparsity:
+    //   3 rows   3080 / 8191 36.0, 35.1 / 33.3, 33.0 / 27.4, 27.9 (75 % 29.6, 30.8)   2304 / 6144 24.1, 23.5 / 23.1, 22.8 / 20.9, 21.1
+    //            2048 / 5461 21.8, 21.1 / 20.8, 20.6 / 19.1, 19.6   4096 / 11008 51.1, 50.5 / - / 35.6, 37.5
+    //   8 rows   4096 / 11008 54.6, 53.6 / 52.0, 51.2 / 42.1, 42.2
+    //            3080 / 8191 38.4, 37.5 / 37.4, 36.8 / 30.8, 32.1   2560 / 6912 31.2, 30.3 / 31.0, 30.3 / 26.4, 26.6   1024 / 10000 23.1, 22.5 / 23.3, 22.6 / 20.2, 20.0
+    //   16 rows  4096 / 14336 71.5, 70.0 / 69.6, 68.2 / 58.6, 58.4   4096 / 11008 60.7, 59.4 / 59.7, 58.6 / 51.3, 50.7   2560 / 6912 34.3, 33.4 / 34.6, 33.8 / 30.4, 31.1
+    // So they pay up to 60 to 75 %, and beyond cost up to what they gave; which it will be the host cannot see.  They are left out where the loss is the
+    // larger: up to eight rows of large matrices (for the few rows among them), and ranges that are half early and
+    // start a multiple of 512 KiB apart, whose early rows all lie on the same part of the memory (2048 / 8192 at 3 rows 26.7, 26.8 / 25.3, 25.8 / 21.9,
+    // 23.1, at 8 28.6, 28.9 / 28.3, 28.6 / 24.8, 25.7; 2048 / 7168 at 3 rows 24.9, 24.1 / 23.6, 23.3, 1920 / 8192 25.3, 24.4 / 24.0, 23.6).
+    const bool alike = a.chunk <= 2 * kDownMmaEarly && ((size_t)a.chunk * a.row_vecs * 16) % (512 << 10) == 0;
+    const bool early = a.mask_bytes && !a.flags && !a.idx && (a.nb > 8 || ((size_t)a.I * a.row_vecs * 16 <= (56u << 20) && !alike));
     auto kern = early ? (zf32 ? down_mma_kernel<DT, true, kDownMmaDepth, true> : down_mma_kernel<DT, false, kDownMmaDepth, true>)
                       : (zf32 ? down_mma_kernel<DT, true, kDownMmaDepth, false> : down_mma_kernel<DT, false, kDownMmaDepth, false>);
     if (hipError_t e = ensure_dynamic_lds((const void*)kern, lds); e != hipSuccess) return e;

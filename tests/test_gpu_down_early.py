@@ -15,6 +15,8 @@ CASES = [
     (4168, 1500, 5, torch.float16),    # nine slabs of 64, the last one of 9
     (4096, 17000, 16, torch.float16),  # more z values than a thread asks for at once
     (8192, 33001, 3, torch.float16),   # ranges of 2064 neurons, whose rows wait for the flags
+    (2048, 8100, 3, torch.float16),    # ranges of 128, 512 KiB apart, whose rows wait too; the next one's do not
+    (2048, 7169, 3, torch.float16),
 ]
 
 
