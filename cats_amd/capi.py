@@ -24,7 +24,7 @@ SYMBOLS = (
     "cats_gate_compact", "cats_read_count", "cats_up_flag", "cats_down_flag", "cats_gate_up", "cats_mlp",
     "cats_mlp_rowmajor_down", "cats_mlp_norm_residual", "cats_up_down", "cats_set_tuning", "cats_mlp_stage", "cats_mlp_noalloc", "cats_up_index", "cats_down_index",
     "cats_probe_read", "cats_mlp_norm_residual_norm", "cats_linear", "cats_attention_step", "cats_mlp_gate_cols", "cats_silu_mask_mul",
-    "cats_prompt_scratch_bytes", "cats_prompt_mlp",
+    "cats_prompt_scratch_bytes", "cats_prompt_mlp", "cats_prompt_plan",
 )
 
 
@@ -53,6 +53,8 @@ def lib() -> ctypes.CDLL:
         L.cats_workspace_init.argtypes = [vp, sz, vp]; L.cats_workspace_init.restype = i32
         L.cats_prompt_scratch_bytes.argtypes = [i32, i32, i32]; L.cats_prompt_scratch_bytes.restype = sz
         L.cats_prompt_mlp.argtypes = [vp, vp, vp, vp, vp, i32, i32, i32, i32, f32, vp, sz, vp]; L.cats_prompt_mlp.restype = i32
+        if hasattr(L, "cats_prompt_plan"):
+            L.cats_prompt_plan.argtypes = [i32, i32, i32, i32, vp]; L.cats_prompt_plan.restype = i32
         L.cats_gate_flag.argtypes = [vp, vp, vp, vp, i32, i32, i32, i32, f32, vp]; L.cats_gate_flag.restype = i32
         L.cats_gate_compact.argtypes = [vp, vp, vp, vp, vp, i32, i32, i32, f32, vp, sz, vp]; L.cats_gate_compact.restype = i32
         L.cats_read_count.argtypes = [vp, vp]; L.cats_read_count.restype = i32
@@ -206,6 +208,13 @@ def mlp_noalloc(x, wgate, wup, wdown_t, threshold, y):
     check(lib().cats_mlp_noalloc(_p(x), _p(wgate), _p(wup), _p(wdown_t), _p(y), B, H, I, DTYPE_CODE[x.dtype], float(threshold),
                                  _stream(x)), "cats_mlp_noalloc")
     return y
+
+
+def prompt_plan(product, M, H, I):
+    """(tile, token blocks, row blocks, steps, ranges of K, steps ahead) of cats_prompt_mlp's product 1 (gate and up) or 2 (down)."""
+    plan = (ctypes.c_int * 6)()
+    check(lib().cats_prompt_plan(product, M, H, I, plan), "cats_prompt_plan")
+    return tuple(plan)
 
 
 def up_down(x, a, wup, wdown_t, threshold, ws: Workspace):

@@ -1473,6 +1473,7 @@ int cats_silu_mask_mul(const void* gate, const void* up, void* z, size_t n, int 
 }
 
 // The plan of the second product: what it needs in the scratch decides its size.
+static PromptPlan prompt_up_plan(int M, int H, int I) { return prompt_plan(true, M, prompt_pitch(I), H, current_device_cus()); }
 static PromptPlan prompt_down_plan(int M, int H, int I) { return prompt_plan(false, M, prompt_sum_pitch(H), I, current_device_cus()); }
 static size_t prompt_z_bytes(int M, int I) { return ((size_t)M * prompt_pitch(I) * 2 + 255) / 256 * 256; }
 
@@ -1483,6 +1484,15 @@ static size_t prompt_bytes(const PromptPlan& down, int M, int H, int I) {
 size_t cats_prompt_scratch_bytes(int M, int H, int I) {
   if (M < 1 || M > CATS_PROMPT_MAX_TOKENS || H < 8 || I < 8 || H > (1 << 28) || I > (1 << 28)) return 0;
   return prompt_bytes(prompt_down_plan(M, H, I), M, H, I);
+}
+
+int cats_prompt_plan(int product, int M, int H, int I, int* plan) {
+  if (!plan) return CATS_ERR_NULL;
+  if ((product != 1 && product != 2) || M < 1 || M > CATS_PROMPT_MAX_TOKENS || H < 8 || I < 8 || H > (1 << 28) || I > (1 << 28)) return CATS_ERR_SHAPE;
+  const PromptPlan p = product == 1 ? prompt_up_plan(M, H, I) : prompt_down_plan(M, H, I);
+  const int v[6] = {p.tile, p.mblocks, p.nblocks, p.steps, p.splits, prompt_steps_ahead(p, current_device_cus())};
+  memcpy(plan, v, sizeof(v));
+  return CATS_OK;
 }
 
 int cats_prompt_mlp(const void* x, const void* wgate, const void* wup, const void* wdown, void* y_out, int M, int H, int I, int dtype,
@@ -1510,7 +1520,7 @@ int cats_prompt_mlp(const void* x, const void* wgate, const void* wup, const voi
   a.M = M; a.N = I; a.K = H;
   a.ldx = H; a.ldo = pitch;
   a.t = round_through(dtype, threshold);
-  const PromptPlan first = prompt_plan(true, M, pitch, H, current_device_cus());
+  const PromptPlan first = prompt_up_plan(M, H, I);
   hipError_t e = dtype == CATS_F16 ? launch_prompt<F16>(true, first, a, s) : launch_prompt<BF16>(true, first, a, s);
   if (e != hipSuccess) return CATS_ERR_LAUNCH;
   float* partial = (float*)((char*)scratch + prompt_z_bytes(M, I));

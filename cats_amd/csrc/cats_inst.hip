@@ -334,13 +334,12 @@ struct PromptLaunch {
     return launch_kernel(kern, dim3(grid), dim3(T::THREADS), T::LDS, stream, a);
   }
   template <bool GATE_UP>
-  static hipError_t run(int t, const PromptArgs& a, hipStream_t stream) {
-    // one workgroup a CU and steps enough: see PromptTile0
-    const bool alone = a.steps >= 10 && (long long)a.mblocks * a.nblocks * a.splits <= current_device_cus();
-    switch (t) {
-      case 0: return alone ? tile<PromptTile0<2>, GATE_UP>(a, stream) : tile<PromptTile0<1>, GATE_UP>(a, stream);
+  static hipError_t run(const PromptPlan& plan, const PromptArgs& a, hipStream_t stream) {
+    const bool two = prompt_steps_ahead(plan, current_device_cus()) == 2;
+    switch (plan.tile) {
+      case 0: return two ? tile<PromptTile0<2>, GATE_UP>(a, stream) : tile<PromptTile0<1>, GATE_UP>(a, stream);
       case 1: return tile<PromptTile1, GATE_UP>(a, stream);
-      case 2: return alone ? tile<PromptTile2<2>, GATE_UP>(a, stream) : tile<PromptTile2<1>, GATE_UP>(a, stream);
+      case 2: return two ? tile<PromptTile2<2>, GATE_UP>(a, stream) : tile<PromptTile2<1>, GATE_UP>(a, stream);
       case 3: return tile<PromptTile3, GATE_UP>(a, stream);
       case 4: return tile<PromptTile4, GATE_UP>(a, stream);
       case 5: return tile<PromptTile5, GATE_UP>(a, stream);
@@ -355,7 +354,7 @@ struct PromptLaunch {
 template <>
 struct PromptLaunch<F32> {
   template <bool GATE_UP>
-  static hipError_t run(int, const PromptArgs&, hipStream_t) { return hipErrorInvalidValue; }
+  static hipError_t run(const PromptPlan&, const PromptArgs&, hipStream_t) { return hipErrorInvalidValue; }
   static hipError_t sum(const PromptSumArgs&, hipStream_t) { return hipErrorInvalidValue; }
 };
 template <>
@@ -364,7 +363,7 @@ hipError_t launch_prompt<CATS_DT>(bool gate_up, const PromptPlan& plan, PromptAr
   a.nblocks = plan.nblocks;
   a.steps = plan.steps;
   a.splits = plan.splits;
-  return gate_up ? PromptLaunch<CATS_DT>::run<true>(plan.tile, a, stream) : PromptLaunch<CATS_DT>::run<false>(plan.tile, a, stream);
+  return gate_up ? PromptLaunch<CATS_DT>::run<true>(plan, a, stream) : PromptLaunch<CATS_DT>::run<false>(plan, a, stream);
 }
 template <>
 hipError_t launch_prompt_sum<CATS_DT>(const PromptSumArgs& a, hipStream_t stream) {

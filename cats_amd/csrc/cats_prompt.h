@@ -307,8 +307,8 @@ typedef PromptTile<4, 2, 4, 4, 64, 1> PromptTile3;
 typedef PromptTile<4, 2, 4, 6, 64, 1> PromptTile4;
 // Half of tile 0: two or three workgroups a CU where tile 0 has one on most and two on some, so the weights come in evenly (4096 / 11008
 // 2 tokens: gate and up 3.4 us less, down 1.6; at 32 tokens, where it reads x twice as often, 0.5 and 0.7).  Up to two blocks of tokens
-// (at 128 tokens of 512 / 1365 13.9 us without it, 14.5 with), and where at most a fifth of the last round's places stay empty: 342
-// workgroups of 2048 / 5461 at 30 tokens, weights in cache, 23.7 us against 22.8.  Whole call at 2, 16 and 32 tokens, before / now: 4096 / 11008 64.2 / 59.6,
+// (at 128 tokens of 512 / 1365 13.9 us without it, 14.5 with), and where it takes more than one round of the CUs only if at most a fifth
+// of the places of all its rounds stay empty: 342 workgroups of 2048 / 5461 at 30 tokens, weights in cache, 23.7 us against 22.8.  Whole call at 2, 16 and 32 tokens, before / now: 4096 / 11008 64.2 / 59.6,
 // 65.0 / 60.9, 66.5 / 63.7; 1024 / 2731 18.5 / 16.5, 19.0 / 17.0, 19.3 / 17.3.
 typedef PromptTile<2, 1, 1, 2, 128, 1> PromptTile5;
 constexpr int kPromptTiles = 6;
@@ -344,6 +344,10 @@ inline PromptPlan prompt_plan(bool gate_up, int M, int N, int K, int cus) {
     }
   }
   return best;
+}
+// Steps of loads in registers: two in the second instances of tiles 0 and 2, see there.
+inline int prompt_steps_ahead(const PromptPlan& p, int cus) {
+  return (p.tile == 0 || p.tile == 2) && p.steps >= 10 && (long long)p.mblocks * p.nblocks * p.splits <= cus ? 2 : 1;
 }
 inline int prompt_pitch(int I) { return (I + 7) / 8 * 8; }   // of z
 inline int prompt_sum_pitch(int H) { return (H + 3) / 4 * 4; }  // of partial sums

@@ -258,6 +258,11 @@ size_t cats_prompt_scratch_bytes(int M, int H, int I);
 int cats_prompt_mlp(const void* x, const void* wgate, const void* wup, const void* wdown, void* y_out, int M, int H, int I, int dtype,
                     float threshold, void* scratch, size_t scratch_bytes, void* stream);
 
+/* What cats_prompt_mlp launches for its first product (1, gate and up) or its second (2, down) on the current device, for tests and
+ * profiles: plan[0..5] = tile (of kPromptShapes), blocks of tokens, blocks of weight rows, steps a workgroup, ranges of K, steps of loads
+ * ahead in registers.  Not in the reference. */
+int cats_prompt_plan(int product, int M, int H, int I, int* plan);
+
 /* One launch of cats_mlp(y_out mode) alone, for per-kernel timing and profiling: stage 1 = the streaming launch (gate, up
  * and, for 1..2 rows, down into per-workgroup partial sums), stage 2 = the launch that finishes y from what stage 1 left in
  * the workspace.  Calling stage 1 then stage 2 with the same arguments is cats_mlp.  Not in the reference. */

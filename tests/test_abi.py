@@ -53,6 +53,7 @@ def test_argument_validation_needs_no_gpu():
     assert L.cats_mlp(p, p, p, p, None, None, None, None, 1, 64, 96, 0, 0.1, p, big, None) == 5  # neither
     assert L.cats_mlp_rowmajor_down(p, p, p, p, p, 1, 64, 100, 0, 0.1, p, big, None) == 3        # wdown rows 200 B
     assert L.cats_down_flag(p, p, p, None, None, 1, 64, 96, 0, p, big, None) == 5
+    assert L.cats_prompt_plan(1, 4, 64, 96, None) == 5 and L.cats_prompt_plan(3, 4, 64, 96, p) == 2
     for code in range(8):
         assert capi.status_string(code) != "unknown status"
     assert capi.status_string(99) == "unknown status"

@@ -45,8 +45,28 @@ def test_prompt_mlp(M, H, I, dtype):
 
 
 @pytest.mark.parametrize("M,H,I", [(2, 640, 515), (32, 641, 1000), (9, 773, 515), (48, 905, 900), (64, 1283, 515), (100, 384, 700), (128, 393, 1041), (200, 520, 2731)])
-def test_two_steps_ahead(M, H, I):
-    """Launches of at most one workgroup a CU, five steps of K and more, odd and even numbers of them, K ending inside and on a step."""
+def test_small_tiles(M, H, I):
+    """Half tiles of 32 tokens and 32 rows, one or two blocks of tokens, and launches of at most one workgroup a CU with too few steps
+    for two ahead; odd and even numbers of steps, K ending inside and on a step."""
+    test_prompt_mlp(M, H, I, torch.float16)
+
+
+AHEAD = [  # product, tokens, H, I, its tile, its steps
+    (1, 128, 1279, 130, 0, 10), (1, 70, 1536, 130, 0, 12), (1, 128, 1409, 130, 0, 12), (1, 100, 1408, 130, 0, 11), (1, 70, 1283, 131, 0, 11),
+    (1, 200, 640, 4099, 2, 10), (1, 160, 630, 5461, 2, 10), (1, 200, 832, 4099, 2, 13), (1, 200, 772, 4099, 2, 13), (1, 192, 2048, 5461, 2, 32),
+    (2, 256, 1400, 1300, 0, 11), (2, 256, 1408, 1408, 0, 11), (2, 130, 3072, 3001, 2, 10), (2, 130, 3072, 3200, 2, 10), (2, 200, 772, 5461, 2, 11),
+    (2, 200, 770, 5632, 2, 11),
+]
+
+
+@pytest.mark.parametrize("product,M,H,I,tile,steps", AHEAD)
+def test_two_steps_ahead(product, M, H, I, tile, steps):
+    """Launches of at most one workgroup a CU and ten steps and more, whose loads are two steps ahead: both tiles that have this, in either
+    product, odd and even numbers of steps, K ending inside and on a step, the second product also in ranges of K."""
+    from cats_amd import capi
+
+    plan = capi.prompt_plan(product, M, H, I)
+    assert (plan[0], plan[3], plan[5]) == (tile, steps, 2), plan
     test_prompt_mlp(M, H, I, torch.float16)
 
 
