@@ -1,5 +1,5 @@
-"""The single-pass kernel on layers with fewer neurons than the chip has row waves: shares of 4 to 24 neurons a workgroup, the last one
-short, some row waves without a neuron, some with a second one."""
+"""Layers with fewer neurons than the chip has row waves, by the kernels of small layers, which take them, and by the single-pass kernel:
+there shares of 4 to 24 neurons a workgroup, the last one short, some row waves without a neuron, some with a second one."""
 import pytest
 import torch
 import torch.nn.functional as F
@@ -7,9 +7,18 @@ import torch.nn.functional as F
 pytestmark = pytest.mark.gpu
 
 
+@pytest.fixture(params=["small", "single pass"])
+def kernels(request):
+    from cats_amd import capi
+
+    capi.set_tuning(gate_variant=0 if request.param == "small" else -1)  # any other than 0 keeps whole calls off the small layers' kernels
+    yield request.param
+    capi.set_tuning()
+
+
 @pytest.mark.parametrize("B", [1, 2])
 @pytest.mark.parametrize("I", [1, 3, 4, 5, 7, 13, 1023, 1025, 1535, 1536, 1537, 2049, 3071, 3073, 6145])
-def test_small_layers(I, B):
+def test_small_layers(I, B, kernels):
     import flash_gemv
 
     H, t = 132, 0.2
