@@ -186,4 +186,11 @@ __device__ __forceinline__ int wave_scan_inclusive(int v, int lane) {
   return v;
 }
 
+// A barrier for LDS only: __syncthreads() would also wait for the weight loads in flight.
+__device__ __forceinline__ void lds_barrier() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
 }  // namespace cats

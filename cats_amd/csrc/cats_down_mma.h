@@ -152,13 +152,6 @@ struct DownMmaStage {
   }
 };
 
-// A barrier for LDS only: __syncthreads() would also wait for the weight loads in flight.
-__device__ __forceinline__ void down_mma_lds_barrier() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-  __builtin_amdgcn_s_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-}
-
 template <class DT, bool ZF32, int DEPTH, bool EARLY>
 __global__ __launch_bounds__(kDownMmaThreads) void down_mma_kernel(DownArgs p) {
   typedef typename DT::st st;
@@ -224,7 +217,7 @@ __global__ __launch_bounds__(kDownMmaThreads) void down_mma_kernel(DownArgs p) {
     const int end = (down_mma_steps_per_wave(n0, DEPTH) + DEPTH) * kDownMmaListWaves * kDownMmaStep;
     for (int i = n0 + lane; i < end; i += kWave) s_list[i] = -1;
   }
-  if constexpr (EARLY) down_mma_lds_barrier();
+  if constexpr (EARLY) lds_barrier();
   else __syncthreads();
   const int n = s_n;
   const int spw = down_mma_steps_per_wave(n, DEPTH);            // steps every list wave runs
@@ -257,7 +250,7 @@ __global__ __launch_bounds__(kDownMmaThreads) void down_mma_kernel(DownArgs p) {
     u32x2 o = {zz[0] | (zz[1] << 16), zz[2] | (zz[3] << 16)};
     s_zop[i] = o;
   }
-  down_mma_lds_barrier();
+  lds_barrier();
   for (int t0 = 0; t0 < spw; t0 += DEPTH) {
 #pragma unroll
     for (int d = 0; d < DEPTH; d++) {

@@ -36,13 +36,6 @@ struct SmallArgs {
   ReduceArgs fin;
 };
 
-// A barrier for LDS only: __syncthreads() would also wait for the weight loads in flight.
-__device__ __forceinline__ void small_lds_barrier() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-  __builtin_amdgcn_s_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-}
-
 // ---- the partial sums of small layers -------------------------------------------------------------------------------------------
 
 // Threads side by side over a row of H columns, four each; the 1024 / quads groups of threads take a range of the partials each.
@@ -194,7 +187,7 @@ __global__ __launch_bounds__(kSmallThreads) void small_rows_kernel(SmallArgs a) 
 #pragma unroll
   for (int e = 0; e < 4; e++) xv[e] = x_in ? xv[e] : 0u;
   if (tid < B * NCH * kWave) xs[tid] = xv;
-  small_lds_barrier();
+  lds_barrier();
   if (p.norm_w) {
     __shared__ float s_scale[B];
     if (wave < B) {
@@ -203,9 +196,9 @@ __global__ __launch_bounds__(kSmallThreads) void small_rows_kernel(SmallArgs a) 
       ss = wave_sum(ss);
       if (lane == 0) s_scale[wave] = rsqrtf(ss / (float)p.K + p.norm_eps);
     }
-    small_lds_barrier();
+    lds_barrier();
     if (x_in) xs[tid] = vec_norm_apply<DT>(xv, s_scale[xb], nw);
-    small_lds_barrier();
+    lds_barrier();
   }
 
   {
@@ -234,7 +227,7 @@ __global__ __launch_bounds__(kSmallThreads) void small_rows_kernel(SmallArgs a) 
       s_any[wave] = any ? 1 : 0;
     }
   }
-  small_lds_barrier();
+  lds_barrier();
   if (wave == 0) {
     const uint64_t live = __ballot(lane < kSmallRows && s_any[lane & (kSmallRows - 1)] != 0);
     if (lane == 0) __hip_atomic_store(&a.counts[blockIdx.x], (int)__popcll(live), __ATOMIC_RELAXED, ONE ? __HIP_MEMORY_SCOPE_AGENT : __HIP_MEMORY_SCOPE_WORKGROUP);
@@ -349,7 +342,7 @@ __global__ __launch_bounds__(kSmallThreads) void small_mma_kernel(SmallArgs a) {
       for (int e = 0; e < 4; e++) xv[g][k][e] = in ? xv[g][k][e] : 0u;
       if (i < xgroup) xs[g * xgroup + i] = xv[g][k];
     }
-  small_lds_barrier();
+  lds_barrier();
   if (p.norm_w) {  // the squares of a batch row in rows_mma_kernel's order
     __shared__ float s_scale[NG * 8];
     if (wave < NG * 8) {
@@ -358,7 +351,7 @@ __global__ __launch_bounds__(kSmallThreads) void small_mma_kernel(SmallArgs a) {
       ss = wave_sum(ss);
       if (lane == 0) s_scale[wave] = rsqrtf(ss / (float)p.K + p.norm_eps);
     }
-    small_lds_barrier();
+    lds_barrier();
 #pragma unroll
     for (int g = 0; g < NG; g++)
 #pragma unroll
@@ -366,7 +359,7 @@ __global__ __launch_bounds__(kSmallThreads) void small_mma_kernel(SmallArgs a) {
         const int i = tid + k * kSmallThreads, b = g * 8 + (i & 7), v = x_vector(i);
         if (b < p.nb && (unsigned)v < (unsigned)p.row_vecs) xs[g * xgroup + i] = vec_norm_apply<DT>(xv[g][k], s_scale[b], nw[k]);
       }
-    small_lds_barrier();
+    lds_barrier();
   }
 
   // ---- gate and up sums ----
@@ -378,7 +371,7 @@ __global__ __launch_bounds__(kSmallThreads) void small_mma_kernel(SmallArgs a) {
     rows.multiply(w[t], 0, acc);
     mma_store_partials<DT, NG>(acc, part + (t * 2 + kind) * NG * kMmaPartGroup, lane, kw);
   }
-  small_lds_barrier();
+  lds_barrier();
   if (wave < T * NG) {  // one wave a tile and group of eight batch rows, one thread per (row rj of the tile, batch row rb)
     const int t = wave / NG, g = wave % NG, rj = lane >> 3, rb = lane & 7, j = t * kMmaTileRows + rj, b = g * 8 + rb;
     const float* sums = part + t * 2 * NG * kMmaPartGroup;
@@ -396,7 +389,7 @@ __global__ __launch_bounds__(kSmallThreads) void small_mma_kernel(SmallArgs a) {
     for (int i = 0; i < 8; i++) bits |= ((bal >> (8 * i)) & 0xffull) ? (1u << i) : 0u;
     if (lane == 0) s_bits[wave] = bits;
   }
-  small_lds_barrier();
+  lds_barrier();
   uint32_t bits = 0u;  // of the sixteen neurons
 #pragma unroll
   for (int i = 0; i < T * NG; i++) bits |= s_bits[i] << (i / NG * 8);
