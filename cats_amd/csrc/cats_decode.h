@@ -8,9 +8,10 @@
 // x may be given before its RMS norm (norm_w), which is then applied while x is staged.  Everything between the weight
 // matrices stays in fp32 and is rounded once where it is stored.  All of it is bound by the weight stream: one wave owns two
 // rows of a matrix, whose loads are all in flight at once, as in rows_kernel.
-// One step of four layers 4096 / 11008, 32 heads, 32000 words, 256 tokens in the cache, fp16, one row: 321 us, of which the MLP
+// One step of four layers 4096 / 11008, 32 heads, 32000 words, 256 tokens in the cache, fp16, one row: 323 us, of which the MLP
 // kernels take 150; with torch's operations in place of these kernels (about 25 launches a layer) it was 761.  Kernel trace: q, k, v
-// 18.9 us with the norm (5.3 TB/s), attention 6.6, output projection 8.4, output head 44 (5.9 TB/s).
+// 19.1 us with the norm (5.3 TB/s), attention 8.0 and the output projection, whose weights it has had fetched, 5.3 (6.6 and 8.1
+// without that), output head 44 (5.9 TB/s).
 #pragma once
 #include "cats_rows.h"
 
@@ -177,8 +178,8 @@ struct AttnArgs {
 // The projection that follows depends on this launch, and attention leaves most CUs and the memory idle.  So the workgroups behind the
 // attending ones read its weights into the caches: the pieces that an XCD's workgroups will ask for on this XCD (workgroups go
 // round the eight XCDs in both launches).  They start about 2 us late, when the cache slots have been asked for: at once they hold
-// those up (attention 10.1 us for 6.6), and as much is fetched as comes in meanwhile.  Step of four layers as above: 327.9 us without
-// (output projection 8.1 us); 24 MiB 320.6, started at once 325 to 335; 32 MiB 322 to 325 (output projection 4.7); 16 MiB 322.1.
+// those up (attention 10.1 us for 6.6), and as much is fetched as comes in meanwhile.  Step of four layers as above, both timed in turn:
+// 327.0 us without, 324.7 with.  Beside each other in one run: 24 MiB 320.6, 32 MiB 322 to 325, 16 MiB 322.1; started at once 325 to 335.
 // Nothing is fetched where the cache slots and the weights together exceed the L2s (eight of 4 MiB): attention then needs the memory
 // itself and its slots take the weights' place.  Steps of two layers 4096 / 11008, one row, without, with, with this limit, in us: 256
 // slots 160.6, 156.5, 156.3;  480 160.9, 158.7, 159.1;  1000 168.2, 171.3, 168.4;  2000 186, 194, 187;  two rows at 480 198.9, 200.9,

@@ -69,7 +69,7 @@ inline size_t down_mma_lds_bytes(int chunk, int nb, int depth) {
 
 // The first 64 neurons of a range, one step of each list wave, are asked for before the flags are there (EARLY: the flags are a byte per
 // neuron, as the whole-MLP calls leave them).  They come to rest behind the mask and z in the same memory trip, in which
-// the memory would otherwise idle, and the union of three rows and more keeps most of them; dead ones are list entries -1.
+// the memory would otherwise idle; dead ones are list entries -1, read for nothing.  Where that pays stands at the launch.
 constexpr int kDownMmaEarly = kDownMmaListWaves * kDownMmaStep;
 constexpr int kDownMmaMaskLoads = 4;  // passes of 512 neurons whose flags wave 0 has in flight together
 constexpr int kDownMmaZLoads = 8;     // z values per thread in flight together

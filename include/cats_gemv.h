@@ -141,9 +141,12 @@ int cats_gate_up(const void* x, const void* wgate, const void* wup, void* out, u
                  int B, int H, int I, int dtype, float threshold, void* stream);
 
 /* Whole CATS MLP with neuron-major down weights.  1..2 rows: one streaming kernel in which every workgroup takes its
- * neurons through gate, up and down; more rows: gate+up kernel, then sparse down kernel.
+ * neurons through gate, up and down; more rows: gate+up kernel, then sparse down kernel.  Small layers (up to about 13
+ * MB a matrix, 23 MB with the partial sums of a batch): one kernel at any number of rows, which reads all rows of all
+ * matrices.
  *   y_out != NULL : (B,H) in dtype.  The workgroups leave fp32 partial sums and a second launch adds them in a fixed
- *                   order: the result is bitwise reproducible from run to run.
+ *                   order: the result is bitwise reproducible from run to run.  (The smallest layers at one row, outside
+ *                   a stream capture: the last workgroup adds them, in the same order, and there is no second launch.)
  *   y_f32 != NULL : fp32 accumulate into the caller's (B,H), which the caller has zeroed (or which holds what the result
  *                   is to be added to) -- the contract of the reference ops named below.  Everything is added with fp32
  *                   atomics, so calls on different streams, each with a workspace of its own, may add into one buffer.
@@ -264,8 +267,8 @@ int cats_prompt_mlp(const void* x, const void* wgate, const void* wup, const voi
 int cats_prompt_plan(int product, int M, int H, int I, int* plan);
 
 /* One launch of cats_mlp(y_out mode) alone, for per-kernel timing and profiling: stage 1 = the streaming launch (gate, up
- * and, for 1..2 rows, down into per-workgroup partial sums), stage 2 = the launch that finishes y from what stage 1 left in
- * the workspace.  Calling stage 1 then stage 2 with the same arguments is cats_mlp.  Not in the reference. */
+ * and, for 1..2 rows and small layers, down into per-workgroup partial sums), stage 2 = what finishes y from what stage 1
+ * left in the workspace (never one launch with stage 1).  Calling stage 1 then stage 2 with the same arguments is cats_mlp.  Not in the reference. */
 int cats_mlp_stage(int stage, const void* x, const void* wgate, const void* wup, const void* wdown_t, void* y_out,
                    int B, int H, int I, int dtype, float threshold, void* ws, size_t ws_bytes, void* stream);
 
@@ -280,8 +283,8 @@ int cats_probe_read(const void* src, size_t bytes, uint32_t* sink, void* stream)
  * resident workgroups per CU (N < 0 keeps 3..16 rows off the matrix-core kernels, gate / up and down); down_groups sets the
  * neuron groups of the sparse down kernels, down_block the workgroup size of the wave-per-row-pair one -- and keeps 3..16 rows
  * on that kernel, off the matrix-core one; path 1 keeps the whole-MLP entry points on the separate gate+up
- * and sparse-down kernels for every batch size (by default 1..2 rows take the single-pass kernel).  Every setting computes
- * the same function.  Process-global and not synchronised: set it before other threads call in.  Not in the reference. */
+ * and sparse-down kernels for every batch size (by default 1..2 rows take the single-pass kernel).  Any value but 0 (path:
+ * 1) keeps whole-MLP calls off the kernels of small layers.  Every setting computes the same function.  Process-global and not synchronised: set it before other threads call in.  Not in the reference. */
 int cats_set_tuning(int gate_variant, int down_groups, int down_block, int path);
 
 #ifdef __cplusplus
