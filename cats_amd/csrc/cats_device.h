@@ -171,6 +171,14 @@ __device__ __forceinline__ float wave_sum(float v) {
   return s;
 }
 
+// Sum over the eight lanes that agree with this one modulo eight, in every lane.
+__device__ __forceinline__ float lanes_sum_mod8(float v) {
+  v = dpp_add<0x128>(v);  // row_ror:8
+  v += __shfl_xor(v, 16, kWave);
+  v += __shfl_xor(v, 32, kWave);
+  return v;
+}
+
 // Number of set bits of a wave ballot below this lane (v_mbcnt_lo/hi).
 __device__ __forceinline__ int ballot_rank(uint64_t ballot) {
   return (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(ballot >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)ballot, 0u));

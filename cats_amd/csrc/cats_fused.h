@@ -41,6 +41,7 @@ static_assert(kFusedWaves == 16 || kFusedWaves == 8, "sixteen waves, or eight fo
 constexpr int fused_down_waves(int batch_template) { return (batch_template == 1 ? 4 : 8) * kFusedWaves / 16; }
 constexpr int kFusedThreads = kFusedWaves * kWave;
 constexpr int kFusedCB = 8;             // 64-lane chunks (of 16 bytes per lane) per block of row loads
+constexpr int kFusedMaxChunks = 128;    // of all staged rows: 128 KiB of x
 constexpr int kFusedMaxKV = 4;          // a down wave covers KV * 64 vectors of a row: rows of up to 4 * DW * 64 vectors
 // Experiment switch, off in the product build: -DCATS_FUSED_POOL=1 compiles the neuron pool described at the kernel
 // (dynamic balancing between the workgroups of a group).  Measured slower than fixed shares on the MI355X, kept so the
@@ -312,7 +313,7 @@ __global__ __launch_bounds__(kFusedThreads) void mlp_fused_kernel(FusedArgs p) {
   __shared__ int s_nfinal;     // slots in use; an upper bound while row waves are still taking tickets
   __shared__ int s_exited;     // row waves that have left
   __shared__ int s_exhausted;  // some row wave has found the group's pool empty
-  __shared__ float s_scale[B];
+  __shared__ __attribute__((aligned(16))) float s_sq[kFusedMaxChunks];  // squares of the staged rows, by chunk
 
   const int tid = threadIdx.x;
   const int lane = tid & (kWave - 1);
@@ -359,7 +360,7 @@ __global__ __launch_bounds__(kFusedThreads) void mlp_fused_kernel(FusedArgs p) {
   // counted in issue order, x goes out first, then (row waves) the first gate block, and only x is waited for before
   // the LDS writes and the barrier -- the weight loads stay in flight across both.
   auto stage = [&](auto&& issue_first) {
-    u32x4 xpre[kXPre];
+    u32x4 xpre[kXPre], nwpre[kXPre];
 #pragma unroll
     for (int k = 0; k < kXPre; k++) {
       const int i = tid + k * kFusedThreads;
@@ -367,17 +368,33 @@ __global__ __launch_bounds__(kFusedThreads) void mlp_fused_kernel(FusedArgs p) {
       xpre[k] = zero4();
       if (i < B * nchv && b < p.nb && v < p.row_vecs) xpre[k] = p.x[(size_t)b * p.row_vecs + v];
     }
+    if (p.norm_w) {  // with x: behind the first gate rows they would come in with these
+#pragma unroll
+      for (int k = 0; k < kXPre; k++) {
+        const int i = tid + k * kFusedThreads;
+        const int b = B == 1 ? 0 : i / nchv, v = i - b * nchv;
+        nwpre[k] = p.norm_w[min(v, vlast)];
+      }
+    }
     issue_first();
+    // The squares of a batch row: by chunk of 64 vectors (a wave's vectors are of one), then over the chunks in their order.
+    auto put = [&](int i, u32x4 val) {
+      xs[i] = val;
+      if (p.norm_w) {
+        const float sq = wave_sum(vec_sumsq<DT>(val, 0.f));
+        if (lane == 0) s_sq[i >> 6] = sq;
+      }
+    };
 #pragma unroll
     for (int k = 0; k < kXPre; k++) {
       const int i = tid + k * kFusedThreads;
-      if (i < B * nchv) xs[i] = xpre[k];
+      if (i < B * nchv) put(i, xpre[k]);
     }
     for (int i = tid + kXPre * kFusedThreads; i < B * nchv; i += kFusedThreads) {
       const int b = i / nchv, v = i - b * nchv;
       u32x4 val = zero4();
       if (b < p.nb && v < p.row_vecs) val = p.x[(size_t)b * p.row_vecs + v];
-      xs[i] = val;
+      put(i, val);
     }
     // given activations: the down waves decide every slot (announced or dead) while they stage the activations.
     // Tickets start at 2 * RW: the slots between a short share and that point are never taken.
@@ -394,17 +411,23 @@ __global__ __launch_bounds__(kFusedThreads) void mlp_fused_kernel(FusedArgs p) {
     }
     __syncthreads();
     if (p.norm_w) {
-      // RMS norm of each batch row, in place in LDS: one wave adds a row's squares (fixed order), everyone rescales.
-      for (int b = wave; b < B; b += kFusedWaves) {
+      auto scale_of = [&](int b) {
         float ss = 0.f;
-        for (int v = lane; v < p.row_vecs; v += kWave) ss = vec_sumsq<DT>(xs[b * nchv + v], ss);
-        ss = wave_sum(ss);
-        if (lane == 0) s_scale[b] = rsqrtf(ss / (float)p.H + p.norm_eps);
-      }
-      __syncthreads();
-      for (int i = tid; i < B * nchv; i += kFusedThreads) {
+        for (int c = 0; c < nchp; c += 4) {
+          const float4 q = *(const float4*)&s_sq[b * nchp + c];
+          ss += (q.x + q.y) + (q.z + q.w);
+        }
+        return rsqrtf(ss / (float)p.H + p.norm_eps);
+      };
+#pragma unroll
+      for (int k = 0; k < kXPre; k++) {
+        const int i = tid + k * kFusedThreads;
         const int b = B == 1 ? 0 : i / nchv, v = i - b * nchv;
-        if (b < p.nb && v < p.row_vecs) xs[i] = vec_norm_apply<DT>(xs[i], s_scale[b], p.norm_w[v]);
+        if (i < B * nchv && b < p.nb && v < p.row_vecs) xs[i] = vec_norm_apply<DT>(xpre[k], scale_of(b), nwpre[k]);
+      }
+      for (int i = tid + kXPre * kFusedThreads; i < B * nchv; i += kFusedThreads) {
+        const int b = i / nchv, v = i - b * nchv;
+        if (b < p.nb && v < p.row_vecs) xs[i] = vec_norm_apply<DT>(xs[i], scale_of(b), p.norm_w[v]);
       }
       __syncthreads();
     }

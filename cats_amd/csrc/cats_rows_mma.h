@@ -254,21 +254,58 @@ struct MmaX {
         v[gb][k] = p.x[in(p, gb, i) ? o : 0u];
       }
   }
+  // What padding slots and batch rows past nb have fetched becomes zero.
+  __device__ __forceinline__ void mask(const RowsArgs& p) {
+#pragma unroll
+    for (int gb = 0; gb < NG; gb++)
+#pragma unroll
+      for (int k = 0; k < NV; k++) {
+        const bool ok = in(p, gb, front * kWave + tid + k * kMmaThreads);
+#pragma unroll
+        for (int e = 0; e < 4; e++) v[gb][k][e] = ok ? v[gb][k][e] : 0u;
+      }
+  }
   // xgroup: slots of one group's operand; the last one is padding where fewer than NV * 512 are needed
-  __device__ __forceinline__ void store(const RowsArgs& p, u32x4* xs, int xgroup) const {
+  __device__ __forceinline__ void store(u32x4* xs, int xgroup) const {
 #pragma unroll
     for (int gb = 0; gb < NG; gb++) {
       if (front && tid < kWave) xs[gb * xgroup + tid] = zero4();
 #pragma unroll
-      for (int k = 0; k < NV; k++) {
-        const int i = front * kWave + tid + k * kMmaThreads;
-        u32x4 o;
-        const bool ok = in(p, gb, i);
-#pragma unroll
-        for (int e = 0; e < 4; e++) o[e] = ok ? v[gb][k][e] : 0u;
-        xs[gb * xgroup + min(i, xgroup - 1)] = o;
-      }
+      for (int k = 0; k < NV; k++) xs[gb * xgroup + min(front * kWave + tid + k * kMmaThreads, xgroup - 1)] = v[gb][k];
       for (int i = front * kWave + tid + NV * kMmaThreads; i < xgroup; i += kMmaThreads) xs[gb * xgroup + i] = zero4();
+    }
+  }
+  // The RMS norm of the masked rows, in registers: slots of one thread, and of the eight lanes that agree modulo eight, are of one batch row.
+  // The squares are added by thread, then over those lanes, then over the waves in their order.  s_sq: 64 floats of LDS a group.
+  // The weights have been asked for with x: behind the first tile they would come in with it.
+  __device__ __forceinline__ void fetch_norm(const RowsArgs& p, u32x4 (&nw)[NV]) const {
+#pragma unroll
+    for (int k = 0; k < NV; k++) {
+      const int q = vector(front * kWave + tid + k * kMmaThreads);
+      nw[k] = p.norm_w[(unsigned)q < (unsigned)p.row_vecs ? q : 0];
+    }
+  }
+  template <class DT>
+  __device__ __forceinline__ void norm(const RowsArgs& p, const u32x4 (&nw)[NV], float* s_sq) {
+    const int lane = tid & (kWave - 1), wave = tid >> 6;
+#pragma unroll
+    for (int gb = 0; gb < NG; gb++) {
+      float ss = 0.f;
+#pragma unroll
+      for (int k = 0; k < NV; k++) ss = vec_sumsq<DT>(v[gb][k], ss);
+      ss = lanes_sum_mod8(ss);
+      if (lane < 8) s_sq[(gb * kMmaWaves + wave) * 8 + lane] = ss;
+    }
+    lds_barrier();
+#pragma unroll
+    for (int gb = 0; gb < NG; gb++) {
+      float ss = 0.f;
+#pragma unroll
+      for (int w = 0; w < kMmaWaves; w++) ss += s_sq[(gb * kMmaWaves + w) * 8 + (lane & 7)];
+      const float scale = rsqrtf(ss / (float)p.K + p.norm_eps);
+#pragma unroll
+      for (int k = 0; k < NV; k++)
+        if (in(p, gb, front * kWave + tid + k * kMmaThreads)) v[gb][k] = vec_norm_apply<DT>(v[gb][k], scale, nw[k]);
     }
   }
 };
@@ -424,11 +461,15 @@ __global__ __launch_bounds__(kMmaThreads) void rows_mma_kernel(RowsArgs p) {
     x.tid = tid;
     x.front = p.mma_front;
     x.fetch(p);
+    u32x4 nw[STEPS * CH];
+    if (UP && p.norm_w) x.fetch_norm(p, nw);
     // the first gate set goes out behind x, before x is waited for: it is a memory round trip ahead when the staging is done
     __builtin_amdgcn_sched_barrier(0);
     issue_gate(0, 0, g0);
     __builtin_amdgcn_sched_barrier(0);
-    x.store(p, xs, xgroup);
+    x.mask(p);
+    if (UP && p.norm_w) x.template norm<DT>(p, nw, part_g);
+    x.store(xs, xgroup);
 #pragma unroll
     for (int c = 0; c < STEPS; c++) u1[c] = zero4();  // defined before the first (unused) up product
     if constexpr (CH == 2) {
@@ -443,25 +484,6 @@ __global__ __launch_bounds__(kMmaThreads) void rows_mma_kernel(RowsArgs p) {
   // The second gate set goes out after the barrier: a wave blocks at issue once the CU's miss queue is full, so
   // everything issued before the barrier delays the moment the staged x becomes usable.
   issue_gate(CH == 2 ? 0 : 1, CH == 2 ? 1 : 0, g1);
-  if (p.norm_w) {
-    // RMS norm in place.  Wave b adds the squares of batch row b (kMmaWaves == 8 rows), in a fixed order.
-    __shared__ float s_scale[NG * 8];
-#pragma unroll
-    for (int gb = 0; gb < NG; gb++) {
-      float ss = 0.f;
-      for (int q = lane; q < xgroup / 8; q += kWave) ss = vec_sumsq<DT>(xs[gb * xgroup + q * 8 + wave], ss);
-      ss = wave_sum(ss);
-      if (lane == 0) s_scale[gb * 8 + wave] = rsqrtf(ss / (float)p.K + p.norm_eps);
-    }
-    __syncthreads();
-#pragma unroll
-    for (int gb = 0; gb < NG; gb++)
-      for (int i = p.mma_front * kWave + tid; i < xgroup; i += kMmaThreads) {
-        const int b = gb * 8 + (i & 7), v = (i >> 6) * 8 + ((i >> 3) & 1) * 4 + ((i >> 4) & 3) - 8 * p.mma_front;
-        if (b < p.nb && v < p.row_vecs) xs[gb * xgroup + i] = vec_norm_apply<DT>(xs[gb * xgroup + i], s_scale[b], p.norm_w[v]);
-      }
-    __syncthreads();
-  }
   CATS_RSTAMP(1);
   if constexpr (kHeld) gate.hold(held);
 
@@ -542,7 +564,8 @@ __global__ __launch_bounds__(kMmaThreads) void rows_mma_up_kernel(RowsArgs p) {
       s_a[e] = av;
       s_f[e] = in && (p.flag_in ? p.flag_in[o] != 0 : fabsf(DT::tof(av)) > p.t) ? 1 : 0;
     }
-    x.store(p, xs, xgroup);
+    x.mask(p);
+    x.store(xs, xgroup);
   }
   __syncthreads();
   // one thread per row of the range: any batch row flagged?  Eight neighbouring lanes make a tile's byte.

@@ -186,20 +186,20 @@ __global__ __launch_bounds__(kSmallThreads) void small_rows_kernel(SmallArgs a) 
   __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
   for (int e = 0; e < 4; e++) xv[e] = x_in ? xv[e] : 0u;
+  if (p.norm_w) {  // NCH waves hold a row
+    __shared__ float s_sq[B * NCH];
+    const float sq = wave_sum(vec_sumsq<DT>(xv, 0.f));
+    if (lane == 0 && xb < B) s_sq[wave] = sq;
+    lds_barrier();
+    if (x_in) {
+      float ss = 0.f;
+#pragma unroll
+      for (int c = 0; c < NCH; c++) ss += s_sq[xb * NCH + c];
+      xv = vec_norm_apply<DT>(xv, rsqrtf(ss / (float)p.K + p.norm_eps), nw);
+    }
+  }
   if (tid < B * NCH * kWave) xs[tid] = xv;
   lds_barrier();
-  if (p.norm_w) {
-    __shared__ float s_scale[B];
-    if (wave < B) {
-      float ss = 0.f;
-      for (int i = lane; i < p.row_vecs; i += kWave) ss = vec_sumsq<DT>(xs[wave * NCH * kWave + i], ss);
-      ss = wave_sum(ss);
-      if (lane == 0) s_scale[wave] = rsqrtf(ss / (float)p.K + p.norm_eps);
-    }
-    lds_barrier();
-    if (x_in) xs[tid] = vec_norm_apply<DT>(xv, s_scale[xb], nw);
-    lds_barrier();
-  }
 
   {
     float z[B];
@@ -332,35 +332,45 @@ __global__ __launch_bounds__(kSmallThreads) void small_mma_kernel(SmallArgs a) {
     wd[r] = load_stream(cols ? a.wd + (size_t)(base + j * p.row_stride) * p.row_vecs + min(dv, p.row_vecs - 1) : a.wd);
   }
   __builtin_amdgcn_sched_barrier(0);
+  auto x_in = [&](int g, int k) {
+    const int i = tid + k * kSmallThreads;
+    return g * 8 + (i & 7) < p.nb && (unsigned)x_vector(i) < (unsigned)p.row_vecs;
+  };
+#pragma unroll
+  for (int g = 0; g < NG; g++)
+#pragma unroll
+    for (int k = 0; k < NV; k++)
+#pragma unroll
+      for (int e = 0; e < 4; e++) xv[g][k][e] = x_in(g, k) ? xv[g][k][e] : 0u;
+  if (p.norm_w) {  // as in MmaX: a thread's vectors are of one batch row
+#pragma unroll
+    for (int g = 0; g < NG; g++) {
+      float ss = 0.f;
+#pragma unroll
+      for (int k = 0; k < NV; k++) ss = vec_sumsq<DT>(xv[g][k], ss);
+      ss = lanes_sum_mod8(ss);
+      if (lane < 8) part[(g * kSmallWaves + wave) * 8 + lane] = ss;
+    }
+    lds_barrier();
+#pragma unroll
+    for (int g = 0; g < NG; g++) {
+      float ss = 0.f;
+#pragma unroll
+      for (int w = 0; w < kSmallWaves; w++) ss += part[(g * kSmallWaves + w) * 8 + (lane & 7)];
+      const float scale = rsqrtf(ss / (float)p.K + p.norm_eps);
+#pragma unroll
+      for (int k = 0; k < NV; k++)
+        if (x_in(g, k)) xv[g][k] = vec_norm_apply<DT>(xv[g][k], scale, nw[k]);
+    }
+  }
 #pragma unroll
   for (int g = 0; g < NG; g++)
 #pragma unroll
     for (int k = 0; k < NV; k++) {
-      const int i = tid + k * kSmallThreads, b = g * 8 + (i & 7), v = x_vector(i);
-      const bool in = b < p.nb && (unsigned)v < (unsigned)p.row_vecs;
-#pragma unroll
-      for (int e = 0; e < 4; e++) xv[g][k][e] = in ? xv[g][k][e] : 0u;
+      const int i = tid + k * kSmallThreads;
       if (i < xgroup) xs[g * xgroup + i] = xv[g][k];
     }
   lds_barrier();
-  if (p.norm_w) {  // the squares of a batch row in rows_mma_kernel's order
-    __shared__ float s_scale[NG * 8];
-    if (wave < NG * 8) {
-      float ss = 0.f;
-      for (int q = lane; q < xgroup / 8; q += kWave) ss = vec_sumsq<DT>(xs[(wave >> 3) * xgroup + q * 8 + kw], ss);
-      ss = wave_sum(ss);
-      if (lane == 0) s_scale[wave] = rsqrtf(ss / (float)p.K + p.norm_eps);
-    }
-    lds_barrier();
-#pragma unroll
-    for (int g = 0; g < NG; g++)
-#pragma unroll
-      for (int k = 0; k < NV; k++) {
-        const int i = tid + k * kSmallThreads, b = g * 8 + (i & 7), v = x_vector(i);
-        if (b < p.nb && (unsigned)v < (unsigned)p.row_vecs) xs[g * xgroup + i] = vec_norm_apply<DT>(xv[g][k], s_scale[b], nw[k]);
-      }
-    lds_barrier();
-  }
 
   // ---- gate and up sums ----
 #pragma unroll
