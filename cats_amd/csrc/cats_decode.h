@@ -38,11 +38,13 @@ struct ProjArgs {
 
 // Two rows per wave.  For kProjQkv they are the two elements of a head that the rotary embedding mixes, d and d + head_dim / 2,
 // so it is applied to the two sums where they are; the wave's number counts these pairs over the three matrices.
-template <class DT, int B, int CB, bool FULL, int MODE, int WAVES>
+// Short rows are taken by blocks of CB = 2 or 4 chunks of 64 vectors instead of eight, and where the result is stored as it is (the output head) by
+// 16 / CB rows a wave: as many loads in flight, and x is staged once for as many weight bytes.
+template <class DT, int B, int CB, int R, bool FULL, int MODE, int WAVES>
 __global__ __launch_bounds__(WAVES* kWave) __attribute__((amdgpu_waves_per_eu(B == 1 && WAVES == 4 && FULL ? 6 : 1, 8)))
 void proj_kernel(ProjArgs a) {
   typedef typename DT::st st;
-  constexpr int R = 2;
+  static_assert(MODE != kProjQkv || R == 2, "a pair of elements a wave");
   constexpr int kThreads = WAVES * kWave;
   const RowsArgs& p = a.r;
   extern __shared__ u32x4 xs[];  // [B][round_up(nch, CB) * 64] vectors

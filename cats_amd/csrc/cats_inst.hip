@@ -1,6 +1,7 @@
 // Kernel instantiations for one dtype.  Compiled three times (-DCATS_DT=F16 / BF16 / F32) so the
 // translation units build in parallel.
 #include "cats_launch.h"
+#include "cats_proj_mma.h"
 #include "cats_rows_mma.h"
 
 #ifndef CATS_DT
@@ -259,19 +260,74 @@ hipError_t launch_fused_b(int grid, const FusedArgs& a, hipStream_t stream) {
   return hipErrorInvalidValue;
 }
 
+template <class DT, int B, int MODE, int CB>
+hipError_t launch_proj_cb(const ProjArgs& a, hipStream_t stream) {
+  constexpr int WAVES = WavesFor<B>::value, R = MODE == kProjPlain ? 2 * kProjCB / CB : 2;
+  const bool full = a.r.K % (kWave * DT::VEC * CB) == 0;
+  auto kern = full ? proj_kernel<DT, B, CB, R, true, MODE, WAVES> : proj_kernel<DT, B, CB, R, false, MODE, WAVES>;
+  const int items = MODE == kProjQkv ? a.r.N / 2 * 3 : (a.r.N + R - 1) / R;
+  const size_t lds = proj_lds_bytes(B, a.r.nch, CB);
+  if (hipError_t e = ensure_dynamic_lds((const void*)kern, lds); e != hipSuccess) return e;
+  return launch_kernel(kern, dim3((items + WAVES - 1) / WAVES), dim3(WAVES * kWave), lds, stream, a);
+}
+// Rows of up to two or four chunks of 64 vectors have instances of their own at one and two rows; batches of such rows are the matrix cores'.
 template <class DT, int B, int MODE>
 hipError_t launch_proj_one(const ProjArgs& a, hipStream_t stream) {
-  constexpr int WAVES = WavesFor<B>::value;
-  const bool full = a.r.K % (kWave * DT::VEC * kProjCB) == 0;
-  auto kern = full ? proj_kernel<DT, B, kProjCB, true, MODE, WAVES> : proj_kernel<DT, B, kProjCB, false, MODE, WAVES>;
-  const int pairs = MODE == kProjQkv ? a.r.N / 2 * 3 : (a.r.N + 1) / 2;
-  const size_t lds = proj_lds_bytes(B, a.r.nch);
-  if (hipError_t e = ensure_dynamic_lds((const void*)kern, lds); e != hipSuccess) return e;
-  return launch_kernel(kern, dim3((pairs + WAVES - 1) / WAVES), dim3(WAVES * kWave), lds, stream, a);
+  if constexpr (B <= 2) {
+    if (a.r.nch <= 2) return launch_proj_cb<DT, B, MODE, 2>(a, stream);
+    if (a.r.nch <= 4) return launch_proj_cb<DT, B, MODE, 4>(a, stream);
+  }
+  return launch_proj_cb<DT, B, MODE, kProjCB>(a, stream);
 }
+
+// Projections of 3..8 rows on the matrix cores: 16-bit types, rows and matrices on whole cache lines, head halves in fours, x operands in LDS.
+template <class DT>
+struct ProjMma {
+  template <int MODE, int STEPS, int CH>
+  static hipError_t run(const ProjArgs& a, int grid, size_t lds, hipStream_t stream) {
+    if constexpr (sizeof(typename DT::st) == 2) {
+      auto kern = proj_mma_kernel<DT, STEPS, CH, MODE>;
+      if (hipError_t e = ensure_dynamic_lds((const void*)kern, lds); e != hipSuccess) return e;
+      return launch_kernel(kern, dim3(grid), dim3(kMmaThreads), lds, stream, a);
+    } else {
+      return hipErrorInvalidValue;
+    }
+  }
+  static bool takes(int mode, const ProjArgs& a) {
+    if (sizeof(typename DT::st) != 2 || a.r.nb < 3 || a.r.nb > 8 || a.r.row_vecs % 8 != 0) return false;
+    uintptr_t w = (uintptr_t)a.r.w;
+    if (mode == kProjQkv) {
+      w |= (uintptr_t)a.wk | (uintptr_t)a.wv;
+      if (a.half % 4 != 0 || 2 * a.half > kProjMaxHeadDim || a.r.N % 8 != 0) return false;
+    }
+    const MmaSplit sp = rows_mma_split(a.r);
+    return w % 128 == 0 && sp.steps > 0 && proj_mma_lds_bytes(sp) <= MmaLaunch<DT>::kMmaMaxLds;
+  }
+  template <int MODE>
+  static hipError_t launch(const ProjArgs& a_in, hipStream_t stream) {
+    ProjArgs a = a_in;
+    const MmaSplit sp = rows_mma_split(a.r);
+    const int ntiles = proj_mma_ntiles(a, MODE), cus = current_device_cus();
+    a.r.rows_per = (ntiles + cus - 1) / cus;
+    a.r.mma_slots = sp.slots;
+    const int grid = (ntiles + a.r.rows_per - 1) / a.r.rows_per;
+    const size_t lds = proj_mma_lds_bytes(sp);
+#define CATS_PROJ_CASE(STEPS, CH) \
+  if (sp.steps == STEPS && sp.chunks == CH) return run<MODE, STEPS, CH>(a, grid, lds, stream);
+    CATS_PROJ_CASE(1, 1) CATS_PROJ_CASE(2, 1) CATS_PROJ_CASE(3, 1) CATS_PROJ_CASE(4, 1) CATS_PROJ_CASE(5, 1) CATS_PROJ_CASE(6, 1) CATS_PROJ_CASE(7, 1)
+    CATS_PROJ_CASE(8, 1) CATS_PROJ_CASE(9, 1) CATS_PROJ_CASE(5, 2) CATS_PROJ_CASE(6, 2) CATS_PROJ_CASE(7, 2) CATS_PROJ_CASE(8, 2) CATS_PROJ_CASE(9, 2)
+#undef CATS_PROJ_CASE
+    return hipErrorInvalidValue;
+  }
+};
 
 template <class DT, int B>
 hipError_t launch_proj_b(int mode, const ProjArgs& a, hipStream_t stream) {
+  if (B >= 4 && ProjMma<DT>::takes(mode, a)) {
+    if (mode == kProjPlain) return ProjMma<DT>::template launch<kProjPlain>(a, stream);
+    if (mode == kProjAdd) return ProjMma<DT>::template launch<kProjAdd>(a, stream);
+    return ProjMma<DT>::template launch<kProjQkv>(a, stream);
+  }
   switch (mode) {
     case kProjPlain: return launch_proj_one<DT, B, kProjPlain>(a, stream);
     case kProjAdd: return launch_proj_one<DT, B, kProjAdd>(a, stream);
@@ -313,7 +369,10 @@ hipError_t launch_attn<CATS_DT>(int head_dim, int bt, AttnArgs a, hipStream_t st
   // the CUs that attention leaves free fetch the next projection's weights, where they are at least three quarters of the chip (half of
   // it: steps of two layers 4096 / 11008, 4 rows of 32 heads, 228.7 / 231.2 us)
   const int ahead = spare ? (cus - a.pairs) / 8 * 8 : 0;
-  a.piece_vecs *= kR * (bt <= 2 ? WavesFor<1>::value : WavesFor<8>::value);  // from vectors of a row to those of a workgroup of proj_kernel
+  // from vectors of a row to those of a workgroup of the projection
+  const int rows = a.pairs / bt * head_dim;
+  if (sizeof(CATS_DT::st) == 2 && bt >= 3 && a.piece_vecs % 8 == 0) a.piece_vecs *= ((rows + 7) / 8 + cus - 1) / cus * 8;
+  else a.piece_vecs *= kR * (bt <= 2 ? WavesFor<1>::value : WavesFor<8>::value);
   return launch_kernel(kern, dim3(a.pairs + ahead), dim3(1024), 0, stream, a);
 }
 

@@ -41,6 +41,36 @@ def test_linear(B, K, N, dtype, norm):
         _check(out, want, dtype, K) if N > 1 else torch.testing.assert_close(out.cpu().double(), want, rtol=4 * EPS[dtype], atol=1e-3)
 
 
+@pytest.mark.parametrize("B,K,N,dtype", [
+    (3, 64, 8, torch.float16), (5, 64, 2000, torch.bfloat16), (4, 512, 4099, torch.float16), (8, 576, 7, torch.bfloat16), (3, 1024, 6001, torch.float16),
+    (7, 1088, 2500, torch.bfloat16), (3, 2048, 4105, torch.float16), (6, 2112, 300, torch.float16), (8, 4608, 100, torch.bfloat16),
+    (4, 4672, 4200, torch.float16), (3, 8192, 520, torch.bfloat16), (8, 8192, 40, torch.float16), (3, 9216, 40, torch.float16), (4, 9280, 24, torch.float16)])
+@pytest.mark.parametrize("norm", [False, True])
+def test_linear_on_the_matrix_cores(B, K, N, dtype, norm):
+    """One to nine steps a wave in one register set and five to nine in two (9280: too long, a wave a row), eight to one tiles a round, rounds
+    in pairs and not, a last tile that is not whole, fewer tiles than CUs and several each."""
+    test_linear(B, K, N, dtype, norm)
+
+
+@pytest.mark.parametrize("B", [1, 2])
+@pytest.mark.parametrize("K,N", [(256, 1000), (1024, 33), (1032, 4099), (2048, 70), (2056, 515)])
+@pytest.mark.parametrize("norm", [False, True])
+def test_linear_over_short_rows(B, K, N, norm):
+    """Blocks of two, four and eight chunks of a row, whole and not, at the rows a wave that goes with them."""
+    test_linear(B, K, N, torch.float16, norm)
+
+
+@pytest.mark.parametrize("offset", [8, 64])
+def test_linear_where_the_matrix_starts(offset):
+    """A matrix that starts inside a cache line keeps the wave-per-row kernel."""
+    import flash_gemv  # noqa: F401
+
+    g = torch.Generator(device="cuda").manual_seed(offset)
+    buf = torch.randn(700 * 640 + 64, generator=g, device="cuda").half() * 0.05
+    w, x = buf[offset:offset + 700 * 640].view(700, 640), torch.randn(4, 640, generator=g, device="cuda").half()
+    _check(torch.ops.flash_gemv.cats_linear(x, None, 1e-5, w), x.cpu().double() @ w.cpu().double().t(), torch.float16, 640)
+
+
 def _reference(h, x, wq, wk, wv, wo, kc, vc, cos, sin, pos):
     B, heads, _, hd = kc.shape
     shp = (B, heads, hd)
@@ -87,6 +117,14 @@ def test_attention_step(B, heads, hd, max_len, pos, dtype):
         out = torch.ops.flash_gemv.cats_attention_step(h.cuda(), x.cuda(), None, 0.0, *[w.cuda() for w in ws], kd, vd, cos.cuda(), sin.cuda(),
                                                        torch.tensor([bad], device="cuda"))
         assert bool(out.isnan().all()) and torch.equal(kd, before)
+
+
+@pytest.mark.parametrize("B,heads,hd,dtype", [(3, 6, 16, torch.float16), (4, 4, 16, torch.bfloat16), (5, 3, 64, torch.float16), (3, 20, 128, torch.bfloat16),
+                                              (8, 16, 256, torch.float16), (4, 32, 128, torch.float16), (3, 40, 128, torch.bfloat16), (2, 4, 64, torch.bfloat16)])
+def test_attention_step_of_batches(B, heads, hd, dtype):
+    """The three projections in tiles of four pairs of a head: one to several tiles a workgroup, of one matrix or of two, rows of 96 elements
+    (no whole cache lines) and two rows with a wave a row; 5120 elements in two register sets."""
+    test_attention_step(B, heads, hd, 50, 33, dtype)
 
 
 @pytest.mark.parametrize("B,heads,hd,max_len,pos", [(5, 13, 16, 40, 20), (5, 13, 128, 600, 513), (1, 20, 128, 600, 255), (1, 20, 128, 600, 256),
