@@ -41,11 +41,10 @@ struct ProjArgs {
 // Short rows are taken by blocks of CB = 2 or 4 chunks of 64 vectors instead of eight, and where the result is stored as it is (the output head) by
 // 16 / CB rows a wave: as many loads in flight, and x is staged once for as many weight bytes.
 template <class DT, int B, int CB, int R, bool FULL, int MODE, int WAVES>
-__global__ __launch_bounds__(WAVES* kWave) __attribute__((amdgpu_waves_per_eu(B == 1 && WAVES == 4 && FULL ? 6 : 1, 8)))
+__global__ __launch_bounds__(WAVES* kWave) __attribute__((amdgpu_waves_per_eu(rows_waves_per_simd(B, FULL), 8)))
 void proj_kernel(ProjArgs a) {
   typedef typename DT::st st;
   static_assert(MODE != kProjQkv || R == 2, "a pair of elements a wave");
-  constexpr int kThreads = WAVES * kWave;
   const RowsArgs& p = a.r;
   extern __shared__ u32x4 xs[];  // [B][round_up(nch, CB) * 64] vectors
   const int lane = threadIdx.x & (kWave - 1);
@@ -77,58 +76,44 @@ void proj_kernel(ProjArgs a) {
   }
   const bool pos_ok = pos >= 0 && pos < (long long)a.max_len;
 
-  // x goes out first, the weights behind it, and only x is waited for before the barrier (see rows_kernel)
+  // What the sums will be joined with is asked for first, and the elements of the rotary embedding behind the weights: after the sums each
+  // would be one more trip.  The weights go out behind x, before x is waited for; at one and two rows half of them when x is staged: its registers.
+  float res[R][B];
+  if (MODE == kProjAdd) {
+#pragma unroll
+    for (int r = 0; r < R; r++)
+#pragma unroll
+      for (int b = 0; b < B; b++) res[r][b] = DT::tof(((const st*)a.residual)[(size_t)min(b, p.nb - 1) * p.N + row[r]]);
+  }
+  constexpr int kXPreAll = (B * CB + WAVES - 1) / WAVES, kXPre = kXPreAll < 4 ? kXPreAll : 4;  // rows of CB chunks
+  constexpr int kFirst = B <= 2 ? R * CB / 2 : R * CB;
   u32x4 wv[R][CB];
-  constexpr int kXPreAll = (B * 512 + kThreads - 1) / kThreads;
-  constexpr int kXPre = kXPreAll < 4 ? kXPreAll : 4;
-  const int nchv = (p.nch + CB - 1) / CB * CB * kWave;
-  u32x4 xpre[kXPre];
-#pragma unroll
-  for (int k = 0; k < kXPre; k++) {
-    const int i = threadIdx.x + k * kThreads;
-    const int b = B == 1 ? 0 : i / nchv, v = i - b * nchv;
-    xpre[k] = zero4();
-    if (i < B * nchv && b < p.nb && v < p.row_vecs) xpre[k] = p.x[(size_t)b * p.row_vecs + v];
-  }
-  rows_issue<R, CB, FULL>(w, row, on, 0, p, lane, wv);
-#pragma unroll
-  for (int k = 0; k < kXPre; k++) {
-    const int i = threadIdx.x + k * kThreads;
-    if (i < B * nchv) xs[i] = xpre[k];
-  }
-  for (int i = threadIdx.x + kXPre * kThreads; i < B * nchv; i += kThreads) {
-    const int b = i / nchv, v = i - b * nchv;
-    u32x4 val = zero4();
-    if (b < p.nb && v < p.row_vecs) val = p.x[(size_t)b * p.row_vecs + v];
-    xs[i] = val;
-  }
-  __syncthreads();
-  if (p.norm_w) {
-    __shared__ float s_scale[B];
-    for (int b = wave; b < B; b += WAVES) {
-      float ss = 0.f;
-      for (int v = lane; v < p.row_vecs; v += kWave) ss = vec_sumsq<DT>(xs[b * nchv + v], ss);
-      ss = wave_sum(ss);
-      if (lane == 0) s_scale[b] = rsqrtf(ss / (float)p.K + p.norm_eps);
-    }
-    __syncthreads();
-    for (int i = threadIdx.x; i < B * nchv; i += kThreads) {
-      const int b = B == 1 ? 0 : i / nchv, v = i - b * nchv;
-      if (b < p.nb && v < p.row_vecs) xs[i] = vec_norm_apply<DT>(xs[i], s_scale[b], p.norm_w[v]);
-    }
-    __syncthreads();
+  __shared__ float s_sq[kRowsMaxChunks + B];
+  RowsX<DT, B, WAVES, kXPre, MODE != kProjAdd> x;
+  x.lane = lane;
+  x.wave = wave;
+  x.nchp = (p.nch + CB - 1) / CB * CB;
+  x.fetch(p);
+  __builtin_amdgcn_sched_barrier(0);
+  rows_issue_all<0, kFirst, R, CB, FULL>(w, row, 0, p, lane, wv);
+  __builtin_amdgcn_sched_barrier(0);
+  x.store(p, xs, s_sq);
+  rows_issue_all<kFirst, R * CB, R, CB, FULL>(w, row, 0, p, lane, wv);
+  float cs = 0.f;  // lane 0: cos of d, 1: of d + half, 2 and 3: sin
+  if (MODE == kProjQkv) {
+    const st* t = (const st*)(lane & 2 ? a.sin_t : a.cos_t);
+    cs = DT::tof(t[(size_t)(pos_ok ? pos : 0) * 2 * a.half + d + (lane & 1) * a.half]);
   }
 
   float g[R][B];
-  rows_dot<DT, B, R, CB, FULL, true>(w, row, on, xs, p.x, p, lane, wv, true, g);
+  rows_dot<DT, B, R, CB, FULL, true, true>(w, row, on, xs, p.x, p, lane, wv, g);
 
+  auto cs_of = [&](int i) { return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(cs), i)); };
+  const float c0 = cs_of(0), c1 = cs_of(1), s0 = cs_of(2), s1 = cs_of(3);
   if (lane != 0) return;
   if (MODE == kProjQkv) {
     if (!on[0]) return;
     if (which == 0 || which == 1) {
-      const st* ct = (const st*)a.cos_t + (size_t)(pos_ok ? pos : 0) * 2 * a.half;
-      const st* sn = (const st*)a.sin_t + (size_t)(pos_ok ? pos : 0) * 2 * a.half;
-      const float c0 = DT::tof(ct[d]), c1 = DT::tof(ct[d + a.half]), s0 = DT::tof(sn[d]), s1 = DT::tof(sn[d + a.half]);
 #pragma unroll
       for (int b = 0; b < B; b++) {
         const float lo = g[0][b], hi = g[1][b];
@@ -157,7 +142,7 @@ void proj_kernel(ProjArgs a) {
         for (int b = 0; b < B; b++)
           if (b < p.nb) {
             const size_t o = (size_t)b * p.N + row[r];
-            out[o] = DT::fromf(MODE == kProjAdd ? g[r][b] + DT::tof(((const st*)a.residual)[o]) : g[r][b]);
+            out[o] = DT::fromf(MODE == kProjAdd ? g[r][b] + res[r][b] : g[r][b]);
           }
       }
   }

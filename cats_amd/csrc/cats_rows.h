@@ -85,12 +85,25 @@ __device__ __forceinline__ void rows_issue(const u32x4* __restrict__ w, const in
   }
 }
 
-// Dot products of R weight rows against the nb staged x rows.  acc[r][b] ends up wave-uniform.  `wv` holds the
-// loads of the first block if `preissued` (the caller started them before x was staged), else it is scratch.
-template <class DT, int B, int R, int CB, bool FULL, bool XLDS>
+// Loads FROM .. TO - 1 of a block, rows one after the other (chunk by chunk they take up to 6 % more of a whole call), whether or not a row is wanted (its index is in range): a load behind a
+// branch may or may not be in flight afterwards, so that waiting for one ahead of it would wait for all.
+template <int FROM, int TO, int R, int CB, bool FULL>
+__device__ __forceinline__ void rows_issue_all(const u32x4* __restrict__ w, const int (&row)[R], int c0, const RowsArgs& p, int lane,
+                                               u32x4 (&wv)[R][CB]) {
+  const int vlast = p.row_vecs - 1;
+#pragma unroll
+  for (int i = FROM; i < TO; i++) {
+    const int r = i / CB, cc = i % CB, v = (c0 + cc) * kWave + lane;
+    wv[r][cc] = load_stream(w + (size_t)row[r] * p.row_vecs + (FULL ? v : min(v, vlast)));
+  }
+}
+
+// Dot products of R weight rows against the nb staged x rows.  acc[r][b] ends up wave-uniform.  ALL: every row is taken, whatever
+// `on` says, and `wv` holds the loads of the first block (the caller started them before x was staged); else it is scratch.
+template <class DT, int B, int R, int CB, bool FULL, bool XLDS, bool ALL>
 __device__ __forceinline__ void rows_dot(const u32x4* __restrict__ w, const int (&row)[R], const bool (&on)[R],
                                          const u32x4* xs, const u32x4* __restrict__ xg, const RowsArgs& p, int lane,
-                                         u32x4 (&wv)[R][CB], bool preissued, float (&acc)[R][B]) {
+                                         u32x4 (&wv)[R][CB], float (&acc)[R][B]) {
 #pragma unroll
   for (int r = 0; r < R; r++)
 #pragma unroll
@@ -99,7 +112,8 @@ __device__ __forceinline__ void rows_dot(const u32x4* __restrict__ w, const int 
   const int vlast = p.row_vecs - 1;
   const int nchp = (p.nch + CB - 1) / CB * CB;
   for (int c0 = 0; c0 < p.nch; c0 += CB) {
-    if (!(preissued && c0 == 0)) rows_issue<R, CB, FULL>(w, row, on, c0, p, lane, wv);
+    if (!ALL) rows_issue<R, CB, FULL>(w, row, on, c0, p, lane, wv);
+    else if (c0 > 0) rows_issue_all<0, R * CB, R, CB, FULL>(w, row, c0, p, lane, wv);
 #pragma unroll
     for (int cc = 0; cc < CB; cc++) {
       const int v = (c0 + cc) * kWave + lane;
@@ -114,22 +128,146 @@ __device__ __forceinline__ void rows_dot(const u32x4* __restrict__ w, const int 
         }
 #pragma unroll
         for (int r = 0; r < R; r++)
-          if (on[r]) acc[r][b] = DT::dot(wv[r][cc], xv, acc[r][b]);
+          if (ALL || on[r]) acc[r][b] = DT::dot(wv[r][cc], xv, acc[r][b]);
       }
+      if (ALL && B >= 4) __builtin_amdgcn_sched_barrier(0);  // else the x of later chunks is read ahead, into twice the registers
     }
   }
 #pragma unroll
   for (int r = 0; r < R; r++)
-    if (on[r]) {
+    if (ALL || on[r]) {
 #pragma unroll
       for (int b = 0; b < B; b++) acc[r][b] = wave_sum(acc[r][b]);
     }
 }
 
+// x of all batch rows on its way into LDS, through the RMS norm if there is one.  Memory returns are counted in issue order: fetch()
+// goes out in front of the first weights, and store() waits for x alone while these stay in flight.  (As loads behind conditions, x
+// was waited for together with all of the weights, and the norm's weights were asked for after that.)  NX vectors a thread are fetched ahead, the rest
+// of longer rows in batches; NORM_AHEAD: so are their norm weights.  All of a wave's 64 vectors are of one chunk of one row.
+// Whole calls, before / now in us: HF layout 4096 / 11008 fp32 1 row 79.8 / 72.6, 2 rows 92.8 / 85.4, fp16 1 row 40.3 / 38.2, bf16 2 rows 48.5 / 42.5,
+// 2000 / 5000 fp16 2 rows 18.0 / 14.6; steps of four layers 4096 / 11008 319 / 306, 2304 / 7097 168.7 / 158.3.  The chunk's row is found by
+// comparisons: divisions took 1 to 3 us of these at two rows, and more than the staging gave at four.
+constexpr int kRowsMaxChunks = 160;  // of 1 KiB: more is not staged
+template <class DT, int B, int WAVES, int NX, bool NORM_AHEAD>
+struct RowsX {
+  static constexpr int U = 2;
+  u32x4 v[NX], nw[NORM_AHEAD ? NX : 1];
+  int lane, wave, nchp;  // nchp: chunks of a row with its padding
+
+  // of chunk c: batch row and vector of this lane
+  __device__ __forceinline__ int row_of(int c) const {
+    int b = 0;
+#pragma unroll
+    for (int i = 1; i < B; i++) b += c >= i * nchp;
+    return b;
+  }
+  __device__ __forceinline__ int vec_of(int c) const { return (c - row_of(c) * nchp) * kWave + lane; }
+  __device__ __forceinline__ bool in(const RowsArgs& p, int c) const {
+    return c < p.nb * nchp && vec_of(c) < p.row_vecs;
+  }
+  __device__ __forceinline__ u32x4 load(const RowsArgs& p, int c) const {
+    return p.x[in(p, c) ? (size_t)row_of(c) * p.row_vecs + vec_of(c) : 0];
+  }
+  __device__ __forceinline__ u32x4 load_norm(const RowsArgs& p, int c) const {
+    return (p.norm_w ? p.norm_w : p.x)[in(p, c) ? vec_of(c) : 0];
+  }
+  __device__ __forceinline__ u32x4 masked(const RowsArgs& p, int c, u32x4 val) const {
+    const bool ok = in(p, c);
+    u32x4 o;
+#pragma unroll
+    for (int e = 0; e < 4; e++) {
+      const uint32_t x = val[e];
+      o[e] = ok ? x : 0u;
+    }
+    return o;
+  }
+  __device__ __forceinline__ void fetch(const RowsArgs& p) {
+#pragma unroll
+    for (int k = 0; k < NX; k++) v[k] = load(p, wave + k * WAVES);
+    if (NORM_AHEAD) {
+#pragma unroll
+      for (int k = 0; k < NX; k++) nw[k] = load_norm(p, wave + k * WAVES);
+    }
+  }
+  // Ends with a barrier.  s_sq: kRowsMaxChunks + B floats.
+  __device__ __forceinline__ void store(const RowsArgs& p, u32x4* xs, float* s_sq) {
+    const int chunks = B * nchp;
+    const bool norm = p.norm_w != nullptr;
+    auto square = [&](int c, u32x4 val) {
+      const float sq = wave_sum(vec_sumsq<DT>(val, 0.f));
+      if (lane == 0) s_sq[c] = sq;
+    };
+#pragma unroll
+    for (int k = 0; k < NX; k++) {
+      const int c = wave + k * WAVES;
+      v[k] = masked(p, c, v[k]);
+      if (c < chunks) {
+        if (norm) square(c, v[k]);
+        else xs[c * kWave + lane] = v[k];
+      }
+    }
+    for (int c0 = wave + NX * WAVES; c0 < chunks; c0 += U * WAVES) {
+      u32x4 t[U];
+#pragma unroll
+      for (int u = 0; u < U; u++) t[u] = load(p, c0 + u * WAVES);
+#pragma unroll
+      for (int u = 0; u < U; u++) {
+        const int c = c0 + u * WAVES;
+        if (c < chunks) {
+          t[u] = masked(p, c, t[u]);
+          xs[c * kWave + lane] = t[u];
+          if (norm) square(c, t[u]);
+        }
+      }
+    }
+    lds_barrier();
+    if (!norm) return;
+    // the squares of a row: by chunk, then over the chunks by lane, then over the lanes
+    auto scale_of = [&](int b) {
+      float ss = 0.f;
+      for (int i = lane; i < nchp; i += kWave) ss += s_sq[b * nchp + i];
+      return rsqrtf(wave_sum(ss) / (float)p.K + p.norm_eps);
+    };
+    float sc = 0.f;
+    if (B == 1) {
+      sc = scale_of(0);
+    } else {
+      for (int b = wave; b < B; b += WAVES) {
+        const float r = scale_of(b);
+        if (lane == 0) s_sq[kRowsMaxChunks + b] = r;
+      }
+      lds_barrier();
+    }
+    auto scale = [&](int c) { return B == 1 ? sc : s_sq[kRowsMaxChunks + row_of(c)]; };
+#pragma unroll
+    for (int k = 0; k < NX; k++) {
+      const int c = wave + k * WAVES;
+      if (c < chunks) {
+        const u32x4 w = NORM_AHEAD ? nw[NORM_AHEAD ? k : 0] : load_norm(p, c);
+        xs[c * kWave + lane] = masked(p, c, vec_norm_apply<DT>(v[k], scale(c), w));
+      }
+    }
+    constexpr int UN = B >= 4 ? 4 : U;
+    for (int c0 = wave + NX * WAVES; c0 < chunks; c0 += UN * WAVES) {
+      u32x4 w[UN];
+#pragma unroll
+      for (int u = 0; u < UN; u++) w[u] = load_norm(p, c0 + u * WAVES);
+#pragma unroll
+      for (int u = 0; u < UN; u++) {
+        const int c = c0 + u * WAVES;
+        if (c < chunks) xs[c * kWave + lane] = masked(p, c, vec_norm_apply<DT>(xs[c * kWave + lane], scale(c), w[u]));
+      }
+    }
+    lds_barrier();
+  }
+};
+
 // B == 1 asks for 6 waves per SIMD (80 VGPRs): 6 workgroups of 4 waves per CU hold all 1376 workgroups of an
 // 11008-row matrix at once, so no workgroup starts late and runs its two dependent passes on a draining machine.
+constexpr int rows_waves_per_simd(int B, bool full) { return B == 1 ? (full ? 6 : 5) : B <= 4 ? 4 : 1; }
 template <class DT, int B, int R, int CB, bool FULL, int MODE, bool XLDS, int WAVES>
-__global__ __launch_bounds__(WAVES* kWave) __attribute__((amdgpu_waves_per_eu(B == 1 && WAVES == 4 && FULL ? 6 : 1, 8)))
+__global__ __launch_bounds__(WAVES* kWave) __attribute__((amdgpu_waves_per_eu(XLDS && MODE != kGemv ? rows_waves_per_simd(B, FULL) : 1, 8)))
 void rows_kernel(RowsArgs p) {
   typedef typename DT::st st;
   extern __shared__ u32x4 xs[];  // [B][round_up(nch, CB) * 64] vectors (XLDS only)
@@ -137,7 +275,6 @@ void rows_kernel(RowsArgs p) {
 
   const int lane = threadIdx.x & (kWave - 1);
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // wave-uniform by construction; say so
-  constexpr int kThreads = WAVES * kWave;
   constexpr int kRowsPerBlock = WAVES * R;
   static_assert(kRowsPerBlock % 8 == 0 && kRowsPerBlock <= 32, "mask bytes are assembled in one 32-bit LDS word");
 
@@ -159,54 +296,31 @@ void rows_kernel(RowsArgs p) {
     }
   }
 
-  // Staging order matters: memory returns are counted in issue order, so the x loads go out first, then the
-  // first block of weight loads, and only the x values are waited for before the LDS writes and the barrier --
-  // the weight loads stay in flight across both.
+  // The first weights go out behind x, before x is waited for.  At one and two rows half of them follows when x is staged: its registers.
+  constexpr bool kPre = MODE != kUp && MODE != kUpIndex;
+  constexpr int kFirst = B <= 2 && MODE != kGemv ? R * CB / 2 : R * CB;
+  constexpr int kXPreAll = (B * CB + WAVES - 1) / WAVES * (16 / DT::VEC / 2);  // rows of 4096 elements
+  constexpr int kXPre = kXPreAll < 4 ? kXPreAll : 4;
   u32x4 wv[R][CB];
-  // x vectors per thread fetched ahead of the weights: all of x for H = 4096 in 16-bit types (B * 512 vectors)
-  constexpr int kXPreAll = (B * 512 + kThreads - 1) / kThreads;
-  constexpr int kXPre = kXPreAll < 4 ? kXPreAll : 4;  // more would spill at B = 8
-  const int nchv = (p.nch + CB - 1) / CB * CB * kWave;  // padded vectors per x row
-  u32x4 xpre[kXPre];
-  if (XLDS) {
-#pragma unroll
-    for (int k = 0; k < kXPre; k++) {
-      const int i = threadIdx.x + k * kThreads;
-      const int b = B == 1 ? 0 : i / nchv, v = i - b * nchv;
-      xpre[k] = zero4();
-      if (i < B * nchv && b < p.nb && v < p.row_vecs) xpre[k] = p.x[(size_t)b * p.row_vecs + v];
-    }
-  }
-  if (MODE != kUp && MODE != kUpIndex) rows_issue<R, CB, FULL>(p.w, row, on, 0, p, lane, wv);
-  if (XLDS) {
-#pragma unroll
-    for (int k = 0; k < kXPre; k++) {
-      const int i = threadIdx.x + k * kThreads;
-      if (i < B * nchv) xs[i] = xpre[k];
-    }
-    for (int i = threadIdx.x + kXPre * kThreads; i < B * nchv; i += kThreads) {
-      const int b = i / nchv, v = i - b * nchv;
-      u32x4 val = zero4();
-      if (b < p.nb && v < p.row_vecs) val = p.x[(size_t)b * p.row_vecs + v];
-      xs[i] = val;
-    }
-  }
   if (threadIdx.x == 0) s_maskbits = 0u;
-  __syncthreads();
-  if (XLDS && p.norm_w) {
-    // RMS norm of each batch row, in place in LDS: one wave adds a row's squares (fixed order), everyone rescales.
-    __shared__ float s_scale[B];
-    for (int b = wave; b < B; b += WAVES) {
-      float ss = 0.f;
-      for (int v = lane; v < p.row_vecs; v += kWave) ss = vec_sumsq<DT>(xs[b * nchv + v], ss);
-      ss = wave_sum(ss);
-      if (lane == 0) s_scale[b] = rsqrtf(ss / (float)p.K + p.norm_eps);
-    }
-    __syncthreads();
-    for (int i = threadIdx.x; i < B * nchv; i += kThreads) {
-      const int b = B == 1 ? 0 : i / nchv, v = i - b * nchv;
-      if (b < p.nb && v < p.row_vecs) xs[i] = vec_norm_apply<DT>(xs[i], s_scale[b], p.norm_w[v]);
-    }
+  if (XLDS) {
+    __shared__ float s_sq[kRowsMaxChunks + B];
+    const int nchp = (p.nch + CB - 1) / CB * CB;
+    auto stage = [&](auto x) {
+      x.lane = lane;
+      x.wave = wave;
+      x.nchp = nchp;
+      x.fetch(p);
+      __builtin_amdgcn_sched_barrier(0);
+      if (kPre) rows_issue_all<0, kFirst, R, CB, FULL>(p.w, row, 0, p, lane, wv);
+      __builtin_amdgcn_sched_barrier(0);
+      x.store(p, xs, s_sq);
+      if (kPre) rows_issue_all<kFirst, R * CB, R, CB, FULL>(p.w, row, 0, p, lane, wv);
+    };
+    // the intermediate rows that kGemv takes: up to 11008 fp32 elements, or two rows of 16-bit ones
+    if (MODE == kGemv && B <= 2 && B * nchp > kXPre * WAVES) stage(RowsX<DT, B, WAVES, 12, false>());
+    else stage(RowsX<DT, B, WAVES, kXPre, (MODE == kGateUp && (B == 2 || B == 4))>());
+  } else {
     __syncthreads();
   }
   CATS_RSTAMP(1);
@@ -251,7 +365,7 @@ void rows_kernel(RowsArgs p) {
     }
   } else {
     float g[R][B];
-    rows_dot<DT, B, R, CB, FULL, XLDS>(p.w, row, on, xs, p.x, p, lane, wv, true, g);
+    rows_dot<DT, B, R, CB, FULL, XLDS, XLDS>(p.w, row, on, xs, p.x, p, lane, wv, g);
     if (MODE == kGemv) {
       if (lane == 0) {
         st* out = (st*)p.zt_out;
@@ -299,7 +413,7 @@ void rows_kernel(RowsArgs p) {
   CATS_RSTAMP(2);
   if (MODE == kGateUp || MODE == kUp || MODE == kUpIndex) {
     float u[R][B];
-    rows_dot<DT, B, R, CB, FULL, XLDS>(MODE == kGateUp ? p.w2 : p.w, row, any, xs, p.x, p, lane, wv, false, u);
+    rows_dot<DT, B, R, CB, FULL, XLDS, false>(MODE == kGateUp ? p.w2 : p.w, row, any, xs, p.x, p, lane, wv, u);
     if (lane == 0) {
 #pragma unroll
       for (int r = 0; r < R; r++)
