@@ -34,6 +34,8 @@ def test_norm_from_registers(oracle, H, I, B, dtype):
 def test_bf16_rounding(B):
     """A sum of two bf16 numbers that fp32 holds exactly leaves as torch rounds it: ties, the carry into the exponent, subnormal results,
     the step to infinity, infinities and NaN."""
+    import flash_gemv  # noqa: F401
+
     pairs = [(1.0, 2.0 ** -8), (1.0 + 2.0 ** -7, 2.0 ** -8), (1.0, -(2.0 ** -9)), (1.0, 2.0 ** -8 + 2.0 ** -14), (2.0 - 2.0 ** -7, 2.0 ** -8),
              (2.0 ** -126, -(2.0 ** -127) + 2.0 ** -133), (2.0 ** -133, 0.0), (3 * 2.0 ** -133, -(2.0 ** -133)),
              (3.3895313892515355e38, 2.0 ** 119), (3.3895313892515355e38, -(2.0 ** 119)), (-3.3895313892515355e38, -(2.0 ** 119)),
