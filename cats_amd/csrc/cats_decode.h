@@ -8,10 +8,10 @@
 // x may be given before its RMS norm (norm_w), which is then applied while x is staged.  Everything between the weight
 // matrices stays in fp32 and is rounded once where it is stored.  All of it is bound by the weight stream: one wave owns two
 // rows of a matrix, whose loads are all in flight at once, as in rows_kernel.
-// One step of four layers 4096 / 11008, 32 heads, 32000 words, 256 tokens in the cache, fp16, one row: 323 us, of which the MLP
+// One step of four layers 4096 / 11008, 32 heads, 32000 words, 256 tokens in the cache, fp16, one row: 306 us, of which the MLP
 // kernels take 150; with torch's operations in place of these kernels (about 25 launches a layer) it was 761.  Kernel trace: q, k, v
-// 19.1 us with the norm (5.3 TB/s), attention 8.0 and the output projection, whose weights it has had fetched, 5.3 (6.6 and 8.1
-// without that), output head 44 (5.9 TB/s).
+// 17.4 us with the norm (5.8 TB/s), attention 7.7 and the output projection, whose weights it has had fetched, 4.8 (8.1
+// without that), output head 40.6 (6.5 TB/s).  With x staged behind the weights: 18.8, 7.6, 5.2 and 42.7.
 #pragma once
 #include "cats_rows.h"
 
