@@ -47,7 +47,8 @@ __device__ inline int small_quads(int H) {
 
 // Batch row `row` of what reduce_partials_kernel does, by one workgroup, the next norm included: no hand-over between workgroups in front of it.
 // Ranges of partials side by side, their sums in range order, then the count.  s_part: a float4 of LDS a thread.
-template <class DT>
+// TAIL: the layer tail, with a residual and perhaps the next norm.
+template <class DT, bool TAIL>
 __device__ __forceinline__ void small_finish_row(const ReduceArgs& p, int row, float4* s_part, float* s_ssq) {
   typedef typename DT::st st;
   const int quads = small_quads(p.H);
@@ -57,13 +58,14 @@ __device__ __forceinline__ void small_finish_row(const ReduceArgs& p, int row, f
   const int per = (p.G + ranges - 1) / ranges, g0 = range * per, g1 = min(p.G, g0 + per);
   const size_t col = (size_t)row * p.H + (on ? quad * 4 : 0);
   const bool mine = range == 0 && on;
-  // what the sums are joined with comes in with the partials (steps of one layer 256 / 640, 4 rows 42.9 us without, 42.3 with; 512 / 1121, 1 row 32.8, 32.6)
+  // What the sums are joined with comes in with the partials: steps of one layer 256 / 640, 4 rows 42.9 us without, 42.3 with; 512 / 1121, 1 row 32.8, 32.6.
+  // In an instance of its own: with these loads behind conditions a plain call of 512 / 1024 took 8.18 us, without any 8.04.
   float residual[4] = {0.f, 0.f, 0.f, 0.f}, norm2[4] = {0.f, 0.f, 0.f, 0.f};
-  if (mine && p.residual && !p.y32_acc) {
+  if (TAIL && mine) {
 #pragma unroll
     for (int e = 0; e < 4; e++) residual[e] = DT::tof(((const st*)p.residual)[col + e]);
   }
-  if (mine && p.norm2_out) {
+  if (TAIL && mine && p.norm2_out) {
 #pragma unroll
     for (int e = 0; e < 4; e++) norm2[e] = DT::tof(((const st*)p.norm2_w)[quad * 4 + e]);
   }
@@ -87,17 +89,17 @@ __device__ __forceinline__ void small_finish_row(const ReduceArgs& p, int row, f
     }
 #pragma unroll
     for (int e = 0; e < 4; e++) {
-      if (p.y32_acc) {
+      if (!TAIL && p.y32_acc) {
         unsafeAtomicAdd(p.y32_acc + col + e, y[e]);  // as in reduce_partials_kernel
       } else {
-        const st o = DT::fromf(p.residual ? DT::rnd(y[e]) + residual[e] : y[e]);
+        const st o = DT::fromf(TAIL ? DT::rnd(y[e]) + residual[e] : y[e]);
         ((st*)p.y_out)[col + e] = o;
         y[e] = DT::tof(o);
         ss = fmaf(y[e], y[e], ss);
       }
     }
   }
-  if (p.norm2_out) {
+  if (TAIL && p.norm2_out) {
     ss = wave_sum(ss);
     if (lane == 0) s_ssq[wave] = ss;
     __syncthreads();
@@ -120,11 +122,11 @@ __device__ __forceinline__ void small_finish_row(const ReduceArgs& p, int row, f
 }
 
 // As a launch: a workgroup per batch row.
-template <class DT>
+template <class DT, bool TAIL>
 __global__ __launch_bounds__(kSmallThreads) void small_tail_kernel(ReduceArgs p) {
   __shared__ float4 s_part[kSmallThreads];
   __shared__ float s_ssq[kSmallWaves];
-  small_finish_row<DT>(p, blockIdx.x, s_part, s_ssq);
+  small_finish_row<DT, TAIL>(p, blockIdx.x, s_part, s_ssq);
 }
 
 // Two neighbouring partial sums.  THROUGH: another workgroup of the same launch reads them, so they are written to the level that all XCDs share.
@@ -137,7 +139,7 @@ __device__ __forceinline__ void small_store2(float* to, float a, float b) {
 
 // The end of a call of one row in one launch, for all threads of the workgroup.  Nobody waits: a workgroup whose sums have been acknowledged counts
 // itself, and the one that finds itself the last adds up everything.  The counter is zero again before the launch ends.
-template <class DT>
+template <class DT, bool TAIL>
 __device__ __forceinline__ void small_arrive(const SmallArgs& a) {
   __shared__ float4 s_part[kSmallThreads];
   __shared__ float s_ssq[kSmallWaves];
@@ -151,7 +153,7 @@ __device__ __forceinline__ void small_arrive(const SmallArgs& a) {
   __syncthreads();
   if (!s_last) return;
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-  small_finish_row<DT>(a.fin, 0, s_part, s_ssq);
+  small_finish_row<DT, TAIL>(a.fin, 0, s_part, s_ssq);
 }
 
 // The sum of lo over this lane and the one W lanes away in the lower of the two, of hi in the upper.
@@ -165,7 +167,8 @@ __device__ __forceinline__ float small_fold(float lo, float hi) {
 // NCH: 64-lane chunks of a row; a wave takes one neuron.
 // Down: a wave owns 1/16 of the columns, CL lanes of one vector each; its 64 / CL lane groups take the neurons in turn and meet in
 // registers, so nothing but z goes through LDS.  (The sums of all lane groups by __shfl_xor, 32 to 64 of them, cost 0.9 us a batch row.)
-template <class DT, int B, int NCH, bool ONE>
+// TAIL: the layer tail, which brings a norm and a residual.
+template <class DT, int B, int NCH, bool ONE, bool TAIL>
 __global__ __launch_bounds__(kSmallThreads) void small_rows_kernel(SmallArgs a) {
   typedef typename DT::st st;
   constexpr int VEC = DT::VEC, CL = NCH == 1 ? 4 : NCH == 2 ? 8 : 16, GR = kWave / CL, DL = kSmallRows / GR;
@@ -182,7 +185,8 @@ __global__ __launch_bounds__(kSmallThreads) void small_rows_kernel(SmallArgs a) 
   const int xb = wave / NCH, xi = tid - xb * NCH * kWave;  // this thread's vector of x
   const bool x_in = xb < B && xb < p.nb && xi < p.row_vecs;
   u32x4 xv = p.x[x_in ? (size_t)xb * p.row_vecs + xi : 0];
-  const u32x4 nw = (p.norm_w ? p.norm_w : p.x)[x_in ? xi : 0];
+  u32x4 nw = zero4();
+  if (TAIL) nw = p.norm_w[x_in ? xi : 0];
   __builtin_amdgcn_sched_barrier(0);
   u32x4 wg[NCH], wu[NCH], wd[DL];
   const size_t own = (size_t)(row0 + min(wave, n - 1)) * p.row_vecs;
@@ -196,7 +200,7 @@ __global__ __launch_bounds__(kSmallThreads) void small_rows_kernel(SmallArgs a) 
   __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
   for (int e = 0; e < 4; e++) xv[e] = x_in ? xv[e] : 0u;
-  if (p.norm_w) {  // NCH waves hold a row
+  if (TAIL) {  // NCH waves hold a row
     __shared__ float s_sq[B * NCH];
     const float sq = wave_sum(vec_sumsq<DT>(xv, 0.f));
     if (lane == 0 && xb < B) s_sq[wave] = sq;
@@ -277,7 +281,7 @@ __global__ __launch_bounds__(kSmallThreads) void small_rows_kernel(SmallArgs a) 
       else *o = s[0];
     }
   }
-  if constexpr (ONE) small_arrive<DT>(a);
+  if constexpr (ONE) small_arrive<DT, TAIL>(a);
 }
 
 // ---- batches on the matrix cores ----------------------------------------------------------------------------------------------

@@ -1,0 +1,63 @@
+"""What the compiler gave the kernels, from the metadata of the built library: registers and scratch.  Needs no GPU."""
+import re
+import struct
+
+import msgpack
+import pytest
+
+from cats_amd.build import KERNEL_LIB
+
+
+def _code_objects(blob):
+    """The gfx950 code objects of the offload bundles in a shared library."""
+    magic, at = b"__CLANG_OFFLOAD_BUNDLE__", 0
+    while (at := blob.find(magic, at)) >= 0:
+        count = struct.unpack_from("<Q", blob, at + 24)[0]
+        o = at + 32
+        for _ in range(count):
+            off, size, n = struct.unpack_from("<QQQ", blob, o)
+            if b"gfx950" in blob[o + 24:o + 24 + n]:
+                yield blob[at + off:at + off + size]
+            o += 24 + n
+        at += 24
+
+
+def _kernels(elf):
+    """amdhsa.kernels of the metadata note (type 32) of a code object."""
+    shoff, = struct.unpack_from("<Q", elf, 0x28)
+    shentsize, shnum = struct.unpack_from("<HH", elf, 0x3A)
+    for i in range(shnum):
+        _, kind, _, _, off, size = struct.unpack_from("<IIQQQQ", elf, shoff + i * shentsize)
+        end = off + size
+        while kind == 7 and off < end:  # SHT_NOTE
+            namesz, descsz, ntype = struct.unpack_from("<III", elf, off)
+            desc = off + 12 + (namesz + 3) // 4 * 4
+            if ntype == 32:
+                yield from msgpack.unpackb(elf[desc:desc + descsz])["amdhsa.kernels"]
+            off = desc + (descsz + 3) // 4 * 4
+
+
+@pytest.fixture(scope="module")
+def kernels():
+    if not KERNEL_LIB.exists():
+        import __graft_entry__
+
+        __graft_entry__.build()
+    found = {k[".name"]: k for elf in _code_objects(KERNEL_LIB.read_bytes()) for k in _kernels(elf)}
+    assert len(found) > 100
+    return found
+
+
+def _pairs(kernels, pattern):
+    """Kernels whose last template argument, a flag, is the only difference: (without, with)."""
+    pairs = [(k, kernels[name.replace(m[0], m[1] + "Lb1EE")]) for name, k in kernels.items() if (m := re.search("(" + pattern + ")Lb0EE", name))]
+    assert pairs
+    return pairs
+
+
+def test_small_layers_hold_no_registers_for_a_tail(kernels):
+    """A plain call of one row has no norm, residual or next norm to hold: fewer registers than a tail's."""
+    for plain, tail in _pairs(kernels, r"small_rows_kernelINS_\w+?ELi1ELi\dELb\dE"):
+        assert plain[".vgpr_count"] < tail[".vgpr_count"], plain[".name"]
+    for plain, tail in _pairs(kernels, r"small_tail_kernelINS_\w+?E"):
+        assert plain[".vgpr_count"] < tail[".vgpr_count"], plain[".name"]
