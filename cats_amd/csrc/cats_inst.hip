@@ -36,12 +36,13 @@ template <class DT>
 struct MmaLaunch {
   static constexpr bool kHasUp = sizeof(typename DT::st) == 2;  // the up pass alone takes 16-bit types
   typedef void (*Kernel)(RowsArgs);
-  enum Which { kGateOnly, kGateAndUp, kUpOnly };
+  enum Which { kGateOnly, kGateAndUp, kNormGateAndUp, kUpOnly };
   template <int STEPS, int CH, int NG>
   static Kernel kernel(Which w) {
     if constexpr (kHasUp)
       if (w == kUpOnly) return rows_mma_up_kernel<DT, STEPS, CH, NG>;
-    return w == kGateAndUp ? rows_mma_kernel<DT, STEPS, CH, true, NG> : rows_mma_kernel<DT, STEPS, CH, false, NG>;
+    if (w == kGateOnly) return rows_mma_kernel<DT, STEPS, CH, false, NG, false>;
+    return w == kNormGateAndUp ? rows_mma_kernel<DT, STEPS, CH, true, NG, CH == 2> : rows_mma_kernel<DT, STEPS, CH, true, NG, false>;
   }
   // One instance per number of steps, so that no load or MFMA sits behind a branch on the row length.
   template <int NG>
@@ -94,12 +95,13 @@ struct MmaLaunch {
     const int ntiles = (a.N + kMmaTileRows - 1) / kMmaTileRows;
     return ntiles < cus ? ntiles : cus;
   }
+  static Which gate_kernel(const RowsArgs& a, bool up) { return !up ? kGateOnly : a.norm_w ? kNormGateAndUp : kGateAndUp; }
   static hipError_t run(const RowsArgs& a, bool up, hipStream_t stream) {
-    return launch(up ? kGateAndUp : kGateOnly, a, 1, rows_mma_lds_bytes(a), stream);
+    return launch(gate_kernel(a, up), a, 1, rows_mma_lds_bytes(a), stream);
   }
   // gate + up (a.w2 set) or the gate pass alone for 9..16 batch rows in one pass over the weights
   static hipError_t run16(const RowsArgs& a, hipStream_t stream) {
-    return launch(a.w2 ? kGateAndUp : kGateOnly, a, 2, rows_mma_lds_bytes(a, 2), stream);
+    return launch(gate_kernel(a, a.w2 != nullptr), a, 2, rows_mma_lds_bytes(a, 2), stream);
   }
   // the up pass alone, gate activations given (kUp)
   static int up_rows_pad(const RowsArgs& a) {

@@ -304,8 +304,11 @@ struct MmaX {
       for (int w = 0; w < kMmaWaves; w++) ss += s_sq[(gb * kMmaWaves + w) * 8 + (lane & 7)];
       const float scale = rsqrtf(ss / (float)p.K + p.norm_eps);
 #pragma unroll
-      for (int k = 0; k < NV; k++)
+      for (int k = 0; k < NV; k++) {
+        // two register sets of bf16: else all of x is taken apart into floats at once, into twice its registers, and spilled
+        if constexpr (NV > 9) asm volatile("" : "+v"(v[gb][k]));
         if (in(p, gb, front * kWave + tid + k * kMmaThreads)) v[gb][k] = vec_norm_apply<DT>(v[gb][k], scale, nw[k]);
+      }
     }
   }
 };
@@ -319,11 +322,17 @@ struct MmaX {
 // staged: read from LDS for every tile they cost a CU 1 KiB (2 KiB at 9..16 rows) of LDS traffic a KiB of weights, 6 us of a 43 us
 // kernel at sixteen rows, part of it in front of the next loads (4096 / 14336 bf16 16 rows: kernel 43.7 / 41.7 us, call 70.6 / 70.0;
 // 3080 / 8191 3 rows 33.25 / 33.0; 4 and 8 rows of 4096 as before).
-template <class DT, int STEPS, int CH, bool UP, int NG = 1>
+// x may be given before its RMS norm (p.norm_w, UP only).  With two register sets that is an instance of its own, NORM: all of x and the
+// norm's weights beside the first set are up to 80 registers more, and whole calls without a norm held them, or spilled: 8160 / 12288 bf16
+// 4 rows 105.4 us, now 101.3, 8 rows 112.8, 109.0; 8192 / 12288 fp16 4 rows 95.6, 94.8; fp32 4512 / 11008 8 rows 123.5, 122.1.  One
+// set takes as many with and without.
+template <class DT, int STEPS, int CH, bool UP, int NG, bool NORM>
 __global__ __launch_bounds__(kMmaThreads) void rows_mma_kernel(RowsArgs p) {
   typedef typename DT::st st;
   typedef MmaRows<DT, STEPS, CH, NG> Rows;
+  static_assert(!NORM || (UP && CH == 2), "an instance of its own where there are two register sets");
   constexpr bool kHeld = CH == 1 && NG * STEPS <= (sizeof(st) == 2 ? 16 : 9);  // more would not fit beside four sets of weights
+  const bool norm = CH == 2 ? NORM : UP && p.norm_w != nullptr;
   extern __shared__ u32x4 xs[];  // [NG][mma_slots][64] x operands, then the partial buffers
   __shared__ uint32_t s_any;
 
@@ -462,13 +471,13 @@ __global__ __launch_bounds__(kMmaThreads) void rows_mma_kernel(RowsArgs p) {
     x.front = p.mma_front;
     x.fetch(p);
     u32x4 nw[STEPS * CH];
-    if (UP && p.norm_w) x.fetch_norm(p, nw);
+    if (norm) x.fetch_norm(p, nw);
     // the first gate set goes out behind x, before x is waited for: it is a memory round trip ahead when the staging is done
     __builtin_amdgcn_sched_barrier(0);
     issue_gate(0, 0, g0);
     __builtin_amdgcn_sched_barrier(0);
     x.mask(p);
-    if (UP && p.norm_w) x.template norm<DT>(p, nw, part_g);
+    if (norm) x.template norm<DT>(p, nw, part_g);
     x.store(xs, xgroup);
 #pragma unroll
     for (int c = 0; c < STEPS; c++) u1[c] = zero4();  // defined before the first (unused) up product
@@ -484,6 +493,7 @@ __global__ __launch_bounds__(kMmaThreads) void rows_mma_kernel(RowsArgs p) {
   // The second gate set goes out after the barrier: a wave blocks at issue once the CU's miss queue is full, so
   // everything issued before the barrier delays the moment the staged x becomes usable.
   issue_gate(CH == 2 ? 0 : 1, CH == 2 ? 1 : 0, g1);
+  if constexpr (CH == 2) __builtin_amdgcn_sched_barrier(0);  // all of it: else its last loads wait behind the first products
   CATS_RSTAMP(1);
   if constexpr (kHeld) gate.hold(held);
 

@@ -61,3 +61,17 @@ def test_small_layers_hold_no_registers_for_a_tail(kernels):
         assert plain[".vgpr_count"] < tail[".vgpr_count"], plain[".name"]
     for plain, tail in _pairs(kernels, r"small_tail_kernelINS_\w+?E"):
         assert plain[".vgpr_count"] < tail[".vgpr_count"], plain[".name"]
+
+
+def test_nothing_spills(kernels):
+    """No kernel has scratch, but for the fp32 wave-per-row passes over rows of x that no workgroup holds in LDS, at eight batch rows."""
+    spilled = {n for n, k in kernels.items() if k[".private_segment_fixed_size"] or k[".vgpr_spill_count"]}
+    assert {n for n in spilled if not re.search(r"rows_kernelINS_3F32ELi8ELi2ELi8ELb0ELi\dELb0E", n)} == set()
+
+
+def test_two_register_sets_hold_no_registers_for_a_norm(kernels):
+    """The matrix-core gate + up pass over long rows: at least as many registers with a norm as without, in each type."""
+    pairs = _pairs(kernels, r"rows_mma_kernelINS_\w+?ELi\dELi2ELb1ELi1E")
+    assert len(pairs) == 15
+    for plain, norm in pairs:
+        assert plain[".vgpr_count"] <= norm[".vgpr_count"], plain[".name"]
