@@ -75,6 +75,7 @@ struct MmaLaunch {
   static bool supported(const RowsArgs& a, int ng = 1) {
     const MmaSplit sp = rows_mma_split(a);
     if (a.mask_out && !a.ubytes_out) return false;  // this kernel writes the union of the flags as bytes only
+    if (a.norm_w && !a.w2) return false;            // ... and has no norm in the gate pass alone
     return sp.steps > 0 && (ng == 1 || sp.chunks == 1) && rows_mma_lds_bytes(a, ng) <= kMmaMaxLds;
   }
   static constexpr size_t kMmaMaxLds = 160 * 1024 - 256;  // the kernels' static LDS takes the rest
