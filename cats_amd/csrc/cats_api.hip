@@ -637,7 +637,7 @@ bool fused_eligible(int B, int H, int I, int dtype, FusedArgs& f, int& grid, boo
   f.rpw = rpw;
   f.spw = rpw;
   f.cap = rpw;
-  return fused_lds_bytes(bt, f.nch, f.cap, vec, dw) <= 128 * 1024;
+  return fused_lds_bytes(bt, f.nch, f.cap, vec, dw) <= kStagedMaxBytes;
 }
 
 // Give the call a neuron pool if its shape allows: a fixed fraction of every workgroup's neurons goes to the pool of
@@ -650,7 +650,7 @@ void fused_enable_pool(FusedArgs& f, int grid, int dtype, int32_t* counters, siz
   const int groups = (grid + kFusedGroup - 1) / kFusedGroup;
   if (spw == f.rpw || spw < 2 * rw || (size_t)groups * kPoolStride * 4 > counter_bytes) return;
   const int cap = fused_slot_cap(spw, f.rpw, rw, true);
-  if (fused_lds_bytes(bt, f.nch, cap, vec_elems(dtype), dw) > 128 * 1024) return;
+  if (fused_lds_bytes(bt, f.nch, cap, vec_elems(dtype), dw) > kStagedMaxBytes) return;
   f.spw = spw;
   f.cap = cap;
   f.pool = counters;
@@ -1072,7 +1072,7 @@ static int mlp_norm_residual_pass(const void* h, const void* norm_weight, float 
   if (!h || !norm_weight || !wgate || !wup || !wdown_t || !out) return CATS_ERR_NULL;
   if (!aligned16(h) || !aligned16(norm_weight) || !aligned16(wgate) || !aligned16(wup) || !aligned16(wdown_t)) return CATS_ERR_ALIGN;
   // the norm works on the LDS copy of h: same bound as the kernels' own x staging
-  if ((size_t)batch_template(B) * (((size_t)H * elem_size(dtype) + 8191) / 8192 * 8192) > 128 * 1024) return CATS_ERR_SHAPE;
+  if ((size_t)batch_template(B) * (((size_t)H * elem_size(dtype) + 8191) / 8192 * 8192) > kStagedMaxBytes) return CATS_ERR_SHAPE;
   WsLayout l;
   st = check_ws(ws, ws_bytes, H, I, l);
   if (st) return st;
@@ -1551,7 +1551,7 @@ static int do_proj(int mode, int dtype, const ProjArgs& a, hipStream_t s) {
 static int check_proj(int B, int K, int N, int dtype) {
   if (int st = check_common(B, K, N, dtype)) return st;
   const int vecs = K / vec_elems(dtype);
-  return proj_lds_bytes(batch_template(B), (vecs + kWave - 1) / kWave) <= kProjMaxLds ? CATS_OK : CATS_ERR_SHAPE;
+  return proj_lds_bytes(batch_template(B), (vecs + kWave - 1) / kWave) <= kStagedMaxBytes ? CATS_OK : CATS_ERR_SHAPE;
 }
 
 int cats_linear(const void* x, const void* norm_weight, float eps, const void* w, const void* residual, void* out, int B, int K, int N,

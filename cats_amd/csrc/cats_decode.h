@@ -88,7 +88,7 @@ void proj_kernel(ProjArgs a) {
   constexpr int kXPreAll = (B * CB + WAVES - 1) / WAVES, kXPre = kXPreAll < 4 ? kXPreAll : 4;  // rows of CB chunks
   constexpr int kFirst = B <= 2 ? R * CB / 2 : R * CB;
   u32x4 wv[R][CB];
-  __shared__ float s_sq[kRowsMaxChunks + B];
+  __shared__ float s_sq[kStagedMaxChunks + B];
   RowsX<DT, B, WAVES, kXPre, MODE != kProjAdd> x;
   x.lane = lane;
   x.wave = wave;

@@ -13,6 +13,10 @@ typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 typedef float f32x2v __attribute__((ext_vector_type(2)));
 
 constexpr int kWave = 64;
+// Of x that a workgroup of the wave-per-row and single-pass kernels holds in LDS, in whole chunks of a wave's 64 vectors; launchers and kernels
+// size by these two.
+constexpr size_t kStagedMaxBytes = 128 * 1024;
+constexpr int kStagedMaxChunks = kStagedMaxBytes / (kWave * sizeof(u32x4));
 
 // Streaming (non-temporal) 128-bit load: weight rows are touched once per call, so they should not
 // displace x, the mask words or the partial sums from L2.

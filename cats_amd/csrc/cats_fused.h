@@ -41,7 +41,6 @@ static_assert(kFusedWaves == 16 || kFusedWaves == 8, "sixteen waves, or eight fo
 constexpr int fused_down_waves(int batch_template) { return (batch_template == 1 ? 4 : 8) * kFusedWaves / 16; }
 constexpr int kFusedThreads = kFusedWaves * kWave;
 constexpr int kFusedCB = 8;             // 64-lane chunks (of 16 bytes per lane) per block of row loads
-constexpr int kFusedMaxChunks = 128;    // of all staged rows: 128 KiB of x
 constexpr int kFusedMaxKV = 4;          // a down wave covers KV * 64 vectors of a row: rows of up to 4 * DW * 64 vectors
 // Experiment switch, off in the product build: -DCATS_FUSED_POOL=1 compiles the neuron pool described at the kernel
 // (dynamic balancing between the workgroups of a group).  Measured slower than fixed shares on the MI355X, kept so the
@@ -313,7 +312,7 @@ __global__ __launch_bounds__(kFusedThreads) void mlp_fused_kernel(FusedArgs p) {
   __shared__ int s_nfinal;     // slots in use; an upper bound while row waves are still taking tickets
   __shared__ int s_exited;     // row waves that have left
   __shared__ int s_exhausted;  // some row wave has found the group's pool empty
-  __shared__ __attribute__((aligned(16))) float s_sq[kFusedMaxChunks];  // squares of the staged rows, by chunk
+  __shared__ __attribute__((aligned(16))) float s_sq[kStagedMaxChunks];  // squares of the staged rows, by chunk
 
   const int tid = threadIdx.x;
   const int lane = tid & (kWave - 1);

@@ -149,7 +149,7 @@ bool takes_mma(int mode, int bt, const RowsArgs& a) {
   // fp32 up to four rows: the wave-per-row kernel keeps up with the weights (gate + up of 4096 / 11008 at 4 rows: 17 us less), as long
   // as it finds x in LDS (dense down, K = 12936: 11 us more).  At eight rows it spends 256 fused multiply-adds a lane on 32 vectors
   // and the matrix cores win (5632 rows of 2048: 54 against 42 us a call, 11008 of 4096: 128 against 115, with a dense down 258 against 120).
-  if (std::is_same<DT, F32>::value && bt == 4 && (mode != kGemv || (size_t)bt * a.K * 4 <= 128 * 1024)) return false;
+  if (std::is_same<DT, F32>::value && bt == 4 && (mode != kGemv || (size_t)bt * a.K * 4 <= kStagedMaxBytes)) return false;
   if (mode == kUp) return MmaLaunch<DT>::supported_up(a);
   if (mode == kGemv) return MmaLaunch<DT>::supported_gemv(a);
   return (mode == kGateUp || mode == kGate) && MmaLaunch<DT>::supported(a);
@@ -160,7 +160,7 @@ hipError_t launch_rows_b(int mode, const RowsArgs& a, hipStream_t stream) {
   if (takes_mma<DT>(mode, B, a))
     return mode == kUp ? MmaLaunch<DT>::run_up(a, stream) : mode == kGemv ? MmaLaunch<DT>::run_gemv(a, stream) : MmaLaunch<DT>::run(a, mode == kGateUp, stream);
   const size_t lds = (size_t)B * ((a.nch + kCB - 1) / kCB * kCB) * kWave * sizeof(u32x4);
-  const bool xlds = lds <= 128 * 1024;
+  const bool xlds = lds <= kStagedMaxBytes;
   const bool full = xlds && (a.K % (kWave * DT::VEC * kCB) == 0);
   switch (mode) {
     case kGate:

@@ -77,8 +77,7 @@ hipError_t launch_small_tail(int rows, const ReduceArgs& r, hipStream_t stream);
 template <class DT>
 hipError_t launch_reduce(const ReduceArgs& r, hipStream_t stream);
 
-// Projections and attention of one decode step (cats_decode.h).  mode is a ProjMode; lds_bytes of x have to fit (proj_lds_bytes).
-constexpr size_t kProjMaxLds = 128 * 1024;
+// Projections and attention of one decode step (cats_decode.h).  mode is a ProjMode; proj_lds_bytes has to be within kStagedMaxBytes.
 constexpr int kProjCB = 8;
 inline size_t proj_lds_bytes(int bt, int nch, int cb = kProjCB) { return (size_t)bt * ((nch + cb - 1) / cb * cb) * kWave * sizeof(u32x4); }
 template <class DT>

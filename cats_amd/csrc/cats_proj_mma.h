@@ -14,7 +14,7 @@
 namespace cats {
 
 constexpr int proj_mma_tiles(int steps, int ch) { return ch == 2 || steps > 4 ? 1 : steps > 2 ? 2 : steps == 2 ? 4 : 8; }
-constexpr int kProjMaxHeadDim = 512;
+constexpr int kProjMaxHeadDim = 256;  // 32 lanes of 8 elements a cache slot, the most that attention takes
 
 // The three matrices as one list of rows, in tiles of eight; a.r as rows_mma_split takes it.
 inline int proj_mma_ntiles(const ProjArgs& a, int mode) { return mode == kProjQkv ? 3 * (a.r.N / 8) : (a.r.N + 7) / 8; }

@@ -148,7 +148,6 @@ __device__ __forceinline__ void rows_dot(const u32x4* __restrict__ w, const int 
 // Whole calls, before / now in us: HF layout 4096 / 11008 fp32 1 row 79.8 / 72.6, 2 rows 92.8 / 85.4, fp16 1 row 40.3 / 38.2, bf16 2 rows 48.5 / 42.5,
 // 2000 / 5000 fp16 2 rows 18.0 / 14.6; steps of four layers 4096 / 11008 319 / 306, 2304 / 7097 168.7 / 158.3.  The chunk's row is found by
 // comparisons: divisions took 1 to 3 us of these at two rows, and more than the staging gave at four.
-constexpr int kRowsMaxChunks = 160;  // of 1 KiB: more is not staged
 template <class DT, int B, int WAVES, int NX, bool NORM_AHEAD>
 struct RowsX {
   static constexpr int U = 2;
@@ -190,7 +189,7 @@ struct RowsX {
       for (int k = 0; k < NX; k++) nw[k] = load_norm(p, wave + k * WAVES);
     }
   }
-  // Ends with a barrier.  s_sq: kRowsMaxChunks + B floats.
+  // Ends with a barrier.  s_sq: kStagedMaxChunks + B floats.
   __device__ __forceinline__ void store(const RowsArgs& p, u32x4* xs, float* s_sq) {
     const int chunks = B * nchp;
     const bool norm = p.norm_w != nullptr;
@@ -235,11 +234,11 @@ struct RowsX {
     } else {
       for (int b = wave; b < B; b += WAVES) {
         const float r = scale_of(b);
-        if (lane == 0) s_sq[kRowsMaxChunks + b] = r;
+        if (lane == 0) s_sq[kStagedMaxChunks + b] = r;
       }
       lds_barrier();
     }
-    auto scale = [&](int c) { return B == 1 ? sc : s_sq[kRowsMaxChunks + row_of(c)]; };
+    auto scale = [&](int c) { return B == 1 ? sc : s_sq[kStagedMaxChunks + row_of(c)]; };
 #pragma unroll
     for (int k = 0; k < NX; k++) {
       const int c = wave + k * WAVES;
@@ -304,7 +303,7 @@ void rows_kernel(RowsArgs p) {
   u32x4 wv[R][CB];
   if (threadIdx.x == 0) s_maskbits = 0u;
   if (XLDS) {
-    __shared__ float s_sq[kRowsMaxChunks + B];
+    __shared__ float s_sq[kStagedMaxChunks + B];
     const int nchp = (p.nch + CB - 1) / CB * CB;
     auto stage = [&](auto x) {
       x.lane = lane;
