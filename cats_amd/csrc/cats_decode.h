@@ -89,7 +89,7 @@ void proj_kernel(ProjArgs a) {
   constexpr int kFirst = B <= 2 ? R * CB / 2 : R * CB;
   u32x4 wv[R][CB];
   __shared__ float s_sq[kStagedMaxChunks + B];
-  RowsX<DT, B, WAVES, kXPre, MODE != kProjAdd> x;
+  RowsX<DT, B, WAVES, kXPre, MODE != kProjAdd ? kNormAhead : kNormLater> x;
   x.lane = lane;
   x.wave = wave;
   x.nchp = (p.nch + CB - 1) / CB * CB;

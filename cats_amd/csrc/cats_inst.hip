@@ -22,7 +22,9 @@ template <int B> struct WavesFor { static constexpr int value = B <= 2 ? 4 : 8; 
 template <class DT, int B, bool FULL, int MODE, bool XLDS>
 hipError_t launch_rows_one(const RowsArgs& a, hipStream_t stream) {
   constexpr int WAVES = WavesFor<B>::value;
-  auto kern = rows_kernel<DT, B, kR, kCB, FULL, MODE, XLDS, WAVES>;
+  auto kern = rows_kernel<DT, B, kR, kCB, FULL, MODE, XLDS, WAVES, true>;
+  if constexpr (rows_norm_apart(MODE, B, XLDS))
+    if (!a.norm_w && (sizeof(typename DT::st) == 4 || a.K <= 4096)) kern = rows_kernel<DT, B, kR, kCB, FULL, MODE, XLDS, WAVES, false>;
   const int rows_per_block = WAVES * kR;
   const int grid = (a.N + rows_per_block - 1) / rows_per_block;
   size_t lds = XLDS ? (size_t)B * ((a.nch + kCB - 1) / kCB * kCB) * kWave * sizeof(u32x4) : 0;

@@ -144,13 +144,19 @@ __device__ __forceinline__ void rows_dot(const u32x4* __restrict__ w, const int 
 // x of all batch rows on its way into LDS, through the RMS norm if there is one.  Memory returns are counted in issue order: fetch()
 // goes out in front of the first weights, and store() waits for x alone while these stay in flight.  (As loads behind conditions, x
 // was waited for together with all of the weights, and the norm's weights were asked for after that.)  NX vectors a thread are fetched ahead, the rest
-// of longer rows in batches; NORM_AHEAD: so are their norm weights.  All of a wave's 64 vectors are of one chunk of one row.
+// of longer rows in batches; RowsNorm says what of the norm's weights.  All of a wave's 64 vectors are of one chunk of one row.
 // Whole calls, before / now in us: HF layout 4096 / 11008 fp32 1 row 79.8 / 72.6, 2 rows 92.8 / 85.4, fp16 1 row 40.3 / 38.2, bf16 2 rows 48.5 / 42.5,
 // 2000 / 5000 fp16 2 rows 18.0 / 14.6; steps of four layers 4096 / 11008 319 / 306, 2304 / 7097 168.7 / 158.3.  The chunk's row is found by
 // comparisons: divisions took 1 to 3 us of these at two rows, and more than the staging gave at four.
-template <class DT, int B, int WAVES, int NX, bool NORM_AHEAD>
+enum RowsNorm {
+  kNoNorm,     // norm_w is not looked at
+  kNormLater,  // norm_w, where given, is asked for when the squares are added
+  kNormAhead   // with x, from x itself where it is not given: a load behind a condition could not be counted
+};
+template <class DT, int B, int WAVES, int NX, RowsNorm NORM>
 struct RowsX {
   static constexpr int U = 2;
+  static constexpr bool NORM_AHEAD = NORM == kNormAhead;
   u32x4 v[NX], nw[NORM_AHEAD ? NX : 1];
   int lane, wave, nchp;  // nchp: chunks of a row with its padding
 
@@ -192,7 +198,7 @@ struct RowsX {
   // Ends with a barrier.  s_sq: kStagedMaxChunks + B floats.
   __device__ __forceinline__ void store(const RowsArgs& p, u32x4* xs, float* s_sq) {
     const int chunks = B * nchp;
-    const bool norm = p.norm_w != nullptr;
+    const bool norm = NORM != kNoNorm && p.norm_w != nullptr;
     auto square = [&](int c, u32x4 val) {
       const float sq = wave_sum(vec_sumsq<DT>(val, 0.f));
       if (lane == 0) s_sq[c] = sq;
@@ -265,7 +271,12 @@ struct RowsX {
 // B == 1 asks for 6 waves per SIMD (80 VGPRs): 6 workgroups of 4 waves per CU hold all 1376 workgroups of an
 // 11008-row matrix at once, so no workgroup starts late and runs its two dependent passes on a draining machine.
 constexpr int rows_waves_per_simd(int B, bool full) { return B == 1 ? (full ? 6 : 5) : B <= 4 ? 4 : 1; }
-template <class DT, int B, int R, int CB, bool FULL, int MODE, bool XLDS, int WAVES>
+// Gate + up at two to four rows has its norm in an instance of its own (NORM).  Asked for ahead, the norm's weights are worth their registers: tails in
+// fp32 with them / later 2048 / 5504 3 rows 33.8 / 34.5 us, 4096 / 11008 4 rows 95.5 / 96.7.  Without a norm they were loads of x that nobody
+// used: fp32 2048 / 5504 4 rows 32.5, now 31.8, HF layout 34.3, 33.8, 1024 / 3072 2 rows 13.0, 12.5; fp16 2048 / 6144 2 rows 17.7, 17.3, 4096 / 11008
+// 44.6, 44.3.  Longer rows of 16-bit types stay with the one instance: 8192 / 12288 bf16 2 rows 87.8 / 88.7 us, 5120 / 13824 70.8 in both.
+constexpr bool rows_norm_apart(int mode, int B, bool xlds) { return mode == kGateUp && xlds && (B == 2 || B == 4); }
+template <class DT, int B, int R, int CB, bool FULL, int MODE, bool XLDS, int WAVES, bool NORM>
 __global__ __launch_bounds__(WAVES* kWave) __attribute__((amdgpu_waves_per_eu(XLDS && MODE != kGemv ? rows_waves_per_simd(B, FULL) : 1, 8)))
 void rows_kernel(RowsArgs p) {
   typedef typename DT::st st;
@@ -317,8 +328,8 @@ void rows_kernel(RowsArgs p) {
       if (kPre) rows_issue_all<kFirst, R * CB, R, CB, FULL>(p.w, row, 0, p, lane, wv);
     };
     // the intermediate rows that kGemv takes: up to 11008 fp32 elements, or two rows of 16-bit ones
-    if (MODE == kGemv && B <= 2 && B * nchp > kXPre * WAVES) stage(RowsX<DT, B, WAVES, 12, false>());
-    else stage(RowsX<DT, B, WAVES, kXPre, (MODE == kGateUp && (B == 2 || B == 4))>());
+    if (MODE == kGemv && B <= 2 && B * nchp > kXPre * WAVES) stage(RowsX<DT, B, WAVES, 12, kNormLater>());
+    else stage(RowsX<DT, B, WAVES, kXPre, !NORM ? kNoNorm : rows_norm_apart(MODE, B, XLDS) ? kNormAhead : kNormLater>());
   } else {
     __syncthreads();
   }

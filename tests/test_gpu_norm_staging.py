@@ -14,6 +14,7 @@ pytestmark = pytest.mark.gpu
     (1288, 5000, 3, torch.bfloat16), (4096, 3000, 8, torch.float16), (6152, 2100, 5, torch.bfloat16),           # matrix-core pass, with and without phases, two register sets
     (8160, 2100, 4, torch.bfloat16), (8192, 2100, 8, torch.float16), (9208, 900, 3, torch.bfloat16), (4096, 1500, 6, torch.float32),             # the longest of these
     (2568, 3500, 9, torch.float16), (4096, 3000, 16, torch.bfloat16), (2056, 2500, 7, torch.float32),
+    (2056, 3000, 2, torch.float32), (4100, 1500, 3, torch.float32), (8192, 601, 4, torch.float32), (12288, 300, 2, torch.float32),               # wave per row
     (384, 777, 4, torch.bfloat16), (264, 500, 11, torch.float16), (1288, 300, 2, torch.float16), (520, 300, 4, torch.float32)])  # small layers
 def test_norm_from_registers(oracle, H, I, B, dtype):
     m = make_mlp(H, I, B, dtype, seed=H + 3 * I + B)

@@ -75,3 +75,11 @@ def test_two_register_sets_hold_no_registers_for_a_norm(kernels):
     assert len(pairs) == 15
     for plain, norm in pairs:
         assert plain[".vgpr_count"] <= norm[".vgpr_count"], plain[".name"]
+
+
+def test_wave_per_row_calls_hold_nothing_for_a_norm(kernels):
+    """Gate + up of two to four rows with x in LDS: the plain instance has no room for the rows' squares."""
+    pairs = _pairs(kernels, r"rows_kernelINS_\w+?ELi[24]ELi2ELi8ELb\dELi1ELb1ELi\dE")
+    assert len(pairs) == 12
+    for plain, norm in pairs:
+        assert plain[".group_segment_fixed_size"] + 512 <= norm[".group_segment_fixed_size"], plain[".name"]
