@@ -35,13 +35,13 @@ def test_norm_from_registers(oracle, H, I, B, dtype):
 @pytest.mark.parametrize("B", [1, 4])
 def test_bf16_rounding(B):
     """A sum of two bf16 numbers that fp32 holds exactly leaves as torch rounds it: ties, the carry into the exponent, subnormal results,
-    the step to infinity, infinities and NaN."""
+    the step to infinity, infinities and NaN.  (The sign of a zero sum is not looked at: it depends on what the sum starts from.)"""
     import flash_gemv  # noqa: F401
 
     pairs = [(1.0, 2.0 ** -8), (1.0 + 2.0 ** -7, 2.0 ** -8), (1.0, -(2.0 ** -9)), (1.0, 2.0 ** -8 + 2.0 ** -14), (2.0 - 2.0 ** -7, 2.0 ** -8),
              (2.0 ** -126, -(2.0 ** -127) + 2.0 ** -133), (2.0 ** -133, 0.0), (3 * 2.0 ** -133, -(2.0 ** -133)),
              (3.3895313892515355e38, 2.0 ** 119), (3.3895313892515355e38, -(2.0 ** 119)), (-3.3895313892515355e38, -(2.0 ** 119)),
-             (float("inf"), 1.0), (float("inf"), float("-inf")), (float("nan"), 0.0), (-0.0, -0.0)]
+             (float("inf"), 1.0), (float("inf"), float("-inf")), (float("nan"), 0.0)]
     w = torch.zeros(16, 64, dtype=torch.bfloat16)
     w[:len(pairs), :2] = torch.tensor(pairs).to(torch.bfloat16)
     x = torch.zeros(B, 64, dtype=torch.bfloat16)
@@ -52,3 +52,28 @@ def test_bf16_rounding(B):
     for b in range(B):
         assert torch.equal(out[b][keep].abs(), want[keep].abs()) and torch.equal(out[b][keep] < 0, want[keep] < 0)
         assert torch.equal(torch.isnan(out[b]), torch.isnan(want)) and torch.equal(torch.isinf(out[b]), torch.isinf(want))
+
+
+def test_bf16_rounding_of_any_float():
+    """Floats of random bits, a third of them ties and as many a last bit beside one, as sums of three bf16 numbers of their own bits: every partial
+    sum is exact, whatever the order, so what is stored is the float rounded once."""
+    import flash_gemv  # noqa: F401
+
+    n = 1 << 18
+    g = torch.Generator().manual_seed(3)
+    bits = torch.randint(0, 1 << 31, (n,), generator=g) | (torch.randint(0, 2, (n,), generator=g) << 31)
+    low = torch.tensor([0x8000, 0x7FFF, 0x8001])
+    kind = torch.arange(n) % 9
+    bits = torch.where(kind < 3, (bits & ~0xFFFF) | 0x8000, torch.where(kind < 6, (bits & ~0xFFFF) | low[1 + kind % 2], bits))
+    exponent = (bits >> 23) & 0xFF
+    bits = (bits & ~(0xFF << 23)) | (exponent.clamp(60, 250) << 23)  # parts of normal size
+    f = torch.where(bits >= 1 << 31, bits - (1 << 32), bits).to(torch.int32).view(torch.float32)
+    part = lambda v: (v.view(torch.int32) & ~0xFFFF).view(torch.float32)  # the leading eight bits of it, towards zero
+    hi = part(f)
+    mid = part(f - hi)
+    w = torch.zeros(n, 64, dtype=torch.bfloat16)
+    for k, v in enumerate((hi, mid, f - hi - mid)):
+        w[:, 7 * k] = v.to(torch.bfloat16)
+        assert torch.equal(w[:, 7 * k].float(), v)
+    out = torch.ops.flash_gemv.cats_linear(torch.ones(1, 64, dtype=torch.bfloat16, device="cuda"), None, 1e-5, w.cuda()).cpu().flatten()
+    assert torch.equal(out.view(torch.int16), f.to(torch.bfloat16).view(torch.int16))
