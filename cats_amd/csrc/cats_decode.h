@@ -6,12 +6,12 @@
 //   proj_kernel<kProjPlain>    out = x . W^T                                                         (the output head)
 //
 // x may be given before its RMS norm (norm_w), which is then applied while x is staged.  Everything between the weight
-// matrices stays in fp32 and is rounded once where it is stored.  All of it is bound by the weight stream: one wave owns two
+// matrices stays in fp32 and is rounded once where it is stored.  All of it is bound by the weight stream: one wave owns two to eight
 // rows of a matrix, whose loads are all in flight at once, as in rows_kernel.
-// One step of four layers 4096 / 11008, 32 heads, 32000 words, 256 tokens in the cache, fp16, one row: 306 us, of which the MLP
-// kernels take 150; with torch's operations in place of these kernels (about 25 launches a layer) it was 761.  Kernel trace: q, k, v
-// 17.4 us with the norm (5.8 TB/s), attention 7.7 and the output projection, whose weights it has had fetched, 4.8 (8.1
-// without that), output head 40.6 (6.5 TB/s).  With x staged behind the weights: 18.8, 7.6, 5.2 and 42.7.
+// One step of four layers 4096 / 11008, 32 heads, 32000 words, 256 tokens in the cache, fp16, one row: 309 us, of which the MLP
+// kernels take 148; with torch's operations in place of these kernels (about 25 launches a layer) it was 761.  Kernel trace: q, k, v
+// 17.4 us with the norm (5.8 TB/s), attention 8.1 and the output projection, whose weights it has had fetched, 4.7 (8.1
+// without that), output head 40.7 (6.4 TB/s).  With x staged behind the weights: 18.8, 7.6, 5.2 and 42.7.
 #pragma once
 #include "cats_rows.h"
 
@@ -36,7 +36,7 @@ struct ProjArgs {
   int max_len;
 };
 
-// Two rows per wave.  For kProjQkv they are the two elements of a head that the rotary embedding mixes, d and d + head_dim / 2,
+// R rows per wave.  For kProjQkv they are two, the elements of a head that the rotary embedding mixes, d and d + head_dim / 2,
 // so it is applied to the two sums where they are; the wave's number counts these pairs over the three matrices.
 // Short rows are taken by blocks of CB = 2 or 4 chunks of 64 vectors instead of eight, and where the result is stored as it is (the output head) by
 // 16 / CB rows a wave: as many loads in flight, and x is staged once for as many weight bytes.

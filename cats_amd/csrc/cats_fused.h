@@ -376,7 +376,8 @@ __global__ __launch_bounds__(kFusedThreads) void mlp_fused_kernel(FusedArgs p) {
       }
     }
     issue_first();
-    // The squares of a batch row: by chunk of 64 vectors (a wave's vectors are of one), then over the chunks in their order.
+    // The squares of a batch row: by chunk of 64 vectors (a wave's vectors are of one), then over the chunks in their order.  x is stored as it is, and
+    // where there is a norm again when the squares are known: what came in ahead from registers, the rest of a longer row read back.
     auto put = [&](int i, u32x4 val) {
       xs[i] = val;
       if (p.norm_w) {

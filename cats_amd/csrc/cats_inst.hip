@@ -286,6 +286,12 @@ hipError_t launch_proj_one(const ProjArgs& a, hipStream_t stream) {
 }
 
 // Projections of 3..8 rows on the matrix cores: 16-bit types, rows and matrices on whole cache lines, head halves in fours, x operands in LDS.
+// Products in fp16 with the weights from memory, a wave a row / matrix cores in us:
+//   2 rows   32000 x 512 8.5, 9.5   32000 x 2048 23.3, 24.9   4096 x 4096 7.5, 8.7   3072 x 1024 4.4, 5.3
+//   3 rows   32000 x 512 26.0, 9.5   32000 x 2048 30.5, 25.0   32000 x 4096 42.5, 43.5   4096 x 4096 8.8, 8.8   3072 x 1024 5.9, 5.3   5120 x 5120 17.8, 13.2
+//   4 rows   32000 x 512 26.1, 9.4   32000 x 2048 31.8, 24.9   32000 x 4096 43.6, 43.6   4096 x 4096 9.1, 8.9   8000 x 2048 9.8, 8.6   32000 x 8192 87.2, 83.4
+//   8 rows   32000 x 512 46.0, 9.4   32000 x 2048 50.5, 24.7   32000 x 4096 63.4, 41.9   4096 x 4096 13.1, 9.0   8000 x 8192 40.2, 28.2
+// So they are taken from three rows on.  At three and four rows 8192 x 8192 alone loses, 25.5, 27.8; 1024 x 8192 10.2, 9.4 and 7168 x 7168 20.5, 19.7 do not.
 template <class DT>
 struct ProjMma {
   template <int MODE, int STEPS, int CH>

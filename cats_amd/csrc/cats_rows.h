@@ -144,9 +144,10 @@ __device__ __forceinline__ void rows_dot(const u32x4* __restrict__ w, const int 
 // x of all batch rows on its way into LDS, through the RMS norm if there is one.  Memory returns are counted in issue order: fetch()
 // goes out in front of the first weights, and store() waits for x alone while these stay in flight.  (As loads behind conditions, x
 // was waited for together with all of the weights, and the norm's weights were asked for after that.)  NX vectors a thread are fetched ahead, the rest
-// of longer rows in batches; RowsNorm says what of the norm's weights.  All of a wave's 64 vectors are of one chunk of one row.
+// of longer rows in batches of U; RowsNorm says what of the norm's weights.  Vectors fetched ahead are stored once, normed; the rest of a longer row is stored
+// as it is and normed in place.  All of a wave's 64 vectors are of one chunk of one row.
 // Whole calls, before / now in us: HF layout 4096 / 11008 fp32 1 row 79.8 / 72.6, 2 rows 92.8 / 85.4, fp16 1 row 40.3 / 38.2, bf16 2 rows 48.5 / 42.5,
-// 2000 / 5000 fp16 2 rows 18.0 / 14.6; steps of four layers 4096 / 11008 319 / 306, 2304 / 7097 168.7 / 158.3.  The chunk's row is found by
+// 2000 / 5000 fp16 2 rows 18.0 / 14.6; steps of four layers 4096 / 11008 324 / 309, 2304 / 7097 with 8000 words 168.7 / 158.3.  The chunk's row is found by
 // comparisons: divisions took 1 to 3 us of these at two rows, and more than the staging gave at four.
 enum RowsNorm {
   kNoNorm,     // norm_w is not looked at
@@ -253,13 +254,12 @@ struct RowsX {
         xs[c * kWave + lane] = masked(p, c, vec_norm_apply<DT>(v[k], scale(c), w));
       }
     }
-    constexpr int UN = B >= 4 ? 4 : U;
-    for (int c0 = wave + NX * WAVES; c0 < chunks; c0 += UN * WAVES) {
-      u32x4 w[UN];
+    for (int c0 = wave + NX * WAVES; c0 < chunks; c0 += U * WAVES) {
+      u32x4 w[U];
 #pragma unroll
-      for (int u = 0; u < UN; u++) w[u] = load_norm(p, c0 + u * WAVES);
+      for (int u = 0; u < U; u++) w[u] = load_norm(p, c0 + u * WAVES);
 #pragma unroll
-      for (int u = 0; u < UN; u++) {
+      for (int u = 0; u < U; u++) {
         const int c = c0 + u * WAVES;
         if (c < chunks) xs[c * kWave + lane] = masked(p, c, vec_norm_apply<DT>(xs[c * kWave + lane], scale(c), w[u]));
       }
@@ -269,7 +269,10 @@ struct RowsX {
 };
 
 // B == 1 asks for 6 waves per SIMD (80 VGPRs): 6 workgroups of 4 waves per CU hold all 1376 workgroups of an
-// 11008-row matrix at once, so no workgroup starts late and runs its two dependent passes on a draining machine.
+// 11008-row matrix at once, so no workgroup starts late and runs its two dependent passes on a draining machine.  Rows that are no
+// whole blocks need more registers for their addresses: 5 (with 6: HF layout 2056 / 5504 fp32 28.6 -> 32.1 us, 3080 / 8192 and 2304 / 7096 in 16 bits as they are).
+// Two to four rows: 4, against none asked for 2048 / 6144 bf16 2 rows 17.4, 17.6, 2048 / 5504 fp32 4 rows 31.7, 31.9, 4096 / 11008 96.4, 96.8, 3080 / 8192 fp16
+// 2 rows 27.4, 27.2.  kGemv asks for none: it holds twelve vectors of x (below).
 constexpr int rows_waves_per_simd(int B, bool full) { return B == 1 ? (full ? 6 : 5) : B <= 4 ? 4 : 1; }
 // Gate + up at two to four rows has its norm in an instance of its own (NORM).  Asked for ahead, the norm's weights are worth their registers: tails in
 // fp32 with them / later 2048 / 5504 3 rows 33.8 / 34.5 us, 4096 / 11008 4 rows 95.5 / 96.7.  Without a norm they were loads of x that nobody
@@ -327,7 +330,10 @@ void rows_kernel(RowsArgs p) {
       x.store(p, xs, s_sq);
       if (kPre) rows_issue_all<kFirst, R * CB, R, CB, FULL>(p.w, row, 0, p, lane, wv);
     };
-    // the intermediate rows that kGemv takes: up to 11008 fp32 elements, or two rows of 16-bit ones
+    // kGemv takes intermediate rows, longer than x: beyond what the others fetch ahead twelve vectors a thread, 48 KiB of four waves, are one trip instead of
+    // six.  The kernel then holds 161 registers at one row and 150 at two, three waves a SIMD, for short rows as well.  That cost nothing: HF layout, before the twelve / with
+    // them, fp16 1 row 1024 / 2048 to 8192 / 28672 (8192 / 12288 81.0, 79.0; 2048 / 4096 11.7, 11.2), fp32 512 / 1024 9.56, 9.51, 2048 / 3072 16.3, 14.6,
+    // 8192 / 12288 164.1, 162.9, two rows 1024 / 2048 bf16 12.6, 9.9, 8192 / 12288 94.8, 87.6 (with the rest of what changed in the staging).
     if (MODE == kGemv && B <= 2 && B * nchp > kXPre * WAVES) stage(RowsX<DT, B, WAVES, 12, kNormLater>());
     else stage(RowsX<DT, B, WAVES, kXPre, !NORM ? kNoNorm : rows_norm_apart(MODE, B, XLDS) ? kNormAhead : kNormLater>());
   } else {
