@@ -561,8 +561,8 @@ bool small_takes(RowsArgs& a, int dtype, size_t room, bool& mma, int& grid) {
 // Sums of a batch row that one workgroup adds up sooner than a launch over all CUs and, for the layer tail, the hand-over in front of its norm
 // (tail with the next norm, one row: 512 / 1024, 131 KB, 7.8 us against 10.1; 704 / 1451, 256 KB, 11.1; 1024 / 1965, 504 KB, 13.2 against 11.8).
 constexpr size_t kSmallTailBytes = 300000;
-// One batch row up to here is one launch: the call then takes 8.0 us instead of 8.7 to 9.2 (the host's pace: 2.1 us a launch), though
-// its kernel takes 1 to 2 us more than the two; 512 / 2048, 262 KB: 10.1 against 8.6.  In a captured graph launches are cheap: two there, with the
+// One batch row up to here is one launch: the call then takes 8.0 us, what its kernel takes (8.2 to 8.6 traced; the host needs 6.1 for the same call over
+// 64 / 64, 5.1 for one projection), instead of 8.7 to 9.2, the host's pace with a second launch, though the kernel takes 1 to 2 us more than the two; 512 / 2048, 262 KB: 10.1 against 8.6.  In a captured graph launches are cheap: two there, with the
 // sums in the same order.
 constexpr size_t kSmallOneLaunchBytes = 131072;
 

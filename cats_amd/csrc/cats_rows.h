@@ -274,7 +274,8 @@ struct RowsX {
 // Two to four rows: 4, against none asked for 2048 / 6144 bf16 2 rows 17.4, 17.6, 2048 / 5504 fp32 4 rows 31.7, 31.9, 4096 / 11008 96.4, 96.8, 3080 / 8192 fp16
 // 2 rows 27.4, 27.2.  kGemv asks for none: it holds twelve vectors of x (below).
 constexpr int rows_waves_per_simd(int B, bool full) { return B == 1 ? (full ? 6 : 5) : B <= 4 ? 4 : 1; }
-// Gate + up at two to four rows has its norm in an instance of its own (NORM).  Asked for ahead, the norm's weights are worth their registers: tails in
+// Gate + up at two to four rows has its norm in an instance of its own (NORM; tails of one row are the single-pass kernel's, of five and more the
+// matrix cores').  Asked for ahead, the norm's weights are worth their registers: tails in
 // fp32 with them / later 2048 / 5504 3 rows 33.8 / 34.5 us, 4096 / 11008 4 rows 95.5 / 96.7.  Without a norm they were loads of x that nobody
 // used: fp32 2048 / 5504 4 rows 32.5, now 31.8, HF layout 34.3, 33.8, 1024 / 3072 2 rows 13.0, 12.5; fp16 2048 / 6144 2 rows 17.7, 17.3, 4096 / 11008
 // 44.6, 44.3.  Longer rows of 16-bit types stay with the one instance: 8192 / 12288 bf16 2 rows 87.8 / 88.7 us, 5120 / 13824 70.8 in both.
@@ -331,7 +332,7 @@ void rows_kernel(RowsArgs p) {
       if (kPre) rows_issue_all<kFirst, R * CB, R, CB, FULL>(p.w, row, 0, p, lane, wv);
     };
     // kGemv takes intermediate rows, longer than x: beyond what the others fetch ahead twelve vectors a thread, 48 KiB of four waves, are one trip instead of
-    // six.  The kernel then holds 161 registers at one row and 150 at two, three waves a SIMD, for short rows as well.  That cost nothing: HF layout, before the twelve / with
+    // five.  The kernel then holds 161 registers at one row and 150 at two, three waves a SIMD, for short rows as well.  That cost nothing: HF layout, before the twelve / with
     // them, fp16 1 row 1024 / 2048 to 8192 / 28672 (8192 / 12288 81.0, 79.0; 2048 / 4096 11.7, 11.2), fp32 512 / 1024 9.56, 9.51, 2048 / 3072 16.3, 14.6,
     // 8192 / 12288 164.1, 162.9, two rows 1024 / 2048 bf16 12.6, 9.9, 8192 / 12288 94.8, 87.6 (with the rest of what changed in the staging).
     if (MODE == kGemv && B <= 2 && B * nchp > kXPre * WAVES) stage(RowsX<DT, B, WAVES, 12, kNormLater>());
